@@ -333,6 +333,74 @@ int we_qkv_rope_kv_attn_fwd(const we_qkv_proj* proj, void* q_out,
                             int32_t dilation, int32_t is_frozen, float scale, int32_t n_splits, int32_t q_tile,
                             int32_t dtype, const we_attn_extras* extras, void* stream);
 
+/*
+ * Check of a call's position ids (the eager-mode checks of src/model/attn.py:25-30 and
+ * src/model/kv_cache.py:112-124) on the device, in front of the call's first write and without
+ * another pass over the stream:
+ *   what     WE_CHECK_FRAME: t_pos >= 0 and constant within each batch row.  WE_CHECK_TABLE:
+ *            y_pos < grid_h, x_pos < grid_w, table row inside [0, table_rows).  0 = no check.
+ *   report   host-coherent memory the device can write: receives 2 * ticket when the ids are in
+ *            order and 2 * ticket + 1 when they are refused, as soon as the call's first kernel
+ *            knows (long before its last kernel ends).
+ *   ticket   any value that tells this call's verdict from an earlier one's in the same word.
+ *   guard    one word of device memory no other call in flight uses.
+ * A refused call leaves kv, `written` and q_out as they were; the attention output is undefined.
+ * The _checked entry points are the ones without the suffix plus this argument (NULL = no check);
+ * waiting for the report is the caller's business.
+ */
+#define WE_CHECK_FRAME 1
+#define WE_CHECK_TABLE 2
+typedef struct we_pos_check {
+  int32_t what;
+  uint64_t* report;
+  uint64_t ticket;
+  uint32_t* guard;
+} we_pos_check;
+
+int we_rope_kv_store_checked(const void* q, const void* k, const void* v,
+                             const int64_t q_strides[3], const int64_t k_strides[3],
+                             const int64_t v_strides[3], void* q_out,
+                             const float* cos_table, const float* sin_table, int64_t table_rows,
+                             const int64_t* t_pos, const int64_t* y_pos, const int64_t* x_pos,
+                             int64_t pos_stride_b, int64_t grid_h, int64_t grid_w,
+                             void* kv, uint8_t* written,
+                             int32_t B, int32_t H, int32_t Hkv, int32_t T, int32_t Dh, int64_t L,
+                             int32_t dilation, int32_t is_frozen, int32_t dtype,
+                             const we_pos_check* check, void* stream);
+
+int we_rope_apply_checked(const void* x, const int64_t x_strides[3], void* x_out,
+                          const float* cos_table, const float* sin_table, int64_t table_rows,
+                          const int64_t* t_pos, const int64_t* y_pos, const int64_t* x_pos,
+                          int64_t pos_stride_b, int64_t grid_h, int64_t grid_w,
+                          int32_t B, int32_t H, int32_t T, int32_t Dh, int32_t dtype,
+                          const we_pos_check* check, void* stream);
+
+int we_rope_kv_attn_fwd_checked(const void* q, const void* k, const void* v,
+                                const int64_t q_strides[3], const int64_t k_strides[3], const int64_t v_strides[3],
+                                void* q_out,
+                                const float* cos_table, const float* sin_table, int64_t table_rows,
+                                const int64_t* t_pos, const int64_t* y_pos, const int64_t* x_pos,
+                                int64_t pos_stride_b, int64_t grid_h, int64_t grid_w,
+                                void* kv, uint8_t* written,
+                                void* out, const int64_t out_strides[3],
+                                void* workspace, size_t workspace_bytes,
+                                int32_t B, int32_t H, int32_t Hkv, int32_t T, int32_t Dh, int64_t L,
+                                int32_t dilation, int32_t is_frozen, float scale, int32_t n_splits, int32_t q_tile,
+                                int32_t dtype, const we_attn_extras* extras, const we_pos_check* check,
+                                void* stream);
+
+int we_qkv_rope_kv_attn_fwd_checked(const we_qkv_proj* proj, void* q_out,
+                                    const float* cos_table, const float* sin_table, int64_t table_rows,
+                                    const int64_t* t_pos, const int64_t* y_pos, const int64_t* x_pos,
+                                    int64_t pos_stride_b, int64_t grid_h, int64_t grid_w,
+                                    void* kv, uint8_t* written,
+                                    void* out, const int64_t out_strides[3],
+                                    void* workspace, size_t workspace_bytes,
+                                    int32_t B, int32_t H, int32_t Hkv, int32_t T, int32_t Dh, int64_t L,
+                                    int32_t dilation, int32_t is_frozen, float scale, int32_t n_splits, int32_t q_tile,
+                                    int32_t dtype, const we_attn_extras* extras, const we_pos_check* check,
+                                    void* stream);
+
 #ifdef __cplusplus
 }
 #endif

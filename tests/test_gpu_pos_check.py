@@ -1,0 +1,93 @@
+"""The position-id check inside the calls' own kernels: whichever way it runs (by the store's workgroups,
+or by the kernel in front of them for many ids), a bad id anywhere is refused with the error the torch
+operations would name, before a row of the cache changes; a good frame passes, also from several threads."""
+import threading
+
+import pytest
+import torch
+
+import world_engine_amd as wea
+from oracle import ring_oracle as ro
+from _harness import to_dev
+
+pytestmark = pytest.mark.gpu
+
+BAD = {  # (name, row from the end of the batch, value at the last token) -> error
+    "t_pos": [(-1, RuntimeError, "non-negative"), (2, RuntimeError, "constant within frame")],
+    "y_pos": [(1000, AssertionError, "pos_ids out of bounds"), (-1000, IndexError, "index out of range")],
+    "x_pos": [(1000, AssertionError, "pos_ids out of bounds")],
+}
+
+
+# 768 ids are the most that the store's workgroups look at themselves
+@pytest.mark.parametrize("B,T", [(1, 8), (1, 257), (1, 768), (4, 192), (1, 769), (3, 512)])
+def test_bad_ids_are_refused_before_anything_is_written(gpu_device, B, T):
+    dev = gpu_device
+    print(f"pos check B={B} T={T}", flush=True)
+    H, Dh, W = 2, 64, 8
+    layer = wea.LayerKVCache(B, H, 2 * T, Dh, torch.bfloat16, T).to(dev)
+    rope = wea.RoPE(*ro.rope_table_1d(4 * T, Dh), -(-T // W), W).to(dev)
+    q, k, v = (torch.randn(B, H, T, Dh, device=dev, dtype=torch.bfloat16) for _ in range(3))
+    w = torch.randn(3 * H * Dh, H * Dh, device=dev, dtype=torch.bfloat16) * 0.05
+    x = torch.randn(B, T, H * Dh, device=dev, dtype=torch.bfloat16)
+    good = to_dev(ro.synth_pos_ids(1, B, T, W), dev)
+    calls = {
+        "attend": lambda pos: layer.rope_upsert_attend(q, k, v, pos, rope, False),
+        "store": lambda pos: layer.rope_upsert(q, k, v, pos, rope, False),
+        "project": lambda pos: layer.qkv_rope_upsert_attend(x, w, H, pos, rope, False),
+        "upsert": lambda pos: layer.upsert_kv(k, v, pos, False),
+        "rope": lambda pos: rope(q, pos),
+    }
+    for name, call in calls.items():
+        call(good)
+        torch.cuda.synchronize()
+        kv, written = layer.kv.clone(), layer.written.clone()
+        for key, bads in BAD.items():
+            if (name == "upsert") != (key == "t_pos") and name in ("upsert", "rope"):
+                continue
+            for value, err, match in bads:
+                pos = {n: p.clone() for n, p in good.items()}
+                pos[key][B - 1, T - 1] = value
+                if key == "t_pos" and name == "rope":
+                    continue
+                with pytest.raises(err, match=match):
+                    call(pos)
+                assert torch.equal(layer.kv, kv) and torch.equal(layer.written, written), f"{name}: {key}={value} wrote"
+        late = dict(good, t_pos=torch.full_like(good["t_pos"], 4))     # one frame past the table
+        if name != "upsert":
+            with pytest.raises(IndexError, match="index out of range"):
+                call(late)
+            assert torch.equal(layer.kv, kv), f"{name}: a frame past the table wrote"
+        call(good)                                                     # and the next good frame passes
+
+
+def test_checked_calls_from_threads_and_streams(gpu_device):
+    """Each thread on its own stream and cache, good and bad frames in turn: verdicts do not cross."""
+    dev = gpu_device
+    T, H, Dh, W = 64, 2, 64, 8
+    tables = ro.rope_table_1d(4 * T, Dh)
+    failures = []
+
+    def work(i):
+        try:
+            stream = torch.cuda.Stream()
+            with torch.cuda.stream(stream):
+                layer = wea.LayerKVCache(1, H, 2 * T, Dh, torch.bfloat16, T).to(dev)
+                rope = wea.RoPE(*tables, T // W, W).to(dev)
+                q = torch.randn(1, H, T, Dh, device=dev, dtype=torch.bfloat16)
+                good = to_dev(ro.synth_pos_ids(1, 1, T, W), dev)
+                bad = dict(good, t_pos=torch.full_like(good["t_pos"], 4))
+                for n in range(40):
+                    if (n + i) % 3 == 0:
+                        with pytest.raises(IndexError):
+                            layer.rope_upsert_attend(q, q, q, bad, rope, False)
+                    else:
+                        layer.rope_upsert_attend(q, q, q, good, rope, False)
+                stream.synchronize()
+        except BaseException as e:      # noqa: BLE001 - reported by the main thread
+            failures.append((i, repr(e)))
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(6)]
+    [t.start() for t in threads]
+    [t.join(60) for t in threads]
+    assert not failures, failures

@@ -1,8 +1,10 @@
 """ctypes binding of the C ABI declared in ``include/we_attn.h`` (``libwe_attn.so``, the product)
 and of the measurement library declared in ``include/we_attn_probe.h`` (``libwe_probe.so``, loaded
-only by the benchmark and by the tests of its entry points).
+only by the benchmark and by the tests of its entry points).  Calls on tensors go through the
+compiled binding on top of the product (``native``, csrc/bindings.cpp); ctypes serves callers of the
+raw ABI, the sizing helpers and the measurement library.
 
-Both are built in-tree by ``world_engine_amd/build.py`` (``hipcc`` for gfx950).  There is no
+All are built in-tree by ``world_engine_amd/build.py`` (``hipcc`` for gfx950).  There is no
 fallback: if a library is missing, every call into it raises.
 """
 from __future__ import annotations
@@ -119,6 +121,11 @@ SIGNATURES = {
     ]),
 }
 
+# the same calls with a we_pos_check* in front of the stream
+for _name in ("we_rope_kv_store", "we_rope_apply", "we_rope_kv_attn_fwd", "we_qkv_rope_kv_attn_fwd"):
+    _res, _args = SIGNATURES[_name]
+    SIGNATURES[_name + "_checked"] = (_res, _args[:-1] + [c_void_p, c_void_p])
+
 # the measurement library exports these on top of everything above; must list every symbol
 # include/we_attn_probe.h declares
 PROBE_SIGNATURES = {
@@ -133,6 +140,24 @@ PROBE_SIGNATURES = {
     ]),
     "we_stream_probe": (c_int32, [c_void_p, c_size_t, c_int32, c_int32, c_int32, c_void_p]),
 }
+
+class _Native:
+    """The compiled binding (``_native.so``): its functions, loaded on first use; raises if it has
+    not been built."""
+
+    def __getattr__(self, name):
+        lib()      # the library it is linked against; says how to build when there is none
+        try:
+            from . import _native
+        except ImportError as e:
+            raise RuntimeError("the compiled binding world_engine_amd/_native.so is missing or cannot be loaded "
+                               f"(run `python -m world_engine_amd.build`): {e}") from e
+        for fn in ("rope_kv_store", "rope_apply", "attn_ring", "attn_ring_static", "rope_kv_attn", "qkv_rope_kv_attn"):
+            setattr(self, fn, getattr(_native, fn))
+        return object.__getattribute__(self, name)
+
+
+native = _Native()
 
 _lib = None
 

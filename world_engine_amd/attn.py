@@ -19,6 +19,7 @@ import torch.nn.functional as F
 from torch import Tensor, nn
 
 from . import ops
+from ._capi import native
 from .kv_cache import RingMask
 
 
@@ -106,8 +107,18 @@ class RoPE(nn.Module):
                              f"select rows {f_min}..{f_max}")
 
     def forward(self, x: Tensor, pos_ids: Mapping[str, Tensor]) -> Tensor:
-        self.check_pos_ids(pos_ids)
-        return ops.rope_apply(x, pos_ids, self.cos, self.sin, self.height, self.width)
+        if torch.compiler.is_compiling():
+            return ops.rope_apply(x, pos_ids, self.cos, self.sin, self.height, self.width)
+        t_pos = pos_ids["t_pos"]
+        if not t_pos.is_cuda:
+            self.check_pos_ids(pos_ids)
+        # (the kernel holds the ids to the same rules; only a refusal looks them over again, to say what is wrong)
+        y = native.rope_apply(x, t_pos, pos_ids["y_pos"], pos_ids["x_pos"], self.cos, self.sin, self.height, self.width,
+                              ops.CHECK_TABLE)
+        if y is False:
+            self.check_pos_ids(pos_ids)
+            raise RuntimeError("position ids were refused (and changed while the call ran)")
+        return y
 
 
 def ring_attention(q: Tensor, k: Tensor, v: Tensor, block_mask: RingMask, enable_gqa: bool = False,
@@ -116,7 +127,8 @@ def ring_attention(q: Tensor, k: Tensor, v: Tensor, block_mask: RingMask, enable
     ``src/model/attn.py:116``: ``k``/``v`` must be the cache planes that ``upsert`` returned
     together with ``block_mask``."""
     kv = block_mask.kv
-    if k.data_ptr() != kv[0].data_ptr() or v.data_ptr() != kv[1].data_ptr():
+    base = kv.data_ptr()
+    if k.data_ptr() != base or v.data_ptr() != base + kv.stride(0) * kv.element_size():
         raise RuntimeError("ring_attention needs the k/v views returned by the cache's upsert")
     if not enable_gqa and q.shape[1] != k.shape[1]:
         raise RuntimeError("query and key head counts differ but enable_gqa is False")

@@ -1,7 +1,7 @@
-"""Build ``libwe_attn.so`` (HIP, gfx950) in-tree: ``python -m world_engine_amd.build``.
+"""Build ``libwe_attn.so`` (HIP, gfx950) and its Python binding in-tree: ``python -m world_engine_amd.build``.
 
 Every source is compiled to its own object, in parallel (the main attention kernel once per
-element type / head dim family), and the objects are linked into the shared library."""
+element type / head dim family), and the objects are linked into the shared library.  The binding is host code: g++ against torch's headers."""
 from __future__ import annotations
 
 import os
@@ -26,9 +26,10 @@ UNITS = _SHARED + _RING + [("device_state.hip", [], "device_state.o"), ("capi.hi
 PROBE_UNITS = _SHARED + [(src, defs + ["-DWE_WITH_PROBES"], "probe_" + obj) for src, defs, obj in _RING] + [
     ("device_state.hip", [], "probe_device_state.o"), ("capi.hip", [], "probe_capi_base.o"),
     ("probe_capi.hip", [], "probe_capi.o"), ("stream_probe.hip", [], "stream_probe.o")]
-SOURCES = sorted({u[0] for u in UNITS + PROBE_UNITS})
+SOURCES = sorted({u[0] for u in UNITS + PROBE_UNITS} | {"bindings.cpp"})
 OUT = os.path.join(HERE, "libwe_attn.so")
 PROBE_OUT = os.path.join(HERE, "libwe_probe.so")
+NATIVE_OUT = os.path.join(HERE, "_native.so")   # Python binding of libwe_attn.so (host code only)
 
 HIPCC_FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC",
@@ -50,8 +51,23 @@ def _run(cmd, verbose):
     return err
 
 
+def _binding_command():
+    """g++ line of the Python binding: torch's headers for the tensors, the library next to it."""
+    import sysconfig
+    from torch.utils import cpp_extension as ext
+    import torch
+    rocm = os.environ.get("ROCM_PATH", "/opt/rocm")
+    inc = [*ext.include_paths(), sysconfig.get_paths()["include"], os.path.join(rocm, "include")]
+    return [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-D__HIP_PLATFORM_AMD__=1",
+            "-DUSE_ROCM=1", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", *[f"-isystem{p}" for p in inc],
+            os.path.join(CSRC, "bindings.cpp"), "-o", NATIVE_OUT, OUT, *[f"-L{p}" for p in ext.library_paths()],
+            "-ltorch", "-ltorch_cpu", "-ltorch_python", "-lc10", "-lc10_hip", f"-L{os.path.join(rocm, 'lib')}", "-lamdhip64",
+            "-Wl,-rpath,$ORIGIN", *[f"-Wl,-rpath,{p}" for p in ext.library_paths()]]
+
+
 def build(verbose: bool = False, jobs: int = 8) -> str:
-    """Compile every unit once and link ``libwe_attn.so`` and ``libwe_probe.so``; returns the product's path."""
+    """Compile every unit once, link ``libwe_attn.so`` and ``libwe_probe.so`` and build the Python binding
+    ``_native.so`` on top; returns the product's path."""
     hipcc = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
     os.makedirs(OBJ_DIR, exist_ok=True)
     units = list({u[2]: u for u in UNITS + PROBE_UNITS}.values())   # one compile per object
@@ -62,6 +78,7 @@ def build(verbose: bool = False, jobs: int = 8) -> str:
     for out, group in ((OUT, UNITS), (PROBE_OUT, PROBE_UNITS)):
         _run([hipcc, "--offload-arch=gfx950", "-shared", "-fPIC", *[os.path.join(OBJ_DIR, u[2]) for u in group], "-o", out],
              verbose)
+    _run(_binding_command(), verbose)
     return OUT
 
 

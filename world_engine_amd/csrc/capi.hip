@@ -71,7 +71,7 @@ int prepare_store(const void* q, const void* k, const void* v, const int64_t* q_
   p.vs_b = v_strides[0]; p.vs_h = v_strides[1]; p.vs_t = v_strides[2];
   p.pos_stride_b = pos_stride_b;
   p.table_rows = table_rows;
-  p.grid_hw = grid_h * grid_w; p.grid_w = grid_w;
+  p.grid_hw = grid_h * grid_w; p.grid_h = grid_h; p.grid_w = grid_w;
   p.cpr_shift = -1;
   for (int sh = 0; sh < 16; ++sh)
     if ((Dh >> 4) == (1 << sh)) p.cpr_shift = sh;
@@ -79,6 +79,35 @@ int prepare_store(const void* q, const void* k, const void* v, const int64_t* q_
   p.B = B; p.H = H; p.Hkv = Hkv; p.T = T; p.Dh = Dh;
   p.dilation = dilation; p.num_buckets = (int)((L / T) / dilation); p.frozen = is_frozen ? 1 : 0;
   p.norm_eps = 0.f; p.v1 = nullptr; p.v_lamb = nullptr; p.v1s_b = p.v1s_h = p.v1s_t = 0;
+  p.check = 0; p.report = nullptr; p.ticket = 0; p.guard = nullptr;
+  return WE_OK;
+}
+
+// Up to this many position ids the store kernel's workgroups look at all of them themselves, beyond
+// it a kernel of its own does.  Measured per eager attention call (16 heads of 128, 4 slots, MI355X),
+// inside / in front / unchecked, us: 64 ids 14.6 / 18.9 / 13.4, 256: 20.3 / 23.4 / 19.1, 512: 24.5 /
+// 26.6 / 22.6, 1024: 34.1 / 33.3 / 29.2 - the extra launch costs 4 us, every id a workgroup looks at
+// costs all of them.
+constexpr int64_t kCheckInStore = 768;
+
+int check_args_ok(const we_pos_check* c, const we::StoreParams& p) {
+  if (!c || c->what == 0) return WE_OK;
+  if (!c->report || !c->guard) return WE_ERR_NULL_POINTER;
+  if ((c->what & ~(WE_CHECK_FRAME | WE_CHECK_TABLE)) != 0) return WE_ERR_UNSUPPORTED;
+  if ((c->what & WE_CHECK_TABLE) != 0 && (!p.cos_t || !p.y_pos || !p.x_pos)) return WE_ERR_NULL_POINTER;
+  return WE_OK;
+}
+
+// Puts the check (arguments already validated) into the call whose store parameters are `p`:
+// inside its kernel, or as a launch in front of it.
+int apply_check(const we_pos_check* c, bool in_kernel, we::StoreParams& p, hipStream_t st) {
+  if (!c || c->what == 0) return WE_OK;
+  p.check = c->what;
+  p.report = c->report;
+  p.ticket = c->ticket;
+  if (in_kernel && (int64_t)p.B * p.T <= kCheckInStore) return WE_OK;
+  if (we::launch_pos_check(p, c->guard, st) != hipSuccess) return WE_ERR_LAUNCH;
+  p.guard = c->guard;
   return WE_OK;
 }
 
@@ -117,7 +146,7 @@ int prepare_proj(const we_qkv_proj* proj, void* q_out, const float* cos_table, c
   p.t_pos = t_pos; p.y_pos = y_pos; p.x_pos = x_pos;
   p.pos_stride_b = pos_stride_b;
   p.table_rows = table_rows;
-  p.grid_hw = grid_h * grid_w; p.grid_w = grid_w;
+  p.grid_hw = grid_h * grid_w; p.grid_h = grid_h; p.grid_w = grid_w;
   p.cpr_shift = Dh == 128 ? 3 : 2;
   p.L = L;
   p.B = B; p.H = H; p.Hkv = Hkv; p.T = T; p.Dh = Dh;
@@ -184,18 +213,41 @@ int we_rope_kv_store(const void* q, const void* k, const void* v, const int64_t 
                      int64_t pos_stride_b, int64_t grid_h, int64_t grid_w, void* kv, uint8_t* written,
                      int32_t B, int32_t H, int32_t Hkv, int32_t T, int32_t Dh, int64_t L,
                      int32_t dilation, int32_t is_frozen, int32_t dtype, void* stream) {
+  return we_rope_kv_store_checked(q, k, v, q_strides, k_strides, v_strides, q_out, cos_table, sin_table, table_rows,
+                                  t_pos, y_pos, x_pos, pos_stride_b, grid_h, grid_w, kv, written, B, H, Hkv, T, Dh, L,
+                                  dilation, is_frozen, dtype, nullptr, stream);
+}
+
+int we_rope_kv_store_checked(const void* q, const void* k, const void* v, const int64_t q_strides[3],
+                             const int64_t k_strides[3], const int64_t v_strides[3], void* q_out,
+                             const float* cos_table, const float* sin_table, int64_t table_rows,
+                             const int64_t* t_pos, const int64_t* y_pos, const int64_t* x_pos,
+                             int64_t pos_stride_b, int64_t grid_h, int64_t grid_w, void* kv, uint8_t* written,
+                             int32_t B, int32_t H, int32_t Hkv, int32_t T, int32_t Dh, int64_t L, int32_t dilation,
+                             int32_t is_frozen, int32_t dtype, const we_pos_check* check, void* stream) {
   we::StoreParams p;
-  const int rc = prepare_store(q, k, v, q_strides, k_strides, v_strides, q_out, cos_table, sin_table, table_rows,
-                               t_pos, y_pos, x_pos, pos_stride_b, grid_h, grid_w, kv, written, B, H, Hkv, T, Dh,
-                               L, dilation, is_frozen, dtype, p);
+  int rc = prepare_store(q, k, v, q_strides, k_strides, v_strides, q_out, cos_table, sin_table, table_rows,
+                         t_pos, y_pos, x_pos, pos_stride_b, grid_h, grid_w, kv, written, B, H, Hkv, T, Dh,
+                         L, dilation, is_frozen, dtype, p);
+  if (rc == WE_OK) rc = check_args_ok(check, p);
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  if (rc == WE_OK) rc = apply_check(check, true, p, st);
   if (rc != WE_OK) return rc;
-  return we::launch_rope_kv_store(p, dtype, static_cast<hipStream_t>(stream)) == hipSuccess ? WE_OK : WE_ERR_LAUNCH;
+  return we::launch_rope_kv_store(p, dtype, st) == hipSuccess ? WE_OK : WE_ERR_LAUNCH;
 }
 
 int we_rope_apply(const void* x, const int64_t x_strides[3], void* x_out, const float* cos_table,
                   const float* sin_table, int64_t table_rows, const int64_t* t_pos, const int64_t* y_pos,
                   const int64_t* x_pos, int64_t pos_stride_b, int64_t grid_h, int64_t grid_w, int32_t B,
                   int32_t H, int32_t T, int32_t Dh, int32_t dtype, void* stream) {
+  return we_rope_apply_checked(x, x_strides, x_out, cos_table, sin_table, table_rows, t_pos, y_pos, x_pos, pos_stride_b,
+                               grid_h, grid_w, B, H, T, Dh, dtype, nullptr, stream);
+}
+
+int we_rope_apply_checked(const void* x, const int64_t x_strides[3], void* x_out, const float* cos_table,
+                          const float* sin_table, int64_t table_rows, const int64_t* t_pos, const int64_t* y_pos,
+                          const int64_t* x_pos, int64_t pos_stride_b, int64_t grid_h, int64_t grid_w, int32_t B,
+                          int32_t H, int32_t T, int32_t Dh, int32_t dtype, const we_pos_check* check, void* stream) {
   if (!x || !x_strides || !x_out || !cos_table || !sin_table || !t_pos || !y_pos || !x_pos)
     return WE_ERR_NULL_POINTER;
   if (dtype != WE_DTYPE_BF16 && dtype != WE_DTYPE_F16 && dtype != WE_DTYPE_F32) return WE_ERR_UNSUPPORTED;
@@ -212,14 +264,18 @@ int we_rope_apply(const void* x, const int64_t x_strides[3], void* x_out, const 
   p.qs_b = x_strides[0]; p.qs_h = x_strides[1]; p.qs_t = x_strides[2];
   p.pos_stride_b = pos_stride_b;
   p.table_rows = table_rows;
-  p.grid_hw = grid_h * grid_w; p.grid_w = grid_w;
+  p.grid_hw = grid_h * grid_w; p.grid_h = grid_h; p.grid_w = grid_w;
   p.cpr_shift = -1;
   for (int sh = 0; sh < 16; ++sh)
     if ((Dh >> 4) == (1 << sh)) p.cpr_shift = sh;
   p.L = T;
   p.B = B; p.H = H; p.Hkv = 0; p.T = T; p.Dh = Dh;
   p.dilation = 1; p.num_buckets = 1; p.frozen = 1;
-  return we::launch_rope_kv_store(p, dtype, static_cast<hipStream_t>(stream)) == hipSuccess ? WE_OK : WE_ERR_LAUNCH;
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  int rc = check_args_ok(check, p);
+  if (rc == WE_OK) rc = apply_check(check, true, p, st);
+  if (rc != WE_OK) return rc;
+  return we::launch_rope_kv_store(p, dtype, st) == hipSuccess ? WE_OK : WE_ERR_LAUNCH;
 }
 
 int we_init(void) { return we::host::init_current_device(); }
@@ -303,6 +359,21 @@ int we_rope_kv_attn_fwd(const void* q, const void* k, const void* v, const int64
                         int32_t H, int32_t Hkv, int32_t T, int32_t Dh, int64_t L, int32_t dilation,
                         int32_t is_frozen, float scale, int32_t n_splits, int32_t q_tile, int32_t dtype,
                         const we_attn_extras* extras, void* stream) {
+  return we_rope_kv_attn_fwd_checked(q, k, v, q_strides, k_strides, v_strides, q_out, cos_table, sin_table, table_rows,
+                                     t_pos, y_pos, x_pos, pos_stride_b, grid_h, grid_w, kv, written, out, out_strides,
+                                     workspace, workspace_bytes, B, H, Hkv, T, Dh, L, dilation, is_frozen, scale,
+                                     n_splits, q_tile, dtype, extras, nullptr, stream);
+}
+
+int we_rope_kv_attn_fwd_checked(const void* q, const void* k, const void* v, const int64_t q_strides[3],
+                                const int64_t k_strides[3], const int64_t v_strides[3], void* q_out,
+                                const float* cos_table, const float* sin_table, int64_t table_rows,
+                                const int64_t* t_pos, const int64_t* y_pos, const int64_t* x_pos,
+                                int64_t pos_stride_b, int64_t grid_h, int64_t grid_w, void* kv, uint8_t* written,
+                                void* out, const int64_t out_strides[3], void* workspace, size_t workspace_bytes,
+                                int32_t B, int32_t H, int32_t Hkv, int32_t T, int32_t Dh, int64_t L, int32_t dilation,
+                                int32_t is_frozen, float scale, int32_t n_splits, int32_t q_tile, int32_t dtype,
+                                const we_attn_extras* extras, const we_pos_check* check, void* stream) {
   if (!q || !q_out || !cos_table) return WE_ERR_NULL_POINTER;
   we::StoreParams sp;
   int rc = prepare_store(q, k, v, q_strides, k_strides, v_strides, q_out, cos_table, sin_table, table_rows, t_pos,
@@ -330,8 +401,14 @@ int we_rope_kv_attn_fwd(const void* q, const void* k, const void* v, const int64
     rc = apply_gate_extras(extras, dtype, p);
     if (rc != WE_OK) return rc;
   }
+  rc = check_args_ok(check, sp);
+  if (rc != WE_OK) return rc;
   if (dev.rc != WE_OK) return dev.rc;
   // Everything is validated before the first launch; the kernels follow each other on the stream.
+  // (A call whose position ids the check refuses stores nothing; its attention output is garbage,
+  // which the caller learns from the report.)
+  rc = apply_check(check, true, sp, st);
+  if (rc != WE_OK) return rc;
   if (we::launch_rope_kv_store(sp, dtype, st) != hipSuccess) return WE_ERR_LAUNCH;
   return launch_attn(p, pl, Dh, dtype, st);
 }
@@ -358,6 +435,20 @@ int we_qkv_rope_kv_attn_fwd(const we_qkv_proj* proj, void* q_out, const float* c
                             int32_t B, int32_t H, int32_t Hkv, int32_t T, int32_t Dh, int64_t L, int32_t dilation,
                             int32_t is_frozen, float scale, int32_t n_splits, int32_t q_tile, int32_t dtype,
                             const we_attn_extras* extras, void* stream) {
+  return we_qkv_rope_kv_attn_fwd_checked(proj, q_out, cos_table, sin_table, table_rows, t_pos, y_pos, x_pos,
+                                         pos_stride_b, grid_h, grid_w, kv, written, out, out_strides, workspace,
+                                         workspace_bytes, B, H, Hkv, T, Dh, L, dilation, is_frozen, scale, n_splits,
+                                         q_tile, dtype, extras, nullptr, stream);
+}
+
+int we_qkv_rope_kv_attn_fwd_checked(const we_qkv_proj* proj, void* q_out, const float* cos_table,
+                                    const float* sin_table, int64_t table_rows, const int64_t* t_pos,
+                                    const int64_t* y_pos, const int64_t* x_pos, int64_t pos_stride_b, int64_t grid_h,
+                                    int64_t grid_w, void* kv, uint8_t* written, void* out,
+                                    const int64_t out_strides[3], void* workspace, size_t workspace_bytes, int32_t B,
+                                    int32_t H, int32_t Hkv, int32_t T, int32_t Dh, int64_t L, int32_t dilation,
+                                    int32_t is_frozen, float scale, int32_t n_splits, int32_t q_tile, int32_t dtype,
+                                    const we_attn_extras* extras, const we_pos_check* check, void* stream) {
   we::ProjParams pp;
   int rc = prepare_proj(proj, q_out, cos_table, sin_table, table_rows, t_pos, y_pos, x_pos, pos_stride_b, grid_h,
                         grid_w, kv, written, B, H, Hkv, T, Dh, L, dilation, is_frozen, dtype, extras, pp);
@@ -371,8 +462,11 @@ int we_qkv_rope_kv_attn_fwd(const we_qkv_proj* proj, void* q_out, const float* c
                     H, Hkv, T, Dh, L, dilation, scale, n_splits, q_tile, dtype, p, pl);
   if (rc != WE_OK) return rc;
   rc = apply_gate_extras(extras, dtype, p);
+  if (rc == WE_OK) rc = check_args_ok(check, pp.s);
   if (rc != WE_OK) return rc;
   if (dev.rc != WE_OK) return dev.rc;
+  rc = apply_check(check, false, pp.s, st);
+  if (rc != WE_OK) return rc;
   if (we::launch_qkv_rope_store(pp, dtype, st) != hipSuccess) return WE_ERR_LAUNCH;
   return launch_attn(p, pl, Dh, dtype, st);
 }

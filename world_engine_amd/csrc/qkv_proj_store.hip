@@ -234,7 +234,7 @@ qkv_rope_store_kernel(ProjParams p) {
   __syncthreads();
 
   // ---- epilogue: the store kernel's work on this thread's item ----
-  if (!e_live) return;
+  if (!e_live || (s.guard != nullptr && *s.guard != 0u)) return;  // (refused position ids: nothing is written)
   Chunk16<Tag> in;
   {
     const u32x4_t* src = reinterpret_cast<const u32x4_t*>(smem + OUT_OFF + e_row * (PN * 2) + (tid & 7) * 32);

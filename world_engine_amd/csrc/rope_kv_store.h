@@ -3,6 +3,7 @@
 #pragma once
 #include "we_common.h"
 #include "we_kernels.h"
+#include "../../include/we_attn.h"
 
 namespace we {
 
@@ -227,18 +228,40 @@ __device__ __forceinline__ void load_item_side(const StoreParams& p, int which, 
   }
 }
 
-// One K or V item of the stand-alone store kernel: load, then the above.
-template <typename Tag>
-__device__ __forceinline__ void store_kv_item(const StoreParams& p, int which, int b, int h, int t, int chunk,
-                                              const SlotInfo& si) {
-  typedef typename Tag::store_t st_t;
-  const st_t* src = which == 1 ? (const st_t*)p.k + b * p.ks_b + h * p.ks_h + t * p.ks_t
-                               : (const st_t*)p.v + b * p.vs_b + h * p.vs_h + t * p.vs_t;
-  Chunk16<Tag> in;
-  load16<Tag>(in, src + chunk * 16);
-  ItemSide<Tag> sd;
-  load_item_side<Tag>(p, which, b, h, t, chunk, sd);
-  finish_kv_chunk<Tag>(p, which, b, h, t, chunk, si, in, sd.rotate, sd.c, sd.s, sd.res, sd.lamb);
+// Whether the position ids of token i (0 .. B * T) break one of the rules asked for: the frame index
+// non-negative and the same over the frame (src/model/kv_cache.py:112-124), the table position
+// inside the table (src/model/attn.py:25-30).
+__device__ __forceinline__ bool pos_id_bad(const StoreParams& p, int i) {
+  const int b = p.B == 1 ? 0 : i / p.T;
+  const int64_t row0 = b * p.pos_stride_b, at = row0 + (i - b * p.T);
+  const int64_t t = p.t_pos[at];
+  bool bad = false;
+  if (p.check & WE_CHECK_FRAME) bad = t < 0 || t != p.t_pos[row0];
+  if (p.check & WE_CHECK_TABLE) {
+    const int64_t y = p.y_pos[at], x = p.x_pos[at];
+    const int64_t row = t * p.grid_hw + y * p.grid_w + x;
+    bad = bad || x >= p.grid_w || y >= p.grid_h || row < 0 || row >= p.table_rows;
+  }
+  return bad;
+}
+
+// The verdict goes to the waiting host as soon as it is known: one relaxed word to host-coherent
+// memory (no fence - the host reads nothing else of this kernel's).
+__device__ __forceinline__ void report_verdict(const StoreParams& p, bool bad) {
+  __hip_atomic_store(p.report, (p.ticket << 1) | (bad ? 1u : 0u), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+// Whether the call's position ids were refused: uniform over the workgroup, which must reach this
+// as a whole.  Without a verdict from the check kernel every workgroup looks at all ids itself (so
+// that none of them writes a row of a refused frame) and the first one reports.
+__device__ __forceinline__ bool frame_refused(const StoreParams& p) {
+  if (p.check == 0) return false;
+  if (p.guard != nullptr) return *p.guard != 0u;
+  bool bad = false;
+  for (int i = threadIdx.x; i < p.B * p.T; i += blockDim.x) bad = pos_id_bad(p, i) || bad;
+  bad = __syncthreads_or(bad) != 0;
+  if (threadIdx.x == 0 && blockIdx.x == 0 && blockIdx.y == 0 && blockIdx.z == 0) report_verdict(p, bad);
+  return bad;
 }
 
 }  // namespace we

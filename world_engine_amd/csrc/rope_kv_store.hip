@@ -24,27 +24,49 @@ __global__ void __launch_bounds__(256) rope_kv_store_kernel(StoreParams p) {
   const int hq = p.q ? p.H : 0;
   const int hkv = p.k ? p.Hkv : 0;  // rotation-only launches carry no k/v
   const int idx = blockIdx.x * 256 + threadIdx.x;
-  if (idx >= p.T * cpr) return;
+  const bool live = idx < p.T * cpr;
   const int t = p.cpr_shift >= 0 ? idx >> p.cpr_shift : idx / cpr;  // head dims are powers of two in practice
   const int chunk = idx - t * cpr;
   const int head_all = blockIdx.y;
   const int b = blockIdx.z;
+  const int which = head_all < hq ? 0 : (head_all < hq + hkv ? 1 : 2);
+  const int h = head_all - (which == 0 ? 0 : (which == 1 ? hq : hq + hkv));
 
-  if (head_all >= hq) {  // K or V row
-    const int64_t frame_t = p.t_pos[0];
-    const int which = head_all < hq + hkv ? 1 : 2;
-    const SlotInfo si = ring_slot(frame_t, p.dilation, p.num_buckets);
-    store_kv_item<Tag>(p, which, b, head_all - hq - (which == 2 ? hkv : 0), t, chunk, si);
-    return;
-  }
-
-  // Q row: rotate (or copy when there is no table) into the contiguous output
-  const int h = head_all;
+  const int64_t frame_t = p.t_pos[0];
   Chunk16<Tag> in;
-  load16<Tag>(in, (const st_t*)p.q + b * p.qs_b + h * p.qs_h + t * p.qs_t + chunk * 16);
   ItemSide<Tag> sd;
-  load_item_side<Tag>(p, 0, b, h, t, chunk, sd);
-  finish_q_chunk<Tag>(p, b, h, t, chunk, in, sd.rotate, sd.c, sd.s);
+  if (live) {
+    const st_t* src = which == 0   ? (const st_t*)p.q + b * p.qs_b + h * p.qs_h + t * p.qs_t
+                      : which == 1 ? (const st_t*)p.k + b * p.ks_b + h * p.ks_h + t * p.ks_t
+                                   : (const st_t*)p.v + b * p.vs_b + h * p.vs_h + t * p.vs_t;
+    load16<Tag>(in, src + chunk * 16);
+    load_item_side<Tag>(p, which, b, h, t, chunk, sd);
+  }
+  // (the row data and the table rows are on their way while the ids are looked at)
+  if (frame_refused(p) || !live) return;
+  if (which == 0) {  // rotate (or copy when there is no table) into the contiguous output
+    finish_q_chunk<Tag>(p, b, h, t, chunk, in, sd.rotate, sd.c, sd.s);
+  } else {
+    const SlotInfo si = ring_slot(frame_t, p.dilation, p.num_buckets);
+    finish_kv_chunk<Tag>(p, which, b, h, t, chunk, si, in, sd.rotate, sd.c, sd.s, sd.res, sd.lamb);
+  }
+}
+
+// The check alone, for frames whose ids are too many for every workgroup of the store to look at.
+__global__ void __launch_bounds__(1024) pos_check_kernel(StoreParams p, uint32_t* guard) {
+  bool bad = false;
+#pragma unroll 4
+  for (int i = threadIdx.x; i < p.B * p.T; i += 1024) bad = pos_id_bad(p, i) || bad;
+  bad = __syncthreads_or(bad) != 0;
+  if (threadIdx.x == 0) {
+    *guard = bad ? 1u : 0u;
+    report_verdict(p, bad);
+  }
+}
+
+hipError_t launch_pos_check(const StoreParams& p, uint32_t* guard, hipStream_t stream) {
+  hipLaunchKernelGGL(pos_check_kernel, dim3(1), dim3(1024), 0, stream, p, guard);
+  return hipGetLastError();
 }
 
 hipError_t launch_rope_kv_store(const StoreParams& p, int dtype, hipStream_t stream) {

@@ -23,7 +23,7 @@ struct StoreParams {
   int64_t vs_b, vs_h, vs_t;
   int64_t pos_stride_b;
   int64_t table_rows;
-  int64_t grid_hw, grid_w;
+  int64_t grid_hw, grid_h, grid_w;
   int64_t L;
   int B, H, Hkv, T, Dh;
   int dilation, num_buckets, frozen;
@@ -33,6 +33,11 @@ struct StoreParams {
   const void* v1;             // value residual [B, Hkv, T, Dh] or null: v = lerp(v, v1, *v_lamb)
   const void* v_lamb;         // device pointer to the lerp weight, element type
   int64_t v1s_b, v1s_h, v1s_t;
+  // optional check of the position ids in front of the call's first write (we_pos_check)
+  int check;               // WE_CHECK_* bits, 0 = no check
+  uint64_t* report;        // host-visible word the verdict goes to
+  uint64_t ticket;
+  const uint32_t* guard;   // set: the check kernel has left its verdict here (non-zero = refused)
 };
 
 // uint64 slots per workgroup of AttnParams::clock_out (measurement library only)
@@ -88,6 +93,8 @@ struct ProjParams {
 };
 
 hipError_t launch_rope_kv_store(const StoreParams& p, int dtype, hipStream_t stream);
+// the check of p's position ids as a kernel of its own: verdict to p.report and *guard
+hipError_t launch_pos_check(const StoreParams& p, uint32_t* guard, hipStream_t stream);
 hipError_t launch_qkv_rope_store(const ProjParams& p, int dtype, hipStream_t stream);
 
 // main kernel, one launcher per (element type, head dim) family: ksplit = 2 -> 128 queries per

@@ -10,8 +10,9 @@ exactly the bits the reference's buffers would.
 What differs by design: ``upsert`` returns a :class:`RingMask` (a view of the cache state) where
 the reference returns a flex-attention ``BlockMask`` (:12-61, :144).  The only consumer of that
 object in the reference is the attention call this package also replaces.  The cache writes are
-one fused kernel launch; the slot is computed on the device from ``t_pos[0, 0]`` (:126-131), so
-no host synchronisation happens outside the optional eager input checks (:112-124).
+one fused kernel launch; the slot is computed on the device from ``t_pos[0, 0]`` (:126-131).  The
+optional eager input checks (:112-124) are done by that launch too: the host waits for its verdict
+on the position ids before it returns, not for the attention behind it.
 """
 from __future__ import annotations
 
@@ -21,6 +22,7 @@ import torch
 from torch import Tensor, nn
 
 from . import ops
+from ._capi import native
 
 
 class RingMask:
@@ -90,31 +92,34 @@ class LayerKVCache(nn.Module):
         self.written.zero_()
         self.written[self.L:].fill_(True)
 
-    # -- input checks of the reference's eager path (src/model/kv_cache.py:112-124) ------------
-    def _check(self, k: Tensor, pos_ids: Mapping[str, Tensor], rope=None) -> None:
+    # -- input checks of the reference's eager path (src/model/kv_cache.py:112-124, src/model/attn.py:25-30) --
+    def _checks(self, rules: int) -> int:
+        """Rules the call's first kernel holds the position ids to (none under ``torch.compile``; the
+        binding drops them under stream capture)."""
+        return rules if self.check_inputs and not torch.compiler.is_compiling() else 0
+
+    def _refuse(self, pos_ids: Mapping[str, Tensor], rope=None) -> None:
+        """The kernel refused the call's position ids and wrote nothing: raise what is wrong with them."""
         t_pos = pos_ids["t_pos"]
-        ops._need_device(k, self.kv, t_pos)
-        if k.size(2) != self.tpf:
-            raise RuntimeError("KV cache expects exactly one frame per upsert")
-        if tuple(t_pos.shape) != (k.size(0), self.tpf):
-            raise RuntimeError("t_pos must be [B, T]")
-        if self.check_inputs and not torch.compiler.is_compiling() and not torch.cuda.is_current_stream_capturing():
-            if not bool((t_pos >= 0).all().item()):
-                raise RuntimeError("t_pos must be non-negative during inference")
-            if not bool((t_pos == t_pos[:, :1]).all().item()):
-                raise RuntimeError("t_pos must be constant within frame")
-            if rope is not None:   # the bounds check of the reference's RoPE (src/model/attn.py:25-30)
-                rope.check_pos_ids(pos_ids)
+        if not bool((t_pos >= 0).all().item()):
+            raise RuntimeError("t_pos must be non-negative during inference")
+        if not bool((t_pos == t_pos[:, :1]).all().item()):
+            raise RuntimeError("t_pos must be constant within frame")
+        if rope is not None:   # the bounds check of the reference's RoPE
+            rope.check_pos_ids(pos_ids)
+        raise RuntimeError("position ids were refused (and changed while the call ran)")
 
     def _mask(self, pos_ids: Mapping[str, Tensor]) -> RingMask:
         return RingMask(self.kv, self.written, pos_ids["t_pos"], self.L, self.tpf, self.pinned_dilation)
 
     def upsert_kv(self, k: Tensor, v: Tensor, pos_ids: Mapping[str, Tensor], is_frozen: bool):
         """Store already-rotated ``k`` and ``v`` ``[B,H,T,Dh]`` (no stacking copy)."""
-        self._check(k, pos_ids)
-        ops.rope_kv_store(None, k, v, pos_ids, None, None, 1, 1, self.kv, self.written, self.L,
-                          self.pinned_dilation, is_frozen)
-        return self.kv[0], self.kv[1], self._mask(pos_ids)
+        kv = self.kv
+        if native.rope_kv_store(None, k, v, pos_ids["t_pos"], None, None, None, None, 1, 1, kv, self.written, self.L,
+                                self.pinned_dilation, is_frozen, self._checks(ops.CHECK_FRAME), self.tpf) is False:
+            self._refuse(pos_ids)
+        k_all, v_all = kv.unbind(0)
+        return k_all, v_all, self._mask(pos_ids)
 
     def upsert(self, kv: Tensor, pos_ids: Mapping[str, Tensor], is_frozen: bool):
         """Reference signature: ``kv`` is ``[2,B,H,T,Dh]`` (``src/model/kv_cache.py:104``)."""
@@ -124,10 +129,14 @@ class LayerKVCache(nn.Module):
                     is_frozen: bool):
         """Fused path used by the attention module: rotate q and k with ``rope``'s tables, store
         k/v, return ``(RoPE(q), k_all, v_all, mask)`` from a single kernel launch."""
-        self._check(k, pos_ids, rope)
-        q_rot = ops.rope_kv_store(q, k, v, pos_ids, rope.cos, rope.sin, rope.height, rope.width,
-                                  self.kv, self.written, self.L, self.pinned_dilation, is_frozen)
-        return q_rot, self.kv[0], self.kv[1], self._mask(pos_ids)
+        kv = self.kv
+        q_rot = native.rope_kv_store(q, k, v, pos_ids["t_pos"], pos_ids["y_pos"], pos_ids["x_pos"], rope.cos, rope.sin,
+                                     rope.height, rope.width, kv, self.written, self.L, self.pinned_dilation, is_frozen,
+                                     self._checks(ops.CHECK_FRAME | ops.CHECK_TABLE), self.tpf)
+        if q_rot is False:
+            self._refuse(pos_ids, rope)
+        k_all, v_all = kv.unbind(0)
+        return q_rot, k_all, v_all, self._mask(pos_ids)
 
     def rope_upsert_attend(self, q: Tensor, k: Tensor, v: Tensor, pos_ids: Mapping[str, Tensor], rope,
                            is_frozen: bool, scale: Optional[float] = None, qk_norm_eps: float = 0.0,
@@ -148,22 +157,16 @@ class LayerKVCache(nn.Module):
                 q, k, v, pos_ids["t_pos"], pos_ids["y_pos"], pos_ids["x_pos"], rope.cos, rope.sin, rope.height,
                 rope.width, self.kv, self.written, self.L, self.pinned_dilation, bool(is_frozen), s,
                 float(qk_norm_eps), v1, v_lamb, gate, gate_x, gate_w)
-        self._check(k, pos_ids, rope)
-        kept = self._reusable(reuse_buffers)
-        bufs = {}
-        if kept is not None:
-            B, H, T, Dh = q.shape
-            key = ("attn", B, H, k.shape[1], T, Dh, q.dtype, q.device)
-            if key not in kept:
-                ws_bytes = ops.attn_workspace_bytes(B, H, k.shape[1], T, Dh, self.L)
-                kept[key] = dict(q_rot=torch.empty((B, H, T, Dh), dtype=q.dtype, device=q.device),
-                                 out=torch.empty((B, T, H, Dh), dtype=q.dtype, device=q.device).transpose(1, 2),
-                                 workspace=torch.empty(ws_bytes, dtype=torch.uint8, device=q.device) if ws_bytes else None)
-            bufs = kept[key]
-        return ops.rope_kv_attn(q, k, v, pos_ids, rope.cos, rope.sin, rope.height, rope.width, self.kv,
-                                self.written, self.L, self.pinned_dilation, is_frozen, scale,
-                                qk_norm_eps=qk_norm_eps, v1=v1, v_lamb=v_lamb, gate=gate, gate_x=gate_x,
-                                gate_w=gate_w, **bufs)[0]
+        q_rot, out, workspace = ops.kept_buffers(self._reusable(reuse_buffers), "attn", q, q.shape[1], k.shape[1], q.shape[2],
+                                                 q.shape[3], self.L)
+        own = self._buffers
+        res = native.rope_kv_attn(q, k, v, pos_ids["t_pos"], pos_ids["y_pos"], pos_ids["x_pos"], rope.cos, rope.sin, rope.height,
+                                  rope.width, own["kv"], own["written"], self.L, self.pinned_dilation, is_frozen, scale, 0, 0,
+                                  out, workspace, q_rot, True, qk_norm_eps, v1, v_lamb, gate, gate_x, gate_w,
+                                  self._checks(ops.CHECK_FRAME | ops.CHECK_TABLE), self.tpf)
+        if res is False:
+            self._refuse(pos_ids, rope)
+        return res[0]
 
     def qkv_rope_upsert_attend(self, x: Tensor, w_qkv: Tensor, n_heads: int, pos_ids: Mapping[str, Tensor], rope,
                                is_frozen: bool, scale: Optional[float] = None, want_v: bool = False,
@@ -182,12 +185,16 @@ class LayerKVCache(nn.Module):
                 rope.height, rope.width, self.kv, self.written, self.L, self.pinned_dilation, bool(is_frozen), s,
                 float(qk_norm_eps), v1, v_lamb, gate_x, gate_w)
             return y, (v if want_v else None)
-        self._check(x.unsqueeze(1), pos_ids, rope)
-        y, _, v = ops.qkv_rope_kv_attn(x, w_qkv, n_heads, n_kv, pos_ids, rope.cos, rope.sin, rope.height, rope.width,
-                                       self.kv, self.written, self.L, self.pinned_dilation, is_frozen, scale,
-                                       want_v=want_v, qk_norm_eps=qk_norm_eps, v1=v1, v_lamb=v_lamb, gate_x=gate_x,
-                                       gate_w=gate_w, buffers=self._reusable(reuse_buffers))
-        return y, v
+        kv = self.kv
+        q_rot, out, workspace = ops.kept_buffers(self._reusable(reuse_buffers), "qkv", x, n_heads, n_kv, x.shape[1], kv.shape[4],
+                                                 self.L)
+        res = native.qkv_rope_kv_attn(x, w_qkv, n_heads, n_kv, pos_ids["t_pos"], pos_ids["y_pos"], pos_ids["x_pos"], rope.cos,
+                                      rope.sin, rope.height, rope.width, kv, self.written, self.L, self.pinned_dilation,
+                                      is_frozen, scale, 0, 0, True, want_v, qk_norm_eps, v1, v_lamb, None, gate_x, gate_w, out,
+                                      workspace, q_rot, self._checks(ops.CHECK_FRAME | ops.CHECK_TABLE), self.tpf)
+        if res is False:
+            self._refuse(pos_ids, rope)
+        return res[0], res[2]
 
 
 class StaticKVCache(nn.Module):
