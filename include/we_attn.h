@@ -33,7 +33,7 @@ extern "C" {
 /* element types of q/k/v, the cache buffer and the attention output */
 #define WE_DTYPE_BF16 0
 #define WE_DTYPE_F16 1
-#define WE_DTYPE_F32 2 /* fp32 caches: the store rotates in fp32, the attention takes a plain one-pass kernel */
+#define WE_DTYPE_F32 2 /* fp32 caches: the store rotates in fp32, the attention takes a one-pass fp32 kernel */
 
 #define WE_OK 0
 #define WE_ERR_NULL_POINTER (-1)
@@ -172,8 +172,8 @@ int we_attn_plan(int32_t B, int32_t H, int32_t Hkv, int32_t T, int32_t Dh, int64
  *   q_tile               queries per workgroup: 0 = choose automatically, or 128 / 256.
  *   scale                softmax scale (> 0); the reference uses 1/sqrt(Dh).
  *
- * Requirements: dtype bf16 or f16 (MFMA kernel) or f32 (plain one-pass kernel on the vector
- * ALUs, fp32 arithmetic throughout, n_splits 0 or 1, q_tile ignored); Dh in {64, 128};
+ * Requirements: dtype bf16 or f16 or f32 (a one-pass kernel of its own, fp32 arithmetic
+ * throughout, n_splits 0 or 1, q_tile ignored); Dh in {64, 128};
  * any T (frames that are not a multiple of the 64-key tile cost one masked tile per slot);
  * L/T <= WE_MAX_SLOTS; H % Hkv == 0; pointers and row starts 16-byte aligned.
  */

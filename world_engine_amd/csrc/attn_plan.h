@@ -30,6 +30,7 @@ struct AttnPlan {
   int n_splits;     // context splits of the units that are split (1: none)
   int units_whole;  // leading (batch, kv head) units that are not split
   int64_t ws_rows;  // query rows that go through the split-context workspace
+  int cus;          // compute units planned for
 };
 
 inline int variant_of(int q_tile) {
@@ -54,6 +55,7 @@ inline int variant_of(int q_tile) {
 inline AttnPlan plan_attn(int B, int H, int Hkv, int T, int64_t L, int n_splits, int variant, int cus) {
   AttnPlan pl;
   if (cus < 8) cus = 8;
+  pl.cus = cus;
   const int64_t wg256 = (int64_t)B * H * ((T + 255) / 256);
   const int64_t wg128 = (int64_t)B * H * ((T + 127) / 128);
   // 256 queries per workgroup when that alone fills the CUs - or when 128 would spill into a
@@ -132,7 +134,7 @@ inline int prepare_attn(const void* q, const int64_t* q_strides, const void* kv,
   if (!(scale > 0.f) || n_splits < 0 || n_splits > 64) return WE_ERR_BAD_SHAPE;
   if (variant_of(q_tile) < 0) return WE_ERR_UNSUPPORTED;
   if (dtype == WE_DTYPE_F32) {
-    // fp32 caches take the plain one-pass kernel: no context splitting, no tile choice
+    // fp32 caches take the one-pass kernel: no context splitting, no tile choice
     if (n_splits > 1 || H > 65535 || B > 65535) return WE_ERR_UNSUPPORTED;
     n_splits = 1;
   }
@@ -175,7 +177,7 @@ inline int prepare_attn(const void* q, const int64_t* q_strides, const void* kv,
 
 // The launches of one planned attention call.
 inline int launch_attn(const AttnParams& p, const AttnPlan& pl, int Dh, int dtype, hipStream_t st) {
-  if (dtype == WE_DTYPE_F32) return launch_attn_ring_f32(p, Dh, st) == hipSuccess ? WE_OK : WE_ERR_LAUNCH;
+  if (dtype == WE_DTYPE_F32) return launch_attn_ring_f32(p, Dh, pl.cus, st) == hipSuccess ? WE_OK : WE_ERR_LAUNCH;
   const int ksplit = pl.variant == 1 ? 2 : 1;
   hipError_t e;
   if (dtype == WE_DTYPE_BF16) e = Dh == 128 ? launch_attn_ring_bf16_128(p, ksplit, st) : launch_attn_ring_bf16_64(p, ksplit, st);

@@ -1,34 +1,84 @@
 // fp32 attention over the KV ring buffer (gfx950): the same visibility rule and ring walk as the
-// MFMA kernel (attn_ring.hip), computed entirely in fp32 on the vector ALUs.
+// half-precision kernel (attn_ring.hip), fp32 throughout (fp32 scores, softmax and P V,
+// src/model/attn.py:116 in eager mode) on the fp32 matrix instructions.
 //
-// fp32 is the reference's CPU plumbing configuration (one layer, 64-token frames), not a serving
-// path; this kernel exists so that the whole interface also works on fp32 caches, with results
-// that follow the reference's fp32 arithmetic (fp32 scores, fp32 softmax, fp32 P V,
-// src/model/attn.py:116 in eager mode).  It is a plain tiled kernel, not tuned.
+// One workgroup = 16 queries of one (batch, head) and NW wavefronts that share out its keys: blocks
+// of 16 keys go round the wavefronts, each keeps its own running (reference, sum, O) and they merge
+// through LDS at the end.  A wavefront's keys are nobody else's, so K and V go from memory straight
+// into the matrix operands' registers, one block ahead, without LDS and without a barrier in the loop:
+//   S^T = K Q^T      v_mfma_f32_16x16x4_f32; the contraction is taken in an order that lets a lane
+//                    load four of its head-dim values at once (lane group g of step (j, i) has value
+//                    16 j + 4 g + i of both operands);
+//   O^T += V^T P^T   the S^T accumulators are the B operand as they are (lane group g, register i =
+//                    key 4 g + i), and output rows are numbered so that a lane's four values of V are
+//                    consecutive: one 16-byte load per key and 64 head-dim values, 256 bytes a row.
 //
-// One workgroup = 64 queries of one (batch, head); a query is shared by 4 lanes that own DH/4
-// head-dim values each.  K/V go through LDS 32 keys at a time; the softmax runs online per tile.
-#include "we_common.h"
+// Bound by the matrix cores (64 MFMAs of 32 cycles per block of 16 keys at Dh = 128, against 16 loads
+// and some 40 vector instructions) and, at 16 queries a workgroup, by the loads' way through the CU's
+// address path beside them: 16 heads of 128, 256 queries, 2048 keys take 54 us = 79 TFLOP/s (a large
+// fp32 matrix product reaches 153 here), 42 us without the loads; 8 heads, 1024 queries and 4096 keys
+// 184 us = 93 TFLOP/s.  The kernel before it (vector ALUs, K and V read from LDS four bytes at a
+// time) took 775 us = 5.5 TFLOP/s for the first; 8 heads of 64, 64 queries, 256 keys: 53 us, now 8.
+#include "attn_mma.h"
 #include "we_kernels.h"
 #include "../../include/we_attn.h"
 
 namespace we {
 
-template <int DH>
-__global__ void __launch_bounds__(256) attn_ring_f32_kernel(AttnParams p) {
-  constexpr int PART = DH / 4;   // head-dim values per lane
-  constexpr int TK = 32;         // keys per tile
-  __shared__ float ks[TK][DH];
-  __shared__ float vs[TK][DH];
+namespace {
+constexpr int F_Q = 16;   // queries per workgroup
+constexpr int F_K = 16;   // keys per block
+}  // namespace
+
+// maximum / sum over the four 16-lane groups of a wavefront, for each lane position in a group
+__device__ __forceinline__ float groups_max(float x) {
+  auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  const float y = fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+  float lo, up;
+  half_wave_pair(y, lo, up);
+  return fmaxf(lo, up);
+}
+__device__ __forceinline__ float groups_sum(float x) {
+  auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  const float y = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+  float lo, up;
+  half_wave_pair(y, lo, up);
+  return lo + up;
+}
+
+template <int DH, int NW>
+__global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2)))
+attn_ring_f32_kernel(AttnParams p) {
+  constexpr int NJ = DH / 16;    // 16-byte loads of K per lane and block
+  constexpr int NH = DH / 64;    // 16-byte loads of V per lane and key
+  constexpr int OROW = DH + 4;   // floats per row of a wavefront's O in LDS (the odd 16 bytes spread the banks)
+  constexpr int NOUT = NW / 2;   // wavefronts whose O is in LDS at a time
+  __shared__ __attribute__((aligned(16))) float osh[NOUT][F_Q][OROW];
+  __shared__ float msh[NW][F_Q], lsh[NW][F_Q];
   __shared__ int vis[WE_MAX_SLOTS + 2];
 
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int qi = tid >> 2, part = tid & 3;
-  const int b = blockIdx.z, h = blockIdx.y, hkv = h / p.group;
-  const int qrow = blockIdx.x * 64 + qi;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int c = lane & 15, g = lane >> 4;
+
+  // ---- which queries ----
+  // (spread over the XCDs by unit where every XCD gets the same number: a unit's workgroups share an L2)
+  const int units = p.B * p.Hkv;
+  int unit, member;
+  if ((units & 7) == 0) {
+    const unsigned j = blockIdx.x >> 3;
+    const unsigned u8 = j / (unsigned)p.members;
+    unit = (int)(u8 * 8 + (blockIdx.x & 7));
+    member = (int)(j - u8 * (unsigned)p.members);
+  } else {
+    unit = (int)(blockIdx.x / (unsigned)p.members);
+    member = (int)(blockIdx.x - (unsigned)unit * (unsigned)p.members);
+  }
+  const int b = unit / p.Hkv, hkv = unit - b * p.Hkv;
+  const int hq_in = member / p.q_tiles, h = hkv * p.group + hq_in;
+  const int q0 = (member - hq_in * p.q_tiles) * F_Q;
 
   // ---- list of visible slots; the tail is pseudo-slot n_slots ----
-  if (tid < 64) {
+  if (wave == 0) {
     const SlotInfo si = ring_slot(p.t_pos[0], p.dilation, p.num_buckets);
     int count = 0;
     for (int base = 0; base < p.n_slots; base += 64) {
@@ -44,86 +94,191 @@ __global__ void __launch_bounds__(256) attn_ring_f32_kernel(AttnParams p) {
       vis[WE_MAX_SLOTS + 1] = count + 1;
     }
   }
+
+  // ---- query c, values 16 j + 4 g + i, pre-multiplied by scale * log2(e) ----
+  f32x4_t qf[NJ];
+  {
+    const int qr = q0 + c < p.T ? q0 + c : p.T - 1;
+    const float* src = reinterpret_cast<const float*>(p.q) + b * p.qs_b + h * p.qs_h + (int64_t)qr * p.qs_t + 4 * g;
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) qf[j] = *reinterpret_cast<const f32x4_t*>(src + 16 * j) * p.scale_log2;
+  }
   __syncthreads();
   const int nvis = vis[WE_MAX_SLOTS + 1];
 
-  // ---- this lane's part of its query, pre-multiplied by scale * log2(e) ----
-  float q[PART];
-  {
-    const int qr = qrow < p.T ? qrow : p.T - 1;
-    const float* src = reinterpret_cast<const float*>(p.q) + b * p.qs_b + h * p.qs_h + (int64_t)qr * p.qs_t + part * PART;
+  f32x4_t o[NH][4];  // o[hh][e] register i: query c, value 64 hh + 16 g + 4 i + e
 #pragma unroll
-    for (int d = 0; d < PART; d += 4) {
-      const f32x4_t x = *reinterpret_cast<const f32x4_t*>(src + d);
-      q[d] = x[0] * p.scale_log2; q[d + 1] = x[1] * p.scale_log2;
-      q[d + 2] = x[2] * p.scale_log2; q[d + 3] = x[3] * p.scale_log2;
-    }
-  }
-  float o[PART];
+  for (int hh = 0; hh < NH; ++hh)
 #pragma unroll
-  for (int d = 0; d < PART; ++d) o[d] = 0.f;
-  float m_run = -INFINITY, l_run = 0.f;
+    for (int e = 0; e < 4; ++e) o[hh][e] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  float m_run = -INFINITY, l_run = 0.f;  // (l_run: this lane group's keys only)
 
   const int64_t cap = p.L + p.T;
   const float* kplane = reinterpret_cast<const float*>(p.kv) + (((int64_t)b * p.Hkv + hkv) * cap) * DH;
   const float* vplane = kplane + (int64_t)p.B * p.Hkv * cap * DH;
 
-  for (int vi = 0; vi < nvis; ++vi) {
-    const int64_t row0 = (int64_t)vis[vi] * p.T;
-    for (int t0 = 0; t0 < p.T; t0 += TK) {
-      __syncthreads();  // the previous tile is no longer read
-      for (int i = tid; i < TK * DH / 4; i += 256) {
-        const int r = i / (DH / 4), c = i % (DH / 4);
-        const int tr = t0 + r < p.T ? t0 + r : p.T - 1;  // a short last tile repeats its last row; masked below
-        *reinterpret_cast<f32x4_t*>(&ks[r][4 * c]) = *reinterpret_cast<const f32x4_t*>(kplane + (row0 + tr) * DH + 4 * c);
-        *reinterpret_cast<f32x4_t*>(&vs[r][4 * c]) = *reinterpret_cast<const f32x4_t*>(vplane + (row0 + tr) * DH + 4 * c);
-      }
-      __syncthreads();
-      float s[TK];
-      float mx = m_run;
+  // Blocks go round the wavefronts in rounds of NW.  The workgroups that share a K/V stream take the
+  // rounds in groups of rot_g, member m starting at round m of every group: they then ask for
+  // different lines at any one time, and each line comes from memory at one member's request (184
+  // against 192 us for the 1024-query shape above; groups of 8 or 16: the same).
+  const int bps = (p.T + F_K - 1) / F_K;  // blocks per slot; the last one may be short
+  const int nblk = nvis * bps, rounds = (nblk + NW - 1) / NW;
+  int rot_g = 1;
+  while (rot_g * 2 <= p.members && rot_g < 4) rot_g *= 2;
+  const int rot_end = (nblk / NW) & ~(rot_g - 1);
+  auto block_of = [&](int k) __attribute__((always_inline)) {
+    const int kk = k < rot_end ? (k & ~(rot_g - 1)) | ((k + member) & (rot_g - 1)) : k;
+    return kk * NW + wave;
+  };
+
+  auto load = [&](f32x4_t(&kf)[NJ], f32x4_t(&vf)[4][NH], int vi_, int sub_) __attribute__((always_inline)) {
+    const int64_t row0 = (int64_t)__builtin_amdgcn_readfirstlane(vis[vi_]) * p.T;
+    const int t0 = sub_ * F_K, last = p.T - 1;  // rows past the frame repeat its last one
+    const float* ks = kplane + (row0 + (t0 + c < last ? t0 + c : last)) * DH + 4 * g;
 #pragma unroll
-      for (int kk = 0; kk < TK; ++kk) {
-        float acc = 0.f;
+    for (int j = 0; j < NJ; ++j) kf[j] = *reinterpret_cast<const f32x4_t*>(ks + 16 * j);
 #pragma unroll
-        for (int d = 0; d < PART; ++d) acc += q[d] * ks[kk][part * PART + d];
-        acc += __shfl_xor(acc, 1);
-        acc += __shfl_xor(acc, 2);
-        if (t0 + kk >= p.T) acc = -INFINITY;
-        s[kk] = acc;
-        mx = fmaxf(mx, acc);
+    for (int i = 0; i < 4; ++i) {
+      const int t = t0 + 4 * g + i;
+      const float* vs = vplane + (row0 + (t < last ? t : last)) * DH + 4 * c;
+#pragma unroll
+      for (int hh = 0; hh < NH; ++hh) vf[i][hh] = *reinterpret_cast<const f32x4_t*>(vs + 64 * hh);
+    }
+  };
+  auto block = [&](const f32x4_t(&kf)[NJ], f32x4_t(&vf)[4][NH], int keys) __attribute__((always_inline)) {
+    f32x4_t s0 = {0.f, 0.f, 0.f, 0.f}, s1 = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int j = 0; j < NJ; j += 2)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        s0 = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[j][i], qf[j][i], s0, 0, 0, 0);
+        s1 = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[j + 1][i], qf[j + 1][i], s1, 0, 0, 0);
       }
-      const float alpha = __builtin_amdgcn_exp2f(m_run - mx);  // 0 on the first tile
+    f32x4_t s = s0 + s1;
+    if (keys < F_K) {  // missing keys: no weight, and nothing for a zero weight to meet but zeros
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        if (4 * g + i >= keys) {
+          s[i] = -INFINITY;
+#pragma unroll
+          for (int hh = 0; hh < NH; ++hh) vf[i][hh] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+        }
+    }
+    const float mx = fmaxf(m_run, groups_max(fmaxf(fmaxf(s[0], s[1]), fmaxf(s[2], s[3]))));
+    if (__ballot(mx != m_run) != 0ull) {
+      const float alpha = __builtin_amdgcn_exp2f(m_run - mx);  // 0 on the first block
       l_run *= alpha;
 #pragma unroll
-      for (int d = 0; d < PART; ++d) o[d] *= alpha;
+      for (int hh = 0; hh < NH; ++hh)
 #pragma unroll
-      for (int kk = 0; kk < TK; ++kk) {
-        const float pr = __builtin_amdgcn_exp2f(s[kk] - mx);
-        l_run += pr;
-#pragma unroll
-        for (int d = 0; d < PART; ++d) o[d] += pr * vs[kk][part * PART + d];
-      }
+        for (int e = 0; e < 4; ++e) o[hh][e] *= alpha;
       m_run = mx;
+    }
+    f32x4_t pr;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) pr[i] = __builtin_amdgcn_exp2f(s[i] - mx);
+    l_run += (pr[0] + pr[1]) + (pr[2] + pr[3]);
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int hh = 0; hh < NH; ++hh)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) o[hh][e] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[i][hh][e], pr[i], o[hh][e], 0, 0, 0);
+  };
+  const int mine_n = rounds - (nblk - (rounds - 1) * NW > wave ? 0 : 1);  // rounds this wavefront takes part in
+  if (mine_n > 0) {
+    f32x4_t ka[NJ], va[4][NH], kb[NJ], vb[4][NH];
+    int at = block_of(0), vi = (int)((unsigned)at / (unsigned)bps), sub = at - vi * bps;
+    load(ka, va, vi, sub);
+    int keys_a = p.T - sub * F_K, keys_b = 0;  // (16 or more = a whole block)
+    for (int k = 1;; k += 2) {
+      if (k < mine_n) {
+        at = block_of(k); vi = (int)((unsigned)at / (unsigned)bps); sub = at - vi * bps;
+        load(kb, vb, vi, sub);
+        keys_b = p.T - sub * F_K;
+      }
+      block(ka, va, keys_a);
+      if (k >= mine_n) break;
+      if (k + 1 < mine_n) {
+        at = block_of(k + 1); vi = (int)((unsigned)at / (unsigned)bps); sub = at - vi * bps;
+        load(ka, va, vi, sub);
+        keys_a = p.T - sub * F_K;
+      }
+      block(kb, vb, keys_b);
+      if (k + 1 >= mine_n) break;
     }
   }
 
-  if (qrow < p.T) {
-    float inv = 1.f / l_run;
-    // fp32: o * inv is the attention output; the gate multiplies that rounded value
-    const float g = p.gate != nullptr ? reinterpret_cast<const float*>(p.gate)[b * p.gs_b + h * p.gs_h + (int64_t)qrow * p.gs_t] : 1.f;
-    float* dst = reinterpret_cast<float*>(p.out) + b * p.os_b + h * p.os_h + (int64_t)qrow * p.os_t + part * PART;
+  // ---- the wavefronts merge ----
+  l_run = groups_sum(l_run);
+  if (g == 0) {
+    msh[wave][c] = m_run;
+    lsh[wave][c] = l_run;
+  }
+  __syncthreads();
+  float mm = -INFINITY, lt = 0.f;
 #pragma unroll
-    for (int d = 0; d < PART; d += 4)
-      *reinterpret_cast<f32x4_t*>(dst + d) = f32x4_t{(o[d] * inv) * g, (o[d + 1] * inv) * g, (o[d + 2] * inv) * g, (o[d + 3] * inv) * g};
+  for (int w = 0; w < NW; ++w)
+    if (lsh[w][c] != 0.f) mm = fmaxf(mm, msh[w][c]);  // (a wavefront without keys has no say)
+#pragma unroll
+  for (int w = 0; w < NW; ++w)
+    if (lsh[w][c] != 0.f) lt += lsh[w][c] * __builtin_amdgcn_exp2f(msh[w][c] - mm);
+  const float mine = l_run != 0.f ? __builtin_amdgcn_exp2f(m_run - mm) : 0.f;
+#pragma unroll
+  for (int hh = 0; hh < NH; ++hh)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) o[hh][e] *= mine;
+  auto row_of = [&](int w, int hh, int i) { return reinterpret_cast<f32x4_t*>(&osh[w][c][64 * hh + 16 * g + 4 * i]); };
+  if (wave >= NOUT) {
+#pragma unroll
+    for (int hh = 0; hh < NH; ++hh)
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        *row_of(wave - NOUT, hh, i) = f32x4_t{o[hh][0][i], o[hh][1][i], o[hh][2][i], o[hh][3][i]};
+  }
+  __syncthreads();
+  if (wave < NOUT) {
+#pragma unroll
+    for (int hh = 0; hh < NH; ++hh)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        f32x4_t* r = row_of(wave, hh, i);
+        *r = f32x4_t{o[hh][0][i], o[hh][1][i], o[hh][2][i], o[hh][3][i]} + *r;
+      }
+  }
+  if (wave == 0 && g == 0) lsh[0][c] = lt;  // (every wavefront has read the sums before the barrier above)
+  __syncthreads();
+  for (int item = tid; item < F_Q * DH / 4; item += 64 * NW) {
+    const int qi = item / (DH / 4), d = (item % (DH / 4)) * 4;
+    const int qrow = q0 + qi;
+    if (qrow >= p.T) continue;
+    f32x4_t y = *reinterpret_cast<const f32x4_t*>(&osh[0][qi][d]);
+#pragma unroll
+    for (int w = 1; w < NOUT; ++w) y += *reinterpret_cast<const f32x4_t*>(&osh[w][qi][d]);
+    y *= 1.f / lsh[0][qi];
+    // the gate multiplies the rounded attention output, as the module's own multiply does
+    if (p.gate != nullptr) y *= reinterpret_cast<const float*>(p.gate)[b * p.gs_b + h * p.gs_h + (int64_t)qrow * p.gs_t];
+    *reinterpret_cast<f32x4_t*>(reinterpret_cast<float*>(p.out) + b * p.os_b + h * p.os_h + (int64_t)qrow * p.os_t + d) = y;
   }
 }
 
-hipError_t launch_attn_ring_f32(const AttnParams& p, int Dh, hipStream_t stream) {
-  const dim3 grid((unsigned)((p.T + 63) / 64), (unsigned)p.H, (unsigned)p.B);
-  if (Dh == 128) hipLaunchKernelGGL(attn_ring_f32_kernel<128>, grid, dim3(256), 0, stream, p);
-  else if (Dh == 64) hipLaunchKernelGGL(attn_ring_f32_kernel<64>, grid, dim3(256), 0, stream, p);
-  else return hipErrorInvalidValue;
+template <int DH>
+static hipError_t launch_f32(AttnParams p, int cus, hipStream_t stream) {
+  p.q_tiles = (p.T + F_Q - 1) / F_Q;
+  p.members = p.group * p.q_tiles;
+  const int64_t wgs = (int64_t)p.B * p.Hkv * p.members;
+  if (wgs > 0x7fffffff) return hipErrorInvalidValue;
+  // eight wavefronts per workgroup (two per SIMD of a CU) while a CU gets one workgroup; two
+  // workgroups of four beyond, which leave a smaller last round
+  if (wgs <= cus) hipLaunchKernelGGL((attn_ring_f32_kernel<DH, 8>), dim3((unsigned)wgs), dim3(512), 0, stream, p);
+  else hipLaunchKernelGGL((attn_ring_f32_kernel<DH, 4>), dim3((unsigned)wgs), dim3(256), 0, stream, p);
   return hipGetLastError();
+}
+
+hipError_t launch_attn_ring_f32(const AttnParams& p, int Dh, int cus, hipStream_t stream) {
+  if (Dh == 128) return launch_f32<128>(p, cus, stream);
+  if (Dh == 64) return launch_f32<64>(p, cus, stream);
+  return hipErrorInvalidValue;
 }
 
 }  // namespace we

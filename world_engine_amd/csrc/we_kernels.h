@@ -103,8 +103,8 @@ hipError_t launch_attn_ring_bf16_128(const AttnParams& p, int ksplit, hipStream_
 hipError_t launch_attn_ring_bf16_64(const AttnParams& p, int ksplit, hipStream_t stream);
 hipError_t launch_attn_ring_f16_128(const AttnParams& p, int ksplit, hipStream_t stream);
 hipError_t launch_attn_ring_f16_64(const AttnParams& p, int ksplit, hipStream_t stream);
-// fp32 caches: plain vector-ALU kernel, one pass, no context splitting
-hipError_t launch_attn_ring_f32(const AttnParams& p, int Dh, hipStream_t stream);
+// fp32 caches: one pass on the fp32 matrix instructions, no context splitting
+hipError_t launch_attn_ring_f32(const AttnParams& p, int Dh, int cus, hipStream_t stream);
 hipError_t launch_attn_combine(const AttnParams& p, int Dh, int dtype, hipStream_t stream);
 // Measurement library only (stream_probe.hip): the 256-token-frame tile stream without the arithmetic.
 hipError_t launch_stream_probe(const void* src, int workgroups, int tiles, int share, hipStream_t stream);
