@@ -105,6 +105,7 @@ int apply_check(const we_pos_check* c, bool in_kernel, we::StoreParams& p, hipSt
   p.check = c->what;
   p.report = c->report;
   p.ticket = c->ticket;
+  if (!p.y_pos || !p.x_pos) p.y_pos = p.x_pos = p.t_pos;  // (no table rules: loaded, not looked at)
   if (in_kernel && (int64_t)p.B * p.T <= kCheckInStore) return WE_OK;
   if (we::launch_pos_check(p, c->guard, st) != hipSuccess) return WE_ERR_LAUNCH;
   p.guard = c->guard;

@@ -230,19 +230,16 @@ __device__ __forceinline__ void load_item_side(const StoreParams& p, int which, 
 
 // Whether the position ids of token i (0 .. B * T) break one of the rules asked for: the frame index
 // non-negative and the same over the frame (src/model/kv_cache.py:112-124), the table position
-// inside the table (src/model/attn.py:25-30).
+// inside the table (src/model/attn.py:25-30).  Free of branches, so that an unrolled loop has the
+// ids of several tokens in flight (without table rules y_pos and x_pos stand for t_pos).
 __device__ __forceinline__ bool pos_id_bad(const StoreParams& p, int i) {
-  const int b = p.B == 1 ? 0 : i / p.T;
+  const int b = p.B == 1 ? 0 : (int)((unsigned)i / (unsigned)p.T);
   const int64_t row0 = b * p.pos_stride_b, at = row0 + (i - b * p.T);
-  const int64_t t = p.t_pos[at];
-  bool bad = false;
-  if (p.check & WE_CHECK_FRAME) bad = t < 0 || t != p.t_pos[row0];
-  if (p.check & WE_CHECK_TABLE) {
-    const int64_t y = p.y_pos[at], x = p.x_pos[at];
-    const int64_t row = t * p.grid_hw + y * p.grid_w + x;
-    bad = bad || x >= p.grid_w || y >= p.grid_h || row < 0 || row >= p.table_rows;
-  }
-  return bad;
+  const int64_t t = p.t_pos[at], t0 = p.t_pos[row0], y = p.y_pos[at], x = p.x_pos[at];
+  const int64_t row = t * p.grid_hw + y * p.grid_w + x;
+  const bool frame = (t < 0) | (t != t0);
+  const bool table = (x >= p.grid_w) | (y >= p.grid_h) | (row < 0) | (row >= p.table_rows);
+  return (frame & ((p.check & WE_CHECK_FRAME) != 0)) | (table & ((p.check & WE_CHECK_TABLE) != 0));
 }
 
 // The verdict goes to the waiting host as soon as it is known: one relaxed word to host-coherent
@@ -255,10 +252,9 @@ __device__ __forceinline__ void report_verdict(const StoreParams& p, bool bad) {
 // as a whole.  Without a verdict from the check kernel every workgroup looks at all ids itself (so
 // that none of them writes a row of a refused frame) and the first one reports.
 __device__ __forceinline__ bool frame_refused(const StoreParams& p) {
-  if (p.check == 0) return false;
   if (p.guard != nullptr) return *p.guard != 0u;
   bool bad = false;
-  for (int i = threadIdx.x; i < p.B * p.T; i += blockDim.x) bad = pos_id_bad(p, i) || bad;
+  for (int i = threadIdx.x; i < p.B * p.T; i += blockDim.x) bad = pos_id_bad(p, i) | bad;
   bad = __syncthreads_or(bad) != 0;
   if (threadIdx.x == 0 && blockIdx.x == 0 && blockIdx.y == 0 && blockIdx.z == 0) report_verdict(p, bad);
   return bad;

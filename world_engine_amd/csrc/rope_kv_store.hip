@@ -15,7 +15,9 @@
 
 namespace we {
 
-template <typename Tag>
+// CHECK: the call's position ids are checked (a variant of its own: the check's code in front of the
+// stores costs an unchecked call 0.5 us).
+template <typename Tag, bool CHECK>
 __global__ void __launch_bounds__(256) rope_kv_store_kernel(StoreParams p) {
   typedef typename Tag::store_t st_t;
   // grid: x = 256-thread slices of the (token, chunk) pairs of one row block, y = head among
@@ -43,7 +45,7 @@ __global__ void __launch_bounds__(256) rope_kv_store_kernel(StoreParams p) {
     load_item_side<Tag>(p, which, b, h, t, chunk, sd);
   }
   // (the row data and the table rows are on their way while the ids are looked at)
-  if (frame_refused(p) || !live) return;
+  if ((CHECK && frame_refused(p)) || !live) return;
   if (which == 0) {  // rotate (or copy when there is no table) into the contiguous output
     finish_q_chunk<Tag>(p, b, h, t, chunk, in, sd.rotate, sd.c, sd.s);
   } else {
@@ -56,7 +58,7 @@ __global__ void __launch_bounds__(256) rope_kv_store_kernel(StoreParams p) {
 __global__ void __launch_bounds__(1024) pos_check_kernel(StoreParams p, uint32_t* guard) {
   bool bad = false;
 #pragma unroll 4
-  for (int i = threadIdx.x; i < p.B * p.T; i += 1024) bad = pos_id_bad(p, i) || bad;
+  for (int i = threadIdx.x; i < p.B * p.T; i += 1024) bad = pos_id_bad(p, i) | bad;
   bad = __syncthreads_or(bad) != 0;
   if (threadIdx.x == 0) {
     *guard = bad ? 1u : 0u;
@@ -69,16 +71,19 @@ hipError_t launch_pos_check(const StoreParams& p, uint32_t* guard, hipStream_t s
   return hipGetLastError();
 }
 
+template <typename Tag>
+static void launch_store(const StoreParams& p, dim3 grid, hipStream_t stream) {
+  if (p.check != 0) hipLaunchKernelGGL((rope_kv_store_kernel<Tag, true>), grid, dim3(256), 0, stream, p);
+  else hipLaunchKernelGGL((rope_kv_store_kernel<Tag, false>), grid, dim3(256), 0, stream, p);
+}
+
 hipError_t launch_rope_kv_store(const StoreParams& p, int dtype, hipStream_t stream) {
   const int hq = p.q ? p.H : 0;
   const int hkv = p.k ? p.Hkv : 0;
   const dim3 grid((unsigned)((p.T * (p.Dh >> 4) + 255) / 256), (unsigned)(hq + 2 * hkv), (unsigned)p.B);
-  if (dtype == 0)
-    hipLaunchKernelGGL(rope_kv_store_kernel<Bf16Tag>, grid, dim3(256), 0, stream, p);
-  else if (dtype == 1)
-    hipLaunchKernelGGL(rope_kv_store_kernel<F16Tag>, grid, dim3(256), 0, stream, p);
-  else
-    hipLaunchKernelGGL(rope_kv_store_kernel<F32Tag>, grid, dim3(256), 0, stream, p);
+  if (dtype == 0) launch_store<Bf16Tag>(p, grid, stream);
+  else if (dtype == 1) launch_store<F16Tag>(p, grid, stream);
+  else launch_store<F32Tag>(p, grid, stream);
   return hipGetLastError();
 }
 
