@@ -334,6 +334,18 @@ int we_qkv_rope_kv_attn_fwd(const we_qkv_proj* proj, void* q_out,
                             int32_t dtype, const we_attn_extras* extras, void* stream);
 
 /*
+ * y = x w^T for the module's projections of one frame (nn.Linear without bias: qkv_proj, out_proj;
+ * src/patch_model.py:116,140): x [M, K], w [N, K], y [M, N], all row-major with the given element
+ * strides between rows (multiples of 8), 16-byte aligned; bf16 / f16, fp32 accumulation, rounded
+ * once; K a multiple of 128, N of 32.  The kernel is made for a few hundred rows, where a GEMM
+ * streams its weights once: we_linear_covers says whether it is the one to use on the current
+ * device (the features per workgroup it would take; 0 = a GEMM library is the better choice).
+ */
+int32_t we_linear_covers(int32_t M, int32_t N, int32_t K, int32_t dtype);
+int we_linear(const void* x, int64_t x_row_stride, const void* w, int64_t w_row_stride,
+              void* y, int64_t y_row_stride, int32_t M, int32_t N, int32_t K, int32_t dtype, void* stream);
+
+/*
  * Check of a call's position ids (the eager-mode checks of src/model/attn.py:25-30 and
  * src/model/kv_cache.py:112-124) on the device, in front of the call's first write and without
  * another pass over the stream:

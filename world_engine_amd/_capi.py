@@ -121,6 +121,9 @@ SIGNATURES = {
     ]),
 }
 
+SIGNATURES["we_linear_covers"] = (c_int32, [c_int32, c_int32, c_int32, c_int32])
+SIGNATURES["we_linear"] = (c_int32, [c_void_p, c_int64, c_void_p, c_int64, c_void_p, c_int64, c_int32, c_int32, c_int32,
+                                     c_int32, c_void_p])
 # the same calls with a we_pos_check* in front of the stream
 for _name in ("we_rope_kv_store", "we_rope_apply", "we_rope_kv_attn_fwd", "we_qkv_rope_kv_attn_fwd"):
     _res, _args = SIGNATURES[_name]
@@ -152,7 +155,7 @@ class _Native:
         except ImportError as e:
             raise RuntimeError("the compiled binding world_engine_amd/_native.so is missing or cannot be loaded "
                                f"(run `python -m world_engine_amd.build`): {e}") from e
-        for fn in ("rope_kv_store", "rope_apply", "attn_ring", "attn_ring_static", "rope_kv_attn", "qkv_rope_kv_attn"):
+        for fn in ("rope_kv_store", "rope_apply", "attn_ring", "attn_ring_static", "rope_kv_attn", "qkv_rope_kv_attn", "linear"):
             setattr(self, fn, getattr(_native, fn))
         return object.__getattribute__(self, name)
 

@@ -3,11 +3,11 @@
 ``RingAttn`` takes the place of ``Attn`` / ``MergedQKVAttn`` (``src/model/attn.py:70-122``,
 ``src/patch_model.py:92-141``): same parameters and state-dict keys, same call signature, same
 order of operations.  The part between the q/k/v projection and the output projection - RoPE,
-cache update, masked attention - runs as two HIP kernel launches (three with context splits)
-instead of the reference's eager/compiled op sequence.  Projections stay ordinary torch ops.  The
-weightless RMS norm, the value-residual lerp and the head gate are torch ops by default and move
-into the two kernels with ``fuse_elementwise=True`` (results then agree to 1 ulp instead of bit
-for bit).
+cache update, masked attention, and with them the value-residual lerp and the head gate - runs as
+two HIP kernel launches (three with context splits) instead of the reference's eager/compiled op
+sequence.  Projections of small half-precision frames run on the library's own kernel, others are
+ordinary torch ops.  The weightless RMS norm is torch's by default (bit for bit what the reference
+stores) and moves into the store kernel with ``fuse_elementwise=True`` (1 ulp).
 """
 from __future__ import annotations
 
@@ -18,7 +18,7 @@ import torch
 import torch.nn.functional as F
 from torch import Tensor, nn
 
-from . import ops
+from . import _capi, ops
 from ._capi import native
 from .kv_cache import RingMask
 
@@ -136,6 +136,33 @@ def ring_attention(q: Tensor, k: Tensor, v: Tensor, block_mask: RingMask, enable
                          block_mask.dilation, scale)
 
 
+def _plain(lin: nn.Module) -> bool:
+    """A linear layer that is nothing but its weight: no bias, no hooks, no replacement of the class."""
+    return type(lin) is nn.Linear and lin.bias is None and not lin._forward_hooks and not lin._forward_pre_hooks
+
+
+@torch.compiler.assume_constant_result
+def _kernel_covers(rows: int, features: int, contraction: int, half: bool) -> bool:
+    dtype = _capi.WE_DTYPE_F16 if half else _capi.WE_DTYPE_BF16
+    return _capi.lib().we_linear_covers(rows, features, contraction, dtype) != 0
+
+
+def _project(lin: nn.Module, x: Tensor) -> Tensor:
+    """``lin(x)``, on the library's own kernel where the frame is small enough for it to be the faster one
+    (one round of workgroups; 256 x 2048 x 2048: 8.2 us against 9.6 on the GPU, and 4 against 19 us of the
+    host's time, most of it the BLAS routine's choice of a kernel).  fp32 sums rounded once, as there."""
+    if _plain(lin) and not torch.is_autocast_enabled():
+        if torch.compiler.is_compiling():        # the opaque op where the kernel covers the shape, for the same bits as eager
+            if (x.dtype in (torch.bfloat16, torch.float16) and lin.weight.dtype == x.dtype and not torch.is_grad_enabled()
+                    and _kernel_covers(x.numel() // x.shape[-1], lin.out_features, x.shape[-1], x.dtype is torch.float16)):
+                return torch.ops.world_engine_amd.linear(x, lin.weight)
+        else:
+            y = native.linear(x, lin.weight)
+            if y is not None:
+                return y
+    return lin(x)
+
+
 class RingAttn(nn.Module):
     """Drop-in for the reference's attention module.
 
@@ -144,10 +171,11 @@ class RingAttn(nn.Module):
     ``merged_qkv`` the three projections are one ``qkv_proj`` as after the reference's inference
     patch (``src/patch_model.py:102-114``); otherwise the keys are ``q_proj/k_proj/v_proj``.
 
-    ``fuse_elementwise`` moves the module's element-wise neighbours of the attention (QK RMS
-    norm, value-residual lerp, head gate incl. its H x H projection and sigmoid) into the two
-    kernels: seven to nine launches fewer per layer, results within 1 ulp of the separate torch operations instead of bit-identical, which
-    is why it is off unless asked for.
+    The value-residual lerp (same bits as torch's) and the head gate incl. its H x H projection and
+    sigmoid (projection sums in another order, then the module's own roundings) are done inside the
+    two kernels.  ``fuse_elementwise`` moves the QK RMS norm there too: one launch and one pass over
+    q, k and v fewer per layer, rows within 1 ulp of torch's norm instead of bit-identical, which is
+    why it is off unless asked for.
 
     ``fuse_projection`` (on top of ``merged_qkv`` and ``fuse_elementwise``) also runs the merged
     q/k/v projection in the library, in one kernel with the cache write: x goes in, the rotated q
@@ -250,7 +278,7 @@ class RingAttn(nn.Module):
                                                self.layer_idx, want_v=first, reuse_buffers=True, **extras)
         if first:
             v1 = v
-        return self.out_proj(y.transpose(1, 2).reshape(B, T, -1)), v1
+        return _project(self.out_proj, y.transpose(1, 2).reshape(B, T, -1)), v1
 
     def projection_workgroups(self, B: int, T: int) -> int:
         """Workgroups the fused projection kernel launches for x ``[B, T, d_model]``."""
@@ -264,49 +292,58 @@ class RingAttn(nn.Module):
         if (self.uses_fused_projection(B, T) and hasattr(kv_cache, "qkv_rope_upsert_attend")
                 and x.dtype in (torch.bfloat16, torch.float16) and x.stride(-1) == 1):
             return self._forward_fused_projection(x, pos_ids, v1, kv_cache)
+        one_call = hasattr(kv_cache, "rope_upsert_attend")
+        fuse = self.fuse_elementwise and one_call and x.dtype != torch.float32
+        H, Hkv, Dh = self.n_heads, self.n_kv_heads, self.d_head
         if self.merged_qkv:
-            q, k, v = self.qkv_proj(x).split((self.q_out, self.kv_out, self.kv_out), dim=-1)
-        else:
-            q, k, v = self.q_proj(x), self.k_proj(x), self.v_proj(x)
-        q = q.reshape(B, T, self.n_heads, self.d_head).transpose(1, 2)
-        k = k.reshape(B, T, self.n_kv_heads, self.d_head).transpose(1, 2)
-        v = v.reshape(B, T, self.n_kv_heads, self.d_head).transpose(1, 2)
-
-        fuse = self.fuse_elementwise and hasattr(kv_cache, "rope_upsert_attend") and x.dtype != torch.float32
-        extras = {}
-        if self.value_residual:
-            first = v1 is None
-            v1 = v if first else v1
+            rows = _project(self.qkv_proj, x).view(B, T, H + 2 * Hkv, Dh)
+            heads = rows.transpose(1, 2)
+            q, k, v = heads.split((H, Hkv, Hkv), dim=1)
             if not fuse:
-                v = torch.lerp(v, v1.view_as(v), self.v_lamb)
-            elif not first:                      # lerp(v, v, w) is v
-                extras.update(v1=v1.view_as(v), v_lamb=self.v_lamb)
+                # The norm is per row, so q and k take it together, as the rows lie in memory: one launch over
+                # the projection's output (the v rows it also covers are not used) where two launches over the
+                # strided q and k views each made a copy first.
+                q, k, _ = F.rms_norm(rows, (Dh,)).transpose(1, 2).split((H, Hkv, Hkv), dim=1)
+        else:
+            q, k, v = (_project(proj, x).reshape(B, T, -1, Dh) for proj in (self.q_proj, self.k_proj, self.v_proj))
+            if not fuse:
+                q, k = F.rms_norm(q, (Dh,)), F.rms_norm(k, (Dh,))
+            q, k, v = q.transpose(1, 2), k.transpose(1, 2), v.transpose(1, 2)
+
+        # The blend and the gate belong into the kernels (torch.compile has fusions of its own for them).
+        inside = one_call and (fuse or not torch.compiler.is_compiling())
+        extras = {}
+        if self.value_residual and v1 is None:
+            v1 = v                               # (lerp(v, v, w) is v)
+        elif self.value_residual and inside:     # same formula in fp32, rounded once: torch.lerp's bits
+            extras.update(v1=v1.view_as(v), v_lamb=self.v_lamb)
+        elif self.value_residual:
+            v = torch.lerp(v, v1.view_as(v), self.v_lamb)
 
         gates = None
-        if self.gated_attn and not fuse:
-            gates = torch.sigmoid(self.gate_proj(x[..., : self.n_heads]))
+        if self.gated_attn:
+            if inside and x.dtype != torch.float32 and (fuse or _plain(self.gate_proj)):
+                # projection, sigmoid and multiply in the kernels' epilogues
+                extras.update(gate_x=x[..., :H], gate_w=self.gate_proj.weight)
+            else:
+                gates = torch.sigmoid(self.gate_proj(x[..., :H])).permute(0, 2, 1)
+                if inside:                       # the epilogue multiplies the rounded output, as `y * gates` would
+                    extras["gate"] = gates
         if fuse:
             extras["qk_norm_eps"] = torch.finfo(torch.float32).eps     # F.rms_norm's epsilon for these inputs
-            if self.gated_attn:      # projection + sigmoid + multiply all happen in the kernels' epilogues
-                extras.update(gate_x=x[..., : self.n_heads], gate_w=self.gate_proj.weight)
-        else:
-            q = F.rms_norm(q, (self.d_head,))
-            k = F.rms_norm(k, (self.d_head,))
 
         # RoPE(q), RoPE(k), cache write (one launch) and attention over the ring (one or two), all
         # behind one library call; a cache without it gets the reference's sequence of calls
-        if hasattr(kv_cache, "rope_upsert_attend"):
+        if one_call:
             # (y lives in the layer's own buffer until this layer's next call; out_proj below reads it now)
             y = kv_cache.rope_upsert_attend(q, k, v, pos_ids, self.rope, self.layer_idx, reuse_buffers=True, **extras)
         else:
             q, k_all, v_all, ring = kv_cache.rope_upsert(q, k, v, pos_ids, self.rope, self.layer_idx)
             y = ring_attention(q, k_all, v_all, ring, enable_gqa=self.enable_gqa)
+        if gates is not None and not inside:
+            y = y * gates.unsqueeze(-1)
 
-        if gates is not None and not fuse:
-            y = y * gates.permute(0, 2, 1).unsqueeze(-1)
-
-        y = y.transpose(1, 2).reshape(B, T, -1)
-        return self.out_proj(y), v1
+        return _project(self.out_proj, y.transpose(1, 2).reshape(B, T, -1)), v1
 
 
 def install_ring_attention(model: nn.Module, rope: Optional[RoPE], attn_types: tuple, merged_qkv: bool = True,

@@ -17,6 +17,7 @@ _RING = [("attn_ring.hip", [f"-DWE_RING_PART={i}"], f"attn_ring_{name}.o")
          for i, name in enumerate(("bf16_128", "bf16_64", "f16_128", "f16_64"))]
 _SHARED = [("rope_kv_store.hip", [], "rope_kv_store.o"),
            ("qkv_proj_store.hip", [], "qkv_proj_store.o"),
+           ("linear_skinny.hip", [], "linear_skinny.o"),
            ("attn_ring_f32.hip", [], "attn_ring_f32.o"),
            ("attn_combine.hip", [], "attn_combine.o")]
 # the product: libwe_attn.so
@@ -60,7 +61,7 @@ def _binding_command():
     inc = [*ext.include_paths(), sysconfig.get_paths()["include"], os.path.join(rocm, "include")]
     return [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-D__HIP_PLATFORM_AMD__=1",
             "-DUSE_ROCM=1", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", *[f"-isystem{p}" for p in inc],
-            os.path.join(CSRC, "bindings.cpp"), "-o", NATIVE_OUT, OUT, *[f"-L{p}" for p in ext.library_paths()],
+            os.path.join(CSRC, "bindings.cpp"), "-o", NATIVE_OUT, f"-L{HERE}", "-l:libwe_attn.so", *[f"-L{p}" for p in ext.library_paths()],
             "-ltorch", "-ltorch_cpu", "-ltorch_python", "-lc10", "-lc10_hip", f"-L{os.path.join(rocm, 'lib')}", "-lamdhip64",
             "-Wl,-rpath,$ORIGIN", *[f"-Wl,-rpath,{p}" for p in ext.library_paths()]]
 

@@ -9,6 +9,7 @@
 #include <torch/csrc/autograd/python_variable.h>
 
 #include <ATen/core/Tensor.h>
+#include <ATen/core/grad_mode.h>
 #include <ATen/ops/empty.h>
 #include <ATen/ops/empty_strided.h>
 #include <c10/hip/HIPStream.h>
@@ -652,7 +653,39 @@ PyObject* qkv_rope_kv_attn(PyObject*, PyObject* const* argv, Py_ssize_t n) {
   });
 }
 
+// x [..., K] times w [N, K] transposed; None where the kernel is not the one to use (shape, layout,
+// element type, a gradient to record): the caller then takes its linear layer.
+PyObject* linear(PyObject*, PyObject* const* argv, Py_ssize_t n) {
+  return guarded([&]() -> PyObject* {
+    Args a("linear", argv, n, 2);
+    const Tensor &x = a.tensor(), &w = a.tensor();
+    if (!x.is_cuda() || w.device() != x.device() || x.dim() < 2 || w.dim() != 2) return none();
+    const at::ScalarType dt = x.scalar_type();
+    if ((dt != at::kBFloat16 && dt != at::kHalf) || w.scalar_type() != dt) return none();
+    if (at::GradMode::is_enabled() && (x.requires_grad() || w.requires_grad())) return none();
+    const int64_t K = x.size(-1), N = w.size(0), M = K > 0 ? x.numel() / K : 0;
+    const int64_t xs = x.stride(-2);
+    if (w.size(1) != K || M <= 0 || M > (1 << 20) || N > (1 << 24) || x.stride(-1) != 1 || w.stride(1) != 1) return none();
+    int64_t step = xs;  // rows of all leading dimensions at one distance
+    for (int64_t d = x.dim() - 3; d >= 0; --d) {
+      step *= x.size(d + 1);
+      if (x.size(d) > 1 && x.stride(d) != step) return none();
+    }
+    const OnDevice on(x.device());
+    if (we_linear_covers((int)M, (int)N, (int)K, dtype_code(x)) == 0) return none();
+    c10::SmallVector<int64_t, 4> shape(x.sizes().begin(), x.sizes().end());
+    shape.back() = N;
+    const Tensor y = at::empty(shape, x.options());
+    const int rc = we_linear(x.data_ptr(), xs, w.data_ptr(), w.stride(0), y.data_ptr(), N, (int)M, (int)N, (int)K,
+                             dtype_code(x), stream_of(x.device()));
+    if (rc == WE_ERR_ALIGNMENT || rc == WE_ERR_UNSUPPORTED || rc == WE_ERR_BAD_SHAPE) return none();
+    if (rc != WE_OK) fail_code("we_linear", rc);
+    return wrap(y);
+  });
+}
+
 PyMethodDef methods[] = {
+    {"linear", (PyCFunction)(void (*)(void))linear, METH_FASTCALL, nullptr},
     {"rope_kv_store", (PyCFunction)(void (*)(void))rope_kv_store, METH_FASTCALL, nullptr},
     {"rope_apply", (PyCFunction)(void (*)(void))rope_apply, METH_FASTCALL, nullptr},
     {"attn_ring", (PyCFunction)(void (*)(void))attn_ring, METH_FASTCALL, nullptr},

@@ -186,6 +186,22 @@ int apply_gate_extras(const we_attn_extras* extras, int dtype, we::AttnParams& p
   return WE_OK;
 }
 
+// Features per workgroup of the skinny projection kernel: the narrowest tile whose workgroups still
+// fit the CUs in one round; 0 where a GEMM library is the better choice.  Over 300 shapes (64 to 4096
+// rows, 128 to 8192 features, 128 to 4096 contraction elements, MI355X) the library won where no tile
+// fits one round, where a workgroup's stream gets long while many rows could share a larger tile
+// (4096 x 512 x 1024: 10.0 against 17.8 us), and where a long contraction leaves most CUs idle that
+// it can split (128 x 256 x 4096: 7.9 against 10.6 us).
+int linear_tile(int M, int N, int K, int cus) {
+  const int64_t m_tiles = ((int64_t)M + 63) / 64;
+  if (K % 128 != 0 || M > 1024 || (int64_t)M * K > (1 << 20) || (K > 2048 && M < 128)) return 0;
+  for (int bn = 32; bn <= 128; bn *= 2) {
+    const int64_t wgs = m_tiles * (N / bn);
+    if (N % bn == 0 && wgs <= cus) return K > 1024 && wgs * 2 < cus ? 0 : bn;
+  }
+  return 0;
+}
+
 }  // namespace
 
 extern "C" {
@@ -470,6 +486,35 @@ int we_qkv_rope_kv_attn_fwd_checked(const we_qkv_proj* proj, void* q_out, const 
   if (rc != WE_OK) return rc;
   if (we::launch_qkv_rope_store(pp, dtype, st) != hipSuccess) return WE_ERR_LAUNCH;
   return launch_attn(p, pl, Dh, dtype, st);
+}
+
+int32_t we_linear_covers(int32_t M, int32_t N, int32_t K, int32_t dtype) {
+  if (M <= 0 || N <= 0 || K <= 0 || (dtype != WE_DTYPE_BF16 && dtype != WE_DTYPE_F16)) return 0;
+  return linear_tile(M, N, K, we::host::compute_units());
+}
+
+int we_linear(const void* x, int64_t x_row_stride, const void* w, int64_t w_row_stride, void* y, int64_t y_row_stride,
+              int32_t M, int32_t N, int32_t K, int32_t dtype, void* stream) {
+  if (!x || !w || !y) return WE_ERR_NULL_POINTER;
+  if (dtype != WE_DTYPE_BF16 && dtype != WE_DTYPE_F16) return WE_ERR_UNSUPPORTED;
+  if (M <= 0 || N <= 0 || K <= 0 || x_row_stride < K || w_row_stride < K || y_row_stride < N) return WE_ERR_BAD_SHAPE;
+  if (N % 32 != 0 || K % 128 != 0) return WE_ERR_UNSUPPORTED;
+  // per-lane offsets are 32-bit: x and a 128-row slab of w stay below 2 GiB
+  if ((uint64_t)M * (uint64_t)x_row_stride * 2u >= (1ull << 31) || 128ull * (uint64_t)w_row_stride * 2u >= (1ull << 31))
+    return WE_ERR_UNSUPPORTED;
+  if (!aligned16(x) || !aligned16(w) || !aligned16(y) || x_row_stride % 8 != 0 || w_row_stride % 8 != 0 || y_row_stride % 8 != 0)
+    return WE_ERR_ALIGNMENT;
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  const Dev dev = dev_for(st);
+  if (dev.rc != WE_OK) return dev.rc;
+  we::LinearParams p{};
+  p.x = x; p.w = w; p.y = y;
+  p.xs = x_row_stride; p.ws = w_row_stride; p.ys = y_row_stride;
+  p.M = M; p.N = N; p.K = K;
+  int bn = linear_tile(M, N, K, dev.state.cus);
+  if (bn == 0) bn = N % 128 == 0 ? 128 : (N % 64 == 0 ? 64 : 32);
+  if ((((int64_t)M + 63) / 64) * 8 * ((N / bn + 7) / 8) >= (1ll << 31)) return WE_ERR_UNSUPPORTED;
+  return we::launch_linear_skinny(p, bn, dtype, st) == hipSuccess ? WE_OK : WE_ERR_LAUNCH;
 }
 
 }  // extern "C"

@@ -92,6 +92,18 @@ struct ProjParams {
   int n_tiles;          // (H + 2 Hkv) Dh / 128
 };
 
+// y [M, N] = x [M, K] W [N, K]^T (linear_skinny.hip)
+struct LinearParams {
+  const void* x;
+  const void* w;
+  void* y;
+  int64_t xs, ws, ys;   // element strides between rows
+  int M, N, K;
+  int m_tiles, n_tiles;
+};
+// bn: features per workgroup, 32, 64 or 128
+hipError_t launch_linear_skinny(const LinearParams& p, int bn, int dtype, hipStream_t stream);
+
 hipError_t launch_rope_kv_store(const StoreParams& p, int dtype, hipStream_t stream);
 // the check of p's position ids as a kernel of its own: verdict to p.report and *guard
 hipError_t launch_pos_check(const StoreParams& p, uint32_t* guard, hipStream_t stream);

@@ -340,3 +340,16 @@ def _qkv_rope_kv_attn_fake(x, w_qkv, n_heads, n_kv_heads, t_pos, y_pos, x_pos, c
     B, T = x.shape[:2]
     Dh = kv.shape[4]
     return (x.new_empty((B, T, n_heads, Dh)).transpose(1, 2), x.new_empty((B, T, n_kv_heads, Dh)).transpose(1, 2))
+
+
+@torch.library.custom_op("world_engine_amd::linear", mutates_args=())
+def linear_op(x: Tensor, w: Tensor) -> Tensor:
+    """``F.linear(x, w)`` on the library's skinny-projection kernel (the BLAS routine where it does not cover the
+    shape on this device)."""
+    y = native.linear(x, w)
+    return torch.nn.functional.linear(x, w) if y is None else y
+
+
+@linear_op.register_fake
+def _linear_fake(x, w):
+    return x.new_empty((*x.shape[:-1], w.shape[0]))
