@@ -180,7 +180,8 @@ inline int launch_attn(const AttnParams& p, const AttnPlan& pl, int Dh, int dtyp
   if (dtype == WE_DTYPE_F32) return launch_attn_ring_f32(p, Dh, pl.cus, st) == hipSuccess ? WE_OK : WE_ERR_LAUNCH;
   const int ksplit = pl.variant == 1 ? 2 : 1;
   hipError_t e;
-  if (dtype == WE_DTYPE_BF16) e = Dh == 128 ? launch_attn_ring_bf16_128(p, ksplit, st) : launch_attn_ring_bf16_64(p, ksplit, st);
+  if (p.T < 64) e = dtype == WE_DTYPE_BF16 ? launch_attn_ring_short_bf16(p, Dh, ksplit, st) : launch_attn_ring_short_f16(p, Dh, ksplit, st);
+  else if (dtype == WE_DTYPE_BF16) e = Dh == 128 ? launch_attn_ring_bf16_128(p, ksplit, st) : launch_attn_ring_bf16_64(p, ksplit, st);
   else e = Dh == 128 ? launch_attn_ring_f16_128(p, ksplit, st) : launch_attn_ring_f16_64(p, ksplit, st);
   if (e != hipSuccess) return WE_ERR_LAUNCH;
   if (pl.n_splits > 1 && launch_attn_combine(p, Dh, dtype, st) != hipSuccess) return WE_ERR_LAUNCH;

@@ -39,8 +39,16 @@
 // so the workgroups that share one K/V stream share an L2.  Start-up code is kept short on purpose:
 // a 256-token frame runs 8 tiles per workgroup and start-up is a third of the kernel.
 //
-// Frame lengths that are not a multiple of 64 use the RAGGED instantiation: the short last tile
-// of a slot is loaded with its missing rows clamped and its missing keys masked to -inf.
+// Frame lengths that are not a multiple of 64 (KEYS_PACKED, 64 tokens and more): the visible keys
+// count through - slot after slot without padding - and a tile is 64 consecutive ones of them, in at
+// most two pieces of memory: the rows behind a slot boundary that is not contiguous (the hidden slot,
+// the step to the tail) get that gap added to their address.  Only the very last tile can be short;
+// the split that owns it takes it first, so that clamped rows and masked keys stay in the prologue and
+// in a peeled first step.  (Before, every slot's last tile was short and every step of the loop
+// carried the masking and some 20 spilled registers; same plan, us: 24 heads of 128, 3600 tokens, 8
+// slots 1395 -> 1338; 24 heads of 64 on 8, 720 tokens, f16 59.7 -> 51.2; 16 heads, 225 tokens, 16 slots
+// 22.2 -> 20.1, in one part 55.1 -> 43.6.)  Frames below 64 tokens
+// (KEYS_SLOT) take a tile per slot, every one of them equally short.
 //
 // Roofline: 4*T*N_vis*Dh flops and 4*N_vis*Dh bytes of K/V per (batch, kv head).
 #include "attn_mma.h"
@@ -94,10 +102,13 @@ __device__ __forceinline__ u32x2_t lds_read_tr(const unsigned char* smem, uint32
   return __builtin_bit_cast(u32x2_t, v);
 }
 
-// RAGGED: the frame length is not a multiple of the 64-key tile (separate instantiation: the
-// masking of the short tiles costs registers the common case cannot spare).
+// How tiles are laid over the visible keys (a separate instantiation each: the ragged ones' few extra
+// instructions and registers are nothing the common case could spare).
+constexpr int KEYS_TILED = 0;   // T % 64 == 0: whole tiles of one slot
+constexpr int KEYS_PACKED = 1;  // T > 64: 64 consecutive visible keys, the last tile short
+constexpr int KEYS_SLOT = 2;    // T < 64: one slot, short
 // CLOCKED: measurement library only - every workgroup reports its duration (p.clock_out).
-template <typename M, int DH, int KSPLIT, bool RAGGED, bool CLOCKED>
+template <typename M, int DH, int KSPLIT, int KEYS, bool CLOCKED>
 __global__ void __attribute__((amdgpu_flat_work_group_size(512, 512), amdgpu_waves_per_eu(2, 2)))
 attn_ring_kernel(AttnParams p) {
   typedef typename M::frag_t frag_t;
@@ -206,17 +217,18 @@ attn_ring_kernel(AttnParams p) {
     ++nvis;
   }
   stamp(0);  // slot list built
-  // tiles per slot; the last one of a slot holds t_last of its 64 keys when T % 64 != 0
-  const int tps = (p.T + BN - 1) / BN;
-  const int t_last = p.T - (tps - 1) * BN;
-  constexpr bool ragged = RAGGED;
-  const int nt = nvis * tps;
+  // tiles of the visible keys; last_keys: keys of the last one
+  const int tps = KEYS == KEYS_TILED ? p.T / BN : 1;
+  const int nt = KEYS == KEYS_PACKED ? (nvis * p.T + BN - 1) / BN : nvis * tps;
+  const int last_keys = nvis * p.T - (nt - 1) * BN;  // (KEYS_PACKED)
   int t_begin = 0, t_end = nt;
   if (nsp > 1) {  // nt <= 257 * T / 64 and nsp <= 64: the products fit 32 bits
     t_begin = (int)((unsigned)split * (unsigned)nt / (unsigned)nsp);
     t_end = (int)((unsigned)(split + 1) * (unsigned)nt / (unsigned)nsp);
   }
   const int ntile = t_end - t_begin;
+  // this split owns a short last tile (and takes it first)
+  const bool shorted = KEYS == KEYS_PACKED && t_end == nt && last_keys < BN && ntile > 0;
 
   const int64_t cap = p.L + p.T;
   const uint64_t kbase = (uint64_t)(uintptr_t)p.kv + (uint64_t)(((int64_t)b * p.Hkv + hkv) * cap) * ROW_B;
@@ -229,13 +241,16 @@ attn_ring_kernel(AttnParams p) {
   for (int i = 0; i < NDMA; ++i) {
     const int row = (wave + i * 8) * RPI + lane / CPR;
     const int phys = lane % CPR;
-    kvoff[i] = row * ROW_B + ((phys ^ k_swz<DH>(row)) << 4);
-    vvoff[i] = row * ROW_B + ((phys ^ v_swz<DH>(row)) << 4);
+    // (a short slot must not read rows of the next one: its missing rows repeat its last)
+    const int src = KEYS == KEYS_SLOT && row >= p.T ? p.T - 1 : row;
+    kvoff[i] = src * ROW_B + ((phys ^ k_swz<DH>(row)) << 4);
+    vvoff[i] = src * ROW_B + ((phys ^ v_swz<DH>(row)) << 4);
   }
   // The split's visible tiles, 64 at a time: lane i of toff holds the byte offset, inside the
   // (batch, kv head) plane, of tile 64*k + i of the split (fits 32 bits, checked on the host).
-  // Bit 0 (row starts are multiples of 128 bytes) marks the short last tile of a slot.  The tile
-  // loop then needs one v_readlane per tile instead of walking slots and tiles with scalar code.
+  // KEYS_PACKED: its low 7 bits (row starts are multiples of 128 bytes) hold the tile row at which
+  // the next slot begins (64: none does), tgap the bytes between the two slots.  The tile loop then
+  // needs one v_readlane (two) per tile instead of walking slots and tiles with scalar code.
   // The workgroups that share this K/V stream (query tiles x grouped query heads) take the tiles
   // in groups of rot_g = 2 or 4, member m starting at tile m of every group: they then ask for
   // different lines at any one time, each line comes from HBM at one member's request and is an
@@ -246,52 +261,67 @@ attn_ring_kernel(AttnParams p) {
   int rot_g = 1;
   while (rot_g * 2 <= p.members && rot_g < 4) rot_g *= 2;
   const unsigned rot_m = (unsigned)(qtile * p.group + hq_in) & (unsigned)(rot_g - 1);
-  const unsigned rot_end = (unsigned)ntile & ~(unsigned)(rot_g - 1);
-  uint32_t toff = 0;
+  const unsigned rot_end = (unsigned)(ntile - (shorted ? 1 : 0)) & ~(unsigned)(rot_g - 1);
+  uint32_t toff = 0, tgap = 0;
+  struct TileAt { uint32_t off, gap; };
   auto load_offsets = [&](int first) __attribute__((always_inline)) {
     unsigned kk = (unsigned)(first + lane);
-    if (!RAGGED && kk < rot_end) kk = (kk & ~(unsigned)(rot_g - 1)) | ((kk + rot_m) & (unsigned)(rot_g - 1));
+    const bool head = shorted && kk == 0;
+    if (shorted && kk > 0) --kk;  // (the short tile stands in front of the others)
+    if (kk < rot_end) kk = (kk & ~(unsigned)(rot_g - 1)) | ((kk + rot_m) & (unsigned)(rot_g - 1));
     unsigned ti = (unsigned)t_begin + kk;
-    if (ti > (unsigned)(t_end - 1)) ti = (unsigned)(t_end - 1);
-    const unsigned sidx = ti / (unsigned)tps;
-    const unsigned sub = ti - sidx * (unsigned)tps;
-    const uint32_t o = ((uint32_t)vis[sidx] * (uint32_t)p.T + sub * BN) * (uint32_t)ROW_B;
-    toff = (ragged && sub == (unsigned)(tps - 1)) ? (o | 1u) : o;
+    if (head || ti > (unsigned)(t_end - 1)) ti = (unsigned)(t_end - 1);
+    if (KEYS == KEYS_PACKED) {
+      const unsigned v0 = ti * BN, T = (unsigned)p.T;
+      const unsigned sidx = v0 / T, in = v0 - sidx * T;
+      const unsigned brk = T - in < BN ? T - in : BN;
+      const int sl = vis[sidx];
+      const int nx = brk < BN && (int)sidx + 1 < nvis ? vis[sidx + 1] : sl + 1;
+      toff = ((uint32_t)sl * T + in) * (uint32_t)ROW_B | brk;
+      tgap = (uint32_t)(nx - sl - 1) * T * (uint32_t)ROW_B;
+    } else {
+      const unsigned sidx = ti / (unsigned)tps;
+      const unsigned sub = ti - sidx * (unsigned)tps;
+      toff = ((uint32_t)vis[sidx] * (uint32_t)p.T + sub * BN) * (uint32_t)ROW_B;
+    }
   };
   int kc = 0;  // tile the K stream requests next; it stays on the last one
   auto next_off = [&]() __attribute__((always_inline)) {
     if ((kc & 63) == 0) load_offsets(kc);
-    const uint32_t o = (uint32_t)__builtin_amdgcn_readlane((int)toff, kc & 63);
+    TileAt t;
+    t.off = (uint32_t)__builtin_amdgcn_readlane((int)toff, kc & 63);
+    t.gap = KEYS == KEYS_PACKED ? (uint32_t)__builtin_amdgcn_readlane((int)tgap, kc & 63) : 0u;
     if (kc < ntile - 1) ++kc;
-    return o;
+    return t;
   };
   const uint64_t kplane = uniform64(kbase), vplane = uniform64(vbase);
   const uint32_t wave_lds = (uint32_t)__builtin_amdgcn_readfirstlane((int)(lds0 + wave * 1024));
-  // A short tile must not read rows of the next slot (or past the end of the buffer): its rows
-  // beyond t_last repeat row t_last - 1; their keys are masked out of the softmax further down.
-  auto clamp_rows = [&](uint32_t voff, int i) __attribute__((always_inline)) {
-    const int row = (wave + i * 8) * RPI + lane / CPR;
-    return row < t_last ? voff : voff - (uint32_t)(row - (t_last - 1)) * ROW_B;
-  };
   // the tile offset is uniform: it goes into the scalar base address, not into every lane's offset
-  auto dma_k = [&](uint32_t off, int slot) __attribute__((always_inline)) {
-    const bool cut = RAGGED && (off & 1u) != 0u;
-    const uint64_t base = kplane + (off & ~1u);
+  const int dma_row = wave * RPI + lane / CPR;  // tile row of this lane's first instruction
+  auto dma_tile = [&](uint64_t plane, const uint32_t(&voff)[NDMA], TileAt t, uint32_t lds) __attribute__((always_inline)) {
+    const uint64_t base = plane + (KEYS == KEYS_PACKED ? t.off & ~127u : t.off);
+    const int brk = (int)(t.off & 127u);
 #pragma unroll
     for (int i = 0; i < NDMA; ++i)
-      dma16(base, cut ? clamp_rows(kvoff[i], i) : kvoff[i], wave_lds + slot * TILE_B + i * 8 * 1024);
+      dma16(base, KEYS == KEYS_PACKED && dma_row >= brk - i * 8 * RPI ? voff[i] + t.gap : voff[i], lds + i * 8 * 1024);
   };
-  auto dma_v = [&](uint32_t off, int slot) __attribute__((always_inline)) {
-    const bool cut = RAGGED && (off & 1u) != 0u;
-    const uint64_t base = vplane + (off & ~1u);
+  // the split's first tile: rows past the keys of a short one repeat its last
+  auto dma_tile0 = [&](uint64_t plane, const uint32_t(&voff)[NDMA], TileAt t, uint32_t lds) __attribute__((always_inline)) {
+    if (KEYS != KEYS_PACKED || !shorted) { dma_tile(plane, voff, t, lds); return; }
+    const uint64_t base = plane + (t.off & ~127u);
+    const int brk = (int)(t.off & 127u);
 #pragma unroll
-    for (int i = 0; i < NDMA; ++i)
-      dma16(base, cut ? clamp_rows(vvoff[i], i) : vvoff[i], wave_lds + L::V_OFF + slot * TILE_B + i * 8 * 1024);
+    for (int i = 0; i < NDMA; ++i) {
+      const int row = dma_row + i * 8 * RPI, src = row < last_keys ? row : last_keys - 1;
+      dma16(base, voff[i] - (uint32_t)(row - src) * ROW_B + (src >= brk ? t.gap : 0u), lds + i * 8 * 1024);
+    }
   };
-  // keys of 32-key block blk of the tile at position sub of its slot that exist (0 .. 32)
-  auto block_keys = [&](int sub, int blk) __attribute__((always_inline)) {
-    if (!RAGGED) return 32;
-    const int n = ((ragged && sub == tps - 1) ? t_last : BN) - 32 * blk;
+  auto dma_k = [&](TileAt t, int slot) __attribute__((always_inline)) { dma_tile(kplane, kvoff, t, wave_lds + slot * TILE_B); };
+  auto dma_v = [&](TileAt t, int slot) __attribute__((always_inline)) { dma_tile(vplane, vvoff, t, wave_lds + L::V_OFF + slot * TILE_B); };
+  // keys that exist in 32-key block blk of the split's first tile (KEYS_SLOT: of every tile)
+  auto block_keys = [&](int blk) __attribute__((always_inline)) {
+    if (KEYS == KEYS_TILED) return 32;
+    const int n = (KEYS == KEYS_SLOT ? p.T : (shorted ? last_keys : BN)) - 32 * blk;
     return n < 0 ? 0 : (n > 32 ? 32 : n);
   };
   // logits of keys that do not exist become -inf (register i of a lane is key row
@@ -368,11 +398,6 @@ attn_ring_kernel(AttnParams p) {
   // (two transposing reads each) - running up to 15 reads ahead of the MFMAs.
   frag_t p_prev[2];
   f32x16_t s_cur;
-  // RAGGED only: this wavefront has not seen a key yet (its first block was an empty block of a
-  // short tile), so its reference exponent is a placeholder; cur_keys = keys of the block whose
-  // probabilities the next step computes.
-  bool ref_unset = false;
-  int cur_keys = 32;
   // Fragment registers live across steps: every step starts with its first PRE reads (all K
   // fragments and the first V^T fragment) already in flight, issued during the previous step.
   constexpr int PRE = KS + 2;
@@ -397,15 +422,14 @@ attn_ring_kernel(AttnParams p) {
     for (int ks = 0; ks < KS; ++ks) read_k(koff_c, ks);
     read_v(voff_c, 0);
   };
-  // nkeys: keys that exist in the block whose logits this step computes (32 = all, 0 = the block
-  // lies past the end of the split)
+  // nkeys: keys that exist in the block whose logits this step computes, where mask_c says that it
+  // may be short
   // (the K fragments at koff_c were requested by the previous step; the offset documents the call)
   // first_c (128-query shape only): the workgroup's very first step has no previous block, so it
   // skips the product and its V reads instead of multiplying a zeroed tile by zeros.
-  auto step = [&](auto /*koff_c*/, auto voff_c, auto nkoff_c, auto nvoff_c, int nkeys, auto&& mid, auto first_c) __attribute__((always_inline)) {
+  auto step = [&](auto /*koff_c*/, auto voff_c, auto nkoff_c, auto nvoff_c, auto mask_c, int nkeys, auto&& mid, auto first_c) __attribute__((always_inline)) {
     constexpr bool FIRST = decltype(first_c)::value;
-    // (logits of a block past the end of the split are never consumed; a short tile's empty block
-    // is masked after its products)
+    // (logits of a block past the end of the split are never consumed)
     // next own V fragment to request / next-step read pairs requested so far
     int vnext = 1, npair = 0;
     constexpr int NPAIR = PRE / 2;            // the next step's first reads go out two at a time
@@ -480,18 +504,13 @@ attn_ring_kernel(AttnParams p) {
 #pragma unroll
     for (int t = 0; t < 4; ++t) rs = M::add_pair(rs, p_cur[1], t);
 
-    // first block with keys of a wavefront that started on an empty block: nothing is accumulated
-    // yet, so the placeholder reference is replaced by this block's own maximum, up or down
-    // (a placeholder far above every real logit would make all of them underflow to zero)
-    const bool seed = RAGGED && ref_unset && cur_keys > 0;
-    if (seed || __ballot(!(rs <= 256.f)) != 0ull) {
+    if (__ballot(!(rs <= 256.f)) != 0ull) {
       // Rare: some probability of this block may exceed 2^8.  Raise the reference of the rows
       // that need it, redo the block's probabilities exactly and rescale the accumulators: they
       // hold the blocks before this one (the last of those products was issued above).
       const float mx = block_max(s_cur);
-      const float m_new = (seed ? mx > -INFINITY : mx > m_ref) ? mx : m_ref;
-      const float alpha = seed ? 1.f : __builtin_amdgcn_exp2f((m_ref - m_new) * lmul);  // seed: sums and accumulators are still zero
-      if (RAGGED) ref_unset = false;
+      const float m_new = mx > m_ref ? mx : m_ref;
+      const float alpha = __builtin_amdgcn_exp2f((m_ref - m_new) * lmul);
       rs = probabilities(p_cur, s_cur, m_new);
       l_run *= alpha;
       m_ref = m_new;
@@ -504,8 +523,7 @@ attn_ring_kernel(AttnParams p) {
     l_run += rs;
     p_prev[0] = p_cur[0];
     p_prev[1] = p_cur[1];
-    if (RAGGED && nkeys < 32) mask_keys(s_next, nkeys);  // short last tile of a slot (or an empty block of it)
-    if (RAGGED) cur_keys = nkeys;
+    if (decltype(mask_c)::value && nkeys < 32) mask_keys(s_next, nkeys);
     s_cur = s_next;
   };
 
@@ -527,8 +545,7 @@ attn_ring_kernel(AttnParams p) {
     // what the iterations before 0 would have.
     constexpr int KA = KSPLIT == 1 ? 3 : 4;
     // The V stream trails the K stream by KA - 2 tiles, so it reuses the K stream's offsets.
-    int csub = t_begin - (t_begin / tps) * tps;  // position in its slot of the tile whose logits are computed next
-    uint32_t off1, off2;  // offsets of the last and the last-but-one tile the K stream visited
+    TileAt off1, off2;  // offsets of the last and the last-but-one tile the K stream visited
     // Q was requested before the slot flags and loads return in order, so it is here; stating a
     // use now keeps the wait for it from landing behind the tile DMAs issued next.
     if (!q_dma) {
@@ -536,18 +553,18 @@ attn_ring_kernel(AttnParams p) {
       for (int ks = 0; ks < KS; ++ks) asm volatile("" ::"v"(qf[ks]));
     }
     {
-      const uint32_t o0 = next_off();
-      const uint32_t o1 = next_off();
-      const uint32_t o2 = next_off();
-      dma_k(o0, 0);
+      const TileAt o0 = next_off();
+      const TileAt o1 = next_off();
+      const TileAt o2 = next_off();
+      dma_tile0(kplane, kvoff, o0, wave_lds);
       dma_k(o1, 1);
       if (KSPLIT == 2) dma_k(o2, 2);
-      dma_v(o0, 0);
+      dma_tile0(vplane, vvoff, o0, wave_lds + L::V_OFF);
       if (KSPLIT == 1) {
         dma_k(o2, 2);
         off1 = o2; off2 = o1;
       } else {
-        const uint32_t o3 = next_off();
+        const TileAt o3 = next_off();
         dma_k(o3, 3);
         off1 = o3; off2 = o2;
       }
@@ -572,14 +589,13 @@ attn_ring_kernel(AttnParams p) {
         const frag_t a = *reinterpret_cast<const frag_t*>(smem + (k_rd ^ (ks << 5)));
         s_cur = M::mma(a, qf[ks], s_cur);
       }
-      const int nk0 = block_keys(csub, hb);
-      if (RAGGED && nk0 < 32) mask_keys(s_cur, nk0);
+      const int nk0 = block_keys(hb);
+      if (KEYS != KEYS_TILED && nk0 < 32) mask_keys(s_cur, nk0);
       const float mx0 = block_max(s_cur);
-      m_ref = mx0 > -INFINITY ? mx0 : 0.f;  // (a block of the first tile may be empty)
-      if (RAGGED) {
-        ref_unset = nk0 == 0;
-        cur_keys = nk0;
-      }
+      // An empty block has no reference to give: one far below any logit makes the first block with
+      // keys exceed every bound and take the rare path, which finds the right one (sums and
+      // accumulators are still zero then).
+      m_ref = mx0 > -INFINITY ? mx0 : (KEYS == KEYS_TILED ? 0.f : -1e30f);
       set_shift();
     }
     // (every wavefront has read its Q fragments before it passes the barrier below: the staging area
@@ -597,31 +613,32 @@ attn_ring_kernel(AttnParams p) {
     // one tile iteration with compile-time ring positions (JM = j mod 4)
     auto iteration = [&](int j, auto jm_c, auto first_c) __attribute__((always_inline)) {
       constexpr int JM = decltype(jm_c)::value;
+      constexpr bool FIRST = decltype(first_c)::value;
       auto issue_dma = [&]() __attribute__((always_inline)) {
-        const uint32_t o = next_off();
+        const TileAt o = next_off();
         dma_k(o, (JM + KA) % NST);                       // K(j+KA)
         dma_v(KA == 3 ? off1 : off2, (JM + 2) % NST);    // V(j+2)
         off2 = off1;
         off1 = o;
       };
       auto nothing = [&]() __attribute__((always_inline)) {};
-      // csub is tile j's position in its slot; nsub tile j+1's
-      const int nsub = csub + 1 == tps ? 0 : csub + 1;
+      typedef std::integral_constant<bool, KEYS == KEYS_SLOT> short_slots;
       if (KSPLIT == 1) {
         // block (j, 0) -> probabilities; logits of (j, 1); product of (j-1, 1)
         step(IntC<JM * TILE_B + KB_B>(), IntC<((JM + 3) % NST) * TILE_B + KB_B>(),
-             IntC<((JM + 1) % NST) * TILE_B>(), IntC<JM * TILE_B>(), block_keys(csub, 1), issue_dma, std::false_type());
+             IntC<((JM + 1) % NST) * TILE_B>(), IntC<JM * TILE_B>(),
+             std::integral_constant<bool, KEYS == KEYS_SLOT || (KEYS == KEYS_PACKED && FIRST)>(), block_keys(1), issue_dma,
+             std::false_type());
         // block (j, 1) -> probabilities; logits of (j+1, 0); product of (j, 0)
         step(IntC<((JM + 1) % NST) * TILE_B>(), IntC<JM * TILE_B>(),
              IntC<((JM + 1) % NST) * TILE_B + KB_B>(), IntC<JM * TILE_B + KB_B>(),
-             j + 1 < ntile ? block_keys(nsub, 0) : 0, nothing, std::false_type());
+             short_slots(), block_keys(0), nothing, std::false_type());
       } else {
         // block (j, hb) -> probabilities; logits of (j+1, hb); product of (j-1, hb)
         step(IntC<((JM + 1) % NST) * TILE_B>(), IntC<((JM + 3) % NST) * TILE_B>(),
              IntC<((JM + 2) % NST) * TILE_B>(), IntC<JM * TILE_B>(),
-             j + 1 < ntile ? block_keys(nsub, __builtin_amdgcn_readfirstlane(hb)) : 0, issue_dma, first_c);
+             short_slots(), block_keys(__builtin_amdgcn_readfirstlane(hb)), issue_dma, first_c);
       }
-      csub = nsub;
       dma_wait<2 * NDMA>();  // all but this iteration's two tiles have landed (this wavefront's part)
       // A bare barrier: __syncthreads() would also wait for every LDS read in flight, i.e. for the
       // next step's fragments requested a moment ago.  Nothing needs that: the tiles arrive by DMA,
@@ -634,9 +651,9 @@ attn_ring_kernel(AttnParams p) {
 
     int j = 0;
     const std::false_type not_first;
-    if (KSPLIT == 2) {
-      // the first tile's step has no product to do: peeled, with the three iterations that bring
-      // the ring position back to zero
+    if (KSPLIT == 2 || KEYS == KEYS_PACKED) {
+      // the first tile's step has no product to do (128 queries) or may have keys to mask: peeled,
+      // with the three iterations that bring the ring position back to zero
       iteration(0, IntC<0>(), std::true_type());
       j = 1;
       if (j < ntile) { iteration(j, IntC<1>(), not_first); ++j; }
@@ -801,49 +818,56 @@ constexpr bool kWithProbes = true;
 constexpr bool kWithProbes = false;
 #endif
 
-template <typename M, int DH, int KSPLIT, bool RAGGED, bool CLOCKED>
+template <typename M, int DH, int KSPLIT, int KEYS, bool CLOCKED>
 static hipError_t launch_ring_c(const AttnParams& p, hipStream_t stream) {
   const int rounds = (p.unit_splits + 7) / 8;
   const dim3 grid((unsigned)(8 * p.q_tiles), (unsigned)p.group, (unsigned)rounds);
-  hipLaunchKernelGGL((attn_ring_kernel<M, DH, KSPLIT, RAGGED, CLOCKED>), grid, dim3(512), RingLds<DH>::kBytes, stream, p);
+  hipLaunchKernelGGL((attn_ring_kernel<M, DH, KSPLIT, KEYS, CLOCKED>), grid, dim3(512), RingLds<DH>::kBytes, stream, p);
   return hipGetLastError();
 }
-template <typename M, int DH, int KSPLIT, bool RAGGED>
+template <typename M, int DH, int KSPLIT, int KEYS>
 static hipError_t launch_ring_r(const AttnParams& p, hipStream_t stream) {
   if constexpr (kWithProbes) {
-    if (p.clock_out != nullptr) return launch_ring_c<M, DH, KSPLIT, RAGGED, true>(p, stream);
+    if (p.clock_out != nullptr) return launch_ring_c<M, DH, KSPLIT, KEYS, true>(p, stream);
   }
-  return launch_ring_c<M, DH, KSPLIT, RAGGED, false>(p, stream);
+  return launch_ring_c<M, DH, KSPLIT, KEYS, false>(p, stream);
 }
 template <typename M, int DH, int KSPLIT>
 static hipError_t launch_ring_t(const AttnParams& p, hipStream_t stream) {
-  return p.T % BN == 0 ? launch_ring_r<M, DH, KSPLIT, false>(p, stream) : launch_ring_r<M, DH, KSPLIT, true>(p, stream);
+  return p.T % BN == 0 ? launch_ring_r<M, DH, KSPLIT, KEYS_TILED>(p, stream) : launch_ring_r<M, DH, KSPLIT, KEYS_PACKED>(p, stream);
 }
 
 // The kernels use more LDS than a launch may ask for by default; the limit is a per-device
 // setting of each kernel, raised once per device by the library's set-up (device_state.hip).
-template <typename M, int DH, int KSPLIT, bool RAGGED, bool CLOCKED>
+template <typename M, int DH, int KSPLIT, int KEYS, bool CLOCKED>
 static hipError_t configure_one() {
-  return hipFuncSetAttribute(reinterpret_cast<const void*>(&attn_ring_kernel<M, DH, KSPLIT, RAGGED, CLOCKED>),
+  return hipFuncSetAttribute(reinterpret_cast<const void*>(&attn_ring_kernel<M, DH, KSPLIT, KEYS, CLOCKED>),
                              hipFuncAttributeMaxDynamicSharedMemorySize, RingLds<DH>::kBytes);
 }
-template <typename M, int DH>
-static hipError_t configure_family() {
-  hipError_t e = configure_one<M, DH, 1, false, false>();
-  if (e == hipSuccess) e = configure_one<M, DH, 1, true, false>();
-  if (e == hipSuccess) e = configure_one<M, DH, 2, false, false>();
-  if (e == hipSuccess) e = configure_one<M, DH, 2, true, false>();
+template <typename M, int DH, int KEYS>
+static hipError_t configure_keys() {
+  hipError_t e = configure_one<M, DH, 1, KEYS, false>();
+  if (e == hipSuccess) e = configure_one<M, DH, 2, KEYS, false>();
   if constexpr (kWithProbes) {
-    if (e == hipSuccess) e = configure_one<M, DH, 1, false, true>();
-    if (e == hipSuccess) e = configure_one<M, DH, 1, true, true>();
-    if (e == hipSuccess) e = configure_one<M, DH, 2, false, true>();
-    if (e == hipSuccess) e = configure_one<M, DH, 2, true, true>();
+    if (e == hipSuccess) e = configure_one<M, DH, 1, KEYS, true>();
+    if (e == hipSuccess) e = configure_one<M, DH, 2, KEYS, true>();
   }
   return e;
 }
+template <typename M, int DH>
+static hipError_t configure_family() {
+  const hipError_t e = configure_keys<M, DH, KEYS_TILED>();
+  return e == hipSuccess ? configure_keys<M, DH, KEYS_PACKED>() : e;
+}
+// frames below one tile
+template <typename M, int DH>
+static hipError_t launch_short(const AttnParams& p, int ksplit, hipStream_t stream) {
+  return ksplit == 2 ? launch_ring_r<M, DH, 2, KEYS_SLOT>(p, stream) : launch_ring_r<M, DH, 1, KEYS_SLOT>(p, stream);
+}
 
 // The four (element type, head dim) families are compiled as separate objects (WE_RING_PART selects
-// one; undefined = all of them in this translation unit) so that they build in parallel.
+// one; undefined = all of them in this translation unit) so that they build in parallel; the short
+// frames' instantiations are parts of their own.
 #if !defined(WE_RING_PART) || WE_RING_PART == 0
 hipError_t launch_attn_ring_bf16_128(const AttnParams& p, int ksplit, hipStream_t stream) {
   return ksplit == 2 ? launch_ring_t<Bf16Mma, 128, 2>(p, stream) : launch_ring_t<Bf16Mma, 128, 1>(p, stream);
@@ -867,6 +891,25 @@ hipError_t launch_attn_ring_f16_64(const AttnParams& p, int ksplit, hipStream_t 
   return ksplit == 2 ? launch_ring_t<F16Mma, 64, 2>(p, stream) : launch_ring_t<F16Mma, 64, 1>(p, stream);
 }
 hipError_t configure_attn_ring_f16_64() { return configure_family<F16Mma, 64>(); }
+#endif
+
+#if defined(WE_RING_PART) && WE_RING_PART == 4
+hipError_t launch_attn_ring_short_bf16(const AttnParams& p, int Dh, int ksplit, hipStream_t stream) {
+  return Dh == 128 ? launch_short<Bf16Mma, 128>(p, ksplit, stream) : launch_short<Bf16Mma, 64>(p, ksplit, stream);
+}
+hipError_t configure_attn_ring_short_bf16() {
+  const hipError_t e = configure_keys<Bf16Mma, 128, KEYS_SLOT>();
+  return e == hipSuccess ? configure_keys<Bf16Mma, 64, KEYS_SLOT>() : e;
+}
+#endif
+#if defined(WE_RING_PART) && WE_RING_PART == 5
+hipError_t launch_attn_ring_short_f16(const AttnParams& p, int Dh, int ksplit, hipStream_t stream) {
+  return Dh == 128 ? launch_short<F16Mma, 128>(p, ksplit, stream) : launch_short<F16Mma, 64>(p, ksplit, stream);
+}
+hipError_t configure_attn_ring_short_f16() {
+  const hipError_t e = configure_keys<F16Mma, 128, KEYS_SLOT>();
+  return e == hipSuccess ? configure_keys<F16Mma, 64, KEYS_SLOT>() : e;
+}
 #endif
 
 }  // namespace we

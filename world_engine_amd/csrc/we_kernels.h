@@ -115,6 +115,9 @@ hipError_t launch_attn_ring_bf16_128(const AttnParams& p, int ksplit, hipStream_
 hipError_t launch_attn_ring_bf16_64(const AttnParams& p, int ksplit, hipStream_t stream);
 hipError_t launch_attn_ring_f16_128(const AttnParams& p, int ksplit, hipStream_t stream);
 hipError_t launch_attn_ring_f16_64(const AttnParams& p, int ksplit, hipStream_t stream);
+// frames below one 64-key tile
+hipError_t launch_attn_ring_short_bf16(const AttnParams& p, int Dh, int ksplit, hipStream_t stream);
+hipError_t launch_attn_ring_short_f16(const AttnParams& p, int Dh, int ksplit, hipStream_t stream);
 // fp32 caches: one pass on the fp32 matrix instructions, no context splitting
 hipError_t launch_attn_ring_f32(const AttnParams& p, int Dh, int cus, hipStream_t stream);
 hipError_t launch_attn_combine(const AttnParams& p, int Dh, int dtype, hipStream_t stream);
