@@ -164,9 +164,9 @@ int we_attn_plan(int32_t B, int32_t H, int32_t Hkv, int32_t T, int32_t Dh, int64
  *                        same sizes, n_splits and q_tile; may be NULL when that is 0.  Nothing in
  *                        it has to start at any value; calls that overlap in time need a
  *                        workspace each.
- *   n_splits             0 = choose automatically (small grids: every (batch, kv head) unit is
- *                        split so that most CUs have work; grids that leave a partial last round
- *                        of workgroups: only that round's units are split); 1 = single pass;
+ *   n_splits             0 = choose automatically (every (batch, kv head) unit in as many parts as
+ *                        fill the CUs' rounds best, or only the units of a partial last round);
+ *                        1 = single pass;
  *                        2..64 = split the visible context of every unit into that many parts.
  *                        Split parts are combined by a second kernel.
  *   q_tile               queries per workgroup: 0 = choose automatically, or 128 / 256.
@@ -194,7 +194,8 @@ int we_attn_ring_fwd(const void* q, const int64_t q_strides[3],
  * is part of the library's device image (every GPU the library runs on holds one copy until the
  * process ends; its address is looked up once per device by that device's set-up, see we_init:
  * under stream capture the device must have been set up beforehand).  Sizes whose
- * we_attn_workspace_bytes(...) exceeds WE_STATIC_SCRATCH_BYTES are
+ * we_attn_workspace_bytes(...) exceeds WE_STATIC_SCRATCH_BYTES run with fewer parts if there is a
+ * plan that fits (the results then differ from we_attn_ring_fwd's in the last bits), else they are
  * rejected with WE_ERR_SCRATCH_LIMIT and nothing is launched.  The call itself performs no
  * hipMalloc / hipFree and calls no allocating library routine.
  * All calls on one GPU share that GPU's buffer: calls that overlap in time on one GPU (different

@@ -42,7 +42,7 @@ inline int variant_of(int q_tile) {
   }
 }
 
-// Pick the kernel shape and the context splitting for a part with `cus` compute units (256 on an
+// The basic choice of kernel shape and context splitting for a part with `cus` compute units (256 on an
 // MI355X; every count below was measured there and is carried to other sizes as a fraction).
 //  * Shape: 256 queries per workgroup when that alone gives at least one workgroup per CU, else
 //    128 queries (two wavefronts share each query block and split every tile's keys).
@@ -52,7 +52,7 @@ inline int variant_of(int q_tile) {
 //    than two 64-key tiles per part.
 //  * Many workgroups that do not divide into whole rounds of CUs (e.g. 384 on 256): only the units
 //    of the last, partial round are split, so that round finishes in a fraction of the time.
-inline AttnPlan plan_attn(int B, int H, int Hkv, int T, int64_t L, int n_splits, int variant, int cus) {
+inline AttnPlan plan_basic(int B, int H, int Hkv, int T, int64_t L, int n_splits, int variant, int cus) {
   AttnPlan pl;
   if (cus < 8) cus = 8;
   pl.cus = cus;
@@ -113,17 +113,92 @@ inline AttnPlan plan_attn(int B, int H, int Hkv, int T, int64_t L, int n_splits,
   return pl;
 }
 
+// What a plan takes, us on an MI355X: every XCD works off its share of the (batch, kv head) unit parts
+// - a unit's workgroups all run on one - in rounds of a workgroup per CU; then the second pass over the
+// partial rows.  Per 64-key tile, per round and per call, with the partial rows' traffic at 3 to 5 TB/s;
+// fitted to 860 timings over 46 shapes (2 to 124 heads, 153 to 3600 tokens, 2 to 64 slots, both tile
+// sizes, 1 to 24 parts), which it meets to 3 to 7 %.
+inline double plan_cost(const AttnPlan& pl, int B, int H, int Hkv, int T, int Dh, int64_t L) {
+  struct Fit { double tile, round, call, comb, comb_mb; };
+  static constexpr Fit kFit[2][2] = {{{0.484, 3.94, 2.21, 2.79, 0.215}, {0.733, 3.01, 2.39, 3.39, 0.331}},
+                                     {{0.872, 2.64, 3.47, 2.61, 0.208}, {1.307, 1.67, 3.41, 3.57, 0.289}}};
+  const Fit& f = kFit[pl.variant == 2][Dh > 64];
+  const int64_t units = (int64_t)B * Hkv, members = (int64_t)(H / Hkv) * ((T + pl.block_m - 1) / pl.block_m);
+  const int64_t nt = (L + 63) / 64, per_xcd = pl.cus / 8 > 0 ? pl.cus / 8 : 1;
+  auto rounds = [&](int64_t parts) { return ((parts + 7) / 8 * members + per_xcd - 1) / per_xcd; };
+  const int64_t split_units = units - pl.units_whole;
+  double c = f.call;
+  if (pl.units_whole > 0) c += (double)rounds(pl.units_whole) * (f.tile * (double)nt + f.round);
+  c += (double)rounds(split_units * pl.n_splits) * (f.tile * (double)((nt + pl.n_splits - 1) / pl.n_splits) + f.round);
+  if (pl.n_splits > 1) c += f.comb + f.comb_mb * 2e-6 * (double)(pl.n_splits * pl.ws_rows) * (Dh * 2 + 16);
+  return c;
+}
+
+// The plan of a call: the basic choice, or the same number of parts for every unit at either tile size
+// where the cost above puts that 5 % lower - the basic rules know neither how units fall on the
+// XCDs (9 units are two rounds on one of them) nor that a context in three parts can fill two rounds of
+// CUs better than one part fills one (144 workgroups).  Against the best of the timings above the basic
+// choice was 11 % slower on average (up to 67 %), this one 2 %.  Frames of up to 256 tokens keep to one
+// round and ask for 15 %: there the parts' fixed costs are most of the time and the basic rules' finer
+// points decide.
+inline AttnPlan plan_attn(int B, int H, int Hkv, int T, int Dh, int64_t L, int n_splits, int variant, int cus) {
+  AttnPlan best = plan_basic(B, H, Hkv, T, L, n_splits, variant, cus);
+  if (n_splits > 0) return best;
+  const double basic = plan_cost(best, B, H, Hkv, T, Dh, L);
+  // (one pass instead of a split: no second launch, a saving the estimate is sure of)
+  double low = (T <= 256 ? 0.85 : 0.95) * basic, low_single = 0.97 * basic;
+  const int64_t nt = (L + 63) / 64;
+  for (int v = 1; v <= 2; ++v) {
+    if (variant != 0 && v != variant) continue;
+    if (v == 2 && T <= 128) continue;
+    const int block_m = v == 2 ? 256 : 128;
+    const int64_t wgs = (int64_t)B * H * ((T + block_m - 1) / block_m);
+    for (int s = 1; s <= 24 && (s == 1 || nt / s >= 2); ++s) {
+      if (s > 1 && wgs * s > (T <= 256 ? best.cus : 8 * (int64_t)best.cus)) break;
+      AttnPlan pl;
+      pl.variant = v; pl.block_m = block_m; pl.n_splits = s; pl.units_whole = 0; pl.cus = best.cus;
+      pl.ws_rows = s > 1 ? (int64_t)B * H * T : 0;
+      const double c = plan_cost(pl, B, H, Hkv, T, Dh, L);
+      if (c < (s == 1 ? low_single : low)) {
+        low_single = c;
+        low = c < low ? c : low;
+        best = pl;
+      }
+    }
+  }
+  return best;
+}
+
+// plan_attn for callers that ask again and again: a thread keeps its last plans (each layer and frame of
+// a model asks twice, and a plan is some fifty cost estimates).
+inline AttnPlan plan_cached(int B, int H, int Hkv, int T, int Dh, int64_t L, int n_splits, int variant, int cus) {
+  struct Entry { int64_t key[9]; AttnPlan plan; };
+  static thread_local Entry kept[16] = {};
+  const int64_t key[9] = {B, H, Hkv, T, Dh, L, n_splits, variant, cus};
+  uint64_t h = 0;
+  for (int64_t k : key) h = (h ^ (uint64_t)k) * 0x9e3779b97f4a7c15ull;
+  Entry& e = kept[h >> 60];
+  for (int i = 0; i < 9; ++i)
+    if (e.key[i] != key[i]) {
+      e.plan = plan_attn(B, H, Hkv, T, Dh, L, n_splits, variant, cus);
+      for (int j = 0; j < 9; ++j) e.key[j] = key[j];
+      break;
+    }
+  return e.plan;
+}
+
 inline size_t workspace_bytes_of(const AttnPlan& pl, int Dh) {
   if (pl.n_splits <= 1 || pl.ws_rows <= 0) return 0;
   return (size_t)pl.n_splits * (size_t)pl.ws_rows * ((size_t)Dh * 2 + 4 * sizeof(float));
 }
 
 // Validation of a we_attn_ring_fwd call, its plan and its kernel parameters.  `cus`: compute units
-// of the device the call will run on.
+// of the device the call will run on.  `workspace_limit`: a plan that needs more gives way to the basic one.
 inline int prepare_attn(const void* q, const int64_t* q_strides, const void* kv, const uint8_t* written,
                         const int64_t* t_pos, void* out, const int64_t* out_strides, void* workspace,
                         size_t workspace_bytes, int B, int H, int Hkv, int T, int Dh, int64_t L, int dilation,
-                        float scale, int n_splits, int q_tile, int dtype, int cus, AttnParams& p, AttnPlan& pl) {
+                        float scale, int n_splits, int q_tile, int dtype, int cus, AttnParams& p, AttnPlan& pl,
+                        size_t workspace_limit = SIZE_MAX) {
   if (!q || !q_strides || !kv || !written || !t_pos || !out || !out_strides) return WE_ERR_NULL_POINTER;
   int rc = ring_shape_ok(B, H, Hkv, T, Dh, L, dilation);
   if (rc != WE_OK) return rc;
@@ -142,7 +217,15 @@ inline int prepare_attn(const void* q, const int64_t* q_strides, const void* kv,
       !strides_ok(out_strides, dtype))
     return WE_ERR_ALIGNMENT;
 
-  pl = plan_attn(B, H, Hkv, T, L, n_splits, variant_of(q_tile), cus);
+  pl = plan_cached(B, H, Hkv, T, Dh, L, n_splits, variant_of(q_tile), cus);
+  if (dilation > 1 && n_splits == 0) {
+    // a dilated ring holds frames in one of `dilation` slots only; the sizing helpers do not know of it,
+    // so the plan for the keys there are is taken where it needs no more workspace
+    const AttnPlan short_ring = plan_cached(B, H, Hkv, T, Dh, L / dilation, 0, variant_of(q_tile), cus);
+    if (workspace_bytes_of(short_ring, Dh) <= workspace_bytes_of(pl, Dh)) pl = short_ring;
+  }
+  if (n_splits == 0 && workspace_bytes_of(pl, Dh) > workspace_limit)
+    pl = plan_basic(B, H, Hkv, T, L, 0, variant_of(q_tile), cus);
   const size_t ws_need = workspace_bytes_of(pl, Dh);
   if (ws_need > 0) {
     if (!workspace || !aligned16(workspace)) return WE_ERR_WORKSPACE;

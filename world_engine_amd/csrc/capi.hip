@@ -11,7 +11,7 @@ using we::host::aligned16;
 using we::host::AttnPlan;
 using we::host::DeviceState;
 using we::host::launch_attn;
-using we::host::plan_attn;
+using we::host::plan_cached;
 using we::host::ring_shape_ok;
 using we::host::strides_ok;
 using we::host::variant_of;
@@ -36,9 +36,9 @@ Dev dev_for(hipStream_t st) {
 int prepare_attn(const DeviceState& ds, const void* q, const int64_t* q_strides, const void* kv, const uint8_t* written,
                  const int64_t* t_pos, void* out, const int64_t* out_strides, void* workspace, size_t workspace_bytes,
                  int B, int H, int Hkv, int T, int Dh, int64_t L, int dilation, float scale, int n_splits, int q_tile,
-                 int dtype, we::AttnParams& p, AttnPlan& pl) {
+                 int dtype, we::AttnParams& p, AttnPlan& pl, size_t workspace_limit = SIZE_MAX) {
   return we::host::prepare_attn(q, q_strides, kv, written, t_pos, out, out_strides, workspace, workspace_bytes, B, H,
-                                Hkv, T, Dh, L, dilation, scale, n_splits, q_tile, dtype, ds.cus, p, pl);
+                                Hkv, T, Dh, L, dilation, scale, n_splits, q_tile, dtype, ds.cus, p, pl, workspace_limit);
 }
 
 // Validation of a we_rope_kv_store call and its kernel parameters.
@@ -298,9 +298,8 @@ int we_rope_apply_checked(const void* x, const int64_t x_strides[3], void* x_out
 int we_init(void) { return we::host::init_current_device(); }
 
 int32_t we_attn_auto_splits(int32_t B, int32_t H, int32_t Hkv, int32_t T, int32_t Dh, int64_t L) {
-  (void)Dh;
-  if (B <= 0 || H <= 0 || Hkv <= 0 || H % Hkv != 0 || T <= 0 || L <= 0) return 1;
-  return plan_attn(B, H, Hkv, T, L, 0, 0, we::host::compute_units()).n_splits;
+  if (B <= 0 || H <= 0 || Hkv <= 0 || H % Hkv != 0 || T <= 0 || Dh <= 0 || L <= 0) return 1;
+  return plan_cached(B, H, Hkv, T, Dh, L, 0, 0, we::host::compute_units()).n_splits;
 }
 
 size_t we_attn_workspace_bytes(int32_t B, int32_t H, int32_t Hkv, int32_t T, int32_t Dh, int64_t L,
@@ -308,7 +307,7 @@ size_t we_attn_workspace_bytes(int32_t B, int32_t H, int32_t Hkv, int32_t T, int
   if (B <= 0 || H <= 0 || Hkv <= 0 || H % Hkv != 0 || T <= 0 || Dh <= 0 || L <= 0 || n_splits < 0) return 0;
   const int variant = variant_of(q_tile);
   if (variant < 0) return 0;
-  return workspace_bytes_of(plan_attn(B, H, Hkv, T, L, n_splits, variant, we::host::compute_units()), Dh);
+  return workspace_bytes_of(plan_cached(B, H, Hkv, T, Dh, L, n_splits, variant, we::host::compute_units()), Dh);
 }
 
 int we_attn_plan(int32_t B, int32_t H, int32_t Hkv, int32_t T, int32_t Dh, int64_t L, int32_t n_splits,
@@ -320,7 +319,7 @@ int we_attn_plan(int32_t B, int32_t H, int32_t Hkv, int32_t T, int32_t Dh, int64
   const int variant = variant_of(q_tile);
   if (variant < 0) return WE_ERR_UNSUPPORTED;
   const int cus = compute_units > 0 ? compute_units : we::host::compute_units();
-  const AttnPlan pl = plan_attn(B, H, Hkv, T, L, n_splits, variant, cus);
+  const AttnPlan pl = plan_cached(B, H, Hkv, T, Dh, L, n_splits, variant, cus);
   const int q_tiles = (T + pl.block_m - 1) / pl.block_m;
   const int64_t wgs = (int64_t)q_tiles * (H / Hkv) * (pl.units_whole + (int64_t)(B * Hkv - pl.units_whole) * pl.n_splits);
   plan[0] = pl.block_m;
@@ -352,7 +351,9 @@ int we_attn_ring_fwd_static(const void* q, const int64_t q_strides[3], const voi
                             int32_t Hkv, int32_t T, int32_t Dh, int64_t L, int32_t dilation, float scale,
                             int32_t n_splits, int32_t q_tile, int32_t dtype, void* stream) {
   // sizes first, so that a call that cannot fit is refused before anything else happens
-  if (we_attn_workspace_bytes(B, H, Hkv, T, Dh, L, n_splits, q_tile) > WE_STATIC_SCRATCH_BYTES && dtype != WE_DTYPE_F32)
+  // (without a given number of parts the basic plan stands in for one that needs too much)
+  if (we_attn_workspace_bytes(B, H, Hkv, T, Dh, L, n_splits, q_tile) > WE_STATIC_SCRATCH_BYTES && dtype != WE_DTYPE_F32 &&
+      (n_splits != 0 || workspace_bytes_of(we::host::plan_basic(B, H, Hkv, T, L, 0, variant_of(q_tile), we::host::compute_units()), Dh) > WE_STATIC_SCRATCH_BYTES))
     return WE_ERR_SCRATCH_LIMIT;
   hipStream_t st = static_cast<hipStream_t>(stream);
   const Dev dev = dev_for(st);
@@ -361,7 +362,8 @@ int we_attn_ring_fwd_static(const void* q, const int64_t q_strides[3], const voi
   we::AttnParams p;
   AttnPlan pl;
   const int rc = prepare_attn(dev.state, q, q_strides, kv, written, t_pos, out, out_strides, ws,
-                              WE_STATIC_SCRATCH_BYTES, B, H, Hkv, T, Dh, L, dilation, scale, n_splits, q_tile, dtype, p, pl);
+                              WE_STATIC_SCRATCH_BYTES, B, H, Hkv, T, Dh, L, dilation, scale, n_splits, q_tile, dtype, p, pl,
+                              WE_STATIC_SCRATCH_BYTES);
   if (rc != WE_OK) return rc;
   if (dev.rc != WE_OK) return dev.rc;
   return launch_attn(p, pl, Dh, dtype, st);
