@@ -248,13 +248,19 @@ __device__ __forceinline__ void report_verdict(const StoreParams& p, bool bad) {
   __hip_atomic_store(p.report, (p.ticket << 1) | (bad ? 1u : 0u), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
-// Whether the call's position ids were refused: uniform over the workgroup, which must reach this
-// as a whole.  Without a verdict from the check kernel every workgroup looks at all ids itself (so
-// that none of them writes a row of a refused frame) and the first one reports.
-__device__ __forceinline__ bool frame_refused(const StoreParams& p) {
-  if (p.guard != nullptr) return *p.guard != 0u;
+// Whether the call's position ids were refused: uniform over the workgroup, which must reach both
+// halves as a whole.  Without a verdict from the check kernel every workgroup looks at all ids itself
+// (so that none of them writes a row of a refused frame) and the first one reports.  The first half
+// requests the ids, ahead of everything else of the call (loads return in order, and the host waits
+// for the report); the second has the verdict.
+__device__ __forceinline__ bool own_ids_bad(const StoreParams& p) {
+  if (p.guard != nullptr) return false;
   bool bad = false;
   for (int i = threadIdx.x; i < p.B * p.T; i += blockDim.x) bad = pos_id_bad(p, i) | bad;
+  return bad;
+}
+__device__ __forceinline__ bool frame_refused(const StoreParams& p, bool bad) {
+  if (p.guard != nullptr) return *p.guard != 0u;
   bad = __syncthreads_or(bad) != 0;
   if (threadIdx.x == 0 && blockIdx.x == 0 && blockIdx.y == 0 && blockIdx.z == 0) report_verdict(p, bad);
   return bad;

@@ -34,6 +34,7 @@ __global__ void __launch_bounds__(256) rope_kv_store_kernel(StoreParams p) {
   const int which = head_all < hq ? 0 : (head_all < hq + hkv ? 1 : 2);
   const int h = head_all - (which == 0 ? 0 : (which == 1 ? hq : hq + hkv));
 
+  const bool bad = CHECK && own_ids_bad(p);
   const int64_t frame_t = p.t_pos[0];
   Chunk16<Tag> in;
   ItemSide<Tag> sd;
@@ -44,8 +45,8 @@ __global__ void __launch_bounds__(256) rope_kv_store_kernel(StoreParams p) {
     load16<Tag>(in, src + chunk * 16);
     load_item_side<Tag>(p, which, b, h, t, chunk, sd);
   }
-  // (the row data and the table rows are on their way while the ids are looked at)
-  if ((CHECK && frame_refused(p)) || !live) return;
+  if (CHECK && frame_refused(p, bad)) return;
+  if (!live) return;
   if (which == 0) {  // rotate (or copy when there is no table) into the contiguous output
     finish_q_chunk<Tag>(p, b, h, t, chunk, in, sd.rotate, sd.c, sd.s);
   } else {
