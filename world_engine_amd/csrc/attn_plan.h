@@ -134,7 +134,7 @@ inline double plan_cost(const AttnPlan& pl, int B, int H, int Hkv, int T, int Dh
   return c;
 }
 
-// The plan of a call: the basic choice, or the same number of parts for every unit at either tile size
+// The plan of a call: the basic choice, or parts for every unit or for the last ones at either tile size
 // where the cost above puts that 5 % lower - the basic rules know neither how units fall on the
 // XCDs (9 units are two rounds on one of them) nor that a context in three parts can fill two rounds of
 // CUs better than one part fills one (144 workgroups).  Against the best of the timings above the basic
@@ -153,17 +153,27 @@ inline AttnPlan plan_attn(int B, int H, int Hkv, int T, int Dh, int64_t L, int n
     if (v == 2 && T <= 128) continue;
     const int block_m = v == 2 ? 256 : 128;
     const int64_t wgs = (int64_t)B * H * ((T + block_m - 1) / block_m);
-    for (int s = 1; s <= 24 && (s == 1 || nt / s >= 2); ++s) {
-      if (s > 1 && wgs * s > (T <= 256 ? best.cus : 8 * (int64_t)best.cus)) break;
+    auto consider = [&](int whole, int s) {
       AttnPlan pl;
-      pl.variant = v; pl.block_m = block_m; pl.n_splits = s; pl.units_whole = 0; pl.cus = best.cus;
-      pl.ws_rows = s > 1 ? (int64_t)B * H * T : 0;
+      pl.variant = v; pl.block_m = block_m; pl.n_splits = s; pl.units_whole = whole; pl.cus = best.cus;
+      pl.ws_rows = s > 1 ? ((int64_t)B * Hkv - whole) * (H / Hkv) * T : 0;
       const double c = plan_cost(pl, B, H, Hkv, T, Dh, L);
       if (c < (s == 1 ? low_single : low)) {
         low_single = c;
         low = c < low ? c : low;
         best = pl;
       }
+    };
+    for (int s = 1; s <= 24 && (s == 1 || nt / s >= 2); ++s) {
+      if (s > 1 && wgs * s > (T <= 256 ? best.cus : 8 * (int64_t)best.cus)) break;
+      consider(0, s);
+    }
+    // or only the units behind the last whole round (of every XCD) in parts: fewer partial rows
+    const int64_t members = (int64_t)(H / Hkv) * ((T + block_m - 1) / block_m), per_xcd = best.cus / 8;
+    for (int r = 1; r <= 3 && T > 256 && members <= r * per_xcd; ++r) {
+      const int64_t whole = r * per_xcd / members * 8;
+      if (whole >= (int64_t)B * Hkv) break;
+      for (int s = 2; s <= 8 && nt / s >= 4; ++s) consider((int)whole, s);
     }
   }
   return best;
