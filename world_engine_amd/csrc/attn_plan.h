@@ -145,8 +145,8 @@ inline AttnPlan plan_attn(int B, int H, int Hkv, int T, int Dh, int64_t L, int n
   AttnPlan best = plan_basic(B, H, Hkv, T, L, n_splits, variant, cus);
   if (n_splits > 0) return best;
   const double basic = plan_cost(best, B, H, Hkv, T, Dh, L);
-  // (one pass instead of a split: no second launch, a saving the estimate is sure of)
-  double low = (T <= 256 ? 0.85 : 0.95) * basic, low_single = 0.97 * basic;
+  // (one pass where every unit was split: no second launch, a saving the estimate is sure of)
+  double low = (T <= 256 ? 0.85 : 0.95) * basic, low_single = best.units_whole == 0 ? 0.97 * basic : low;
   const int64_t nt = (L + 63) / 64;
   for (int v = 1; v <= 2; ++v) {
     if (variant != 0 && v != variant) continue;
