@@ -62,3 +62,28 @@ def test_plans_over_several_rounds_and_the_static_scratch(gpu_device):
         out = torch.full_like(q, float("nan"))
         ops.attn_ring_static(q, kv, written, t_pos, n * T, d, out)
         assert (out.float() - one).abs().max().item() <= 2e-3
+
+
+@pytest.mark.parametrize("group,T,kw", [(2, 129, {}), (3, 143, {"q_tile": 128}), (4, 180, {"q_tile": 256}), (3, 255, {"n_splits": 3}),
+                                        (5, 257, {"q_tile": 256, "n_splits": 2}), (4, 96, {}), (4, 192, {}), (3, 320, {"q_tile": 128, "n_splits": 2})])
+def test_grouped_heads_share_query_tiles(gpu_device, group, T, kw):
+    """Query rows of a group's heads count through the tiles: rotated q (one stride through all heads) and strided
+    projection views, a gate per (head, token), tiles that hold the end of one head and the start of the next."""
+    print(f"grouped {group} T={T} {kw}", flush=True)
+    B, Hkv, Dh, n = 2, 8, 128, 3
+    H = group * Hkv
+    p = Pair(gpu_device, torch.bfloat16, B=B, H=H, Hkv=Hkv, T=T, Dh=Dh, n_slots=n, cfg_id=94)
+    g = torch.Generator(gpu_device).manual_seed(T)
+    for t in range(n + 1):
+        q, k, v, pos = p.inputs(t)
+        (q_o, k_all, v_all, mask), (q_h, ring) = p.store(q, k, v, pos)
+        ref = ro.attention_fp32(q_o, k_all, v_all, mask)
+        assert_attn_close(p.attend(q_h, ring, **kw), ref, f"t={t}")
+        strided = q_h.transpose(1, 2).contiguous().transpose(1, 2)          # [B, T, H, Dh] memory
+        assert_attn_close(p.attend(strided, ring, **kw), ref, f"t={t}, strided q")
+    gate = torch.rand(B, H, T, device=gpu_device, generator=g).bfloat16()
+    args = [x.to(gpu_device) for x in (q, k, v)] + [{n: i.to(gpu_device) for n, i in pos.items()}, p.rope.cos, p.rope.sin,
+                                                    p.rope.height, p.rope.width, ring.kv, ring.written, ring.L, 1, True]
+    plain, _ = ops.rope_kv_attn(*args, **kw)
+    gated, _ = ops.rope_kv_attn(*args, **kw, gate=gate)
+    assert (gated.float() - plain.float() * gate.float().unsqueeze(-1)).abs().max().item() <= 2e-2

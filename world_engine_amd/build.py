@@ -14,7 +14,7 @@ CSRC = os.path.join(HERE, "csrc")
 OBJ_DIR = os.path.join(HERE, "_obj")
 # (source, extra defines, object name)
 _RING = [("attn_ring.hip", [f"-DWE_RING_PART={i}"], f"attn_ring_{name}.o")
-         for i, name in enumerate(("bf16_128", "bf16_64", "f16_128", "f16_64", "short_bf16", "short_f16"))]
+         for i, name in enumerate(("bf16_128", "bf16_64", "f16_128", "f16_64", "short_bf16", "short_f16", "shared_bf16", "shared_f16"))]
 _SHARED = [("rope_kv_store.hip", [], "rope_kv_store.o"),
            ("qkv_proj_store.hip", [], "qkv_proj_store.o"),
            ("linear_skinny.hip", [], "linear_skinny.o"),

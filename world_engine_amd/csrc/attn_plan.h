@@ -42,6 +42,20 @@ inline int variant_of(int q_tile) {
   }
 }
 
+// Workgroups of a (batch, kv head) unit, which share its K/V stream: the query tiles of its heads.  The heads of
+// a group fill the tiles together where that saves one (3 heads of 143 queries: four tiles of 128 where each by
+// itself takes two) and tiles are what takes the time: not in frames of up to 128 tokens, nor in calls whose rows
+// fill less than a quarter of the CUs with tiles of 128, from 257 tokens an eighth.  (28 heads of 64 on 7, 374
+// tokens, 16 slots 32.8 -> 29.3 us; 24 of 128 on 12, 180 tokens, batch 2 28.0 -> 23.8; 60 on 15, 308 tokens,
+// batch 2 69.0 -> 59.  16 on 4, 192 tokens would be 18.1 -> 18.6, 6 on 2, 320 tokens 11.4 -> 11.9.)
+inline int64_t members_of(int units, int group, int T, int block_m, int cus, bool* shared = nullptr) {
+  const int64_t apart = group * (((int64_t)T + block_m - 1) / block_m);
+  const int64_t together = ((int64_t)group * T + block_m - 1) / block_m;
+  const bool share = together < apart && T > 128 && (int64_t)units * group * T >= (int64_t)cus * (T > 256 ? 16 : 32);
+  if (shared != nullptr) *shared = share;
+  return share ? together : apart;
+}
+
 // The basic choice of kernel shape and context splitting for a part with `cus` compute units (256 on an
 // MI355X; every count below was measured there and is carried to other sizes as a fraction).
 //  * Shape: 256 queries per workgroup when that alone gives at least one workgroup per CU, else
@@ -56,8 +70,8 @@ inline AttnPlan plan_basic(int B, int H, int Hkv, int T, int64_t L, int n_splits
   AttnPlan pl;
   if (cus < 8) cus = 8;
   pl.cus = cus;
-  const int64_t wg256 = (int64_t)B * H * ((T + 255) / 256);
-  const int64_t wg128 = (int64_t)B * H * ((T + 127) / 128);
+  const int64_t wg256 = (int64_t)B * Hkv * members_of(B * Hkv, H / Hkv, T, 256, cus);
+  const int64_t wg128 = (int64_t)B * Hkv * members_of(B * Hkv, H / Hkv, T, 128, cus);
   // 256 queries per workgroup when that alone fills the CUs - or when 128 would spill into a
   // second round that 256 avoids (136 to 256 heads of a 256-token frame: one round of fat
   // workgroups beats one and a bit rounds of thin ones by 5 to 17 %)
@@ -65,8 +79,7 @@ inline AttnPlan plan_basic(int B, int H, int Hkv, int T, int64_t L, int n_splits
   pl.block_m = pl.variant == 2 ? 256 : 128;
   const int units = B * Hkv;
   const int group = H / Hkv;
-  const int q_tiles = (T + pl.block_m - 1) / pl.block_m;
-  const int members = group * q_tiles;
+  const int members = (int)members_of(units, group, T, pl.block_m, cus);
   const int64_t wgs = (int64_t)units * members;
   const int64_t tiles = L / 64;  // visible 64-key tiles at steady state
   const int64_t max_s = tiles / 2 > 0 ? tiles / 2 : 1;
@@ -123,7 +136,7 @@ inline double plan_cost(const AttnPlan& pl, int B, int H, int Hkv, int T, int Dh
   static constexpr Fit kFit[2][2] = {{{0.484, 3.94, 2.21, 2.79, 0.215}, {0.733, 3.01, 2.39, 3.39, 0.331}},
                                      {{0.872, 2.64, 3.47, 2.61, 0.208}, {1.307, 1.67, 3.41, 3.57, 0.289}}};
   const Fit& f = kFit[pl.variant == 2][Dh > 64];
-  const int64_t units = (int64_t)B * Hkv, members = (int64_t)(H / Hkv) * ((T + pl.block_m - 1) / pl.block_m);
+  const int64_t units = (int64_t)B * Hkv, members = members_of((int)units, H / Hkv, T, pl.block_m, pl.cus);
   const int64_t nt = (L + 63) / 64, per_xcd = pl.cus / 8 > 0 ? pl.cus / 8 : 1;
   auto rounds = [&](int64_t parts) { return ((parts + 7) / 8 * members + per_xcd - 1) / per_xcd; };
   const int64_t split_units = units - pl.units_whole;
@@ -152,7 +165,7 @@ inline AttnPlan plan_attn(int B, int H, int Hkv, int T, int Dh, int64_t L, int n
     if (variant != 0 && v != variant) continue;
     if (v == 2 && T <= 128) continue;
     const int block_m = v == 2 ? 256 : 128;
-    const int64_t wgs = (int64_t)B * H * ((T + block_m - 1) / block_m);
+    const int64_t members = members_of(B * Hkv, H / Hkv, T, block_m, best.cus), wgs = (int64_t)B * Hkv * members, per_xcd = best.cus / 8;
     auto consider = [&](int whole, int s) {
       AttnPlan pl;
       pl.variant = v; pl.block_m = block_m; pl.n_splits = s; pl.units_whole = whole; pl.cus = best.cus;
@@ -169,7 +182,6 @@ inline AttnPlan plan_attn(int B, int H, int Hkv, int T, int Dh, int64_t L, int n
       consider(0, s);
     }
     // or only the units behind the last whole round (of every XCD) in parts: fewer partial rows
-    const int64_t members = (int64_t)(H / Hkv) * ((T + block_m - 1) / block_m), per_xcd = best.cus / 8;
     for (int r = 1; r <= 3 && T > 256 && members <= r * per_xcd; ++r) {
       const int64_t whole = r * per_xcd / members * 8;
       if (whole >= (int64_t)B * Hkv) break;
@@ -253,17 +265,20 @@ inline int prepare_attn(const void* q, const int64_t* q_strides, const void* kv,
   p.n_splits = pl.n_splits;
   p.units_whole = pl.units_whole;
   p.ws_row0 = (int64_t)B * H * T - pl.ws_rows;
-  p.q_tiles = (T + pl.block_m - 1) / pl.block_m;
   p.group = H / Hkv;
-  p.members = p.group * p.q_tiles;
+  bool shared = false;
+  p.members = (int)members_of(B * Hkv, p.group, T, pl.block_m, pl.cus, &shared);
+  p.q_heads = shared ? 1 : p.group;
   p.unit_splits = pl.units_whole + (B * Hkv - pl.units_whole) * pl.n_splits;
   p.scale_log2 = scale * 1.4426950408889634f;
   p.gate = nullptr; p.gs_b = p.gs_h = p.gs_t = 0;
   p.gate_x = nullptr; p.gate_w = nullptr; p.gx_b = p.gx_t = 0;
   p.clock_out = nullptr;
-  p.q_dma = (q_strides[2] > 0 && (uint64_t)T * (uint64_t)q_strides[2] * 2u < (1ull << 31)) ? 1 : 0;
+  // the Q tile by DMA: 32-bit row offsets, and rows one stride apart throughout the tile
+  p.q_dma = (q_strides[2] > 0 && (uint64_t)T * (shared ? p.group : 1) * (uint64_t)q_strides[2] * 2u < (1ull << 31) &&
+             (!shared || q_strides[1] == (int64_t)T * q_strides[2])) ? 1 : 0;
 
-  if ((p.unit_splits + 7) / 8 > 65535 || p.group > 65535 || (int64_t)B * H - (int64_t)pl.units_whole * p.group > 65535)
+  if ((p.unit_splits + 7) / 8 > 65535 || p.q_heads > 65535 || 8ll * p.members > 0x7fffffff || (int64_t)B * H - (int64_t)pl.units_whole * p.group > 65535)
     return WE_ERR_UNSUPPORTED;  // grid y / z limits of the two launches
   return WE_OK;
 }
@@ -274,6 +289,7 @@ inline int launch_attn(const AttnParams& p, const AttnPlan& pl, int Dh, int dtyp
   const int ksplit = pl.variant == 1 ? 2 : 1;
   hipError_t e;
   if (p.T < 64) e = dtype == WE_DTYPE_BF16 ? launch_attn_ring_short_bf16(p, Dh, ksplit, st) : launch_attn_ring_short_f16(p, Dh, ksplit, st);
+  else if (p.q_heads != p.group) e = dtype == WE_DTYPE_BF16 ? launch_attn_ring_shared_bf16(p, Dh, ksplit, st) : launch_attn_ring_shared_f16(p, Dh, ksplit, st);
   else if (dtype == WE_DTYPE_BF16) e = Dh == 128 ? launch_attn_ring_bf16_128(p, ksplit, st) : launch_attn_ring_bf16_64(p, ksplit, st);
   else e = Dh == 128 ? launch_attn_ring_f16_128(p, ksplit, st) : launch_attn_ring_f16_64(p, ksplit, st);
   if (e != hipSuccess) return WE_ERR_LAUNCH;

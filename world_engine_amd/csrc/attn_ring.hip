@@ -34,7 +34,7 @@
 // (batch, kv head) units are context-split (see the planner in attn_plan.h); split workgroups leave
 // normalised partial outputs that a second kernel merges (attn_combine.hip).
 //
-// The grid is 3-D (8 * query tiles, query heads per kv head, rounds of 8 units): no division by
+// The grid is 3-D (8 * query tiles, heads with tiles of their own, rounds of 8 units): no division by
 // run-time values is needed to find a workgroup's unit, and blockIdx.x % 8 is the XCD it runs on,
 // so the workgroups that share one K/V stream share an L2.  Start-up code is kept short on purpose:
 // a 256-token frame runs 8 tiles per workgroup and start-up is a third of the kernel.
@@ -102,15 +102,27 @@ __device__ __forceinline__ u32x2_t lds_read_tr(const unsigned char* smem, uint32
   return __builtin_bit_cast(u32x2_t, v);
 }
 
+// The kernel's argument, read anew: what only the epilogue needs then takes no scalar registers through the
+// tile loop.  Short frames and shared query tiles need more of those than there are (70 moved to vector lanes
+// and back, 21 with this; 24 heads of 36 tokens, 64 slots: 18.1 -> 17.7 us).
+template <typename P>
+__device__ __forceinline__ const P& reread_args() {
+  uint64_t at = (uint64_t)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(at));
+  return *(const P*)(const __attribute__((address_space(4))) P*)at;
+}
+
 // How tiles are laid over the visible keys (a separate instantiation each: the ragged ones' few extra
 // instructions and registers are nothing the common case could spare).
 constexpr int KEYS_TILED = 0;   // T % 64 == 0: whole tiles of one slot
 constexpr int KEYS_PACKED = 1;  // T > 64: 64 consecutive visible keys, the last tile short
 constexpr int KEYS_SLOT = 2;    // T < 64: one slot, short
+constexpr int KEYS_SHARED = 3;  // as KEYS_PACKED, any T > 64, and grouped heads share query tiles
 // CLOCKED: measurement library only - every workgroup reports its duration (p.clock_out).
 template <typename M, int DH, int KSPLIT, int KEYS, bool CLOCKED>
 __global__ void __attribute__((amdgpu_flat_work_group_size(512, 512), amdgpu_waves_per_eu(2, 2)))
 attn_ring_kernel(AttnParams p) {
+  constexpr bool SHARED = KEYS == KEYS_SHARED, RUN = KEYS == KEYS_PACKED || SHARED;
   typedef typename M::frag_t frag_t;
   typedef RingLds<DH> L;
   constexpr int KS = DH / 16;               // contraction steps of K Q^T
@@ -148,7 +160,7 @@ attn_ring_kernel(AttnParams p) {
   uint8_t flag = lane < p.n_slots ? p.written[(int64_t)lane * p.T] : (uint8_t)0;
 
   // ---- which (batch, head, query tile, split) this workgroup owns ----
-  // The grid is (8 * query tiles, query heads per kv head, rounds): workgroups are dispatched
+  // The grid is (8 * query tiles, heads with tiles of their own, rounds): workgroups are dispatched
   // to XCDs round-robin in linear order, so XCD = blockIdx.x % 8, and the workgroups that share
   // one K/V stream (the x * y of one round) all land on the same XCD and its L2.
   const int xcd = blockIdx.x & 7, qtile = blockIdx.x >> 3, hq_in = blockIdx.y;
@@ -165,7 +177,11 @@ attn_ring_kernel(AttnParams p) {
     unit = p.units_whole + r / p.n_splits; split = r % p.n_splits; nsp = p.n_splits;
   }
   const int b = unit / p.Hkv, hkv = unit - b * p.Hkv;
-  const int h = hkv * p.group + hq_in;
+  // Query rows of this workgroup's heads.  Where grouped heads share tiles the rows count
+  // through all of them: row r is token r % T of head r / T of the group.  Rows past the last token are
+  // computed and not stored.
+  const int row0 = qtile * BM;
+  const int h0 = hkv * p.group + hq_in;
 
   // ---- raw Q fragments ----
   // A lane's fragment loads touch 32 rows x 32 bytes each: 512 small requests per wavefront, which
@@ -177,23 +193,25 @@ attn_ring_kernel(AttnParams p) {
   constexpr int Q_OFF = L::V_OFF + 2 * TILE_B;
   const bool q_dma = KSPLIT == 2 && p.q_dma != 0;
   frag_t qf[KS];
-  const int qrow = qtile * BM + qb * 32 + l32;
+  const unsigned qrow = (unsigned)(row0 + qb * 32 + l32);
   if (!q_dma) {
-    const uint16_t* qbase = reinterpret_cast<const uint16_t*>(p.q) + b * p.qs_b + h * p.qs_h;
-    const int qr = qrow < p.T ? qrow : p.T - 1;
-    const uint16_t* src = qbase + (int64_t)qr * p.qs_t + hh * 8;
+    int hq = SHARED ? (int)(qrow / (unsigned)p.T) : 0, qr = (int)qrow - hq * p.T;
+    if (SHARED && hq >= p.group) { hq = p.group - 1; qr = p.T - 1; }
+    qr = qr < p.T ? qr : p.T - 1;
+    const uint16_t* src = reinterpret_cast<const uint16_t*>(p.q) + b * p.qs_b + (h0 + hq) * p.qs_h + (int64_t)qr * p.qs_t + hh * 8;
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) qf[ks] = *reinterpret_cast<const frag_t*>(src + ks * 16);
   }
   if (us_raw >= p.unit_splits) return;
   if (KSPLIT == 2 && q_dma) {
-    const uint64_t qplane = uniform64((uint64_t)(uintptr_t)p.q + (uint64_t)(((int64_t)b * p.qs_b + (int64_t)h * p.qs_h) * 2));
+    const int limit = SHARED ? p.group * p.T : p.T;
+    const uint64_t qplane = uniform64((uint64_t)(uintptr_t)p.q + (uint64_t)(((int64_t)b * p.qs_b + (int64_t)h0 * p.qs_h) * 2));
     const uint32_t q_lds = (uint32_t)__builtin_amdgcn_readfirstlane((int)(lds0 + Q_OFF + wave * 1024));
 #pragma unroll
     for (int i = 0; i < 2 * NDMA; ++i) {
       const int row = (wave + i * 8) * RPI + lane / CPR;   // row of the 128-query tile
-      int qr = qtile * BM + row;
-      qr = qr < p.T ? qr : p.T - 1;
+      int qr = row0 + row;
+      qr = qr < limit ? qr : limit - 1;
       dma16(qplane, (uint32_t)qr * (uint32_t)(p.qs_t * 2) + (uint32_t)(((lane % CPR) ^ k_swz<DH>(row)) << 4), q_lds + i * 8 * 1024);
     }
   }
@@ -219,8 +237,8 @@ attn_ring_kernel(AttnParams p) {
   stamp(0);  // slot list built
   // tiles of the visible keys; last_keys: keys of the last one
   const int tps = KEYS == KEYS_TILED ? p.T / BN : 1;
-  const int nt = KEYS == KEYS_PACKED ? (nvis * p.T + BN - 1) / BN : nvis * tps;
-  const int last_keys = nvis * p.T - (nt - 1) * BN;  // (KEYS_PACKED)
+  const int nt = RUN ? (nvis * p.T + BN - 1) / BN : nvis * tps;
+  const int last_keys = nvis * p.T - (nt - 1) * BN;  // (RUN)
   int t_begin = 0, t_end = nt;
   if (nsp > 1) {  // nt <= 257 * T / 64 and nsp <= 64: the products fit 32 bits
     t_begin = (int)((unsigned)split * (unsigned)nt / (unsigned)nsp);
@@ -228,7 +246,7 @@ attn_ring_kernel(AttnParams p) {
   }
   const int ntile = t_end - t_begin;
   // this split owns a short last tile (and takes it first)
-  const bool shorted = KEYS == KEYS_PACKED && t_end == nt && last_keys < BN && ntile > 0;
+  const bool shorted = RUN && t_end == nt && last_keys < BN && ntile > 0;
 
   const int64_t cap = p.L + p.T;
   const uint64_t kbase = (uint64_t)(uintptr_t)p.kv + (uint64_t)(((int64_t)b * p.Hkv + hkv) * cap) * ROW_B;
@@ -248,7 +266,7 @@ attn_ring_kernel(AttnParams p) {
   }
   // The split's visible tiles, 64 at a time: lane i of toff holds the byte offset, inside the
   // (batch, kv head) plane, of tile 64*k + i of the split (fits 32 bits, checked on the host).
-  // KEYS_PACKED: its low 7 bits (row starts are multiples of 128 bytes) hold the tile row at which
+  // RUN: its low 7 bits (row starts are multiples of 128 bytes) hold the tile row at which
   // the next slot begins (64: none does), tgap the bytes between the two slots.  The tile loop then
   // needs one v_readlane (two) per tile instead of walking slots and tiles with scalar code.
   // The workgroups that share this K/V stream (query tiles x grouped query heads) take the tiles
@@ -260,7 +278,7 @@ attn_ring_kernel(AttnParams p) {
   // keys does not matter to a softmax.
   int rot_g = 1;
   while (rot_g * 2 <= p.members && rot_g < 4) rot_g *= 2;
-  const unsigned rot_m = (unsigned)(qtile * p.group + hq_in) & (unsigned)(rot_g - 1);
+  const unsigned rot_m = (unsigned)(qtile * p.q_heads + hq_in) & (unsigned)(rot_g - 1);
   const unsigned rot_end = (unsigned)(ntile - (shorted ? 1 : 0)) & ~(unsigned)(rot_g - 1);
   uint32_t toff = 0, tgap = 0;
   struct TileAt { uint32_t off, gap; };
@@ -271,7 +289,7 @@ attn_ring_kernel(AttnParams p) {
     if (kk < rot_end) kk = (kk & ~(unsigned)(rot_g - 1)) | ((kk + rot_m) & (unsigned)(rot_g - 1));
     unsigned ti = (unsigned)t_begin + kk;
     if (head || ti > (unsigned)(t_end - 1)) ti = (unsigned)(t_end - 1);
-    if (KEYS == KEYS_PACKED) {
+    if (RUN) {
       const unsigned v0 = ti * BN, T = (unsigned)p.T;
       const unsigned sidx = v0 / T, in = v0 - sidx * T;
       const unsigned brk = T - in < BN ? T - in : BN;
@@ -290,7 +308,7 @@ attn_ring_kernel(AttnParams p) {
     if ((kc & 63) == 0) load_offsets(kc);
     TileAt t;
     t.off = (uint32_t)__builtin_amdgcn_readlane((int)toff, kc & 63);
-    t.gap = KEYS == KEYS_PACKED ? (uint32_t)__builtin_amdgcn_readlane((int)tgap, kc & 63) : 0u;
+    t.gap = RUN ? (uint32_t)__builtin_amdgcn_readlane((int)tgap, kc & 63) : 0u;
     if (kc < ntile - 1) ++kc;
     return t;
   };
@@ -299,15 +317,15 @@ attn_ring_kernel(AttnParams p) {
   // the tile offset is uniform: it goes into the scalar base address, not into every lane's offset
   const int dma_row = wave * RPI + lane / CPR;  // tile row of this lane's first instruction
   auto dma_tile = [&](uint64_t plane, const uint32_t(&voff)[NDMA], TileAt t, uint32_t lds) __attribute__((always_inline)) {
-    const uint64_t base = plane + (KEYS == KEYS_PACKED ? t.off & ~127u : t.off);
+    const uint64_t base = plane + (RUN ? t.off & ~127u : t.off);
     const int brk = (int)(t.off & 127u);
 #pragma unroll
     for (int i = 0; i < NDMA; ++i)
-      dma16(base, KEYS == KEYS_PACKED && dma_row >= brk - i * 8 * RPI ? voff[i] + t.gap : voff[i], lds + i * 8 * 1024);
+      dma16(base, RUN && dma_row >= brk - i * 8 * RPI ? voff[i] + t.gap : voff[i], lds + i * 8 * 1024);
   };
   // the split's first tile: rows past the keys of a short one repeat its last
   auto dma_tile0 = [&](uint64_t plane, const uint32_t(&voff)[NDMA], TileAt t, uint32_t lds) __attribute__((always_inline)) {
-    if (KEYS != KEYS_PACKED || !shorted) { dma_tile(plane, voff, t, lds); return; }
+    if (!RUN || !shorted) { dma_tile(plane, voff, t, lds); return; }
     const uint64_t base = plane + (t.off & ~127u);
     const int brk = (int)(t.off & 127u);
 #pragma unroll
@@ -627,7 +645,7 @@ attn_ring_kernel(AttnParams p) {
         // block (j, 0) -> probabilities; logits of (j, 1); product of (j-1, 1)
         step(IntC<JM * TILE_B + KB_B>(), IntC<((JM + 3) % NST) * TILE_B + KB_B>(),
              IntC<((JM + 1) % NST) * TILE_B>(), IntC<JM * TILE_B>(),
-             std::integral_constant<bool, KEYS == KEYS_SLOT || (KEYS == KEYS_PACKED && FIRST)>(), block_keys(1), issue_dma,
+             std::integral_constant<bool, KEYS == KEYS_SLOT || (RUN && FIRST)>(), block_keys(1), issue_dma,
              std::false_type());
         // block (j, 1) -> probabilities; logits of (j+1, 0); product of (j, 0)
         step(IntC<((JM + 1) % NST) * TILE_B>(), IntC<JM * TILE_B>(),
@@ -651,7 +669,7 @@ attn_ring_kernel(AttnParams p) {
 
     int j = 0;
     const std::false_type not_first;
-    if (KSPLIT == 2 || KEYS == KEYS_PACKED) {
+    if (KSPLIT == 2 || RUN) {
       // the first tile's step has no product to do (128 queries) or may have keys to mask: peeled,
       // with the three iterations that bring the ring position back to zero
       iteration(0, IntC<0>(), std::true_type());
@@ -736,13 +754,16 @@ attn_ring_kernel(AttnParams p) {
 
   stamp(3);  // pair merged
   // ---- epilogue ----
-  const int64_t rows = (int64_t)p.B * p.H * p.T - p.ws_row0;  // rows in the workspace
-  const bool valid = qrow < p.T;
+  const AttnParams& ep = KEYS != KEYS_SLOT && !SHARED ? p : reread_args<AttnParams>();
+  const int64_t rows = (int64_t)ep.B * ep.H * ep.T - ep.ws_row0;  // rows in the workspace
+  const int hq = SHARED ? (int)(qrow / (unsigned)ep.T) : 0, qt = (int)qrow - hq * ep.T;
+  const int h = h0 + hq;
+  const bool valid = qt < ep.T && (!SHARED || hq < ep.group);
   const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
-  const int64_t row = ((int64_t)b * p.H + h) * p.T + qrow;
+  const int64_t row = ((int64_t)b * ep.H + h) * ep.T + qt;
   float gate_v = 1.f;
-  const bool gated = p.gate != nullptr || p.gate_w != nullptr;
-  if (gated && nsp == 1 && qrow < p.T) gate_v = head_gate<typename M::elem_t>(p, b, h, qrow);
+  const bool gated = ep.gate != nullptr || ep.gate_w != nullptr;
+  if (gated && nsp == 1 && valid) gate_v = head_gate<typename M::elem_t>(ep, b, h, qt);
   // A split leaves its partial output as fp16 values in [-1, 1] plus one fp32 scale per row (the
   // row's largest normalised magnitude): 11 significant bits whatever the element type, for the
   // bytes of a bf16 row, and no overflow for any finite V.  A row that holds an infinity keeps the
@@ -768,7 +789,7 @@ attn_ring_kernel(AttnParams p) {
       row_scale = 1.f;
     }
     if (valid && hh == 0)
-      *reinterpret_cast<f32x4_t*>(p.ws_ml + ((int64_t)split * rows + (row - p.ws_row0)) * 4) =
+      *reinterpret_cast<f32x4_t*>(ep.ws_ml + ((int64_t)split * rows + (row - ep.ws_row0)) * 4) =
           f32x4_t{l_tot > 0.f ? m_ref : -INFINITY, l_tot, row_scale, 0.f};
   }
 #pragma unroll
@@ -788,8 +809,8 @@ attn_ring_kernel(AttnParams p) {
       const int d0 = 32 * db + 8 * (c + hh);
       if (valid) {
         if (nsp == 1) {
-          uint16_t* dst = reinterpret_cast<uint16_t*>(p.out) + b * p.os_b + h * p.os_h +
-                          (int64_t)qrow * p.os_t + d0;
+          uint16_t* dst = reinterpret_cast<uint16_t*>(ep.out) + b * ep.os_b + h * ep.os_h +
+                          (int64_t)qt * ep.os_t + d0;
           frag_t y = M::pack8(f[0], f[1], f[2], f[3], f[4], f[5], f[6], f[7]);
           if (gated) {  // y * gate on element-type values, as the module's own multiply
             y = M::pack8((float)y[0] * gate_v, (float)y[1] * gate_v, (float)y[2] * gate_v, (float)y[3] * gate_v,
@@ -797,7 +818,7 @@ attn_ring_kernel(AttnParams p) {
           }
           *reinterpret_cast<frag_t*>(dst) = y;
         } else {
-          uint16_t* dst = p.ws_o + ((int64_t)split * rows + (row - p.ws_row0)) * DH + d0;
+          uint16_t* dst = ep.ws_o + ((int64_t)split * rows + (row - ep.ws_row0)) * DH + d0;
           *reinterpret_cast<f16x8_t*>(dst) = F16Mma::pack8(f[0], f[1], f[2], f[3], f[4], f[5], f[6], f[7]);
         }
       }
@@ -821,7 +842,7 @@ constexpr bool kWithProbes = false;
 template <typename M, int DH, int KSPLIT, int KEYS, bool CLOCKED>
 static hipError_t launch_ring_c(const AttnParams& p, hipStream_t stream) {
   const int rounds = (p.unit_splits + 7) / 8;
-  const dim3 grid((unsigned)(8 * p.q_tiles), (unsigned)p.group, (unsigned)rounds);
+  const dim3 grid((unsigned)(8 * (p.members / p.q_heads)), (unsigned)p.q_heads, (unsigned)rounds);
   hipLaunchKernelGGL((attn_ring_kernel<M, DH, KSPLIT, KEYS, CLOCKED>), grid, dim3(512), RingLds<DH>::kBytes, stream, p);
   return hipGetLastError();
 }
@@ -859,15 +880,21 @@ static hipError_t configure_family() {
   const hipError_t e = configure_keys<M, DH, KEYS_TILED>();
   return e == hipSuccess ? configure_keys<M, DH, KEYS_PACKED>() : e;
 }
-// frames below one tile
-template <typename M, int DH>
-static hipError_t launch_short(const AttnParams& p, int ksplit, hipStream_t stream) {
-  return ksplit == 2 ? launch_ring_r<M, DH, 2, KEYS_SLOT>(p, stream) : launch_ring_r<M, DH, 1, KEYS_SLOT>(p, stream);
+// frames below one tile, and grouped heads that share query tiles
+template <typename M, int KEYS>
+static hipError_t launch_keys(const AttnParams& p, int Dh, int ksplit, hipStream_t stream) {
+  if (Dh == 128) return ksplit == 2 ? launch_ring_r<M, 128, 2, KEYS>(p, stream) : launch_ring_r<M, 128, 1, KEYS>(p, stream);
+  return ksplit == 2 ? launch_ring_r<M, 64, 2, KEYS>(p, stream) : launch_ring_r<M, 64, 1, KEYS>(p, stream);
+}
+template <typename M, int KEYS>
+static hipError_t configure_both() {
+  const hipError_t e = configure_keys<M, 128, KEYS>();
+  return e == hipSuccess ? configure_keys<M, 64, KEYS>() : e;
 }
 
 // The four (element type, head dim) families are compiled as separate objects (WE_RING_PART selects
 // one; undefined = all of them in this translation unit) so that they build in parallel; the short
-// frames' instantiations are parts of their own.
+// frames' and the shared tiles' instantiations are parts of their own.
 #if !defined(WE_RING_PART) || WE_RING_PART == 0
 hipError_t launch_attn_ring_bf16_128(const AttnParams& p, int ksplit, hipStream_t stream) {
   return ksplit == 2 ? launch_ring_t<Bf16Mma, 128, 2>(p, stream) : launch_ring_t<Bf16Mma, 128, 1>(p, stream);
@@ -895,21 +922,27 @@ hipError_t configure_attn_ring_f16_64() { return configure_family<F16Mma, 64>();
 
 #if defined(WE_RING_PART) && WE_RING_PART == 4
 hipError_t launch_attn_ring_short_bf16(const AttnParams& p, int Dh, int ksplit, hipStream_t stream) {
-  return Dh == 128 ? launch_short<Bf16Mma, 128>(p, ksplit, stream) : launch_short<Bf16Mma, 64>(p, ksplit, stream);
+  return launch_keys<Bf16Mma, KEYS_SLOT>(p, Dh, ksplit, stream);
 }
-hipError_t configure_attn_ring_short_bf16() {
-  const hipError_t e = configure_keys<Bf16Mma, 128, KEYS_SLOT>();
-  return e == hipSuccess ? configure_keys<Bf16Mma, 64, KEYS_SLOT>() : e;
-}
+hipError_t configure_attn_ring_short_bf16() { return configure_both<Bf16Mma, KEYS_SLOT>(); }
 #endif
 #if defined(WE_RING_PART) && WE_RING_PART == 5
 hipError_t launch_attn_ring_short_f16(const AttnParams& p, int Dh, int ksplit, hipStream_t stream) {
-  return Dh == 128 ? launch_short<F16Mma, 128>(p, ksplit, stream) : launch_short<F16Mma, 64>(p, ksplit, stream);
+  return launch_keys<F16Mma, KEYS_SLOT>(p, Dh, ksplit, stream);
 }
-hipError_t configure_attn_ring_short_f16() {
-  const hipError_t e = configure_keys<F16Mma, 128, KEYS_SLOT>();
-  return e == hipSuccess ? configure_keys<F16Mma, 64, KEYS_SLOT>() : e;
+hipError_t configure_attn_ring_short_f16() { return configure_both<F16Mma, KEYS_SLOT>(); }
+#endif
+#if defined(WE_RING_PART) && WE_RING_PART == 6
+hipError_t launch_attn_ring_shared_bf16(const AttnParams& p, int Dh, int ksplit, hipStream_t stream) {
+  return launch_keys<Bf16Mma, KEYS_SHARED>(p, Dh, ksplit, stream);
 }
+hipError_t configure_attn_ring_shared_bf16() { return configure_both<Bf16Mma, KEYS_SHARED>(); }
+#endif
+#if defined(WE_RING_PART) && WE_RING_PART == 7
+hipError_t launch_attn_ring_shared_f16(const AttnParams& p, int Dh, int ksplit, hipStream_t stream) {
+  return launch_keys<F16Mma, KEYS_SHARED>(p, Dh, ksplit, stream);
+}
+hipError_t configure_attn_ring_shared_f16() { return configure_both<F16Mma, KEYS_SHARED>(); }
 #endif
 
 }  // namespace we

@@ -62,7 +62,7 @@ attn_ring_f32_kernel(AttnParams p) {
 
   // ---- which queries ----
   // (spread over the XCDs by unit where every XCD gets the same number: a unit's workgroups share an L2)
-  const int units = p.B * p.Hkv;
+  const int units = p.B * p.Hkv, q_tiles = (p.T + F_Q - 1) / F_Q;
   int unit, member;
   if ((units & 7) == 0) {
     const unsigned j = blockIdx.x >> 3;
@@ -74,8 +74,8 @@ attn_ring_f32_kernel(AttnParams p) {
     member = (int)(blockIdx.x - (unsigned)unit * (unsigned)p.members);
   }
   const int b = unit / p.Hkv, hkv = unit - b * p.Hkv;
-  const int hq_in = member / p.q_tiles, h = hkv * p.group + hq_in;
-  const int q0 = (member - hq_in * p.q_tiles) * F_Q;
+  const int hq_in = member / q_tiles, h = hkv * p.group + hq_in;
+  const int q0 = (member - hq_in * q_tiles) * F_Q;
 
   // ---- list of visible slots; the tail is pseudo-slot n_slots ----
   if (wave == 0) {
@@ -264,8 +264,7 @@ attn_ring_f32_kernel(AttnParams p) {
 
 template <int DH>
 static hipError_t launch_f32(AttnParams p, int cus, hipStream_t stream) {
-  p.q_tiles = (p.T + F_Q - 1) / F_Q;
-  p.members = p.group * p.q_tiles;
+  p.members = p.group * ((p.T + F_Q - 1) / F_Q);
   const int64_t wgs = (int64_t)p.B * p.Hkv * p.members;
   if (wgs > 0x7fffffff) return hipErrorInvalidValue;
   // eight wavefronts per workgroup (two per SIMD of a CU) while a CU gets one workgroup; two

@@ -320,8 +320,7 @@ int we_attn_plan(int32_t B, int32_t H, int32_t Hkv, int32_t T, int32_t Dh, int64
   if (variant < 0) return WE_ERR_UNSUPPORTED;
   const int cus = compute_units > 0 ? compute_units : we::host::compute_units();
   const AttnPlan pl = plan_cached(B, H, Hkv, T, Dh, L, n_splits, variant, cus);
-  const int q_tiles = (T + pl.block_m - 1) / pl.block_m;
-  const int64_t wgs = (int64_t)q_tiles * (H / Hkv) * (pl.units_whole + (int64_t)(B * Hkv - pl.units_whole) * pl.n_splits);
+  const int64_t wgs = we::host::members_of(B * Hkv, H / Hkv, T, pl.block_m, pl.cus) * (pl.units_whole + (int64_t)(B * Hkv - pl.units_whole) * pl.n_splits);
   plan[0] = pl.block_m;
   plan[1] = pl.n_splits;
   plan[2] = pl.units_whole;

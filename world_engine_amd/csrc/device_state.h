@@ -32,6 +32,8 @@ hipError_t configure_attn_ring_f16_128();
 hipError_t configure_attn_ring_f16_64();
 hipError_t configure_attn_ring_short_bf16();
 hipError_t configure_attn_ring_short_f16();
+hipError_t configure_attn_ring_shared_bf16();
+hipError_t configure_attn_ring_shared_f16();
 hipError_t configure_qkv_rope_store();
 hipError_t configure_linear_skinny();
 

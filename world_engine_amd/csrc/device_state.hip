@@ -53,6 +53,7 @@ int init_current_device() {
   if (configure_attn_ring_bf16_128() != hipSuccess || configure_attn_ring_bf16_64() != hipSuccess ||
       configure_attn_ring_f16_128() != hipSuccess || configure_attn_ring_f16_64() != hipSuccess ||
       configure_attn_ring_short_bf16() != hipSuccess || configure_attn_ring_short_f16() != hipSuccess ||
+      configure_attn_ring_shared_bf16() != hipSuccess || configure_attn_ring_shared_f16() != hipSuccess ||
       configure_qkv_rope_store() != hipSuccess || configure_linear_skinny() != hipSuccess)
     return WE_ERR_LAUNCH;
   void* p = nullptr;

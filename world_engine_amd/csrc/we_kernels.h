@@ -59,9 +59,9 @@ struct AttnParams {
   int n_splits;     // context splits of the units that are split (1 = nothing is split)
   int units_whole;  // leading (batch, kv head) units processed unsplit, writing the output directly
   int64_t ws_row0;  // first query row covered by the split-context workspace
-  int q_tiles;      // ceil(T / queries per workgroup)
+  int q_heads;      // heads of a group that have query tiles of their own: group, or 1 when they share tiles
   int group;        // query heads per kv head, H / Hkv
-  int members;      // workgroups that share one K/V stream: group * q_tiles
+  int members;      // workgroups that share one K/V stream
   int unit_splits;  // units_whole + (B * Hkv - units_whole) * n_splits
   float scale_log2;  // softmax scale * log2(e), applied to the raw logits in fp32
   // optional per (batch, head, token) output gate, element type (src/model/attn.py:117-119): either
@@ -118,6 +118,9 @@ hipError_t launch_attn_ring_f16_64(const AttnParams& p, int ksplit, hipStream_t 
 // frames below one 64-key tile
 hipError_t launch_attn_ring_short_bf16(const AttnParams& p, int Dh, int ksplit, hipStream_t stream);
 hipError_t launch_attn_ring_short_f16(const AttnParams& p, int Dh, int ksplit, hipStream_t stream);
+// grouped heads that share query tiles (q_heads != group)
+hipError_t launch_attn_ring_shared_bf16(const AttnParams& p, int Dh, int ksplit, hipStream_t stream);
+hipError_t launch_attn_ring_shared_f16(const AttnParams& p, int Dh, int ksplit, hipStream_t stream);
 // fp32 caches: one pass on the fp32 matrix instructions, no context splitting
 hipError_t launch_attn_ring_f32(const AttnParams& p, int Dh, int cus, hipStream_t stream);
 hipError_t launch_attn_combine(const AttnParams& p, int Dh, int dtype, hipStream_t stream);
