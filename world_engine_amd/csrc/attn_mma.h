@@ -67,6 +67,13 @@ __device__ __forceinline__ void dma16(uint64_t gbase, uint32_t voff, uint32_t ld
                : "v"(voff), "s"(gbase), "s"(lds_addr)
                : "memory", "m0");
 }
+// The same for 4 bytes per lane, each from an address of its own.
+__device__ __forceinline__ void dma4(const void* src, uint32_t lds_addr) {
+  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off"
+               :
+               : "v"((uint64_t)(uintptr_t)src), "s"(lds_addr)
+               : "memory", "m0");
+}
 template <int N>
 __device__ __forceinline__ void dma_wait() {
   asm volatile("s_waitcnt vmcnt(%0)" : : "n"(N) : "memory");

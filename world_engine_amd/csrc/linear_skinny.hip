@@ -141,38 +141,34 @@ linear_skinny_kernel(LinearParams p) {
   }
 
   // ---- the contraction shares add up through LDS ----
-  // vector v of lane l of block (fb, mb) of share k sits at ((((k * NF + fb) * 2 + mb) * 4 + v) * 64 + l) * 16
+  // Vector v of lane l of block (fb, mb) of share k - features 4 pc .. 4 pc + 3 of the tile, pc = 8 fb + 2 v + l / 32,
+  // of row 32 mb + l % 32 - sits at ((((k * NF + fb) * 2 + mb) * 4 + v) * 64 + (l ^ swz(pc))) * 16: a quarter
+  // wavefront of the readers, who take the vectors row by row as the output wants them, finds 16 bank groups.
   __syncthreads();  // everybody is done with the ring
+  constexpr int PCR = BN / 4;                  // vectors per row
+  auto swz = [](int pc) { return BN == 32 ? 2 * pc : pc & 15; };
   f32x4_t* xch = reinterpret_cast<f32x4_t*>(smem);
 #pragma unroll
   for (int mb = 0; mb < 2; ++mb)
 #pragma unroll
     for (int v = 0; v < 4; ++v)
-      xch[(((kg * NF + fb) * 2 + mb) * 4 + v) * 64 + lane] =
+      xch[(((kg * NF + fb) * 2 + mb) * 4 + v) * 64 + (lane ^ swz(fb * 8 + 2 * v + hh))] =
           f32x4_t{acc[mb][4 * v], acc[mb][4 * v + 1], acc[mb][4 * v + 2], acc[mb][4 * v + 3]};
   __syncthreads();
-  constexpr int SHARE_V = NF * 2 * 4 * 64;             // vectors of one share
-  constexpr int OUT_OFF = KG * SHARE_V * 16;           // the rounded tile [64][BN] behind them
-  static_assert(OUT_OFF + LM * BN * 2 <= L::kBytes, "exchange area and output tile reuse the ring");
+  constexpr int SHARE_V = NF * 2 * 4 * 64;     // vectors of one share
+  static_assert(KG * SHARE_V * 16 <= L::kBytes && SHARE_V == LM * PCR, "the exchange area reuses the ring");
 #pragma unroll
   for (int i = tid; i < SHARE_V; i += 512) {
-    f32x4_t r = xch[i];
+    const int row = i / PCR, pc = i % PCR;
+    const int at = (((pc >> 3) * 2 + (row >> 5)) * 4 + ((pc >> 1) & 3)) * 64 + ((((pc & 1) << 5) | (row & 31)) ^ swz(pc));
+    f32x4_t r = xch[at];
 #pragma unroll
-    for (int k = 1; k < KG; ++k) r += xch[k * SHARE_V + i];
-    // vector v of lane l: features 8 v + 4 (l / 32) + 0..3 of the block, row l % 32
-    const int l = i & 63, v = (i >> 6) & 3, mb = (i >> 8) & 1, f = i >> 9;
+    for (int k = 1; k < KG; ++k) r += xch[k * SHARE_V + at];
     typedef typename M::elem_t E;
     typedef E e4_t __attribute__((ext_vector_type(4)));
-    *reinterpret_cast<e4_t*>(smem + OUT_OFF + (mb * 32 + (l & 31)) * (BN * 2) + (f * 32 + 8 * v + 4 * (l >> 5)) * 2) =
-        e4_t{(E)r[0], (E)r[1], (E)r[2], (E)r[3]};
-  }
-  __syncthreads();
-  constexpr int CPR = BN / 8;  // 16-byte chunks per row of the tile
-  for (int i = tid; i < LM * CPR; i += 512) {
-    const int row = i / CPR, ch = i % CPR;
     if (m0 + row < p.M)
-      *reinterpret_cast<u32x4_t*>(reinterpret_cast<uint16_t*>(p.y) + (int64_t)(m0 + row) * p.ys + n0 + ch * 8) =
-          *reinterpret_cast<const u32x4_t*>(smem + OUT_OFF + i * 16);
+      *reinterpret_cast<e4_t*>(reinterpret_cast<uint16_t*>(p.y) + (int64_t)(m0 + row) * p.ys + n0 + pc * 4) =
+          e4_t{(E)r[0], (E)r[1], (E)r[2], (E)r[3]};
   }
 }
 

@@ -12,12 +12,16 @@
 // bytes, 16-byte chunks XOR-swizzled with (row & 15) on the global side of the DMA.  Wavefront w
 // takes feature half (w & 1) and the contraction steps (w >> 1) and (w >> 1) + 4 of every slot:
 // per slot 8 fragment reads (ds_read_b128) feed 8 v_mfma_f32_32x32x16 (A = W rows, B = x rows, so
-// a lane owns one token and registers run along features).  The four partial sums of a tile are
-// added through LDS in a fixed order, rounded to the element type as the GEMM's output tensor
-// would be, and laid out as a [64][128] tile in LDS; then every thread takes one 16-element item
-// exactly like a thread of the store kernel (same functions, same bits): RMS norm, rotation,
-// value blend, tail / ring-slot rows, `written`.  cos / sin values, position ids and the value
-// residual of a thread's item are requested before the main loop.
+// a lane owns one token and registers run along features).  The four partial sums of a tile go
+// through LDS; every thread adds those of one 16-element item in a fixed order, rounds them to the
+// element type as the GEMM's output tensor would be, and goes on exactly like a thread of the store
+// kernel (same functions, same bits): RMS norm, rotation, value blend, tail / ring-slot rows,
+// `written`.
+//
+// What runs outside the loop is a third of the time, so it waits for as little as it can: the position
+// ids come by DMA ahead of the first slot, cos / sin values and the value residual of a thread's item
+// are requested behind the second one, and the sums reach the items without a staging tile (256 x 6144
+// x 2048, weights out of HBM: 18.96 -> 18.36 us; 11.2 of it is the tiles' intake alone).
 //
 // The grid is 1-D: workgroup id % 8 is the XCD, and the token tiles of one feature tile follow
 // each other on one XCD, so a weight slab is fetched from HBM once and re-read from that L2.
@@ -38,10 +42,9 @@ constexpr int X_TILE_B = PM * P_ROW_B;       // 16 KB
 constexpr int W_TILE_B = PN * P_ROW_B;       // 32 KB
 constexpr int SLOT_B = X_TILE_B + W_TILE_B;  // 48 KB
 constexpr int NSLOT = 3;
-constexpr int BLK_B = 32 * 32 * 4;           // one 32 x 32 fp32 block of partial sums
-constexpr int OUT_OFF = 2 * 4 * 4 * BLK_B;   // the element-type output tile sits behind the exchange area
-constexpr int PROJ_LDS_B = NSLOT * SLOT_B;
-static_assert(OUT_OFF + PM * PN * 2 <= PROJ_LDS_B, "exchange area and output tile reuse the ring");
+constexpr int IDS_OFF = NSLOT * SLOT_B;      // position ids: [wavefront][t, y, x][8 tokens], padded to 256 bytes each
+constexpr int PROJ_LDS_B = IDS_OFF + 8 * 256;
+static_assert(2 * 4 * 4 * (32 * 32 * 4) <= IDS_OFF, "the exchange area (4 shares of 8 fp32 blocks) reuses the ring");
 }  // namespace
 
 template <typename M, typename Tag>
@@ -122,12 +125,18 @@ qkv_rope_store_kernel(ProjParams p) {
   const int G = mt_all >= 8 ? 8 : (mt_all >= 4 ? 4 : (mt_all >= 2 ? 2 : 1));
   const int rot = mi & (G - 1), ncg = nc & ~(G - 1);
   auto chunk = [&](int c) __attribute__((always_inline)) { return c < ncg ? (c & ~(G - 1)) | ((c + rot) & (G - 1)) : c; };
+  // the position ids of this wavefront's 8 items' tokens: lane 16 a + 2 k + half takes 4 bytes of array a's
+  // id of token k (the last lanes repeat lane 47)
+  {
+    const int l = lane < 48 ? lane : 47, a = l >> 4;
+    int tok = m0 + wave * 8 + ((l & 15) >> 1);
+    tok = tok < s.T ? tok : s.T - 1;
+    const int64_t* ids = a == 0 ? s.t_pos : (a == 1 ? s.y_pos : s.x_pos);
+    dma4(reinterpret_cast<const uint32_t*>(ids + b * s.pos_stride_b + tok) + (l & 1),
+         (uint32_t)__builtin_amdgcn_readfirstlane((int)(lds0 + IDS_OFF + wave * 256)));
+  }
   dma_slot(chunk(0), 0);
   if (nc > 1) dma_slot(chunk(1), 1);
-
-  // ---- what the item needs besides the projection: requested now, used after the loop ----
-  ItemSide<Tag> side;
-  load_item_side<Tag>(s, which, b, e_h, e_tc, e_chunk, side);
 
   // ---- fragment read addresses: row l32 of a 32-row block, logical chunk 2 * step + hh ----
   uint32_t a_rd[2], b_rd[2];
@@ -146,14 +155,42 @@ qkv_rope_store_kernel(ProjParams p) {
 #pragma unroll
       for (int i = 0; i < 16; ++i) acc[nb][mb][i] = 0.f;
 
+  // ---- what the item needs besides the projection (as it comes: a conversion here would wait for it) ----
+  ItemSide<Tag> side;
+  u32x4_t res_raw[2];
+  st_t lamb_raw;
+  uint32_t guard;
+  side.rotate = which != 2;
+  const bool blend = which == 2 && s.v1 != nullptr;
+  auto request_side = [&]() __attribute__((always_inline)) {
+    if (side.rotate) {
+      const int64_t* ids = reinterpret_cast<const int64_t*>(smem + IDS_OFF + wave * 256) + (e_row & 7);
+      const int64_t at = rope_table_row(s, ids[0], ids[8], ids[16]) * (s.Dh >> 1);
+      load_cos_sin(s.cos_t + at, s.sin_t + at, e_chunk, side.c, side.s);
+    }
+    if (blend) {
+      const u32x4_t* src = reinterpret_cast<const u32x4_t*>((const st_t*)s.v1 + b * s.v1s_b + e_h * s.v1s_h + e_tc * s.v1s_t + e_chunk * 16);
+      res_raw[0] = src[0];
+      res_raw[1] = src[1];
+    }
+    // (requested whether there are any or not - a value merged with another is waited for on the spot - and
+    // by a lane's own load, for the same reason)
+    int zero = 0;
+    asm volatile("" : "+v"(zero));
+    lamb_raw = *(reinterpret_cast<const st_t*>(blend ? s.v_lamb : p.w) + zero);
+    guard = *((s.guard != nullptr ? s.guard : reinterpret_cast<const uint32_t*>(s.t_pos)) + zero);
+  };
+
   // ---- main loop: one barrier per slot ----
   uint32_t slot_off = 0;   // byte offset of the slot being consumed
   int fill = 2 % NSLOT;    // slot the next DMA goes to
-  for (int c = 0; c < nc; ++c) {
+  auto consume = [&](int c, auto with_side) __attribute__((always_inline)) {
     if (c + 1 < nc) dma_wait<NDMA>(); else dma_wait<0>();  // this wavefront's part of slot c has landed
     // every wavefront's part has landed, and everybody is done with the slot refilled next
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
+    // (in front of the next slot's request: the counter wait for the slot after this one covers it)
+    if (decltype(with_side)::value) request_side();
     if (c + 2 < nc) dma_slot(chunk(c + 2), fill);
     fill = fill + 1 == NSLOT ? 0 : fill + 1;
 #pragma unroll
@@ -169,78 +206,49 @@ qkv_rope_store_kernel(ProjParams p) {
       acc[1][0] = M::mma(a1, b0, acc[1][0]);
       acc[1][1] = M::mma(a1, b1, acc[1][1]);
     }
-    slot_off = slot_off + SLOT_B == (uint32_t)PROJ_LDS_B ? 0u : slot_off + SLOT_B;
-  }
+    slot_off = slot_off + SLOT_B == (uint32_t)(NSLOT * SLOT_B) ? 0u : slot_off + SLOT_B;
+  };
+  int c0 = 0;
+  if (nc > 1) consume(c0++, std::false_type());
+  consume(c0++, std::true_type());
+  for (int c = c0; c < nc; ++c) consume(c, std::false_type());
 
   // ---- the four contraction groups add their partial sums through LDS ----
-  // Block (nb, mb) of feature half nh belongs to the wavefront with kg == 2 * nb + mb.  Vector g
-  // of lane l of the block that group k hands to that owner sits at
-  // ((((nh * 4 + k) * 4 + block) * 4 + g) * 64 + l) * 16.
+  // Vector g (features 8 g + 4 hh + 0..3 of the lane's token) of lane l of block (nb, mb) of feature half nh,
+  // group k, sits at ((((nh * 4 + k) * 4 + 2 * nb + mb) * 4 + g) * 64 + (l ^ 2 * item)) * 16, item being the
+  // 16-feature item of the tile that it belongs to: a quarter wavefront then reads 16 bank groups below.
   __syncthreads();  // everybody is done with the ring
   f32x4_t* xch = reinterpret_cast<f32x4_t*>(smem);
 #pragma unroll
   for (int nb = 0; nb < 2; ++nb)
 #pragma unroll
-    for (int mb = 0; mb < 2; ++mb) {
-      const int blk = 2 * nb + mb;
-      if (blk != kg) {
-        f32x4_t* dst = xch + (((nh * 4 + kg) * 4 + blk) * 4) * 64 + lane;
+    for (int mb = 0; mb < 2; ++mb)
 #pragma unroll
-        for (int g = 0; g < 4; ++g)
-          dst[g * 64] = f32x4_t{acc[nb][mb][4 * g], acc[nb][mb][4 * g + 1], acc[nb][mb][4 * g + 2], acc[nb][mb][4 * g + 3]};
-      }
-    }
+      for (int g = 0; g < 4; ++g)
+        xch[(((nh * 4 + kg) * 4 + 2 * nb + mb) * 4 + g) * 64 + (lane ^ (2 * (nh * 4 + nb * 2 + (g >> 1))))] =
+            f32x4_t{acc[nb][mb][4 * g], acc[nb][mb][4 * g + 1], acc[nb][mb][4 * g + 2], acc[nb][mb][4 * g + 3]};
   __syncthreads();
-#pragma unroll
-  for (int nb = 0; nb < 2; ++nb)
-#pragma unroll
-    for (int mb = 0; mb < 2; ++mb) {
-      const int blk = 2 * nb + mb;
-      if (blk == kg) {
-        // sum in the order of the contraction groups, whoever the owner is
-        f32x16_t r;
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-          f32x16_t part;
-          if (k == kg) {
-            part = acc[nb][mb];
-          } else {
-            const f32x4_t* src = xch + (((nh * 4 + k) * 4 + blk) * 4) * 64 + lane;
-#pragma unroll
-            for (int g = 0; g < 4; ++g) {
-              const f32x4_t v = src[g * 64];
-              part[4 * g] = v[0]; part[4 * g + 1] = v[1]; part[4 * g + 2] = v[2]; part[4 * g + 3] = v[3];
-            }
-          }
-          if (k == 0) r = part;
-          else
-#pragma unroll
-            for (int i = 0; i < 16; ++i) r[i] += part[i];
-        }
-        // register 4 g + e of a lane is feature 8 g + 4 hh + e of the block, for token l32
-        unsigned char* orow = smem + OUT_OFF + (mb * 32 + l32) * (PN * 2) + (nh * 64 + nb * 32 + 4 * hh) * 2;
-#pragma unroll
-        for (int g = 0; g < 4; ++g) {
-          uint16_t e4[4];
-#pragma unroll
-          for (int e = 0; e < 4; ++e) e4[e] = Tag::from_f32(r[4 * g + e]);
-          u32x2_t pk;
-          pk[0] = (uint32_t)e4[0] | ((uint32_t)e4[1] << 16);
-          pk[1] = (uint32_t)e4[2] | ((uint32_t)e4[3] << 16);
-          *reinterpret_cast<u32x2_t*>(orow + g * 16) = pk;
-        }
-      }
-    }
-  __syncthreads();
-
-  // ---- epilogue: the store kernel's work on this thread's item ----
-  if (!e_live || (s.guard != nullptr && *s.guard != 0u)) return;  // (refused position ids: nothing is written)
   Chunk16<Tag> in;
   {
-    const u32x4_t* src = reinterpret_cast<const u32x4_t*>(smem + OUT_OFF + e_row * (PN * 2) + (tid & 7) * 32);
-    u32x4_t* dst = reinterpret_cast<u32x4_t*>(in.e);
-    dst[0] = src[0];
-    dst[1] = src[1];
+    const int item = tid & 7, blk = (item & 2) + (e_row >> 5);
+    const f32x4_t* src = xch + ((item >> 2) * 16 + blk) * 256 + (item & 1) * 128;
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {   // features 4 v .. 4 v + 3 of the item
+      const int at = (v >> 1) * 64 + (((v & 1) * 32 + (e_row & 31)) ^ (2 * item));
+      f32x4_t r = src[at];
+#pragma unroll
+      for (int k = 1; k < 4; ++k) r += src[k * 1024 + at];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) in.e[4 * v + e] = Tag::from_f32(r[e]);
+    }
+  }
+
+  // ---- epilogue: the store kernel's work on this thread's item ----
+  if (!e_live || (s.guard != nullptr && guard != 0u)) return;  // (refused position ids: nothing is written)
+  if (blend) {
+    *reinterpret_cast<u32x4_t*>(side.res.e) = res_raw[0];
+    *reinterpret_cast<u32x4_t*>(side.res.e + 8) = res_raw[1];
+    side.lamb = Tag::to_f32(lamb_raw);
   }
   if (which == 0) {
     finish_q_chunk<Tag>(s, b, e_h, e_t, e_chunk, in, side.rotate, side.c, side.s);

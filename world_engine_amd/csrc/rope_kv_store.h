@@ -97,10 +97,13 @@ __device__ __forceinline__ void lerp_chunk(Chunk16<Tag>& v, const Chunk16<Tag>& 
 
 // Row of the cos / sin tables for token t of batch element b (src/model/attn.py:33-36): the
 // three position ids select one row of the flattened [frames, height, width] table.
-__device__ __forceinline__ int64_t rope_table_row(const StoreParams& p, int b, int t) {
-  int64_t pos = p.t_pos[b * p.pos_stride_b + t] * p.grid_hw + p.y_pos[b * p.pos_stride_b + t] * p.grid_w +
-                p.x_pos[b * p.pos_stride_b + t];
+__device__ __forceinline__ int64_t rope_table_row(const StoreParams& p, int64_t t_id, int64_t y_id, int64_t x_id) {
+  const int64_t pos = t_id * p.grid_hw + y_id * p.grid_w + x_id;
   return pos < 0 ? 0 : (pos >= p.table_rows ? p.table_rows - 1 : pos);
+}
+__device__ __forceinline__ int64_t rope_table_row(const StoreParams& p, int b, int t) {
+  const int64_t at = b * p.pos_stride_b + t;
+  return rope_table_row(p, p.t_pos[at], p.y_pos[at], p.x_pos[at]);
 }
 
 // cos / sin of the 8 pairs of chunk `chunk` of a table row.
