@@ -75,16 +75,9 @@ class LayerKVCache(nn.Module):
         # per-layer call buffers (rotated q, attention output, split-context workspace) of the eager
         # path, sized on first use and dropped whenever the module is moved or cast
         self._call_buffers = {}
-        self._fresh = self.kv._version   # the ring as it was made, all zeros, has this version
 
     def _apply(self, fn, *args, **kwargs):
         self._call_buffers = {}
-        kv = self.kv
-        if kv.device.type == "cpu" and not kv.is_inference() and kv._version == self._fresh:
-            # an unused ring moves to a GPU as zeros made there (a model's rings are a gigabyte to copy)
-            moved = fn(kv.new_zeros(1))
-            if moved.is_cuda:
-                self.kv = torch.zeros(kv.shape, dtype=moved.dtype, device=moved.device)
         return super()._apply(fn, *args, **kwargs)
 
     def _reusable(self, reuse: bool):
