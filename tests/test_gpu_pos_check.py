@@ -91,3 +91,34 @@ def test_checked_calls_from_threads_and_streams(gpu_device):
     [t.start() for t in threads]
     [t.join(60) for t in threads]
     assert not failures, failures
+
+
+def test_ids_on_another_device_are_refused_before_any_launch(gpu_device):
+    """Every id tensor of a call has to be on the call's device: one left on the host is an error, not a pointer
+    for a kernel."""
+    dev = gpu_device
+    T, H, Dh, W = 64, 2, 64, 8
+    layer = wea.LayerKVCache(1, H, 2 * T, Dh, torch.bfloat16, T).to(dev)
+    rope = wea.RoPE(*ro.rope_table_1d(4 * T, Dh), T // W, W).to(dev)
+    q = torch.randn(1, H, T, Dh, device=dev, dtype=torch.bfloat16)
+    w = torch.randn(3 * H * Dh, H * Dh, device=dev, dtype=torch.bfloat16)
+    x = torch.randn(1, T, H * Dh, device=dev, dtype=torch.bfloat16)
+    good = to_dev(ro.synth_pos_ids(1, 1, T, W), dev)
+    calls = {
+        "attend": lambda pos: layer.rope_upsert_attend(q, q, q, pos, rope, False),
+        "store": lambda pos: layer.rope_upsert(q, q, q, pos, rope, False),
+        "project": lambda pos: layer.qkv_rope_upsert_attend(x, w, H, pos, rope, False),
+        "rope": lambda pos: rope(q, pos),
+        "store op": lambda pos: wea.ops.rope_kv_store(q, q, q, pos, rope.cos, rope.sin, rope.height, rope.width, layer.kv,
+                                                      layer.written, layer.L, 1, False),
+        "rope op": lambda pos: wea.ops.rope_apply(q, pos, rope.cos, rope.sin, rope.height, rope.width),
+    }
+    kv = layer.kv.clone()
+    for name, call in calls.items():
+        for key in good:
+            with pytest.raises(RuntimeError, match="on a ROCm GPU only|on the same device"):
+                call(dict(good, **{key: good[key].cpu()}))
+        assert torch.equal(layer.kv, kv), name
+    layer.check_inputs = False
+    with pytest.raises(RuntimeError, match="on a ROCm GPU only"):
+        calls["attend"](dict(good, y_pos=good["y_pos"].cpu()))

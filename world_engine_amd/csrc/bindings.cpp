@@ -398,7 +398,8 @@ PyObject* rope_kv_store(PyObject*, PyObject* const* argv, Py_ssize_t n) {
     const bool frozen = a.flag();
     const int what = (int)a.integer();
     const int64_t tpf = a.integer();
-    const c10::Device dev = need_device({&k, &v, &kv, &written, q, cos, sin, &tp});
+    const c10::Device dev = need_device({&k, &v, &kv, &written, q, cos, sin, &tp, cos != nullptr ? yp : nullptr,
+                                         cos != nullptr ? xp : nullptr});
     if (k.dim() != 4 || k.sizes() != v.sizes()) fail("k and v must both be [B, Hkv, T, Dh]");
     const int64_t B = k.size(0), Hkv = k.size(1), T = k.size(2), Dh = k.size(3);
     if (tpf > 0 && T != tpf) fail("KV cache expects exactly one frame per upsert");
@@ -438,7 +439,7 @@ PyObject* rope_apply(PyObject*, PyObject* const* argv, Py_ssize_t n) {
     const Tensor &cos_in = a.tensor(), &sin_in = a.tensor();
     const int64_t gh = a.integer(), gw = a.integer();
     const int what = (int)a.integer();
-    const c10::Device dev = need_device({&x, &cos_in, &sin_in, &tp});
+    const c10::Device dev = need_device({&x, &cos_in, &sin_in, &tp, &yp, &xp});
     if (x.dim() != 4) fail("x must be [B, H, T, Dh]");
     const int64_t B = x.size(0), H = x.size(1), T = x.size(2), Dh = x.size(3);
     if (cos_in.scalar_type() != at::kFloat || sin_in.scalar_type() != at::kFloat) fail("cos/sin tables must be fp32");
@@ -532,7 +533,7 @@ PyObject* rope_kv_attn(PyObject*, PyObject* const* argv, Py_ssize_t n) {
     const Tensor &kv = a.tensor(), &written = a.tensor();
     const int64_t L = a.integer(), dilation = a.integer();
     const bool frozen = a.flag();
-    const c10::Device dev = need_device({&q, &k, &v, &kv, &written, &cos, &sin, &tp});
+    const c10::Device dev = need_device({&q, &k, &v, &kv, &written, &cos, &sin, &tp, &yp, &xp});
     if (k.dim() != 4 || k.sizes() != v.sizes()) fail("k and v must both be [B, Hkv, T, Dh]");
     const int64_t B = k.size(0), Hkv = k.size(1), T = k.size(2), Dh = k.size(3);
     const float scale = (float)a.scale(Dh);
@@ -591,7 +592,7 @@ PyObject* qkv_rope_kv_attn(PyObject*, PyObject* const* argv, Py_ssize_t n) {
     const Tensor &kv = a.tensor(), &written = a.tensor();
     const int64_t L = a.integer(), dilation = a.integer();
     const bool frozen = a.flag();
-    const c10::Device dev = need_device({&x, &w, &kv, &written, &cos, &sin, &tp});
+    const c10::Device dev = need_device({&x, &w, &kv, &written, &cos, &sin, &tp, &yp, &xp});
     if (x.dim() != 3 || x.stride(2) != 1) fail("x must be [B, T, d_model] with contiguous channels");
     const int64_t B = x.size(0), T = x.size(1), d_model = x.size(2);
     if (kv.dim() != 5) fail("kv must be [2, B, Hkv, L+T, Dh]");
