@@ -122,3 +122,37 @@ def test_ids_on_another_device_are_refused_before_any_launch(gpu_device):
     layer.check_inputs = False
     with pytest.raises(RuntimeError, match="on a ROCm GPU only"):
         calls["attend"](dict(good, y_pos=good["y_pos"].cpu()))
+
+
+def test_more_checked_calls_at_once_than_records(gpu_device):
+    """More threads in a checked call than the binding has records for: the ones that wait for a record let the
+    ones that hold one finish (every call is behind 50 ms of work on its stream, so that they pile up)."""
+    dev = gpu_device
+    T, H, Dh, W = 64, 2, 64, 8
+    threads_n = 40
+    rope = wea.RoPE(*ro.rope_table_1d(4 * T, Dh), T // W, W).to(dev)
+    good = to_dev(ro.synth_pos_ids(1, 1, T, W), dev)
+    layers = [wea.LayerKVCache(1, H, 2 * T, Dh, torch.bfloat16, T).to(dev) for _ in range(threads_n)]
+    q = torch.randn(1, H, T, Dh, device=dev, dtype=torch.bfloat16)
+    gate = torch.cuda.Event()
+    torch.cuda.synchronize()
+    torch.cuda._sleep(100_000_000)      # (cycles: tens of milliseconds, then it ends by itself)
+    gate.record()
+    outs, failures = [None] * threads_n, []
+
+    def work(i):
+        try:
+            stream = torch.cuda.Stream()
+            with torch.cuda.stream(stream):
+                stream.wait_event(gate)
+                for _ in range(3):
+                    outs[i] = layers[i].rope_upsert_attend(q, q, q, good, rope, True)
+                stream.synchronize()
+        except BaseException as e:      # noqa: BLE001 - reported by the main thread
+            failures.append((i, repr(e)))
+
+    threads = [threading.Thread(target=work, args=(i,), daemon=True) for i in range(threads_n)]
+    [t.start() for t in threads]
+    [t.join(60) for t in threads]
+    assert not failures and not any(t.is_alive() for t in threads), failures
+    assert all(torch.equal(o, outs[0]) for o in outs)

@@ -24,6 +24,7 @@
 #include <string>
 
 #include "../../include/we_attn.h"
+#include "record_slots.h"
 
 namespace {
 
@@ -32,6 +33,21 @@ using at::Tensor;
 [[noreturn]] void fail(const std::string& what) { throw std::runtime_error(what); }
 [[noreturn]] void fail_code(const char* fn, int code) {
   fail(std::string(fn) + " failed: " + we_error_string(code) + " (code " + std::to_string(code) + ")");
+}
+
+// Without the interpreter's lock for as long as it lives: around everything that can wait (a launch
+// into a full queue, a verdict, a free record), so that other threads of the program go on.
+struct NoGil {
+  PyThreadState* state = PyEval_SaveThread();
+  ~NoGil() { PyEval_RestoreThread(state); }
+  NoGil() = default;
+  NoGil(const NoGil&) = delete;
+  NoGil& operator=(const NoGil&) = delete;
+};
+template <typename F>
+int call_library(F&& f) {
+  const NoGil off;
+  return f();
 }
 
 // ---- arguments -----------------------------------------------------------------------------
@@ -252,14 +268,14 @@ struct Extras {
 };
 
 // ---- verdicts of the position-id check -------------------------------------------------------
-// A call that checks holds one of kVerdicts records while it runs: a word of host-coherent memory
+// A call that checks holds one of a device's records while it runs: a word of host-coherent memory
 // the device reports to and a word of device memory the kernels pass the verdict on in.  The
-// records are made on a device's first checked call and live as long as the process; calls from
-// more threads than there are records wait for one.
-constexpr int kVerdicts = 32;
+// records are made on a device's first checked call and live as long as the process; a call that
+// finds all of them out waits for one, without the interpreter's lock.
+constexpr int kVerdicts = we::RecordSlots::kCount;
 constexpr int kMaxDevices = 64;
 struct Verdicts {
-  std::atomic<uint32_t> busy{0};
+  we::RecordSlots slots;
   uint64_t* report = nullptr;   // kVerdicts words, one per 64 bytes
   uint32_t* guard = nullptr;    // likewise, on the device
   uint64_t ticket[kVerdicts] = {};
@@ -293,13 +309,10 @@ class PosCheck {
   PosCheck(int what, c10::Device dev, hipStream_t st) : st_(st) {
     if (what == 0 || capturing(st)) return;
     v_ = &verdicts(dev);
-    for (;;) {
-      uint32_t b = v_->busy.load(std::memory_order_relaxed);
-      if (~b != 0u) {
-        slot_ = __builtin_ctz(~b);
-        if (v_->busy.compare_exchange_weak(b, b | (1u << slot_), std::memory_order_acquire)) break;
-      }
-    }
+    slot_ = v_->slots.take([](auto&& wait) {
+      const NoGil off;
+      wait();
+    });
     c_.what = what;
     c_.report = v_->report + slot_ * 8;
     c_.guard = v_->guard + slot_ * 16;
@@ -307,19 +320,22 @@ class PosCheck {
   }
   ~PosCheck() {
     if (v_ == nullptr) return;
-    if (!awaited_) (void)hipStreamSynchronize(st_);  // (a call that failed half-way: nothing may report to the record later)
-    v_->busy.fetch_and(~(1u << slot_), std::memory_order_release);
+    if (!awaited_) {  // (a call that failed half-way: nothing may report to the record later)
+      const NoGil off;
+      (void)hipStreamSynchronize(st_);
+    }
+    v_->slots.give_back(slot_);
   }
   PosCheck(const PosCheck&) = delete;
   PosCheck& operator=(const PosCheck&) = delete;
   const we_pos_check* arg() const { return v_ != nullptr ? &c_ : nullptr; }
-  // Waits for the verdict of the launched call; true = refused.
+  // Waits for the verdict of the launched call, without the interpreter's lock; true = refused.
   bool refused() {
     if (v_ == nullptr) return false;
     awaited_ = true;
+    const NoGil off;
     const volatile uint64_t* word = c_.report;
     uint64_t got = 0;
-    PyThreadState* save = PyEval_SaveThread();
     const auto began = std::chrono::steady_clock::now();
     bool there = false;
     for (int spin = 1; !there; ++spin) {
@@ -336,7 +352,6 @@ class PosCheck {
       got = *word;
       there = (got >> 1) == c_.ticket;
     }
-    PyEval_RestoreThread(save);
     if (!there) fail(std::string("the position-id check did not report: ") + hipGetErrorString(e));
     std::atomic_thread_fence(std::memory_order_acquire);
     return (got & 1u) != 0;
@@ -420,12 +435,12 @@ PyObject* rope_kv_store(PyObject*, PyObject* const* argv, Py_ssize_t n) {
     Tensor q_out;
     if (q != nullptr) q_out = new_heads(*q, B, H, T, Dh);
     PosCheck check(what, dev, st);
-    const int rc = we_rope_kv_store_checked(
+    const int rc = call_library([&] { return we_rope_kv_store_checked(
         q != nullptr ? q->data_ptr() : nullptr, k.data_ptr(), v.data_ptr(), q != nullptr ? qs.s : nullptr, ks.s, vs.s,
         q != nullptr ? q_out.data_ptr() : nullptr, rotate ? cos->const_data_ptr<float>() : nullptr,
         rotate ? sin->const_data_ptr<float>() : nullptr, rotate ? cos->size(0) : 0, pos.tp(), pos.yp(), pos.xp(),
         pos.row_stride, gh, gw, kv.data_ptr(), static_cast<uint8_t*>(written.data_ptr()), (int)B, (int)H, (int)Hkv,
-        (int)T, (int)Dh, L, (int)dilation, frozen ? 1 : 0, code_t, check.arg(), st);
+        (int)T, (int)Dh, L, (int)dilation, frozen ? 1 : 0, code_t, check.arg(), st); });
     if (rc != WE_OK) fail_code("we_rope_kv_store", rc);
     if (check.refused()) return refused_result();
     return q != nullptr ? wrap(q_out) : none();
@@ -453,9 +468,9 @@ PyObject* rope_apply(PyObject*, PyObject* const* argv, Py_ssize_t n) {
     const Tensor cos = cos_in.contiguous(), sin = sin_in.contiguous();
     const Tensor out = new_heads(x, B, H, T, Dh);
     PosCheck check(what, dev, st);
-    const int rc = we_rope_apply_checked(x.data_ptr(), xs.s, out.data_ptr(), cos.const_data_ptr<float>(),
+    const int rc = call_library([&] { return we_rope_apply_checked(x.data_ptr(), xs.s, out.data_ptr(), cos.const_data_ptr<float>(),
                                          sin.const_data_ptr<float>(), cos.size(0), pos.tp(), pos.yp(), pos.xp(),
-                                         pos.row_stride, gh, gw, (int)B, (int)H, (int)T, (int)Dh, code_t, check.arg(), st);
+                                         pos.row_stride, gh, gw, (int)B, (int)H, (int)T, (int)Dh, code_t, check.arg(), st); });
     if (rc != WE_OK) fail_code("we_rope_apply", rc);
     if (check.refused()) return refused_result();
     return wrap(out);
@@ -491,10 +506,10 @@ PyObject* attn_ring(PyObject*, PyObject* const* argv, Py_ssize_t n) {
     const Workspace ws(ws_in, B, H, Hkv, T, Dh, L, splits, q_tile, q);
     const Tensor out = output_or_new(out_in, token_major, q, dev, B, H, T, Dh);
     const Strides os(out, "out");
-    const int rc = we_attn_ring_fwd(q.data_ptr(), qs.s, kv.data_ptr(), static_cast<const uint8_t*>(written.data_ptr()),
+    const int rc = call_library([&] { return we_attn_ring_fwd(q.data_ptr(), qs.s, kv.data_ptr(), static_cast<const uint8_t*>(written.data_ptr()),
                                     t_pos.const_data_ptr<int64_t>(), out.data_ptr(), os.s, ws.ptr, ws.bytes, (int)B, (int)H,
                                     (int)Hkv, (int)T, (int)Dh, L, (int)dilation, scale, splits, q_tile, dtype_code(q),
-                                    stream_of(dev));
+                                    stream_of(dev)); });
     if (rc != WE_OK) fail_code("we_attn_ring_fwd", rc);
     return wrap(out);
   });
@@ -515,10 +530,10 @@ PyObject* attn_ring_static(PyObject*, PyObject* const* argv, Py_ssize_t n) {
       fail("out must be [B, H, T, Dh] of q's element type on q's device");
     const Strides qs(q, "q"), os(out, "out");
     const OnDevice on(dev);
-    const int rc = we_attn_ring_fwd_static(q.data_ptr(), qs.s, kv.data_ptr(), static_cast<const uint8_t*>(written.data_ptr()),
+    const int rc = call_library([&] { return we_attn_ring_fwd_static(q.data_ptr(), qs.s, kv.data_ptr(), static_cast<const uint8_t*>(written.data_ptr()),
                                            t_pos.const_data_ptr<int64_t>(), out.data_ptr(), os.s, (int)B, (int)H, (int)Hkv,
                                            (int)T, (int)Dh, L, (int)dilation, scale, splits, q_tile, dtype_code(q),
-                                           stream_of(dev));
+                                           stream_of(dev)); });
     if (rc != WE_OK) fail_code("we_attn_ring_fwd_static", rc);
     return none();
   });
@@ -571,11 +586,11 @@ PyObject* rope_kv_attn(PyObject*, PyObject* const* argv, Py_ssize_t n) {
     const Tensor out = output_or_new(out_in, token_major, q, dev, B, H, T, Dh);
     const Strides os(out, "out");
     PosCheck check(what, dev, st);
-    const int rc = we_rope_kv_attn_fwd_checked(
+    const int rc = call_library([&] { return we_rope_kv_attn_fwd_checked(
         q.data_ptr(), k.data_ptr(), v.data_ptr(), qs.s, ks.s, vs.s, q_rot.data_ptr(), cos.const_data_ptr<float>(),
         sin.const_data_ptr<float>(), cos.size(0), pos.tp(), pos.yp(), pos.xp(), pos.row_stride, gh, gw, kv.data_ptr(),
         static_cast<uint8_t*>(written.data_ptr()), out.data_ptr(), os.s, ws.ptr, ws.bytes, (int)B, (int)H, (int)Hkv, (int)T,
-        (int)Dh, L, (int)dilation, frozen ? 1 : 0, scale, splits, q_tile, code_t, extras.ptr(), check.arg(), st);
+        (int)Dh, L, (int)dilation, frozen ? 1 : 0, scale, splits, q_tile, code_t, extras.ptr(), check.arg(), st); });
     if (rc != WE_OK) fail_code("we_rope_kv_attn_fwd", rc);
     if (check.refused()) return refused_result();
     return pack({&out, &q_rot});
@@ -633,20 +648,20 @@ PyObject* qkv_rope_kv_attn(PyObject*, PyObject* const* argv, Py_ssize_t n) {
     Tensor out;
     PosCheck check(what, dev, st);
     if (!attend) {
-      const int rc = we_qkv_rope_kv_store(&proj, q_rot.data_ptr(), cos.const_data_ptr<float>(), sin.const_data_ptr<float>(),
+      const int rc = call_library([&] { return we_qkv_rope_kv_store(&proj, q_rot.data_ptr(), cos.const_data_ptr<float>(), sin.const_data_ptr<float>(),
                                           cos.size(0), pos.tp(), pos.yp(), pos.xp(), pos.row_stride, gh, gw, kv.data_ptr(),
                                           static_cast<uint8_t*>(written.data_ptr()), (int)B, (int)H, (int)Hkv, (int)T, (int)Dh,
-                                          L, (int)dilation, frozen ? 1 : 0, code_t, extras.ptr(), st);
+                                          L, (int)dilation, frozen ? 1 : 0, code_t, extras.ptr(), st); });
       if (rc != WE_OK) fail_code("we_qkv_rope_kv_store", rc);
     } else {
       const Workspace ws(ws_in, B, H, Hkv, T, Dh, L, splits, q_tile, x);
       out = output_or_new(out_in, true, x, dev, B, H, T, Dh);
       const Strides os(out, "out");
-      const int rc = we_qkv_rope_kv_attn_fwd_checked(
+      const int rc = call_library([&] { return we_qkv_rope_kv_attn_fwd_checked(
           &proj, q_rot.data_ptr(), cos.const_data_ptr<float>(), sin.const_data_ptr<float>(), cos.size(0), pos.tp(), pos.yp(),
           pos.xp(), pos.row_stride, gh, gw, kv.data_ptr(), static_cast<uint8_t*>(written.data_ptr()), out.data_ptr(), os.s,
           ws.ptr, ws.bytes, (int)B, (int)H, (int)Hkv, (int)T, (int)Dh, L, (int)dilation, frozen ? 1 : 0, scale, splits, q_tile,
-          code_t, extras.ptr(), check.arg(), st);
+          code_t, extras.ptr(), check.arg(), st); });
       if (rc != WE_OK) fail_code("we_qkv_rope_kv_attn_fwd", rc);
       if (check.refused()) return refused_result();
     }
@@ -677,8 +692,8 @@ PyObject* linear(PyObject*, PyObject* const* argv, Py_ssize_t n) {
     c10::SmallVector<int64_t, 4> shape(x.sizes().begin(), x.sizes().end());
     shape.back() = N;
     const Tensor y = at::empty(shape, x.options());
-    const int rc = we_linear(x.data_ptr(), xs, w.data_ptr(), w.stride(0), y.data_ptr(), N, (int)M, (int)N, (int)K,
-                             dtype_code(x), stream_of(x.device()));
+    const int rc = call_library([&] { return we_linear(x.data_ptr(), xs, w.data_ptr(), w.stride(0), y.data_ptr(), N, (int)M, (int)N, (int)K,
+                             dtype_code(x), stream_of(x.device())); });
     if (rc == WE_ERR_ALIGNMENT || rc == WE_ERR_UNSUPPORTED || rc == WE_ERR_BAD_SHAPE) return none();
     if (rc != WE_OK) fail_code("we_linear", rc);
     return wrap(y);
