@@ -356,7 +356,9 @@ int we_linear(const void* x, int64_t x_row_stride, const void* w, int64_t w_row_
  *            order and 2 * ticket + 1 when they are refused, as soon as the call's first kernel
  *            knows (long before its last kernel ends).
  *   ticket   any value that tells this call's verdict from an earlier one's in the same word.
- *   guard    one word of device memory no other call in flight uses.
+ *   guard    we_pos_check_guard_bytes(...) bytes of device memory that are the call's own until its last
+ *            kernel is done - well after the report: the kernels behind the first read the verdict
+ *            there.  Nothing in it has to start at any value; may be NULL when that is 0.
  * A refused call leaves kv, `written` and q_out as they were; the attention output is undefined.
  * The _checked entry points are the ones without the suffix plus this argument (NULL = no check);
  * waiting for the report is the caller's business.
@@ -369,6 +371,13 @@ typedef struct we_pos_check {
   uint64_t ticket;
   uint32_t* guard;
 } we_pos_check;
+
+/*
+ * Bytes `guard` has to have for a checked call on B x T position ids (with_projection: for
+ * we_qkv_rope_kv_attn_fwd_checked).  0: the workgroups of the call's first kernel all look at the ids
+ * themselves and pass nothing on.
+ */
+size_t we_pos_check_guard_bytes(int32_t B, int32_t T, int32_t with_projection);
 
 int we_rope_kv_store_checked(const void* q, const void* k, const void* v,
                              const int64_t q_strides[3], const int64_t k_strides[3],

@@ -270,6 +270,24 @@ def test_one_call_entry_point_validates_both_halves():
     assert lib.we_rope_kv_attn_fwd(*args(extras=ctypes.byref(ex))) == -2
 
 
+def test_guard_memory_of_the_position_id_check():
+    """A check whose verdict goes to later kernels needs a word of the call's own; one that the store's workgroups
+    make themselves needs none."""
+    lib = _capi.lib()
+
+    class PosCheck(ctypes.Structure):
+        _fields_ = [("what", ctypes.c_int32), ("report", ctypes.c_void_p), ("ticket", ctypes.c_uint64), ("guard", ctypes.c_void_p)]
+
+    for B, T, proj, need in ((1, 768, 0, 0), (3, 256, 0, 0), (1, 769, 0, 4), (4, 193, 0, 4), (1, 8, 1, 4)):
+        assert lib.we_pos_check_guard_bytes(B, T, proj) == need, (B, T, proj)
+    s3 = _capi.i64x3(16, 16, 16)
+    fake = ctypes.c_void_p(4096)     # never dereferenced: validation fails first
+    args = lambda T, check: [fake, s3, fake, fake, fake, 10, fake, fake, fake, T, 8, 8, 1, 1, T, 64, 0, ctypes.byref(check), None]
+    assert lib.we_rope_apply_checked(*args(1024, PosCheck(2, 4096, 1, None))) == -1
+    assert lib.we_rope_apply_checked(*args(64, PosCheck(2, None, 1, 4096))) == -1
+    assert lib.we_rope_apply_checked(*args(64, PosCheck(4, 4096, 1, 4096))) == -3
+
+
 def test_stream_probe_validates_before_launching():
     """The tile-stream probe of the measurement library refuses bad arguments with a status code (no GPU needed)."""
     lib = _capi.probe_lib()

@@ -156,3 +156,48 @@ def test_more_checked_calls_at_once_than_records(gpu_device):
     [t.join(60) for t in threads]
     assert not failures and not any(t.is_alive() for t in threads), failures
     assert all(torch.equal(o, outs[0]) for o in outs)
+
+
+@pytest.mark.parametrize("path,T", [("store", 1024), ("project", 256)])
+def test_a_verdict_stays_with_its_call(gpu_device, path, T):
+    """Calls whose verdict goes through device memory (many ids, or a projection in front), good ones on one stream
+    and refused ones on another at the same time: every good frame is stored whole, no refused one at all."""
+    dev = gpu_device
+    H, Dh, W, calls = 8, 64, 32, 60
+    rope = wea.RoPE(*ro.rope_table_1d(4 * T, Dh), T // W, W).to(dev)
+    good = to_dev(ro.synth_pos_ids(1, 1, T, W), dev)
+    bad = dict(good, t_pos=torch.full_like(good["t_pos"], 4))
+    layers = [wea.LayerKVCache(1, H, 2 * T, Dh, torch.bfloat16, T).to(dev) for _ in range(2)]
+    v = [torch.full((1, H, T, Dh), 1.0 + n, device=dev, dtype=torch.bfloat16) for n in range(calls)]
+    eye = torch.cat([torch.eye(H * Dh, device=dev, dtype=torch.bfloat16)] * 3)      # q = k = v = x
+    x = [t.transpose(1, 2).reshape(1, T, H * Dh) for t in v]
+    tails, failures = [], []
+    torch.cuda.synchronize()
+
+    def call(layer, n, pos):
+        if path == "store":
+            layer.rope_upsert(v[n], v[n], v[n], pos, rope, True)
+        else:
+            layer.qkv_rope_upsert_attend(x[n], eye, H, pos, rope, True)
+
+    def work(which):
+        try:
+            stream = torch.cuda.Stream()
+            with torch.cuda.stream(stream):
+                for n in range(calls):
+                    if which == 0:
+                        call(layers[0], n, good)
+                        tails.append(layers[0].kv[1, :, :, layers[0].L:].clone())
+                    else:
+                        with pytest.raises(IndexError):
+                            call(layers[1], n, bad)
+                stream.synchronize()
+        except BaseException as e:      # noqa: BLE001 - reported by the main thread
+            failures.append((which, repr(e)))
+
+    threads = [threading.Thread(target=work, args=(i,), daemon=True) for i in range(2)]
+    [t.start() for t in threads]
+    [t.join(60) for t in threads]
+    assert not failures and not any(t.is_alive() for t in threads), failures
+    assert all(torch.equal(t, v[n]) for n, t in enumerate(tails)), "a good frame was not stored whole"
+    assert not layers[1].kv.any(), "a refused frame was stored"

@@ -268,16 +268,18 @@ struct Extras {
 };
 
 // ---- verdicts of the position-id check -------------------------------------------------------
-// A call that checks holds one of a device's records while it runs: a word of host-coherent memory
-// the device reports to and a word of device memory the kernels pass the verdict on in.  The
-// records are made on a device's first checked call and live as long as the process; a call that
-// finds all of them out waits for one, without the interpreter's lock.
+// A call that checks holds one of a device's records until it has its verdict: a word of host-coherent
+// memory, which one of the call's kernels writes once.  The records are made on a device's first
+// checked call and live as long as the process; a call that finds all of them out waits for one,
+// without the interpreter's lock.
+// The device word in which the verdict goes on to the call's later kernels is read long after the
+// host has had its report, so it cannot be a record's: it is memory from torch's allocator, which
+// hands it out again only to work that the stream runs behind this call's.
 constexpr int kVerdicts = we::RecordSlots::kCount;
 constexpr int kMaxDevices = 64;
 struct Verdicts {
   we::RecordSlots slots;
   uint64_t* report = nullptr;   // kVerdicts words, one per 64 bytes
-  uint32_t* guard = nullptr;    // likewise, on the device
   uint64_t ticket[kVerdicts] = {};
 };
 std::atomic<Verdicts*> g_verdicts[kMaxDevices];
@@ -291,13 +293,11 @@ Verdicts& verdicts(c10::Device dev) {
   std::lock_guard<std::mutex> lock(g_mu);
   p = g_verdicts[d].load(std::memory_order_acquire);
   if (p != nullptr) return *p;
-  void *host = nullptr, *dv = nullptr;
-  if (hipHostMalloc(&host, kVerdicts * 64, hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess ||
-      hipMalloc(&dv, kVerdicts * 64) != hipSuccess)
+  void* host = nullptr;
+  if (hipHostMalloc(&host, kVerdicts * 64, hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess)
     fail("cannot allocate the position-id check's records");
   Verdicts* made = new Verdicts;
   made->report = static_cast<uint64_t*>(host);
-  made->guard = static_cast<uint32_t*>(dv);
   for (int i = 0; i < kVerdicts * 8; ++i) made->report[i] = 0;
   g_verdicts[d].store(made, std::memory_order_release);
   return *made;
@@ -305,9 +305,12 @@ Verdicts& verdicts(c10::Device dev) {
 
 class PosCheck {
  public:
-  // what: WE_CHECK_* bits; nothing is checked under stream capture (the verdict could not be waited for)
-  PosCheck(int what, c10::Device dev, hipStream_t st) : st_(st) {
+  // what: WE_CHECK_* bits, for a call on B x T ids on dev's current stream st; nothing is checked under
+  // stream capture (the verdict could not be waited for)
+  PosCheck(int what, c10::Device dev, hipStream_t st, int64_t B, int64_t T, bool with_projection) : st_(st) {
     if (what == 0 || capturing(st)) return;
+    const size_t bytes = we_pos_check_guard_bytes((int)B, (int)T, with_projection ? 1 : 0);
+    if (bytes != 0) guard_ = at::empty({(int64_t)bytes}, at::TensorOptions().dtype(at::kByte).device(dev));
     v_ = &verdicts(dev);
     slot_ = v_->slots.take([](auto&& wait) {
       const NoGil off;
@@ -315,7 +318,7 @@ class PosCheck {
     });
     c_.what = what;
     c_.report = v_->report + slot_ * 8;
-    c_.guard = v_->guard + slot_ * 16;
+    c_.guard = guard_.defined() ? reinterpret_cast<uint32_t*>(guard_.data_ptr()) : nullptr;
     c_.ticket = ++v_->ticket[slot_];
   }
   ~PosCheck() {
@@ -362,6 +365,7 @@ class PosCheck {
   Verdicts* v_ = nullptr;
   int slot_ = 0;
   bool awaited_ = false;
+  Tensor guard_;
   we_pos_check c_{};
 };
 
@@ -434,7 +438,7 @@ PyObject* rope_kv_store(PyObject*, PyObject* const* argv, Py_ssize_t n) {
     const int64_t H = q != nullptr ? q->size(1) : Hkv;
     Tensor q_out;
     if (q != nullptr) q_out = new_heads(*q, B, H, T, Dh);
-    PosCheck check(what, dev, st);
+    PosCheck check(what, dev, st, B, T, false);
     const int rc = call_library([&] { return we_rope_kv_store_checked(
         q != nullptr ? q->data_ptr() : nullptr, k.data_ptr(), v.data_ptr(), q != nullptr ? qs.s : nullptr, ks.s, vs.s,
         q != nullptr ? q_out.data_ptr() : nullptr, rotate ? cos->const_data_ptr<float>() : nullptr,
@@ -467,7 +471,7 @@ PyObject* rope_apply(PyObject*, PyObject* const* argv, Py_ssize_t n) {
     const hipStream_t st = stream_of(dev);
     const Tensor cos = cos_in.contiguous(), sin = sin_in.contiguous();
     const Tensor out = new_heads(x, B, H, T, Dh);
-    PosCheck check(what, dev, st);
+    PosCheck check(what, dev, st, B, T, false);
     const int rc = call_library([&] { return we_rope_apply_checked(x.data_ptr(), xs.s, out.data_ptr(), cos.const_data_ptr<float>(),
                                          sin.const_data_ptr<float>(), cos.size(0), pos.tp(), pos.yp(), pos.xp(),
                                          pos.row_stride, gh, gw, (int)B, (int)H, (int)T, (int)Dh, code_t, check.arg(), st); });
@@ -585,7 +589,7 @@ PyObject* rope_kv_attn(PyObject*, PyObject* const* argv, Py_ssize_t n) {
     }
     const Tensor out = output_or_new(out_in, token_major, q, dev, B, H, T, Dh);
     const Strides os(out, "out");
-    PosCheck check(what, dev, st);
+    PosCheck check(what, dev, st, B, T, false);
     const int rc = call_library([&] { return we_rope_kv_attn_fwd_checked(
         q.data_ptr(), k.data_ptr(), v.data_ptr(), qs.s, ks.s, vs.s, q_rot.data_ptr(), cos.const_data_ptr<float>(),
         sin.const_data_ptr<float>(), cos.size(0), pos.tp(), pos.yp(), pos.xp(), pos.row_stride, gh, gw, kv.data_ptr(),
@@ -646,7 +650,7 @@ PyObject* qkv_rope_kv_attn(PyObject*, PyObject* const* argv, Py_ssize_t n) {
       for (int i = 0; i < 3; ++i) proj.v_out_strides[i] = s.s[i];
     }
     Tensor out;
-    PosCheck check(what, dev, st);
+    PosCheck check(what, dev, st, B, T, true);
     if (!attend) {
       const int rc = call_library([&] { return we_qkv_rope_kv_store(&proj, q_rot.data_ptr(), cos.const_data_ptr<float>(), sin.const_data_ptr<float>(),
                                           cos.size(0), pos.tp(), pos.yp(), pos.xp(), pos.row_stride, gh, gw, kv.data_ptr(),

@@ -90,23 +90,26 @@ int prepare_store(const void* q, const void* k, const void* v, const int64_t* q_
 // costs all of them.
 constexpr int64_t kCheckInStore = 768;
 
-int check_args_ok(const we_pos_check* c, const we::StoreParams& p) {
+bool checked_in_store(int64_t B, int64_t T, bool with_projection) { return !with_projection && B * T <= kCheckInStore; }
+
+int check_args_ok(const we_pos_check* c, bool with_projection, const we::StoreParams& p) {
   if (!c || c->what == 0) return WE_OK;
-  if (!c->report || !c->guard) return WE_ERR_NULL_POINTER;
+  if (!c->report || (!c->guard && !checked_in_store(p.B, p.T, with_projection))) return WE_ERR_NULL_POINTER;
   if ((c->what & ~(WE_CHECK_FRAME | WE_CHECK_TABLE)) != 0) return WE_ERR_UNSUPPORTED;
   if ((c->what & WE_CHECK_TABLE) != 0 && (!p.cos_t || !p.y_pos || !p.x_pos)) return WE_ERR_NULL_POINTER;
   return WE_OK;
 }
 
 // Puts the check (arguments already validated) into the call whose store parameters are `p`:
-// inside its kernel, or as a launch in front of it.
-int apply_check(const we_pos_check* c, bool in_kernel, we::StoreParams& p, hipStream_t st) {
+// inside its kernel, or as a launch in front of it whose verdict the call's other kernels read from the
+// guard word (which therefore has to be the call's own until the last of them is done).
+int apply_check(const we_pos_check* c, bool with_projection, we::StoreParams& p, hipStream_t st) {
   if (!c || c->what == 0) return WE_OK;
   p.check = c->what;
   p.report = c->report;
   p.ticket = c->ticket;
   if (!p.y_pos || !p.x_pos) p.y_pos = p.x_pos = p.t_pos;  // (no table rules: loaded, not looked at)
-  if (in_kernel && (int64_t)p.B * p.T <= kCheckInStore) return WE_OK;
+  if (checked_in_store(p.B, p.T, with_projection)) return WE_OK;
   if (we::launch_pos_check(p, c->guard, st) != hipSuccess) return WE_ERR_LAUNCH;
   p.guard = c->guard;
   return WE_OK;
@@ -246,9 +249,9 @@ int we_rope_kv_store_checked(const void* q, const void* k, const void* v, const 
   int rc = prepare_store(q, k, v, q_strides, k_strides, v_strides, q_out, cos_table, sin_table, table_rows,
                          t_pos, y_pos, x_pos, pos_stride_b, grid_h, grid_w, kv, written, B, H, Hkv, T, Dh,
                          L, dilation, is_frozen, dtype, p);
-  if (rc == WE_OK) rc = check_args_ok(check, p);
+  if (rc == WE_OK) rc = check_args_ok(check, false, p);
   hipStream_t st = static_cast<hipStream_t>(stream);
-  if (rc == WE_OK) rc = apply_check(check, true, p, st);
+  if (rc == WE_OK) rc = apply_check(check, false, p, st);
   if (rc != WE_OK) return rc;
   return we::launch_rope_kv_store(p, dtype, st) == hipSuccess ? WE_OK : WE_ERR_LAUNCH;
 }
@@ -289,10 +292,14 @@ int we_rope_apply_checked(const void* x, const int64_t x_strides[3], void* x_out
   p.B = B; p.H = H; p.Hkv = 0; p.T = T; p.Dh = Dh;
   p.dilation = 1; p.num_buckets = 1; p.frozen = 1;
   hipStream_t st = static_cast<hipStream_t>(stream);
-  int rc = check_args_ok(check, p);
-  if (rc == WE_OK) rc = apply_check(check, true, p, st);
+  int rc = check_args_ok(check, false, p);
+  if (rc == WE_OK) rc = apply_check(check, false, p, st);
   if (rc != WE_OK) return rc;
   return we::launch_rope_kv_store(p, dtype, st) == hipSuccess ? WE_OK : WE_ERR_LAUNCH;
+}
+
+size_t we_pos_check_guard_bytes(int32_t B, int32_t T, int32_t with_projection) {
+  return checked_in_store(B, T, with_projection != 0) ? 0 : sizeof(uint32_t);
 }
 
 int we_init(void) { return we::host::init_current_device(); }
@@ -419,13 +426,13 @@ int we_rope_kv_attn_fwd_checked(const void* q, const void* k, const void* v, con
     rc = apply_gate_extras(extras, dtype, p);
     if (rc != WE_OK) return rc;
   }
-  rc = check_args_ok(check, sp);
+  rc = check_args_ok(check, false, sp);
   if (rc != WE_OK) return rc;
   if (dev.rc != WE_OK) return dev.rc;
   // Everything is validated before the first launch; the kernels follow each other on the stream.
   // (A call whose position ids the check refuses stores nothing; its attention output is garbage,
   // which the caller learns from the report.)
-  rc = apply_check(check, true, sp, st);
+  rc = apply_check(check, false, sp, st);
   if (rc != WE_OK) return rc;
   if (we::launch_rope_kv_store(sp, dtype, st) != hipSuccess) return WE_ERR_LAUNCH;
   return launch_attn(p, pl, Dh, dtype, st);
@@ -480,10 +487,10 @@ int we_qkv_rope_kv_attn_fwd_checked(const we_qkv_proj* proj, void* q_out, const 
                     H, Hkv, T, Dh, L, dilation, scale, n_splits, q_tile, dtype, p, pl);
   if (rc != WE_OK) return rc;
   rc = apply_gate_extras(extras, dtype, p);
-  if (rc == WE_OK) rc = check_args_ok(check, pp.s);
+  if (rc == WE_OK) rc = check_args_ok(check, true, pp.s);
   if (rc != WE_OK) return rc;
   if (dev.rc != WE_OK) return dev.rc;
-  rc = apply_check(check, false, pp.s, st);
+  rc = apply_check(check, true, pp.s, st);
   if (rc != WE_OK) return rc;
   if (we::launch_qkv_rope_store(pp, dtype, st) != hipSuccess) return WE_ERR_LAUNCH;
   return launch_attn(p, pl, Dh, dtype, st);
