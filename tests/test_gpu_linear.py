@@ -3,12 +3,17 @@ of contraction slots: operands whose fp32 sums are exact must give the product's
 shapes that do not fit one round of workgroups are left to the library."""
 import pytest
 import torch
+from torch import nn
+from torch.utils._python_dispatch import TorchDispatchMode
+from torch.overrides import TorchFunctionMode
 
 from world_engine_amd._capi import native
+from world_engine_amd.attn import _plain, _project
 
-pytestmark = pytest.mark.gpu
+gpu = pytest.mark.gpu
 
 
+@gpu
 @pytest.mark.parametrize("M,N,K,dtype", [
     (1, 32, 128, torch.bfloat16), (63, 32, 256, torch.float16), (64, 96, 384, torch.bfloat16), (65, 64, 512, torch.bfloat16),
     (130, 4096, 640, torch.float16), (256, 4096, 768, torch.bfloat16), (257, 6144, 896, torch.bfloat16), (64, 4096, 2048, torch.float16),
@@ -25,6 +30,7 @@ def test_linear_is_exact_on_exact_operands(gpu_device, M, N, K, dtype):
         assert torch.equal(y.reshape(M, N), ref)
 
 
+@gpu
 def test_linear_leaves_other_shapes_to_the_library(gpu_device):
     x = torch.zeros(1025, 256, device=gpu_device, dtype=torch.bfloat16)
     assert native.linear(x, torch.zeros(32, 256, device=gpu_device, dtype=torch.bfloat16)) is None         # many rows
@@ -36,3 +42,89 @@ def test_linear_leaves_other_shapes_to_the_library(gpu_device):
     assert native.linear(x[:8], w) is None                                                                  # a gradient to record
     with torch.no_grad():
         assert native.linear(x[:8], w).shape == (8, 32)
+
+
+class Doubled(torch.Tensor):
+    """A weight whose product is not that of its memory, as a quantised or distributed tensor's is not."""
+    @classmethod
+    def __torch_function__(cls, func, types, args=(), kwargs=None):
+        out = super().__torch_function__(func, types, args, kwargs)
+        return out.as_subclass(torch.Tensor) * 2 if func is nn.functional.linear else out
+
+
+def _doubling_forward(lin):
+    inner = lin.forward
+    lin.forward = lambda x: inner(x) * 2
+
+
+def _doubling_subclass(lin):
+    w = lin.weight.detach().as_subclass(Doubled)
+    del lin.weight
+    lin.weight = w
+
+
+# how -> change of a layer that doubles what a call of it returns; the hook of every module is undone by the caller
+DOUBLING = {
+    "instance forward": _doubling_forward,
+    "forward hook": lambda lin: lin.register_forward_hook(lambda m, a, y: y * 2),
+    "forward pre-hook": lambda lin: lin.register_forward_pre_hook(lambda m, a: (a[0] * 2,)),
+    "hook of every module": lambda lin: nn.modules.module.register_module_forward_hook(lambda m, a, y: y * 2),
+    "class forward": lambda lin: setattr(nn.Linear, "forward", lambda self, x: nn.functional.linear(x, self.weight) * 2),
+    "weight subclass": _doubling_subclass,
+    "subclass of the layer": lambda lin: setattr(lin, "__class__", type("Twice", (nn.Linear,), {
+        "forward": lambda self, x: nn.functional.linear(x, self.weight) * 2})),
+}
+
+
+@pytest.mark.parametrize("how", DOUBLING)
+def test_a_layer_that_is_more_than_its_weight_is_called(how, device="cpu"):
+    lin = nn.Linear(256, 64, bias=False, dtype=torch.bfloat16, device=device).requires_grad_(False)
+    x = torch.randn(8, 256, dtype=torch.bfloat16, device=device)
+    assert _plain(lin)
+    want = _project(lin, x) * 2
+    forward, undo = nn.Linear.forward, DOUBLING[how](lin)
+    try:
+        assert not _plain(lin)
+        got = _project(lin, x)
+    finally:
+        nn.Linear.forward = forward
+        if hasattr(undo, "remove"):
+            undo.remove()
+    assert torch.allclose(got.float(), want.float(), rtol=2 ** -7, atol=2 ** -7)   # (two kernels' order of additions: 1 ulp)
+
+
+@gpu
+@pytest.mark.parametrize("how", DOUBLING)
+def test_a_layer_that_is_more_than_its_weight_is_called_on_the_gpu(gpu_device, how):
+    test_a_layer_that_is_more_than_its_weight_is_called(how, gpu_device)
+
+
+@gpu
+def test_linear_leaves_watched_operations_to_torch(gpu_device):
+    """Modes that see torch's operations, forward-mode tangents and functorch's wrappers: the operation stays torch's."""
+    class Watch(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            seen.append(str(func))
+            return func(*args, **(kwargs or {}))
+
+    class WatchFunctions(TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            seen.append(getattr(func, "__name__", ""))
+            return func(*args, **(kwargs or {}))
+
+    seen = []
+    lin = nn.Linear(256, 64, bias=False, dtype=torch.bfloat16, device=gpu_device).requires_grad_(False)
+    x = torch.randn(8, 256, dtype=torch.bfloat16, device=gpu_device)
+    assert native.linear(x, lin.weight) is not None
+    with Watch():
+        _project(lin, x)
+    assert any("mm" in s for s in seen), seen
+    seen.clear()
+    with WatchFunctions():
+        _project(lin, x)
+    assert "linear" in seen, seen
+    t = torch.randn_like(x)
+    y, dy = torch.func.jvp(lambda a: _project(lin, a), (x,), (t,))
+    assert torch.allclose(dy.float(), nn.functional.linear(t, lin.weight).float(), rtol=2 ** -7, atol=2 ** -7)
+    z = torch.func.vmap(lambda a: _project(lin, a))(torch.stack([x, t]))
+    assert torch.allclose(z[1].float(), dy.float(), rtol=2 ** -7, atol=2 ** -7)

@@ -136,9 +136,18 @@ def ring_attention(q: Tensor, k: Tensor, v: Tensor, block_mask: RingMask, enable
                          block_mask.dilation, scale)
 
 
+_LINEAR_FORWARD = nn.Linear.forward
+
+
 def _plain(lin: nn.Module) -> bool:
-    """A linear layer that is nothing but its weight: no bias, no hooks, no replacement of the class."""
-    return type(lin) is nn.Linear and lin.bias is None and not lin._forward_hooks and not lin._forward_pre_hooks
+    """A linear layer that is nothing but its weight, so that the product alone stands for a call of it: no bias, no
+    other class or ``forward`` in its place (of the class or of this instance, which is how wrapping libraries hook
+    in), no hook of its own or of every module, and an ordinary tensor as weight (a subclass - quantised, distributed
+    - has a product of its own)."""
+    return (type(lin) is nn.Linear and lin.bias is None and "forward" not in lin.__dict__
+            and nn.Linear.forward is _LINEAR_FORWARD and type(lin.weight) in (nn.Parameter, Tensor)
+            and not (lin._forward_hooks or lin._forward_pre_hooks or lin._backward_hooks or lin._backward_pre_hooks)
+            and not nn.modules.module._has_any_global_hook())
 
 
 @torch.compiler.assume_constant_result
@@ -151,7 +160,7 @@ def _project(lin: nn.Module, x: Tensor) -> Tensor:
     """``lin(x)``, on the library's own kernel where the frame is small enough for it to be the faster one
     (one round of workgroups; 256 x 2048 x 2048: 8.2 us against 9.6 on the GPU, and 4 against 19 us of the
     host's time, most of it the BLAS routine's choice of a kernel).  fp32 sums rounded once, as there."""
-    if _plain(lin) and not torch.is_autocast_enabled():
+    if type(x) is Tensor and _plain(lin) and not torch.is_autocast_enabled():
         if torch.compiler.is_compiling():        # the opaque op where the kernel covers the shape, for the same bits as eager
             if (x.dtype in (torch.bfloat16, torch.float16) and lin.weight.dtype == x.dtype and not torch.is_grad_enabled()
                     and _kernel_covers(x.numel() // x.shape[-1], lin.out_features, x.shape[-1], x.dtype is torch.float16)):

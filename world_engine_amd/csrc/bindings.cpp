@@ -8,10 +8,12 @@
 // that kernel's verdict only, while the attention behind it is already running.
 #include <torch/csrc/autograd/python_variable.h>
 
+#include <ATen/PythonTorchFunctionTLS.h>
 #include <ATen/core/Tensor.h>
 #include <ATen/core/grad_mode.h>
 #include <ATen/ops/empty.h>
 #include <ATen/ops/empty_strided.h>
+#include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <c10/hip/HIPStream.h>
 #include <hip/hip_runtime_api.h>
 
@@ -673,13 +675,21 @@ PyObject* qkv_rope_kv_attn(PyObject*, PyObject* const* argv, Py_ssize_t n) {
   });
 }
 
+// A tensor that is its memory and nothing else: no Python subclass or functorch wrapper that would
+// see the operation, no tangent, no lazily negated view.
+bool plain_memory(const Tensor& t) {
+  return t.has_storage() && !t.unsafeGetTensorImpl()->is_python_dispatch() && !t.is_neg() && !t._fw_grad(/*level=*/0).defined();
+}
+
 // x [..., K] times w [N, K] transposed; None where the kernel is not the one to use (shape, layout,
-// element type, a gradient to record): the caller then takes its linear layer.
+// element type, a gradient to record, somebody who watches torch's operations): the caller then takes
+// its linear layer.
 PyObject* linear(PyObject*, PyObject* const* argv, Py_ssize_t n) {
   return guarded([&]() -> PyObject* {
     Args a("linear", argv, n, 2);
     const Tensor &x = a.tensor(), &w = a.tensor();
-    if (!x.is_cuda() || w.device() != x.device() || x.dim() < 2 || w.dim() != 2) return none();
+    if (c10::impl::TorchDispatchModeTLS::any_modes_set() || at::impl::torch_function_mode_enabled()) return none();
+    if (!x.is_cuda() || w.device() != x.device() || !plain_memory(x) || !plain_memory(w) || x.dim() < 2 || w.dim() != 2) return none();
     const at::ScalarType dt = x.scalar_type();
     if ((dt != at::kBFloat16 && dt != at::kHalf) || w.scalar_type() != dt) return none();
     if (at::GradMode::is_enabled() && (x.requires_grad() || w.requires_grad())) return none();
