@@ -296,6 +296,19 @@ class RingAttn(nn.Module):
     def uses_fused_projection(self, B: int, T: int) -> bool:
         return self.fuse_projection and self.projection_workgroups(B, T) <= self.fused_projection_max_workgroups
 
+    def _records(self, x: Tensor) -> bool:
+        """Whether this call's operations are recorded for a backward pass (through the gate and ``out_proj``:
+        nothing is recorded through the attention)."""
+        return torch.is_grad_enabled() and (x.requires_grad or any(p.requires_grad for p in self.parameters()))
+
+    def _gate_is_the_kernels(self, x: Tensor, q: Tensor) -> bool:
+        """Whether the attention kernels' epilogue can stand for ``sigmoid(gate_proj(x[..., :H]))`` and the product
+        with it: the layer is its weight alone, all of one half-precision type and in the layout the kernels read,
+        and nothing of it is recorded."""
+        return (x.dtype != torch.float32 and x.stride(-1) == 1 and _plain(self.gate_proj) and not torch.is_autocast_enabled()
+                and self.gate_proj.weight.is_contiguous() and not self._records(x)
+                and native.plain(x, self.gate_proj.weight, q))
+
     def forward(self, x: Tensor, pos_ids: Mapping[str, Tensor], v1: Optional[Tensor], kv_cache):
         B, T = x.shape[:2]
         if (self.uses_fused_projection(B, T) and hasattr(kv_cache, "qkv_rope_upsert_attend")
@@ -331,13 +344,14 @@ class RingAttn(nn.Module):
 
         gates = None
         if self.gated_attn:
-            if inside and x.dtype != torch.float32 and (fuse or _plain(self.gate_proj)):
+            if fuse or (inside and self._gate_is_the_kernels(x, q)):
                 # projection, sigmoid and multiply in the kernels' epilogues
                 extras.update(gate_x=x[..., :H], gate_w=self.gate_proj.weight)
             else:
                 gates = torch.sigmoid(self.gate_proj(x[..., :H])).permute(0, 2, 1)
-                if inside:                       # the epilogue multiplies the rounded output, as `y * gates` would
-                    extras["gate"] = gates
+                if inside and not self._records(x) and native.plain(gates, q):
+                    extras["gate"] = gates       # the epilogue multiplies the rounded output, as `y * gates` would
+                    gates = None
         if fuse:
             extras["qk_norm_eps"] = torch.finfo(torch.float32).eps     # F.rms_norm's epsilon for these inputs
 
@@ -349,7 +363,7 @@ class RingAttn(nn.Module):
         else:
             q, k_all, v_all, ring = kv_cache.rope_upsert(q, k, v, pos_ids, self.rope, self.layer_idx)
             y = ring_attention(q, k_all, v_all, ring, enable_gqa=self.enable_gqa)
-        if gates is not None and not inside:
+        if gates is not None:
             y = y * gates.unsqueeze(-1)
 
         return _project(self.out_proj, y.transpose(1, 2).reshape(B, T, -1)), v1

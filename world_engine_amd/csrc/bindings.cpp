@@ -371,6 +371,15 @@ class PosCheck {
   we_pos_check c_{};
 };
 
+// A tensor that is its memory and nothing else: no Python subclass or functorch wrapper that would
+// see the operation, no tangent, no lazily negated view.
+bool plain_memory(const Tensor& t) {
+  return t.has_storage() && !t.unsafeGetTensorImpl()->is_python_dispatch() && !t.is_neg() && !t._fw_grad(/*level=*/0).defined();
+}
+// Somebody sees every operation of this thread (dispatch and function modes).
+bool watched() { return c10::impl::TorchDispatchModeTLS::any_modes_set() || at::impl::torch_function_mode_enabled(); }
+bool to_record(const Tensor& t) { return at::GradMode::is_enabled() && t.requires_grad(); }
+
 // ---- results -------------------------------------------------------------------------------
 
 PyObject* wrap(const Tensor& t) { return THPVariable_Wrap(t); }
@@ -675,10 +684,21 @@ PyObject* qkv_rope_kv_attn(PyObject*, PyObject* const* argv, Py_ssize_t n) {
   });
 }
 
-// A tensor that is its memory and nothing else: no Python subclass or functorch wrapper that would
-// see the operation, no tangent, no lazily negated view.
-bool plain_memory(const Tensor& t) {
-  return t.has_storage() && !t.unsafeGetTensorImpl()->is_python_dispatch() && !t.is_neg() && !t._fw_grad(/*level=*/0).defined();
+// plain(t, ...): whether an operation on these tensors can be done on their memory without anybody
+// missing it - one element type and device, nobody watching, no gradient or tangent to carry on.
+PyObject* plain(PyObject*, PyObject* const* argv, Py_ssize_t n) {
+  return guarded([&]() -> PyObject* {
+    Args a("plain", argv, n, n);
+    bool ok = !watched();
+    const Tensor* first = nullptr;
+    for (Py_ssize_t i = 0; i < n && ok; ++i) {
+      const Tensor& t = a.tensor();
+      if (first == nullptr) first = &t;
+      ok = plain_memory(t) && !to_record(t) &&
+           t.scalar_type() == first->scalar_type() && t.device() == first->device();
+    }
+    return PyBool_FromLong(ok ? 1 : 0);
+  });
 }
 
 // x [..., K] times w [N, K] transposed; None where the kernel is not the one to use (shape, layout,
@@ -688,11 +708,11 @@ PyObject* linear(PyObject*, PyObject* const* argv, Py_ssize_t n) {
   return guarded([&]() -> PyObject* {
     Args a("linear", argv, n, 2);
     const Tensor &x = a.tensor(), &w = a.tensor();
-    if (c10::impl::TorchDispatchModeTLS::any_modes_set() || at::impl::torch_function_mode_enabled()) return none();
+    if (watched()) return none();
     if (!x.is_cuda() || w.device() != x.device() || !plain_memory(x) || !plain_memory(w) || x.dim() < 2 || w.dim() != 2) return none();
     const at::ScalarType dt = x.scalar_type();
     if ((dt != at::kBFloat16 && dt != at::kHalf) || w.scalar_type() != dt) return none();
-    if (at::GradMode::is_enabled() && (x.requires_grad() || w.requires_grad())) return none();
+    if (to_record(x) || to_record(w)) return none();
     const int64_t K = x.size(-1), N = w.size(0), M = K > 0 ? x.numel() / K : 0;
     const int64_t xs = x.stride(-2);
     if (w.size(1) != K || M <= 0 || M > (1 << 20) || N > (1 << 24) || x.stride(-1) != 1 || w.stride(1) != 1) return none();
@@ -715,6 +735,7 @@ PyObject* linear(PyObject*, PyObject* const* argv, Py_ssize_t n) {
 }
 
 PyMethodDef methods[] = {
+    {"plain", (PyCFunction)(void (*)(void))plain, METH_FASTCALL, nullptr},
     {"linear", (PyCFunction)(void (*)(void))linear, METH_FASTCALL, nullptr},
     {"rope_kv_store", (PyCFunction)(void (*)(void))rope_kv_store, METH_FASTCALL, nullptr},
     {"rope_apply", (PyCFunction)(void (*)(void))rope_apply, METH_FASTCALL, nullptr},
