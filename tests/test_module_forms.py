@@ -100,6 +100,38 @@ def test_the_gate_of_another_type_or_layout_stays_torchs():
     assert "gate_w" not in cache.asked and torch.equal(y, ref)
 
 
+def residual_rows(odd, device="cpu"):
+    """Value rows [1, H, T, DH] as an earlier layer hands them on, or the same values where a row starts off a 16-byte
+    boundary or its elements are not neighbours."""
+    r = torch.randn(1, H, T, DH, generator=torch.Generator().manual_seed(9)).to(device, torch.bfloat16)
+    if odd == "offset":
+        return F.pad(r, (1, 7))[..., 1:DH + 1]
+    if odd == "row stride":
+        return F.pad(r, (0, 1))[..., :DH]
+    return r.transpose(-1, -2).contiguous().transpose(-1, -2) if odd == "columns" else r
+
+
+@pytest.mark.parametrize("odd", ["offset", "row stride", "columns"])
+def test_value_rows_of_another_layout_are_blended_by_torch(odd):
+    cache, m = StandIn(), module().requires_grad_(False)
+    x = torch.randn(1, T, D, dtype=torch.bfloat16)
+    want, _ = m(x, None, residual_rows(""), cache)
+    assert "v1" in cache.asked
+    got, _ = m(x, None, residual_rows(odd), cache)
+    assert "v1" not in cache.asked and torch.equal(got, want)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("odd", ["offset", "row stride", "columns"])
+def test_value_rows_of_another_layout_on_the_kernels(gpu_device, odd):
+    m, cache, pos = on_gpu(gpu_device, value_residual=True)
+    x = torch.randn(1, T, D, device=gpu_device, dtype=torch.bfloat16)
+    with torch.no_grad():
+        want, _ = m(x, pos, residual_rows("", gpu_device), cache)
+        got, _ = m(x, pos, residual_rows(odd, gpu_device), cache)
+    assert torch.equal(got, want)
+
+
 def on_gpu(device, value_residual=False, **kw):
     m = module(device=device, value_residual=value_residual, **kw)
     cache = wea.StaticKVCache(config(value_residual=value_residual), 1, torch.bfloat16).to(device)

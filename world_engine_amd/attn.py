@@ -337,10 +337,12 @@ class RingAttn(nn.Module):
         extras = {}
         if self.value_residual and v1 is None:
             v1 = v                               # (lerp(v, v, w) is v)
-        elif self.value_residual and inside:     # same formula in fp32, rounded once: torch.lerp's bits
-            extras.update(v1=v1.view_as(v), v_lamb=self.v_lamb)
         elif self.value_residual:
-            v = torch.lerp(v, v1.view_as(v), self.v_lamb)
+            res = v1.view_as(v)
+            if fuse or (inside and native.plain(v, res, self.v_lamb) and native.aligned_rows(res)):
+                extras.update(v1=res, v_lamb=self.v_lamb)      # same formula in fp32, rounded once: torch.lerp's bits
+            else:
+                v = torch.lerp(v, res, self.v_lamb)
 
         gates = None
         if self.gated_attn:

@@ -701,6 +701,18 @@ PyObject* plain(PyObject*, PyObject* const* argv, Py_ssize_t n) {
   });
 }
 
+// aligned_rows(t): t is [B, H, T, Dh] with rows as the kernels read them, contiguous and 16-byte aligned.
+PyObject* aligned_rows(PyObject*, PyObject* const* argv, Py_ssize_t n) {
+  return guarded([&]() -> PyObject* {
+    Args a("aligned_rows", argv, n, 1);
+    const Tensor& t = a.tensor();
+    const int64_t per16 = 16 / (int64_t)t.element_size();
+    const bool ok = t.dim() == 4 && t.stride(3) == 1 && t.stride(0) % per16 == 0 && t.stride(1) % per16 == 0 &&
+                    t.stride(2) % per16 == 0 && (reinterpret_cast<uintptr_t>(t.const_data_ptr()) & 15u) == 0;
+    return PyBool_FromLong(ok ? 1 : 0);
+  });
+}
+
 // x [..., K] times w [N, K] transposed; None where the kernel is not the one to use (shape, layout,
 // element type, a gradient to record, somebody who watches torch's operations): the caller then takes
 // its linear layer.
@@ -736,6 +748,7 @@ PyObject* linear(PyObject*, PyObject* const* argv, Py_ssize_t n) {
 
 PyMethodDef methods[] = {
     {"plain", (PyCFunction)(void (*)(void))plain, METH_FASTCALL, nullptr},
+    {"aligned_rows", (PyCFunction)(void (*)(void))aligned_rows, METH_FASTCALL, nullptr},
     {"linear", (PyCFunction)(void (*)(void))linear, METH_FASTCALL, nullptr},
     {"rope_kv_store", (PyCFunction)(void (*)(void))rope_kv_store, METH_FASTCALL, nullptr},
     {"rope_apply", (PyCFunction)(void (*)(void))rope_apply, METH_FASTCALL, nullptr},
