@@ -89,6 +89,25 @@ def test_the_gate_keeps_its_gradient(dtype, trained):
     assert torch.allclose(leaf.grad.float(), ref.float(), rtol=2e-2, atol=2e-2 * ref.abs().max().item())
 
 
+@pytest.mark.parametrize("gated", [False, True])
+def test_a_later_call_leaves_a_recorded_output_alone(gated):
+    """What ``out_proj`` (or the gate's product) saved for the backward pass is not the layer's reused buffer."""
+    cache, m = StandIn(), module(gated_attn=gated)
+    xs = [torch.randn(1, T, D, dtype=torch.bfloat16) for _ in range(2)]
+    grads = []
+    for later_call in (False, True):
+        m.zero_grad()
+        y, _ = m(xs[0], None, None, cache)
+        if later_call:
+            m(xs[1], None, None, cache)
+        y.float().sum().backward()
+        grads.append(m.out_proj.weight.grad.clone())
+    assert torch.equal(grads[0], grads[1])
+    with torch.no_grad():
+        m(xs[0], None, None, cache)
+    assert cache.asked["reuse_buffers"]
+
+
 def test_the_gate_of_another_type_or_layout_stays_torchs():
     cache, m = StandIn(), module().requires_grad_(False)
     x = torch.randn(1, D, T, dtype=torch.bfloat16).transpose(1, 2)            # channels not contiguous

@@ -284,7 +284,7 @@ class RingAttn(nn.Module):
         if self.gated_attn:
             extras.update(gate_x=x[..., : self.n_heads], gate_w=self.gate_proj.weight)
         y, v = kv_cache.qkv_rope_upsert_attend(x, self.qkv_proj.weight, self.n_heads, pos_ids, self.rope,
-                                               self.layer_idx, want_v=first, reuse_buffers=True, **extras)
+                                               self.layer_idx, want_v=first, reuse_buffers=not self._records(x), **extras)
         if first:
             v1 = v
         return _project(self.out_proj, y.transpose(1, 2).reshape(B, T, -1)), v1
@@ -298,15 +298,16 @@ class RingAttn(nn.Module):
 
     def _records(self, x: Tensor) -> bool:
         """Whether this call's operations are recorded for a backward pass (through the gate and ``out_proj``:
-        nothing is recorded through the attention)."""
-        return torch.is_grad_enabled() and (x.requires_grad or any(p.requires_grad for p in self.parameters()))
+        nothing is recorded through the attention).  Under ``torch.compile`` the choices that hang on it are not made."""
+        return (not torch.compiler.is_compiling() and torch.is_grad_enabled()
+                and (x.requires_grad or any(p.requires_grad for p in self.parameters())))
 
-    def _gate_is_the_kernels(self, x: Tensor, q: Tensor) -> bool:
+    def _gate_is_the_kernels(self, x: Tensor, q: Tensor, records: bool) -> bool:
         """Whether the attention kernels' epilogue can stand for ``sigmoid(gate_proj(x[..., :H]))`` and the product
         with it: the layer is its weight alone, all of one half-precision type and in the layout the kernels read,
         and nothing of it is recorded."""
         return (x.dtype != torch.float32 and x.stride(-1) == 1 and _plain(self.gate_proj) and not torch.is_autocast_enabled()
-                and self.gate_proj.weight.is_contiguous() and not self._records(x)
+                and self.gate_proj.weight.is_contiguous() and not records
                 and native.plain(x, self.gate_proj.weight, q))
 
     def forward(self, x: Tensor, pos_ids: Mapping[str, Tensor], v1: Optional[Tensor], kv_cache):
@@ -334,6 +335,7 @@ class RingAttn(nn.Module):
 
         # The blend and the gate belong into the kernels (torch.compile has fusions of its own for them).
         inside = one_call and (fuse or not torch.compiler.is_compiling())
+        records = self._records(x)
         extras = {}
         if self.value_residual and v1 is None:
             v1 = v                               # (lerp(v, v, w) is v)
@@ -346,12 +348,12 @@ class RingAttn(nn.Module):
 
         gates = None
         if self.gated_attn:
-            if fuse or (inside and self._gate_is_the_kernels(x, q)):
+            if fuse or (inside and self._gate_is_the_kernels(x, q, records)):
                 # projection, sigmoid and multiply in the kernels' epilogues
                 extras.update(gate_x=x[..., :H], gate_w=self.gate_proj.weight)
             else:
                 gates = torch.sigmoid(self.gate_proj(x[..., :H])).permute(0, 2, 1)
-                if inside and not self._records(x) and native.plain(gates, q):
+                if inside and not records and native.plain(gates, q):
                     extras["gate"] = gates       # the epilogue multiplies the rounded output, as `y * gates` would
                     gates = None
         if fuse:
@@ -360,8 +362,10 @@ class RingAttn(nn.Module):
         # RoPE(q), RoPE(k), cache write (one launch) and attention over the ring (one or two), all
         # behind one library call; a cache without it gets the reference's sequence of calls
         if one_call:
-            # (y lives in the layer's own buffer until this layer's next call; out_proj below reads it now)
-            y = kv_cache.rope_upsert_attend(q, k, v, pos_ids, self.rope, self.layer_idx, reuse_buffers=True, **extras)
+            # (y lives in the layer's own buffer until this layer's next call; out_proj below reads it now - a
+            # backward pass would read it later)
+            y = kv_cache.rope_upsert_attend(q, k, v, pos_ids, self.rope, self.layer_idx,
+                                            reuse_buffers=not records, **extras)
         else:
             q, k_all, v_all, ring = kv_cache.rope_upsert(q, k, v, pos_ids, self.rope, self.layer_idx)
             y = ring_attention(q, k_all, v_all, ring, enable_gqa=self.enable_gqa)
