@@ -108,6 +108,16 @@ def test_a_later_call_leaves_a_recorded_output_alone(gated):
     assert cache.asked["reuse_buffers"]
 
 
+@pytest.mark.parametrize("gated", [False, True])
+def test_a_later_call_leaves_what_a_hook_kept_alone(gated):
+    cache, m = StandIn(), module(gated_attn=gated).requires_grad_(False)
+    kept = []
+    m.out_proj.register_forward_pre_hook(lambda lin, args: kept.append(args[0]))
+    for _ in range(2):
+        m(torch.randn(1, T, D, dtype=torch.bfloat16), None, None, cache)
+    assert not torch.equal(kept[0], kept[1])
+
+
 def test_the_gate_of_another_type_or_layout_stays_torchs():
     cache, m = StandIn(), module().requires_grad_(False)
     x = torch.randn(1, D, T, dtype=torch.bfloat16).transpose(1, 2)            # channels not contiguous

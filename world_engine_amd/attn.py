@@ -284,7 +284,8 @@ class RingAttn(nn.Module):
         if self.gated_attn:
             extras.update(gate_x=x[..., : self.n_heads], gate_w=self.gate_proj.weight)
         y, v = kv_cache.qkv_rope_upsert_attend(x, self.qkv_proj.weight, self.n_heads, pos_ids, self.rope,
-                                               self.layer_idx, want_v=first, reuse_buffers=not self._records(x), **extras)
+                                               self.layer_idx, want_v=first,
+                                               reuse_buffers=self._reads_output_at_once(self._records(x)), **extras)
         if first:
             v1 = v
         return _project(self.out_proj, y.transpose(1, 2).reshape(B, T, -1)), v1
@@ -301,6 +302,12 @@ class RingAttn(nn.Module):
         nothing is recorded through the attention).  Under ``torch.compile`` the choices that hang on it are not made."""
         return (not torch.compiler.is_compiling() and torch.is_grad_enabled()
                 and (x.requires_grad or any(p.requires_grad for p in self.parameters())))
+
+    def _reads_output_at_once(self, records: bool) -> bool:
+        """Whether nothing of this call reads the attention's output after ``out_proj``, so that it can live in the
+        layer's own buffer until the layer's next call: a backward pass would, and hooks or layers of another kind
+        may keep what they are given."""
+        return not records and _plain(self.out_proj)
 
     def _gate_is_the_kernels(self, x: Tensor, q: Tensor, records: bool) -> bool:
         """Whether the attention kernels' epilogue can stand for ``sigmoid(gate_proj(x[..., :H]))`` and the product
@@ -362,10 +369,8 @@ class RingAttn(nn.Module):
         # RoPE(q), RoPE(k), cache write (one launch) and attention over the ring (one or two), all
         # behind one library call; a cache without it gets the reference's sequence of calls
         if one_call:
-            # (y lives in the layer's own buffer until this layer's next call; out_proj below reads it now - a
-            # backward pass would read it later)
             y = kv_cache.rope_upsert_attend(q, k, v, pos_ids, self.rope, self.layer_idx,
-                                            reuse_buffers=not records, **extras)
+                                            reuse_buffers=self._reads_output_at_once(records), **extras)
         else:
             q, k_all, v_all, ring = kv_cache.rope_upsert(q, k, v, pos_ids, self.rope, self.layer_idx)
             y = ring_attention(q, k_all, v_all, ring, enable_gqa=self.enable_gqa)
