@@ -136,6 +136,14 @@ size_t we_attn_workspace_bytes(int32_t B, int32_t H, int32_t Hkv, int32_t T, int
                                int32_t n_splits, int32_t q_tile);
 
 /*
+ * The same for an element type: what lets an f16 call keep its partial results in fp32 (about twice
+ * the bytes above; an f16 call with a shorter workspace splits less where it can, and holds them in
+ * 16 bits otherwise), 0 for fp32 calls, which split nothing.
+ */
+size_t we_attn_workspace_bytes_for(int32_t B, int32_t H, int32_t Hkv, int32_t T, int32_t Dh, int64_t L,
+                                   int32_t n_splits, int32_t q_tile, int32_t dtype);
+
+/*
  * What the library would do with an attention call of these sizes (inspection helper without a
  * counterpart in the reference; launches nothing): plan[0] = queries per workgroup, [1] = context
  * parts of the units that are split, [2] = leading (batch, kv head) units left whole, [3] =
@@ -160,7 +168,8 @@ int we_attn_plan(int32_t B, int32_t H, int32_t Hkv, int32_t T, int32_t Dh, int64
  *   q    [B, H, T, Dh]   element strides q_strides = {batch, head, token}; Dh contiguous.
  *   kv, written, t_pos   as in we_rope_kv_store, after that call for the same frame.
  *   out  [B, H, T, Dh]   element strides out_strides = {batch, head, token}; Dh contiguous.
- *   workspace            device scratch of at least we_attn_workspace_bytes(...) bytes for the
+ *   workspace            device scratch of at least we_attn_workspace_bytes(...) bytes (f16: better
+ *                        we_attn_workspace_bytes_for) for the
  *                        same sizes, n_splits and q_tile; may be NULL when that is 0.  Nothing in
  *                        it has to start at any value; calls that overlap in time need a
  *                        workspace each.
@@ -189,8 +198,8 @@ int we_attn_ring_fwd(const void* q, const int64_t q_strides[3],
  * we_attn_ring_fwd for callers that cannot allocate device memory, not even a workspace: code
  * under HIP graph capture, tight serving loops, harnesses that forbid hipMalloc.  It has no
  * counterpart in the reference (whose attention call allocates through torch as it pleases).
- * Arguments, requirements and results are those of we_attn_ring_fwd, bit for bit, without the
- * workspace pair: the split-context partial results go to a buffer of WE_STATIC_SCRATCH_BYTES that
+ * Arguments, requirements and results are those of we_attn_ring_fwd with a workspace of
+ * WE_STATIC_SCRATCH_BYTES, bit for bit, without the workspace pair: the split-context partial results go to a buffer of WE_STATIC_SCRATCH_BYTES that
  * is part of the library's device image (every GPU the library runs on holds one copy until the
  * process ends; its address is looked up once per device by that device's set-up, see we_init:
  * under stream capture the device must have been set up beforehand).  Sizes whose

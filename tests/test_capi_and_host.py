@@ -111,6 +111,16 @@ def test_workspace_and_split_planning():
     assert lib.we_attn_auto_splits(1, 1, 1, 64, 64, 128) <= 1
 
 
+def test_workspace_of_an_element_type():
+    """f16 partial rows are fp32; bf16 ones 16 bits, as the size helper without a type has them; fp32 splits nothing."""
+    for sizes in ((1, 16, 16, 256, 128, 4096), (1, 24, 8, 720, 64, 16 * 720), (4, 24, 24, 1024, 128, 8192)):
+        Dh, plain = sizes[4], ops.attn_workspace_bytes(*sizes)
+        assert plain > 0 and ops.attn_workspace_bytes(*sizes, dtype=torch.bfloat16) == plain
+        assert ops.attn_workspace_bytes(*sizes, dtype=torch.float16) == plain // (Dh * 2 + 16) * (Dh * 4 + 16)
+        assert ops.attn_workspace_bytes(*sizes, dtype=torch.float32) == 0
+    assert ops.attn_workspace_bytes(1, 80, 80, 256, 128, 4096, dtype=torch.float16) == 0      # one pass
+
+
 def test_planner_over_other_shapes_and_cu_counts():
     """Invariants of the split planner over shapes and parts other than the benchmark's: a split
     call never launches more workgroups than there are CUs, every part keeps at least two 64-key

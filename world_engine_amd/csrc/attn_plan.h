@@ -209,9 +209,10 @@ inline AttnPlan plan_cached(int B, int H, int Hkv, int T, int Dh, int64_t L, int
   return e.plan;
 }
 
-inline size_t workspace_bytes_of(const AttnPlan& pl, int Dh) {
+// Partial rows of 16-bit values, or of fp32 ones (`wide`).
+inline size_t workspace_bytes_of(const AttnPlan& pl, int Dh, bool wide = false) {
   if (pl.n_splits <= 1 || pl.ws_rows <= 0) return 0;
-  return (size_t)pl.n_splits * (size_t)pl.ws_rows * ((size_t)Dh * 2 + 4 * sizeof(float));
+  return (size_t)pl.n_splits * (size_t)pl.ws_rows * ((size_t)Dh * (wide ? 4 : 2) + 4 * sizeof(float));
 }
 
 // Validation of a we_attn_ring_fwd call, its plan and its kernel parameters.  `cus`: compute units
@@ -248,15 +249,31 @@ inline int prepare_attn(const void* q, const int64_t* q_strides, const void* kv,
   }
   if (n_splits == 0 && workspace_bytes_of(pl, Dh) > workspace_limit)
     pl = plan_basic(B, H, Hkv, T, L, 0, variant_of(q_tile), cus);
-  const size_t ws_need = workspace_bytes_of(pl, Dh);
+  // An f16 output has the 11 significant bits of a 16-bit partial row itself, which would round it once
+  // more: its partial rows are fp32.  (24 heads of 64 on 8, 720 tokens, 16 slots, dilation 2, relative
+  // error against 64 bits: one pass 2.93e-4; three parts with fp16 rows 3.50e-4, with fp32 rows 2.93e-4.
+  // A bf16 output has 8 bits: 2.347e-3 in one pass, 2.352e-3 with fp16 rows.)  A workspace that holds
+  // 16-bit rows only gets the basic plan, which splits less, where it holds that one's.
+  bool wide = false;
+  const size_t given = workspace_bytes < workspace_limit ? workspace_bytes : workspace_limit;
+  if (dtype == WE_DTYPE_F16 && workspace_bytes_of(pl, Dh) > 0 && workspace_bytes_of(pl, Dh) <= given) {
+    wide = workspace_bytes_of(pl, Dh, true) <= given;
+    const AttnPlan basic = plan_basic(B, H, Hkv, T, L, n_splits, variant_of(q_tile), cus);
+    if (!wide && workspace_bytes_of(basic, Dh) <= given) {
+      pl = basic;
+      wide = workspace_bytes_of(pl, Dh, true) <= given;
+    }
+  }
+  const size_t ws_need = workspace_bytes_of(pl, Dh, wide);
   if (ws_need > 0) {
     if (!workspace || !aligned16(workspace)) return WE_ERR_WORKSPACE;
     if (workspace_bytes < ws_need) return WE_ERR_WORKSPACE;
   }
 
   p.q = q; p.kv = kv; p.written = written; p.t_pos = t_pos; p.out = out;
-  p.ws_o = ws_need ? static_cast<uint16_t*>(workspace) : nullptr;
-  p.ws_ml = ws_need ? reinterpret_cast<float*>(p.ws_o + (size_t)pl.n_splits * (size_t)pl.ws_rows * Dh) : nullptr;
+  p.ws_o = ws_need ? workspace : nullptr;
+  p.ws_ml = ws_need ? reinterpret_cast<float*>(static_cast<char*>(workspace) + (size_t)pl.n_splits * (size_t)pl.ws_rows * Dh * (wide ? 4 : 2)) : nullptr;
+  p.ws_f32 = wide ? 1 : 0;
   p.qs_b = q_strides[0]; p.qs_h = q_strides[1]; p.qs_t = q_strides[2];
   p.os_b = out_strides[0]; p.os_h = out_strides[1]; p.os_t = out_strides[2];
   p.L = L;

@@ -123,6 +123,7 @@ template <typename M, int DH, int KSPLIT, int KEYS, bool CLOCKED>
 __global__ void __attribute__((amdgpu_flat_work_group_size(512, 512), amdgpu_waves_per_eu(2, 2)))
 attn_ring_kernel(AttnParams p) {
   constexpr bool SHARED = KEYS == KEYS_SHARED, RUN = KEYS == KEYS_PACKED || SHARED;
+  constexpr bool PARTS_F32 = std::is_same<M, F16Mma>::value;
   typedef typename M::frag_t frag_t;
   typedef RingLds<DH> L;
   constexpr int KS = DH / 16;               // contraction steps of K Q^T
@@ -764,9 +765,11 @@ attn_ring_kernel(AttnParams p) {
   float gate_v = 1.f;
   const bool gated = ep.gate != nullptr || ep.gate_w != nullptr;
   if (gated && nsp == 1 && valid) gate_v = head_gate<typename M::elem_t>(ep, b, h, qt);
-  // A split leaves its partial output as fp16 values in [-1, 1] plus one fp32 scale per row (the
-  // row's largest normalised magnitude): 11 significant bits whatever the element type, for the
-  // bytes of a bf16 row, and no overflow for any finite V.  A row that holds an infinity keeps the
+  // A split leaves its partial output as values in [-1, 1] plus one fp32 scale per row (the row's
+  // largest normalised magnitude).  For a bf16 output they are fp16: 11 significant bits for the bytes
+  // of a bf16 row, three more than the output has, and no overflow for any finite V.  For an f16 output
+  // that would be its own precision once more per part, so they are fp32 (PARTS_F32; ws_f32 is off only
+  // where a caller's workspace is too short for it).  A row that holds an infinity keeps the
   // plain normalised values (scale 1), so that only the columns concerned turn non-finite, as in a
   // single pass; a row whose largest magnitude is too small for its reciprocal is scaled by 2^100.
   float mul = inv;
@@ -818,8 +821,14 @@ attn_ring_kernel(AttnParams p) {
           }
           *reinterpret_cast<frag_t*>(dst) = y;
         } else {
-          uint16_t* dst = ep.ws_o + ((int64_t)split * rows + (row - ep.ws_row0)) * DH + d0;
-          *reinterpret_cast<f16x8_t*>(dst) = F16Mma::pack8(f[0], f[1], f[2], f[3], f[4], f[5], f[6], f[7]);
+          const int64_t at = ((int64_t)split * rows + (row - ep.ws_row0)) * DH + d0;
+          if (PARTS_F32 && ep.ws_f32 != 0) {
+            f32x4_t* dst = reinterpret_cast<f32x4_t*>(static_cast<float*>(ep.ws_o) + at);
+            dst[0] = f32x4_t{f[0], f[1], f[2], f[3]};
+            dst[1] = f32x4_t{f[4], f[5], f[6], f[7]};
+          } else {
+            *reinterpret_cast<f16x8_t*>(static_cast<uint16_t*>(ep.ws_o) + at) = F16Mma::pack8(f[0], f[1], f[2], f[3], f[4], f[5], f[6], f[7]);
+          }
         }
       }
     }

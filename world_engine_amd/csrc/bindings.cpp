@@ -222,8 +222,7 @@ struct Workspace {
   size_t bytes = 0;
   Workspace(const Tensor* given, int64_t B, int64_t H, int64_t Hkv, int64_t T, int64_t Dh, int64_t L, int splits,
             int q_tile, const Tensor& like) {
-    if (like.scalar_type() == at::kFloat) return;  // (the fp32 kernel splits nothing)
-    const size_t need = we_attn_workspace_bytes((int)B, (int)H, (int)Hkv, (int)T, (int)Dh, L, splits, q_tile);
+    const size_t need = we_attn_workspace_bytes_for((int)B, (int)H, (int)Hkv, (int)T, (int)Dh, L, splits, q_tile, dtype_code(like));
     if (need == 0) return;
     if (given != nullptr && (size_t)given->numel() * given->element_size() >= need) t = *given;
     else t = at::empty({(int64_t)need}, like.options().dtype(at::kByte));

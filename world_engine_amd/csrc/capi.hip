@@ -317,6 +317,14 @@ size_t we_attn_workspace_bytes(int32_t B, int32_t H, int32_t Hkv, int32_t T, int
   return workspace_bytes_of(plan_cached(B, H, Hkv, T, Dh, L, n_splits, variant, we::host::compute_units()), Dh);
 }
 
+size_t we_attn_workspace_bytes_for(int32_t B, int32_t H, int32_t Hkv, int32_t T, int32_t Dh, int64_t L, int32_t n_splits,
+                                   int32_t q_tile, int32_t dtype) {
+  if (dtype == WE_DTYPE_F32) return 0;
+  if (dtype != WE_DTYPE_F16) return we_attn_workspace_bytes(B, H, Hkv, T, Dh, L, n_splits, q_tile);
+  if (we_attn_workspace_bytes(B, H, Hkv, T, Dh, L, n_splits, q_tile) == 0) return 0;
+  return workspace_bytes_of(plan_cached(B, H, Hkv, T, Dh, L, n_splits, variant_of(q_tile), we::host::compute_units()), Dh, true);
+}
+
 int we_attn_plan(int32_t B, int32_t H, int32_t Hkv, int32_t T, int32_t Dh, int64_t L, int32_t n_splits,
                  int32_t q_tile, int32_t compute_units, int32_t plan[WE_PLAN_FIELDS]) {
   if (!plan) return WE_ERR_NULL_POINTER;

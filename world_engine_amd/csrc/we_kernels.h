@@ -49,7 +49,7 @@ struct AttnParams {
   const uint8_t* written;
   const int64_t* t_pos;
   void* out;
-  uint16_t* ws_o;  // [n_splits][rows >= ws_row0][Dh] normalised partial outputs / row scale, fp16 in [-1, 1]
+  void* ws_o;      // [n_splits][rows >= ws_row0][Dh] normalised partial outputs / row scale, in [-1, 1]: fp32 or fp16 (ws_f32)
   float* ws_ml;    // [n_splits][rows >= ws_row0][4]  softmax reference (log2 domain), sum, row scale, unused
   int64_t qs_b, qs_h, qs_t;
   int64_t os_b, os_h, os_t;
@@ -75,6 +75,7 @@ struct AttnParams {
   // of the main kernel leaves its duration as (shader-clock cycles, ticks of the constant 100 MHz
   // counter) at [2 * linear workgroup id]
   uint64_t* clock_out;
+  int ws_f32;           // f16 caches: ws_o holds fp32 values
   int q_dma;            // 128-query workgroups fetch their Q tile by DMA (row offsets fit 32 bits)
 };
 

@@ -117,9 +117,12 @@ def attn_auto_splits(B: int, H: int, Hkv: int, T: int, Dh: int, L: int) -> int:
 
 
 def attn_workspace_bytes(B: int, H: int, Hkv: int, T: int, Dh: int, L: int, n_splits: int = 0,
-                         q_tile: int = 0) -> int:
-    """Bytes of split-context workspace ``attn_ring`` needs for these sizes and knobs."""
-    return int(_capi.lib().we_attn_workspace_bytes(B, H, Hkv, T, Dh, L, n_splits, q_tile))
+                         q_tile: int = 0, dtype: Optional[torch.dtype] = None) -> int:
+    """Bytes of split-context workspace ``attn_ring`` needs for these sizes and knobs, for q's element type where
+    it is given (float16 holds its partial results in fp32 and needs twice the bytes of bfloat16, the default)."""
+    if dtype is None:
+        return int(_capi.lib().we_attn_workspace_bytes(B, H, Hkv, T, Dh, L, n_splits, q_tile))
+    return int(_capi.lib().we_attn_workspace_bytes_for(B, H, Hkv, T, Dh, L, n_splits, q_tile, _DTYPE_CODE[dtype]))
 
 
 def attn_plan(B: int, H: int, Hkv: int, T: int, Dh: int, L: int, n_splits: int = 0, q_tile: int = 0,
@@ -143,7 +146,8 @@ def attn_ring(q: Tensor, kv: Tensor, written: Tensor, t_pos: Tensor, L: int, dil
     ``[2,B,Hkv,L+T,Dh]``, ``written`` ``[L+T]`` bool, ``t_pos`` int64 with the frame index at
     element 0.  Returns ``[B,H,T,Dh]``; with ``token_major_out`` its memory is ``[B,T,H,Dh]`` so
     that ``y.transpose(1, 2).reshape(B, T, H*Dh)`` is a view (``src/patch_model.py:139``).
-    ``workspace`` (split-context scratch, uint8, ``attn_workspace_bytes`` long) is allocated when not given.
+    ``workspace`` (split-context scratch, uint8, ``attn_workspace_bytes`` long for q's element type) is allocated
+    when not given, or when it is shorter.
     ``clocks`` (int64 device tensor): the call goes through the measurement library
     (``libwe_probe.so``, ``we_attn_ring_fwd_clocked``), which also leaves, per workgroup of the main
     kernel, its duration in shader-clock cycles and in ticks of the constant 100 MHz counter.
@@ -159,7 +163,7 @@ def attn_ring(q: Tensor, kv: Tensor, written: Tensor, t_pos: Tensor, L: int, dil
         raise RuntimeError("kv must be a contiguous [2, B, Hkv, L+T, Dh] of q's element type and written [L+T]")
     lib = _capi.probe_lib()
     with torch.cuda.device(dev):      # (the size depends on the device's compute-unit count)
-        ws_bytes = int(lib.we_attn_workspace_bytes(B, H, Hkv, T, Dh, L, n_splits, q_tile))
+        ws_bytes = int(lib.we_attn_workspace_bytes_for(B, H, Hkv, T, Dh, L, n_splits, q_tile, _dtype_code(q)))
     if ws_bytes and (workspace is None or workspace.numel() * workspace.element_size() < ws_bytes):
         workspace = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
     if out is None:
@@ -260,7 +264,7 @@ def kept_buffers(buffers: Optional[dict], kind: str, like: Tensor, H: int, Hkv: 
     kept = buffers.get(key)
     if kept is None:
         with torch.cuda.device(dev):      # (the size depends on the device's compute-unit count)
-            ws_bytes = attn_workspace_bytes(B, H, Hkv, T, Dh, L, n_splits, q_tile)
+            ws_bytes = attn_workspace_bytes(B, H, Hkv, T, Dh, L, n_splits, q_tile, dtype)
         kept = buffers[key] = (torch.empty((B, H, T, Dh), dtype=dtype, device=dev),
                                torch.empty((B, T, H, Dh), dtype=dtype, device=dev).transpose(1, 2),
                                torch.empty(ws_bytes, dtype=torch.uint8, device=dev) if ws_bytes else None)
