@@ -7,6 +7,7 @@ import pytest
 import torch
 
 import world_engine_amd as wea
+from world_engine_amd._capi import native
 from oracle import ring_oracle as ro
 from _harness import to_dev
 
@@ -122,6 +123,25 @@ def test_ids_on_another_device_are_refused_before_any_launch(gpu_device):
     layer.check_inputs = False
     with pytest.raises(RuntimeError, match="on a ROCm GPU only"):
         calls["attend"](dict(good, y_pos=good["y_pos"].cpu()))
+
+
+def test_a_check_that_cannot_be_made_is_refused(gpu_device):
+    """The projection and store without attention has no check: one that is asked for is an error, not left out."""
+    dev = gpu_device
+    T, H, Dh, W = 64, 2, 64, 8
+    layer = wea.LayerKVCache(1, H, 2 * T, Dh, torch.bfloat16, T).to(dev)
+    rope = wea.RoPE(*ro.rope_table_1d(4 * T, Dh), T // W, W).to(dev)
+    x = torch.randn(1, T, H * Dh, device=dev, dtype=torch.bfloat16)
+    w = torch.randn(3 * H * Dh, H * Dh, device=dev, dtype=torch.bfloat16)
+    pos = to_dev(ro.synth_pos_ids(1, 1, T, W), dev)
+    call = lambda check: native.qkv_rope_kv_attn(
+        x, w, H, H, pos["t_pos"], pos["y_pos"], pos["x_pos"], rope.cos, rope.sin, rope.height, rope.width, layer.kv,
+        layer.written, layer.L, 1, False, None, 0, 0, False, False, 0.0, None, None, None, None, None, None, None, None, check, T)
+    with pytest.raises(RuntimeError, match="no check"):
+        call(wea.ops.CHECK_FRAME)
+    assert not layer.kv.any()
+    call(0)
+    assert layer.kv.any()
 
 
 def test_more_checked_calls_at_once_than_records(gpu_device):

@@ -636,6 +636,7 @@ PyObject* qkv_rope_kv_attn(PyObject*, PyObject* const* argv, Py_ssize_t n) {
     const int what = (int)a.integer();
     const int64_t tpf = a.integer();
     if (tpf > 0 && T != tpf) fail("KV cache expects exactly one frame per upsert");
+    if (!attend && what != 0) fail("qkv_rope_kv_attn: a call without attention has no check of its position ids");
     if (w.dim() != 2 || !is_shape(w, {(H + 2 * Hkv) * Dh, d_model}) || w.stride(1) != 1)
       fail("w_qkv must be [(H + 2 Hkv) * Dh, d_model] with contiguous rows");
     if (x.scalar_type() != kv.scalar_type() || w.scalar_type() != kv.scalar_type())
