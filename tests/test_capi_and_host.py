@@ -160,6 +160,22 @@ def test_no_cpu_fallback():
         ops.attn_ring(k, cache.kv, cache.written, pos["t_pos"], 128, 1)
 
 
+def test_half_of_a_rotation_is_refused():
+    """A table or an id tensor left out of a rotating store is an error of the call."""
+    cache = wea.LayerKVCache(1, 2, 128, 64, torch.bfloat16, 64)
+    k = torch.zeros(1, 2, 64, 64, dtype=torch.bfloat16)
+    ids, table = torch.zeros(1, 64, dtype=torch.long), torch.zeros(64, 32)
+    whole = {"y_pos": ids, "x_pos": ids, "cos": table, "sin": table}
+    for gone in ("y_pos", "x_pos", "sin"):      # (without cos nothing is rotated)
+        a = dict(whole, **{gone: None})
+        with pytest.raises(RuntimeError, match="together"):
+            ops.native.rope_kv_store(k, k, k, ids, a["y_pos"], a["x_pos"], a["cos"], a["sin"], 8, 8, cache.kv, cache.written,
+                                     128, 1, False, 0, 0)
+    with pytest.raises(RuntimeError, match="together"):
+        ops.rope_kv_store(k, k, k, {"t_pos": ids, "y_pos": ids, "x_pos": None}, table, table, 8, 8, cache.kv, cache.written, 128,
+                          1, False)
+
+
 def test_missing_library_fails_loudly(monkeypatch):
     monkeypatch.setattr(_capi, "_lib", None)
     monkeypatch.setattr(_capi, "LIB_PATH", "/nonexistent/libwe_attn.so")

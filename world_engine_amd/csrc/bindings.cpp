@@ -427,8 +427,10 @@ PyObject* rope_kv_store(PyObject*, PyObject* const* argv, Py_ssize_t n) {
     const bool frozen = a.flag();
     const int what = (int)a.integer();
     const int64_t tpf = a.integer();
-    const c10::Device dev = need_device({&k, &v, &kv, &written, q, cos, sin, &tp, cos != nullptr ? yp : nullptr,
-                                         cos != nullptr ? xp : nullptr});
+    const bool rotate = cos != nullptr;
+    if (rotate && (sin == nullptr || yp == nullptr || xp == nullptr))
+      fail("a rotation takes the cos and sin tables and y_pos and x_pos together");
+    const c10::Device dev = need_device({&k, &v, &kv, &written, q, cos, sin, &tp, rotate ? yp : nullptr, rotate ? xp : nullptr});
     if (k.dim() != 4 || k.sizes() != v.sizes()) fail("k and v must both be [B, Hkv, T, Dh]");
     const int64_t B = k.size(0), Hkv = k.size(1), T = k.size(2), Dh = k.size(3);
     if (tpf > 0 && T != tpf) fail("KV cache expects exactly one frame per upsert");
@@ -438,7 +440,6 @@ PyObject* rope_kv_store(PyObject*, PyObject* const* argv, Py_ssize_t n) {
     check_cache(kv, written, B, Hkv, T, Dh, L);
     if (q != nullptr && (q->dim() != 4 || q->size(0) != B || q->size(2) != T || q->size(3) != Dh))
       fail("q must be [B, H, T, Dh] matching k");
-    const bool rotate = cos != nullptr;
     if (rotate) check_tables(*cos, *sin, Dh);
     const PosIds pos(tp, rotate ? yp : nullptr, rotate ? xp : nullptr, B, T);
     const Strides qs = q != nullptr ? Strides(*q, "q") : Strides(), ks(k, "k"), vs(v, "v");
