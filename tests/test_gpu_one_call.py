@@ -275,6 +275,21 @@ def test_eager_loop_reuses_its_per_layer_buffers(gpu_device):
     assert len(p.hip.layers[0]._call_buffers) == 0, "moving or casting the cache drops the call buffers"
 
 
+def test_workspace_of_another_device_or_in_pieces(gpu_device):
+    """A workspace on the host is an error before any launch; one whose elements are not all its own memory is not
+    used."""
+    p = Pair(gpu_device, torch.bfloat16, B=1, H=4, Hkv=4, T=128, Dh=64, n_slots=4, cfg_id=64)
+    q, k, v, pos = p.inputs(0)
+    (_, _, _, _), (q_h, ring) = p.store(q, k, v, pos)
+    need = ops.attn_workspace_bytes(1, 4, 4, 128, 64, 512, 2)
+    want = p.attend(q_h, ring, n_splits=2)
+    with pytest.raises(RuntimeError, match="workspace must be on"):
+        p.attend(q_h, ring, n_splits=2, workspace=torch.empty(need, dtype=torch.uint8))
+    one = torch.full((16,), 7, dtype=torch.uint8, device=gpu_device)
+    assert torch.equal(p.attend(q_h, ring, n_splits=2, workspace=one[:1].expand(need)), want)
+    assert bool((one == 7).all())
+
+
 def _alloc_events_of_reusing_calls(p, frame):
     """Allocator events (torch.cuda.memory_stats) caused by one more frame through the reusing path."""
     q, k, v, pos = frame

@@ -215,7 +215,7 @@ Tensor output_or_new(const Tensor* out, bool token_major, const Tensor& like, c1
   return *out;
 }
 
-// The caller's split-context workspace where it is long enough, else a new one.
+// The caller's split-context workspace where it is long enough and in one piece, else a new one.
 struct Workspace {
   Tensor t;
   void* ptr = nullptr;
@@ -224,7 +224,8 @@ struct Workspace {
             int q_tile, const Tensor& like) {
     const size_t need = we_attn_workspace_bytes_for((int)B, (int)H, (int)Hkv, (int)T, (int)Dh, L, splits, q_tile, dtype_code(like));
     if (need == 0) return;
-    if (given != nullptr && (size_t)given->numel() * given->element_size() >= need) t = *given;
+    if (given != nullptr && given->device() != like.device()) fail("workspace must be on the call's device, " + like.device().str());
+    if (given != nullptr && given->is_contiguous() && (size_t)given->numel() * given->element_size() >= need) t = *given;
     else t = at::empty({(int64_t)need}, like.options().dtype(at::kByte));
     ptr = t.data_ptr();
     bytes = (size_t)t.numel() * t.element_size();
