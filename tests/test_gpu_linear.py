@@ -8,7 +8,7 @@ from torch.utils._python_dispatch import TorchDispatchMode
 from torch.overrides import TorchFunctionMode
 
 from world_engine_amd._capi import native
-from world_engine_amd.attn import _plain, _project
+from world_engine_amd.attn import _plain_weight, _project
 
 gpu = pytest.mark.gpu
 
@@ -42,6 +42,10 @@ def test_linear_leaves_other_shapes_to_the_library(gpu_device):
     assert native.linear(x[:8], w) is None                                                                  # a gradient to record
     with torch.no_grad():
         assert native.linear(x[:8], w).shape == (8, 32)
+
+
+def project(lin, x):
+    return _project(lin, x, _plain_weight(lin))
 
 
 class Doubled(torch.Tensor):
@@ -80,12 +84,12 @@ DOUBLING = {
 def test_a_layer_that_is_more_than_its_weight_is_called(how, device="cpu"):
     lin = nn.Linear(256, 64, bias=False, dtype=torch.bfloat16, device=device).requires_grad_(False)
     x = torch.randn(8, 256, dtype=torch.bfloat16, device=device)
-    assert _plain(lin)
-    want = _project(lin, x) * 2
+    assert _plain_weight(lin) is lin.weight
+    want = project(lin, x) * 2
     forward, undo = nn.Linear.forward, DOUBLING[how](lin)
     try:
-        assert not _plain(lin)
-        got = _project(lin, x)
+        assert _plain_weight(lin) is None
+        got = project(lin, x)
     finally:
         nn.Linear.forward = forward
         if hasattr(undo, "remove"):
@@ -117,14 +121,14 @@ def test_linear_leaves_watched_operations_to_torch(gpu_device):
     x = torch.randn(8, 256, dtype=torch.bfloat16, device=gpu_device)
     assert native.linear(x, lin.weight) is not None
     with Watch():
-        _project(lin, x)
+        project(lin, x)
     assert any("mm" in s for s in seen), seen
     seen.clear()
     with WatchFunctions():
-        _project(lin, x)
+        project(lin, x)
     assert "linear" in seen, seen
     t = torch.randn_like(x)
-    y, dy = torch.func.jvp(lambda a: _project(lin, a), (x,), (t,))
+    y, dy = torch.func.jvp(lambda a: project(lin, a), (x,), (t,))
     assert torch.allclose(dy.float(), nn.functional.linear(t, lin.weight).float(), rtol=2 ** -7, atol=2 ** -7)
-    z = torch.func.vmap(lambda a: _project(lin, a))(torch.stack([x, t]))
+    z = torch.func.vmap(lambda a: project(lin, a))(torch.stack([x, t]))
     assert torch.allclose(z[1].float(), dy.float(), rtol=2 ** -7, atol=2 ** -7)

@@ -139,15 +139,19 @@ def ring_attention(q: Tensor, k: Tensor, v: Tensor, block_mask: RingMask, enable
 _LINEAR_FORWARD = nn.Linear.forward
 
 
-def _plain(lin: nn.Module) -> bool:
-    """A linear layer that is nothing but its weight, so that the product alone stands for a call of it: no bias, no
-    other class or ``forward`` in its place (of the class or of this instance, which is how wrapping libraries hook
-    in), no hook of its own or of every module, and an ordinary tensor as weight (a subclass - quantised, distributed
-    - has a product of its own)."""
-    return (type(lin) is nn.Linear and lin.bias is None and "forward" not in lin.__dict__
-            and nn.Linear.forward is _LINEAR_FORWARD and type(lin.weight) in (nn.Parameter, Tensor)
-            and not (lin._forward_hooks or lin._forward_pre_hooks or lin._backward_hooks or lin._backward_pre_hooks)
-            and not nn.modules.module._has_any_global_hook())
+def _plain_weight(lin: nn.Module) -> Optional[Tensor]:
+    """The weight of a linear layer that is nothing else, so that the product alone stands for a call of it; None for
+    any other: a bias, another class or ``forward`` in its place (of the class or of this instance, which is how
+    wrapping libraries hook in), a hook of its own or of every module, or a weight that is no ordinary tensor (a
+    subclass - quantised, distributed - has a product of its own)."""
+    own = lin.__dict__
+    if (type(lin) is not nn.Linear or "forward" in own or nn.Linear.forward is not _LINEAR_FORWARD or own["_forward_hooks"]
+            or own["_forward_pre_hooks"] or own["_backward_hooks"] or own["_backward_pre_hooks"]
+            or nn.modules.module._has_any_global_hook()):
+        return None
+    params = own["_parameters"]
+    w = params.get("weight")
+    return w if type(w) in (nn.Parameter, Tensor) and params.get("bias", w) is None else None
 
 
 @torch.compiler.assume_constant_result
@@ -156,17 +160,18 @@ def _kernel_covers(rows: int, features: int, contraction: int, half: bool) -> bo
     return _capi.lib().we_linear_covers(rows, features, contraction, dtype) != 0
 
 
-def _project(lin: nn.Module, x: Tensor) -> Tensor:
+def _project(lin: nn.Module, x: Tensor, w: Optional[Tensor]) -> Tensor:
     """``lin(x)``, on the library's own kernel where the frame is small enough for it to be the faster one
     (one round of workgroups; 256 x 2048 x 2048: 8.2 us against 9.6 on the GPU, and 4 against 19 us of the
-    host's time, most of it the BLAS routine's choice of a kernel).  fp32 sums rounded once, as there."""
-    if type(x) is Tensor and _plain(lin) and not torch.is_autocast_enabled():
+    host's time, most of it the BLAS routine's choice of a kernel).  fp32 sums rounded once, as there.  ``w`` is the
+    layer's ``_plain_weight``."""
+    if w is not None and type(x) is Tensor and not torch.is_autocast_enabled():
         if torch.compiler.is_compiling():        # the opaque op where the kernel covers the shape, for the same bits as eager
-            if (x.dtype in (torch.bfloat16, torch.float16) and lin.weight.dtype == x.dtype and not torch.is_grad_enabled()
-                    and _kernel_covers(x.numel() // x.shape[-1], lin.out_features, x.shape[-1], x.dtype is torch.float16)):
-                return torch.ops.world_engine_amd.linear(x, lin.weight)
+            if (x.dtype in (torch.bfloat16, torch.float16) and w.dtype == x.dtype and not torch.is_grad_enabled()
+                    and _kernel_covers(x.numel() // x.shape[-1], w.shape[0], x.shape[-1], x.dtype is torch.float16)):
+                return torch.ops.world_engine_amd.linear(x, w)
         else:
-            y = native.linear(x, lin.weight)
+            y = native.linear(x, w)
             if y is not None:
                 return y
     return lin(x)
@@ -283,12 +288,14 @@ class RingAttn(nn.Module):
             extras.update(v1=v1.view(B, self.n_kv_heads, T, self.d_head), v_lamb=self.v_lamb)
         if self.gated_attn:
             extras.update(gate_x=x[..., : self.n_heads], gate_w=self.gate_proj.weight)
-        y, v = kv_cache.qkv_rope_upsert_attend(x, self.qkv_proj.weight, self.n_heads, pos_ids, self.rope,
-                                               self.layer_idx, want_v=first,
-                                               reuse_buffers=self._reads_output_at_once(self._records(x)), **extras)
+        out_proj = self.out_proj
+        out_w = _plain_weight(out_proj)
+        # (the output may live in the layer's buffer, see forward)
+        y, v = kv_cache.qkv_rope_upsert_attend(x, self.qkv_proj.weight, self.n_heads, pos_ids, self.rope, self.layer_idx,
+                                               want_v=first, reuse_buffers=out_w is not None and not self._records(x), **extras)
         if first:
             v1 = v
-        return _project(self.out_proj, y.transpose(1, 2).reshape(B, T, -1)), v1
+        return _project(out_proj, y.transpose(1, 2).reshape(B, T, -1), out_w), v1
 
     def projection_workgroups(self, B: int, T: int) -> int:
         """Workgroups the fused projection kernel launches for x ``[B, T, d_model]``."""
@@ -303,20 +310,6 @@ class RingAttn(nn.Module):
         return (not torch.compiler.is_compiling() and torch.is_grad_enabled()
                 and (x.requires_grad or any(p.requires_grad for p in self.parameters())))
 
-    def _reads_output_at_once(self, records: bool) -> bool:
-        """Whether nothing of this call reads the attention's output after ``out_proj``, so that it can live in the
-        layer's own buffer until the layer's next call: a backward pass would, and hooks or layers of another kind
-        may keep what they are given."""
-        return not records and _plain(self.out_proj)
-
-    def _gate_is_the_kernels(self, x: Tensor, q: Tensor, records: bool) -> bool:
-        """Whether the attention kernels' epilogue can stand for ``sigmoid(gate_proj(x[..., :H]))`` and the product
-        with it: the layer is its weight alone, all of one half-precision type and in the layout the kernels read,
-        and nothing of it is recorded."""
-        return (x.dtype != torch.float32 and x.stride(-1) == 1 and _plain(self.gate_proj) and not torch.is_autocast_enabled()
-                and self.gate_proj.weight.is_contiguous() and not records
-                and native.plain(x, self.gate_proj.weight, q))
-
     def forward(self, x: Tensor, pos_ids: Mapping[str, Tensor], v1: Optional[Tensor], kv_cache):
         B, T = x.shape[:2]
         if (self.uses_fused_projection(B, T) and hasattr(kv_cache, "qkv_rope_upsert_attend")
@@ -326,7 +319,8 @@ class RingAttn(nn.Module):
         fuse = self.fuse_elementwise and one_call and x.dtype != torch.float32
         H, Hkv, Dh = self.n_heads, self.n_kv_heads, self.d_head
         if self.merged_qkv:
-            rows = _project(self.qkv_proj, x).view(B, T, H + 2 * Hkv, Dh)
+            qkv_proj = self.qkv_proj
+            rows = _project(qkv_proj, x, _plain_weight(qkv_proj)).view(B, T, H + 2 * Hkv, Dh)
             heads = rows.transpose(1, 2)
             q, k, v = heads.split((H, Hkv, Hkv), dim=1)
             if not fuse:
@@ -335,7 +329,7 @@ class RingAttn(nn.Module):
                 # strided q and k views each made a copy first.
                 q, k, _ = F.rms_norm(rows, (Dh,)).transpose(1, 2).split((H, Hkv, Hkv), dim=1)
         else:
-            q, k, v = (_project(proj, x).reshape(B, T, -1, Dh) for proj in (self.q_proj, self.k_proj, self.v_proj))
+            q, k, v = (_project(proj, x, _plain_weight(proj)).reshape(B, T, -1, Dh) for proj in (self.q_proj, self.k_proj, self.v_proj))
             if not fuse:
                 q, k = F.rms_norm(q, (Dh,)), F.rms_norm(k, (Dh,))
             q, k, v = q.transpose(1, 2), k.transpose(1, 2), v.transpose(1, 2)
@@ -347,19 +341,23 @@ class RingAttn(nn.Module):
         if self.value_residual and v1 is None:
             v1 = v                               # (lerp(v, v, w) is v)
         elif self.value_residual:
-            res = v1.view_as(v)
-            if fuse or (inside and native.plain(v, res, self.v_lamb) and native.aligned_rows(res)):
-                extras.update(v1=res, v_lamb=self.v_lamb)      # same formula in fp32, rounded once: torch.lerp's bits
+            res, lamb = v1.view_as(v), self.v_lamb
+            if fuse or (inside and native.blend_ready(v, res, lamb)):
+                extras.update(v1=res, v_lamb=lamb)      # same formula in fp32, rounded once: torch.lerp's bits
             else:
-                v = torch.lerp(v, res, self.v_lamb)
+                v = torch.lerp(v, res, lamb)
 
         gates = None
         if self.gated_attn:
-            if fuse or (inside and self._gate_is_the_kernels(x, q, records)):
-                # projection, sigmoid and multiply in the kernels' epilogues
-                extras.update(gate_x=x[..., :H], gate_w=self.gate_proj.weight)
+            gate_proj = self.gate_proj
+            gate_w = gate_proj.weight if fuse else _plain_weight(gate_proj)
+            # Projection, sigmoid and multiply in the kernels' epilogues, where the layer is its weight alone, all of it
+            # one half-precision type in the layout the kernels read, and nothing of it is recorded.
+            if fuse or (inside and gate_w is not None and not records and not torch.is_autocast_enabled()
+                        and native.gate_ready(x, gate_w, q)):
+                extras.update(gate_x=x[..., :H], gate_w=gate_w)
             else:
-                gates = torch.sigmoid(self.gate_proj(x[..., :H])).permute(0, 2, 1)
+                gates = torch.sigmoid(gate_proj(x[..., :H])).permute(0, 2, 1)
                 if inside and not records and native.plain(gates, q):
                     extras["gate"] = gates       # the epilogue multiplies the rounded output, as `y * gates` would
                     gates = None
@@ -368,16 +366,20 @@ class RingAttn(nn.Module):
 
         # RoPE(q), RoPE(k), cache write (one launch) and attention over the ring (one or two), all
         # behind one library call; a cache without it gets the reference's sequence of calls
+        out_proj = self.out_proj
+        out_w = _plain_weight(out_proj)
         if one_call:
+            # The output may live in the layer's own buffer until the layer's next call if nothing reads it after
+            # out_proj: a backward pass would, and hooks or layers of another kind may keep what they are given.
             y = kv_cache.rope_upsert_attend(q, k, v, pos_ids, self.rope, self.layer_idx,
-                                            reuse_buffers=self._reads_output_at_once(records), **extras)
+                                            reuse_buffers=out_w is not None and not records, **extras)
         else:
             q, k_all, v_all, ring = kv_cache.rope_upsert(q, k, v, pos_ids, self.rope, self.layer_idx)
             y = ring_attention(q, k_all, v_all, ring, enable_gqa=self.enable_gqa)
         if gates is not None:
             y = y * gates.unsqueeze(-1)
 
-        return _project(self.out_proj, y.transpose(1, 2).reshape(B, T, -1)), v1
+        return _project(out_proj, y.transpose(1, 2).reshape(B, T, -1), out_w), v1
 
 
 def install_ring_attention(model: nn.Module, rope: Optional[RoPE], attn_types: tuple, merged_qkv: bool = True,

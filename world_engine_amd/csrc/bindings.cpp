@@ -46,11 +46,6 @@ struct NoGil {
   NoGil(const NoGil&) = delete;
   NoGil& operator=(const NoGil&) = delete;
 };
-template <typename F>
-int call_library(F&& f) {
-  const NoGil off;
-  return f();
-}
 
 // ---- arguments -----------------------------------------------------------------------------
 
@@ -334,11 +329,10 @@ class PosCheck {
   PosCheck(const PosCheck&) = delete;
   PosCheck& operator=(const PosCheck&) = delete;
   const we_pos_check* arg() const { return v_ != nullptr ? &c_ : nullptr; }
-  // Waits for the verdict of the launched call, without the interpreter's lock; true = refused.
+  // Waits for the verdict of the launched call (not under the interpreter's lock); true = refused.
   bool refused() {
     if (v_ == nullptr) return false;
     awaited_ = true;
-    const NoGil off;
     const volatile uint64_t* word = c_.report;
     uint64_t got = 0;
     const auto began = std::chrono::steady_clock::now();
@@ -370,6 +364,15 @@ class PosCheck {
   Tensor guard_;
   we_pos_check c_{};
 };
+
+// A library call and, where it checks, the wait for its verdict, without the interpreter's lock; true = refused.
+template <typename F>
+bool run(const char* fn, PosCheck* check, F&& call) {
+  const NoGil off;
+  const int rc = call();
+  if (rc != WE_OK) fail_code(fn, rc);
+  return check != nullptr && check->refused();
+}
 
 // A tensor that is its memory and nothing else: no Python subclass or functorch wrapper that would
 // see the operation, no tangent, no lazily negated view.
@@ -451,14 +454,13 @@ PyObject* rope_kv_store(PyObject*, PyObject* const* argv, Py_ssize_t n) {
     Tensor q_out;
     if (q != nullptr) q_out = new_heads(*q, B, H, T, Dh);
     PosCheck check(what, dev, st, B, T, false);
-    const int rc = call_library([&] { return we_rope_kv_store_checked(
+    const bool refused = run("we_rope_kv_store", &check, [&] { return we_rope_kv_store_checked(
         q != nullptr ? q->data_ptr() : nullptr, k.data_ptr(), v.data_ptr(), q != nullptr ? qs.s : nullptr, ks.s, vs.s,
         q != nullptr ? q_out.data_ptr() : nullptr, rotate ? cos->const_data_ptr<float>() : nullptr,
         rotate ? sin->const_data_ptr<float>() : nullptr, rotate ? cos->size(0) : 0, pos.tp(), pos.yp(), pos.xp(),
         pos.row_stride, gh, gw, kv.data_ptr(), static_cast<uint8_t*>(written.data_ptr()), (int)B, (int)H, (int)Hkv,
         (int)T, (int)Dh, L, (int)dilation, frozen ? 1 : 0, code_t, check.arg(), st); });
-    if (rc != WE_OK) fail_code("we_rope_kv_store", rc);
-    if (check.refused()) return refused_result();
+    if (refused) return refused_result();
     return q != nullptr ? wrap(q_out) : none();
   });
 }
@@ -484,11 +486,10 @@ PyObject* rope_apply(PyObject*, PyObject* const* argv, Py_ssize_t n) {
     const Tensor cos = cos_in.contiguous(), sin = sin_in.contiguous();
     const Tensor out = new_heads(x, B, H, T, Dh);
     PosCheck check(what, dev, st, B, T, false);
-    const int rc = call_library([&] { return we_rope_apply_checked(x.data_ptr(), xs.s, out.data_ptr(), cos.const_data_ptr<float>(),
+    const bool refused = run("we_rope_apply", &check, [&] { return we_rope_apply_checked(x.data_ptr(), xs.s, out.data_ptr(), cos.const_data_ptr<float>(),
                                          sin.const_data_ptr<float>(), cos.size(0), pos.tp(), pos.yp(), pos.xp(),
                                          pos.row_stride, gh, gw, (int)B, (int)H, (int)T, (int)Dh, code_t, check.arg(), st); });
-    if (rc != WE_OK) fail_code("we_rope_apply", rc);
-    if (check.refused()) return refused_result();
+    if (refused) return refused_result();
     return wrap(out);
   });
 }
@@ -522,11 +523,10 @@ PyObject* attn_ring(PyObject*, PyObject* const* argv, Py_ssize_t n) {
     const Workspace ws(ws_in, B, H, Hkv, T, Dh, L, splits, q_tile, q);
     const Tensor out = output_or_new(out_in, token_major, q, dev, B, H, T, Dh);
     const Strides os(out, "out");
-    const int rc = call_library([&] { return we_attn_ring_fwd(q.data_ptr(), qs.s, kv.data_ptr(), static_cast<const uint8_t*>(written.data_ptr()),
+    run("we_attn_ring_fwd", nullptr, [&] { return we_attn_ring_fwd(q.data_ptr(), qs.s, kv.data_ptr(), static_cast<const uint8_t*>(written.data_ptr()),
                                     t_pos.const_data_ptr<int64_t>(), out.data_ptr(), os.s, ws.ptr, ws.bytes, (int)B, (int)H,
                                     (int)Hkv, (int)T, (int)Dh, L, (int)dilation, scale, splits, q_tile, dtype_code(q),
                                     stream_of(dev)); });
-    if (rc != WE_OK) fail_code("we_attn_ring_fwd", rc);
     return wrap(out);
   });
 }
@@ -546,11 +546,10 @@ PyObject* attn_ring_static(PyObject*, PyObject* const* argv, Py_ssize_t n) {
       fail("out must be [B, H, T, Dh] of q's element type on q's device");
     const Strides qs(q, "q"), os(out, "out");
     const OnDevice on(dev);
-    const int rc = call_library([&] { return we_attn_ring_fwd_static(q.data_ptr(), qs.s, kv.data_ptr(), static_cast<const uint8_t*>(written.data_ptr()),
+    run("we_attn_ring_fwd_static", nullptr, [&] { return we_attn_ring_fwd_static(q.data_ptr(), qs.s, kv.data_ptr(), static_cast<const uint8_t*>(written.data_ptr()),
                                            t_pos.const_data_ptr<int64_t>(), out.data_ptr(), os.s, (int)B, (int)H, (int)Hkv,
                                            (int)T, (int)Dh, L, (int)dilation, scale, splits, q_tile, dtype_code(q),
                                            stream_of(dev)); });
-    if (rc != WE_OK) fail_code("we_attn_ring_fwd_static", rc);
     return none();
   });
 }
@@ -602,13 +601,12 @@ PyObject* rope_kv_attn(PyObject*, PyObject* const* argv, Py_ssize_t n) {
     const Tensor out = output_or_new(out_in, token_major, q, dev, B, H, T, Dh);
     const Strides os(out, "out");
     PosCheck check(what, dev, st, B, T, false);
-    const int rc = call_library([&] { return we_rope_kv_attn_fwd_checked(
+    const bool refused = run("we_rope_kv_attn_fwd", &check, [&] { return we_rope_kv_attn_fwd_checked(
         q.data_ptr(), k.data_ptr(), v.data_ptr(), qs.s, ks.s, vs.s, q_rot.data_ptr(), cos.const_data_ptr<float>(),
         sin.const_data_ptr<float>(), cos.size(0), pos.tp(), pos.yp(), pos.xp(), pos.row_stride, gh, gw, kv.data_ptr(),
         static_cast<uint8_t*>(written.data_ptr()), out.data_ptr(), os.s, ws.ptr, ws.bytes, (int)B, (int)H, (int)Hkv, (int)T,
         (int)Dh, L, (int)dilation, frozen ? 1 : 0, scale, splits, q_tile, code_t, extras.ptr(), check.arg(), st); });
-    if (rc != WE_OK) fail_code("we_rope_kv_attn_fwd", rc);
-    if (check.refused()) return refused_result();
+    if (refused) return refused_result();
     return pack({&out, &q_rot});
   });
 }
@@ -665,22 +663,20 @@ PyObject* qkv_rope_kv_attn(PyObject*, PyObject* const* argv, Py_ssize_t n) {
     Tensor out;
     PosCheck check(what, dev, st, B, T, true);
     if (!attend) {
-      const int rc = call_library([&] { return we_qkv_rope_kv_store(&proj, q_rot.data_ptr(), cos.const_data_ptr<float>(), sin.const_data_ptr<float>(),
+      run("we_qkv_rope_kv_store", nullptr, [&] { return we_qkv_rope_kv_store(&proj, q_rot.data_ptr(), cos.const_data_ptr<float>(), sin.const_data_ptr<float>(),
                                           cos.size(0), pos.tp(), pos.yp(), pos.xp(), pos.row_stride, gh, gw, kv.data_ptr(),
                                           static_cast<uint8_t*>(written.data_ptr()), (int)B, (int)H, (int)Hkv, (int)T, (int)Dh,
                                           L, (int)dilation, frozen ? 1 : 0, code_t, extras.ptr(), st); });
-      if (rc != WE_OK) fail_code("we_qkv_rope_kv_store", rc);
     } else {
       const Workspace ws(ws_in, B, H, Hkv, T, Dh, L, splits, q_tile, x);
       out = output_or_new(out_in, true, x, dev, B, H, T, Dh);
       const Strides os(out, "out");
-      const int rc = call_library([&] { return we_qkv_rope_kv_attn_fwd_checked(
+      const bool refused = run("we_qkv_rope_kv_attn_fwd", &check, [&] { return we_qkv_rope_kv_attn_fwd_checked(
           &proj, q_rot.data_ptr(), cos.const_data_ptr<float>(), sin.const_data_ptr<float>(), cos.size(0), pos.tp(), pos.yp(),
           pos.xp(), pos.row_stride, gh, gw, kv.data_ptr(), static_cast<uint8_t*>(written.data_ptr()), out.data_ptr(), os.s,
           ws.ptr, ws.bytes, (int)B, (int)H, (int)Hkv, (int)T, (int)Dh, L, (int)dilation, frozen ? 1 : 0, scale, splits, q_tile,
           code_t, extras.ptr(), check.arg(), st); });
-      if (rc != WE_OK) fail_code("we_qkv_rope_kv_attn_fwd", rc);
-      if (check.refused()) return refused_result();
+      if (refused) return refused_result();
     }
     return pack({&out, &q_rot, &v_raw});
   });
@@ -703,15 +699,28 @@ PyObject* plain(PyObject*, PyObject* const* argv, Py_ssize_t n) {
   });
 }
 
-// aligned_rows(t): t is [B, H, T, Dh] with rows as the kernels read them, contiguous and 16-byte aligned.
-PyObject* aligned_rows(PyObject*, PyObject* const* argv, Py_ssize_t n) {
+// The same for what the store kernel's blend reads: v, the value rows it is blended with (contiguous rows on
+// 16-byte boundaries) and the weight.
+PyObject* blend_ready(PyObject* self, PyObject* const* argv, Py_ssize_t n) {
   return guarded([&]() -> PyObject* {
-    Args a("aligned_rows", argv, n, 1);
+    Args a("blend_ready", argv, n, 3);
+    a.tensor();
     const Tensor& t = a.tensor();
     const int64_t per16 = 16 / (int64_t)t.element_size();
-    const bool ok = t.dim() == 4 && t.stride(3) == 1 && t.stride(0) % per16 == 0 && t.stride(1) % per16 == 0 &&
-                    t.stride(2) % per16 == 0 && (reinterpret_cast<uintptr_t>(t.const_data_ptr()) & 15u) == 0;
-    return PyBool_FromLong(ok ? 1 : 0);
+    if (t.dim() != 4 || t.stride(3) != 1 || t.stride(0) % per16 != 0 || t.stride(1) % per16 != 0 || t.stride(2) % per16 != 0 ||
+        !t.has_storage() || (reinterpret_cast<uintptr_t>(t.const_data_ptr()) & 15u) != 0)
+      Py_RETURN_FALSE;
+    return plain(self, argv, n);
+  });
+}
+// And for the head gate in the attention's epilogue: x (contiguous channels), gate_proj's weight (contiguous), q; one
+// half-precision type.
+PyObject* gate_ready(PyObject* self, PyObject* const* argv, Py_ssize_t n) {
+  return guarded([&]() -> PyObject* {
+    Args a("gate_ready", argv, n, 3);
+    const Tensor &x = a.tensor(), &w = a.tensor();
+    if ((x.scalar_type() != at::kBFloat16 && x.scalar_type() != at::kHalf) || x.stride(-1) != 1 || !w.is_contiguous()) Py_RETURN_FALSE;
+    return plain(self, argv, n);
   });
 }
 
@@ -740,8 +749,12 @@ PyObject* linear(PyObject*, PyObject* const* argv, Py_ssize_t n) {
     c10::SmallVector<int64_t, 4> shape(x.sizes().begin(), x.sizes().end());
     shape.back() = N;
     const Tensor y = at::empty(shape, x.options());
-    const int rc = call_library([&] { return we_linear(x.data_ptr(), xs, w.data_ptr(), w.stride(0), y.data_ptr(), N, (int)M, (int)N, (int)K,
-                             dtype_code(x), stream_of(x.device())); });
+    int rc = WE_OK;
+    {
+      const NoGil off;
+      rc = we_linear(x.data_ptr(), xs, w.data_ptr(), w.stride(0), y.data_ptr(), N, (int)M, (int)N, (int)K, dtype_code(x),
+                     stream_of(x.device()));
+    }
     if (rc == WE_ERR_ALIGNMENT || rc == WE_ERR_UNSUPPORTED || rc == WE_ERR_BAD_SHAPE) return none();
     if (rc != WE_OK) fail_code("we_linear", rc);
     return wrap(y);
@@ -750,7 +763,8 @@ PyObject* linear(PyObject*, PyObject* const* argv, Py_ssize_t n) {
 
 PyMethodDef methods[] = {
     {"plain", (PyCFunction)(void (*)(void))plain, METH_FASTCALL, nullptr},
-    {"aligned_rows", (PyCFunction)(void (*)(void))aligned_rows, METH_FASTCALL, nullptr},
+    {"blend_ready", (PyCFunction)(void (*)(void))blend_ready, METH_FASTCALL, nullptr},
+    {"gate_ready", (PyCFunction)(void (*)(void))gate_ready, METH_FASTCALL, nullptr},
     {"linear", (PyCFunction)(void (*)(void))linear, METH_FASTCALL, nullptr},
     {"rope_kv_store", (PyCFunction)(void (*)(void))rope_kv_store, METH_FASTCALL, nullptr},
     {"rope_apply", (PyCFunction)(void (*)(void))rope_apply, METH_FASTCALL, nullptr},
