@@ -199,8 +199,8 @@ int we_attn_ring_fwd(const void* q, const int64_t q_strides[3],
  * under HIP graph capture, tight serving loops, harnesses that forbid hipMalloc.  It has no
  * counterpart in the reference (whose attention call allocates through torch as it pleases).
  * Arguments, requirements and results are those of we_attn_ring_fwd with a workspace of
- * WE_STATIC_SCRATCH_BYTES, bit for bit, without the workspace pair: the split-context partial results go to a buffer of WE_STATIC_SCRATCH_BYTES that
- * is part of the library's device image (every GPU the library runs on holds one copy until the
+ * WE_STATIC_SCRATCH_BYTES, bit for bit, without the workspace pair: the split-context partial
+ * results go to a buffer of WE_STATIC_SCRATCH_BYTES that is part of the library's device image (every GPU the library runs on holds one copy until the
  * process ends; its address is looked up once per device by that device's set-up, see we_init:
  * under stream capture the device must have been set up beforehand).  Sizes whose
  * we_attn_workspace_bytes(...) exceeds WE_STATIC_SCRATCH_BYTES run with fewer parts if there is a
@@ -241,9 +241,8 @@ int we_attn_ring_fwd_static(const void* q, const int64_t q_strides[3],
  *                {batch, token}), gate_w at gate_proj.weight [H, H] row-major (out, in).  The
  *                projection's output and the sigmoid's are rounded to the element type like the
  *                module's tensors.  Both NULL = off; not together with `gate`; bf16 / f16 only.
- * Results equal the separate torch operations up to the last bit of the row reduction, of the
- * lerp's fused multiply-add and of the gate's dot product (1 ulp of the element type); the gate
- * multiply itself is exact.
+ * Results equal the separate torch operations up to the last bit of the norm's row reduction and of
+ * the gate's dot product (1 ulp of the element type); the lerp and the gate multiply have their bits.
  */
 typedef struct we_attn_extras {
   float qk_norm_eps;

@@ -6,7 +6,7 @@ import pytest
 import torch
 
 from oracle import ring_oracle as ro
-from _harness import Pair, assert_attn_close, assert_bits_equal, assert_ulp_close, merged_views, to_dev
+from _harness import Pair, assert_attn_close, assert_bits_equal, merged_views, to_dev
 import world_engine_amd as wea
 from world_engine_amd import _capi, ops
 
@@ -123,7 +123,7 @@ def test_non_finite_values_in_v_poison_the_same_columns_however_the_context_is_s
 def test_value_blend_weight_signs_and_the_switch_point(gpu_device, lamb):
     """torch.lerp switches formula at |w| = 0.5 (ATen/native/Lerp.h), not at w = 0.5: a learned
     v_lamb at or below -0.5 takes the second formula.  Cache rows against the oracle's value_lerp
-    (pinned to torch.lerp bit for bit) within 1 ulp (the kernel's fused multiply-add)."""
+    (pinned to torch.lerp bit for bit), bit for bit."""
     dev = gpu_device
     dtype = torch.bfloat16
     p = Pair(dev, dtype, B=1, H=2, Hkv=2, T=64, Dh=64, n_slots=2, cfg_id=95)
@@ -139,6 +139,22 @@ def test_value_blend_weight_signs_and_the_switch_point(gpu_device, lamb):
         out, _ = ops.rope_kv_attn(qd, kd, vd, to_dev(pos, dev), p.rope.cos, p.rope.sin, p.rope.height, p.rope.width,
                                   layer.kv, layer.written, layer.L, 1, False, v1=v1.to(dev), v_lamb=w.to(dev))
         assert_bits_equal(layer.kv[0], p.oracle.layers[0].kv[0], f"K plane t={t}")
-        frac = assert_ulp_close(layer.kv[1], p.oracle.layers[0].kv[1], f"blended V plane, weight {lamb}, t={t}")
-        assert frac < 0.05, frac
+        assert_bits_equal(layer.kv[1], p.oracle.layers[0].kv[1], f"blended V plane, weight {lamb}, t={t}")
         assert_attn_close(out, ref, f"weight {lamb} t={t}")
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+def test_value_blend_has_the_bits_of_torch_lerp(gpu_device, dtype):
+    """Values of any size against each other, on this device: what the attention module's default rests on, which
+    blends in the store kernel."""
+    dev = gpu_device
+    p = Pair(dev, dtype, B=1, H=8, Hkv=8, T=128, Dh=128, n_slots=2, cfg_id=96)
+    layer, pos = p.hip.layers[0], to_dev(p.inputs(0)[3], dev)
+    g = torch.Generator(dev).manual_seed(12)
+    for lamb in (-0.75, -0.5, 0.0, 0.01, 0.3, 0.498046875, 0.5, 0.7, 1.0):
+        v, v1 = (torch.randn(1, 8, 128, 128, device=dev, generator=g)
+                 * torch.exp2(torch.randint(-8, 9, (1, 8, 128, 128), device=dev, generator=g).float()) for _ in range(2))
+        v, v1, w = v.to(dtype), v1.to(dtype), torch.tensor(lamb, dtype=dtype, device=dev)
+        ops.rope_kv_attn(v, v, v, pos, p.rope.cos, p.rope.sin, p.rope.height, p.rope.width, layer.kv, layer.written, layer.L,
+                         1, True, v1=v1, v_lamb=w)
+        assert_bits_equal(layer.kv[1, :, :, layer.L:], torch.lerp(v, v1, w), f"weight {lamb}")

@@ -9,7 +9,8 @@ import torch.nn.functional as F
 
 import world_engine_amd as wea
 from oracle import ring_oracle as ro
-from _harness import to_dev
+from _harness import assert_bits_equal, to_dev
+from world_engine_amd.attn import _project
 
 H, DH, T = 4, 64, 64
 D = H * DH
@@ -178,6 +179,30 @@ def test_the_gates_gradient_on_the_kernels(gpu_device):
     y.float().square().sum().backward()
     assert m.gate_proj.weight.grad is not None and m.gate_proj.weight.grad.abs().sum() > 0
     assert torch.allclose(y.float(), want.float(), rtol=2e-2, atol=2e-2)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+def test_the_default_module_stores_the_bits_of_the_separate_operations(gpu_device, dtype):
+    """From the projection's rows on: the norm over q and k in one launch, the blend in the store kernel and the gate
+    in the attention's epilogue, against each operation by itself."""
+    m = module(dtype, gpu_device).requires_grad_(False)
+    m.v_lamb.fill_(0.3)
+    caches = [wea.StaticKVCache(config(), 1, dtype).to(gpu_device) for _ in range(2)]
+    for c in caches:
+        c.set_frozen(False)
+    for t in range(4):
+        pos = to_dev(ro.synth_pos_ids(t, 1, T, 8), gpu_device)
+        x, v1 = torch.randn(1, T, D, device=gpu_device).to(dtype), torch.randn(1, H, T, DH, device=gpu_device).to(dtype)
+        got, _ = m(x, pos, v1, caches[0])
+        rows = _project(m.qkv_proj, x, m.qkv_proj.weight).view(1, T, 3 * H, DH).transpose(1, 2)
+        q, k, v = (r.contiguous() for r in rows.split(H, dim=1))
+        y = caches[1].rope_upsert_attend(F.rms_norm(q, (DH,)), F.rms_norm(k, (DH,)), torch.lerp(v, v1, m.v_lamb), pos, m.rope, 0)
+        y = y * torch.sigmoid(F.linear(x[..., :H], m.gate_proj.weight)).permute(0, 2, 1).unsqueeze(-1)
+        assert_bits_equal(caches[0].layers[0].kv, caches[1].layers[0].kv, f"cache rows, frame {t}")
+        want = _project(m.out_proj, y.transpose(1, 2).reshape(1, T, D), m.out_proj.weight)
+        eps = torch.finfo(dtype).eps                 # the gate's dot product may round the other way: 1 ulp of a factor
+        assert torch.allclose(got.float(), want.float(), rtol=2 * eps, atol=2 * eps * want.abs().max().item())
 
 
 @pytest.mark.gpu

@@ -5,9 +5,11 @@
 order of operations.  The part between the q/k/v projection and the output projection - RoPE,
 cache update, masked attention, and with them the value-residual lerp and the head gate - runs as
 two HIP kernel launches (three with context splits) instead of the reference's eager/compiled op
-sequence.  Projections of small half-precision frames run on the library's own kernel, others are
-ordinary torch ops.  The weightless RMS norm is torch's by default (bit for bit what the reference
-stores) and moves into the store kernel with ``fuse_elementwise=True`` (1 ulp).
+sequence.  Projections of small half-precision frames run on the library's own kernel (fp32 sums
+rounded once, in another order of additions than a BLAS routine's), others are ordinary torch ops.
+The weightless RMS norm is torch's by default and moves into the store kernel with
+``fuse_elementwise=True`` (1 ulp).  From the projections' rows on, the default module stores the
+bits that the reference's operations give on the same device.
 """
 from __future__ import annotations
 
@@ -185,9 +187,11 @@ class RingAttn(nn.Module):
     ``merged_qkv`` the three projections are one ``qkv_proj`` as after the reference's inference
     patch (``src/patch_model.py:102-114``); otherwise the keys are ``q_proj/k_proj/v_proj``.
 
-    The value-residual lerp (same bits as torch's) and the head gate incl. its H x H projection and
+    In eager mode the value-residual lerp (torch's bits) and the head gate incl. its H x H projection and
     sigmoid (projection sums in another order, then the module's own roundings) are done inside the
-    two kernels.  ``fuse_elementwise`` moves the QK RMS norm there too: one launch and one pass over
+    two kernels, unless a gradient is recorded, a type or layout is not theirs, or a layer is more than its
+    weight; ``torch.compile`` fuses the torch operations itself and rounds between them where it
+    chooses to.  ``fuse_elementwise`` moves the QK RMS norm there too: one launch and one pass over
     q, k and v fewer per layer, rows within 1 ulp of torch's norm instead of bit-identical, which is
     why it is off unless asked for.
 

@@ -901,9 +901,9 @@ static hipError_t configure_both() {
   return e == hipSuccess ? configure_keys<M, 64, KEYS>() : e;
 }
 
-// The four (element type, head dim) families are compiled as separate objects (WE_RING_PART selects
-// one; undefined = all of them in this translation unit) so that they build in parallel; the short
-// frames' and the shared tiles' instantiations are parts of their own.
+// The four (element type, head dim) families (parts 0 to 3) and the short frames' and the shared tiles'
+// instantiations (4 to 7) are compiled as separate objects, one per WE_RING_PART, so that they build in
+// parallel.  Without it this translation unit holds parts 0 to 3.
 #if !defined(WE_RING_PART) || WE_RING_PART == 0
 hipError_t launch_attn_ring_bf16_128(const AttnParams& p, int ksplit, hipStream_t stream) {
   return ksplit == 2 ? launch_ring_t<Bf16Mma, 128, 2>(p, stream) : launch_ring_t<Bf16Mma, 128, 1>(p, stream);
