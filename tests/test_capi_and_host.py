@@ -119,6 +119,8 @@ def test_workspace_of_an_element_type():
         assert ops.attn_workspace_bytes(*sizes, dtype=torch.float16) == plain // (Dh * 2 + 16) * (Dh * 4 + 16)
         assert ops.attn_workspace_bytes(*sizes, dtype=torch.float32) == 0
     assert ops.attn_workspace_bytes(1, 80, 80, 256, 128, 4096, dtype=torch.float16) == 0      # one pass
+    with pytest.raises(RuntimeError, match="unsupported element type"):
+        ops.attn_workspace_bytes(1, 16, 16, 256, 128, 4096, dtype=torch.float64)
 
 
 def test_planner_over_other_shapes_and_cu_counts():

@@ -260,10 +260,12 @@ inline int prepare_attn(const void* q, const int64_t* q_strides, const void* kv,
   const size_t given = workspace_bytes < workspace_limit ? workspace_bytes : workspace_limit;
   if (dtype == WE_DTYPE_F16 && workspace_bytes_of(pl, Dh) > 0 && workspace_bytes_of(pl, Dh) <= given) {
     wide = workspace_bytes_of(pl, Dh, true) <= given;
-    const AttnPlan basic = plan_basic(B, H, Hkv, T, L, n_splits, variant_of(q_tile), cus);
-    if (!wide && workspace_bytes_of(basic, Dh) <= given) {
-      pl = basic;
-      wide = workspace_bytes_of(pl, Dh, true) <= given;
+    if (!wide) {
+      const AttnPlan basic = plan_basic(B, H, Hkv, T, L, n_splits, variant_of(q_tile), cus);
+      if (workspace_bytes_of(basic, Dh) <= given) {
+        pl = basic;
+        wide = workspace_bytes_of(pl, Dh, true) <= given;
+      }
     }
   }
   const size_t ws_need = workspace_bytes_of(pl, Dh, wide);

@@ -149,7 +149,7 @@ class LayerKVCache(nn.Module):
 
         ``reuse_buffers``: the rotated q, the output and the split-context workspace live in
         per-layer tensors that the next eager call of this layer uses again, so a serving loop
-        allocates nothing after its first frame.  The returned tensor is then only valid until
+        asks the allocator for none of them after its first frame.  The returned tensor is then only valid until
         that next call (the attention module consumes it at once); off by default."""
         if torch.compiler.is_compiling():
             s = float(scale) if scale is not None else float(q.shape[-1]) ** -0.5

@@ -21,11 +21,11 @@ _DTYPE_CODE = {torch.bfloat16: _capi.WE_DTYPE_BF16, torch.float16: _capi.WE_DTYP
                torch.float32: _capi.WE_DTYPE_F32}
 
 
-def _dtype_code(t: Tensor) -> int:
+def _dtype_code(dtype: torch.dtype) -> int:
     try:
-        return _DTYPE_CODE[t.dtype]
+        return _DTYPE_CODE[dtype]
     except KeyError:
-        raise RuntimeError(f"unsupported element type {t.dtype}") from None
+        raise RuntimeError(f"unsupported element type {dtype}") from None
 
 
 def _need_device(*tensors: Tensor) -> torch.device:
@@ -122,7 +122,7 @@ def attn_workspace_bytes(B: int, H: int, Hkv: int, T: int, Dh: int, L: int, n_sp
     it is given (float16 holds its partial results in fp32 and needs twice the bytes of bfloat16, the default)."""
     if dtype is None:
         return int(_capi.lib().we_attn_workspace_bytes(B, H, Hkv, T, Dh, L, n_splits, q_tile))
-    return int(_capi.lib().we_attn_workspace_bytes_for(B, H, Hkv, T, Dh, L, n_splits, q_tile, _DTYPE_CODE[dtype]))
+    return int(_capi.lib().we_attn_workspace_bytes_for(B, H, Hkv, T, Dh, L, n_splits, q_tile, _dtype_code(dtype)))
 
 
 def attn_plan(B: int, H: int, Hkv: int, T: int, Dh: int, L: int, n_splits: int = 0, q_tile: int = 0,
@@ -163,7 +163,7 @@ def attn_ring(q: Tensor, kv: Tensor, written: Tensor, t_pos: Tensor, L: int, dil
         raise RuntimeError("kv must be a contiguous [2, B, Hkv, L+T, Dh] of q's element type and written [L+T]")
     lib = _capi.probe_lib()
     with torch.cuda.device(dev):      # (the size depends on the device's compute-unit count)
-        ws_bytes = int(lib.we_attn_workspace_bytes_for(B, H, Hkv, T, Dh, L, n_splits, q_tile, _dtype_code(q)))
+        ws_bytes = int(lib.we_attn_workspace_bytes_for(B, H, Hkv, T, Dh, L, n_splits, q_tile, _dtype_code(q.dtype)))
     if ws_bytes and (workspace is None or workspace.numel() * workspace.element_size() < ws_bytes):
         workspace = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
     if out is None:
@@ -172,7 +172,7 @@ def attn_ring(q: Tensor, kv: Tensor, written: Tensor, t_pos: Tensor, L: int, dil
     code = _call(dev, lib.we_attn_ring_fwd_clocked, q.data_ptr(), _bhtd_strides(q, "q"), kv.data_ptr(), written.data_ptr(),
                  t_pos.data_ptr(), out.data_ptr(), _bhtd_strides(out, "out"), workspace.data_ptr() if ws_bytes else None,
                  workspace.numel() * workspace.element_size() if ws_bytes else 0, B, H, Hkv, T, Dh, L, dilation,
-                 1.0 / math.sqrt(Dh) if scale is None else float(scale), n_splits, q_tile, _dtype_code(q),
+                 1.0 / math.sqrt(Dh) if scale is None else float(scale), n_splits, q_tile, _dtype_code(q.dtype),
                  clocks.data_ptr(), clocks.numel(), _stream_ptr(dev), probe=True)
     _capi.check(code, "we_attn_ring_fwd_clocked")
     return out
