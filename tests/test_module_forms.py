@@ -130,6 +130,25 @@ def test_the_gate_of_another_type_or_layout_stays_torchs():
     assert "gate_w" not in cache.asked and torch.equal(y, ref)
 
 
+class Doubled(torch.Tensor):
+    """A tensor whose linear products are not those of its memory."""
+    @classmethod
+    def __torch_function__(cls, func, types, args=(), kwargs=None):
+        out = super().__torch_function__(func, types, args, kwargs)
+        return out * 2 if func is F.linear else out
+
+
+def test_inputs_that_are_more_than_their_memory_stay_torchs():
+    cache, m = StandIn(), module().requires_grad_(False)
+    x, rows = torch.randn(1, T, D, dtype=torch.bfloat16), residual_rows("")
+    m(x.as_subclass(Doubled), None, None, cache)
+    assert "gate_w" not in cache.asked
+    m(x, None, rows.as_subclass(Doubled), cache)
+    assert "gate_w" in cache.asked and "v1" not in cache.asked
+    m(x, None, rows, cache)
+    assert "gate_w" in cache.asked and "v1" in cache.asked
+
+
 def residual_rows(odd, device="cpu"):
     """Value rows [1, H, T, DH] as an earlier layer hands them on, or the same values where a row starts off a 16-byte
     boundary or its elements are not neighbours."""

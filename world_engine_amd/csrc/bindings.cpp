@@ -683,7 +683,8 @@ PyObject* qkv_rope_kv_attn(PyObject*, PyObject* const* argv, Py_ssize_t n) {
 }
 
 // plain(t, ...): whether an operation on these tensors can be done on their memory without anybody
-// missing it - one element type and device, nobody watching, no gradient or tangent to carry on.
+// missing it - tensors (or parameters) of no other class, of one element type and device, nobody
+// watching, no gradient or tangent to carry on.
 PyObject* plain(PyObject*, PyObject* const* argv, Py_ssize_t n) {
   return guarded([&]() -> PyObject* {
     Args a("plain", argv, n, n);
@@ -692,8 +693,8 @@ PyObject* plain(PyObject*, PyObject* const* argv, Py_ssize_t n) {
     for (Py_ssize_t i = 0; i < n && ok; ++i) {
       const Tensor& t = a.tensor();
       if (first == nullptr) first = &t;
-      ok = plain_memory(t) && !to_record(t) &&
-           t.scalar_type() == first->scalar_type() && t.device() == first->device();
+      ok = THPVariable_CheckExact(argv[i]) && plain_memory(t) && !to_record(t) && t.scalar_type() == first->scalar_type() &&
+           t.device() == first->device();
     }
     return PyBool_FromLong(ok ? 1 : 0);
   });
