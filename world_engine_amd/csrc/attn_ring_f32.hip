@@ -57,7 +57,7 @@ attn_ring_f32_kernel(AttnParams p) {
   __shared__ float msh[NW][F_Q], lsh[NW][F_Q];
   __shared__ int vis[WE_MAX_SLOTS + 2];
 
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int c = lane & 15, g = lane >> 4;
 
   // ---- which queries ----
@@ -131,18 +131,20 @@ attn_ring_f32_kernel(AttnParams p) {
     return kk * NW + wave;
   };
 
+  // (uniform base and 32-bit lane offsets; rows past the frame repeat its last one)
   auto load = [&](f32x4_t(&kf)[NJ], f32x4_t(&vf)[4][NH], int vi_, int sub_) __attribute__((always_inline)) {
-    const int64_t row0 = (int64_t)__builtin_amdgcn_readfirstlane(vis[vi_]) * p.T;
-    const int t0 = sub_ * F_K, last = p.T - 1;  // rows past the frame repeat its last one
-    const float* ks = kplane + (row0 + (t0 + c < last ? t0 + c : last)) * DH + 4 * g;
+    const int64_t row0 = (int64_t)__builtin_amdgcn_readfirstlane(vis[vi_]) * p.T + sub_ * F_K;
+    const int last = p.T - 1 - sub_ * F_K;
+    const char* kb = reinterpret_cast<const char*>(kplane + row0 * DH);
+    const char* vb = reinterpret_cast<const char*>(vplane + row0 * DH);
+    const uint32_t ko = (uint32_t)((c < last ? c : last) * DH + 4 * g) * 4u;
 #pragma unroll
-    for (int j = 0; j < NJ; ++j) kf[j] = *reinterpret_cast<const f32x4_t*>(ks + 16 * j);
+    for (int j = 0; j < NJ; ++j) kf[j] = *reinterpret_cast<const f32x4_t*>(kb + ko + 64 * j);
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const int t = t0 + 4 * g + i;
-      const float* vs = vplane + (row0 + (t < last ? t : last)) * DH + 4 * c;
+      const uint32_t vo = (uint32_t)((4 * g + i < last ? 4 * g + i : last) * DH + 4 * c) * 4u;
 #pragma unroll
-      for (int hh = 0; hh < NH; ++hh) vf[i][hh] = *reinterpret_cast<const f32x4_t*>(vs + 64 * hh);
+      for (int hh = 0; hh < NH; ++hh) vf[i][hh] = *reinterpret_cast<const f32x4_t*>(vb + vo + 256 * hh);
     }
   };
   auto block = [&](const f32x4_t(&kf)[NJ], f32x4_t(&vf)[4][NH], int keys) __attribute__((always_inline)) {
@@ -188,22 +190,21 @@ attn_ring_f32_kernel(AttnParams p) {
   const int mine_n = rounds - (nblk - (rounds - 1) * NW > wave ? 0 : 1);  // rounds this wavefront takes part in
   if (mine_n > 0) {
     f32x4_t ka[NJ], va[4][NH], kb[NJ], vb[4][NH];
-    int at = block_of(0), vi = (int)((unsigned)at / (unsigned)bps), sub = at - vi * bps;
-    load(ka, va, vi, sub);
-    int keys_a = p.T - sub * F_K, keys_b = 0;  // (16 or more = a whole block)
+    // The next block is requested whether there is one or not (the last one again then): behind a branch the
+    // compiler counts the loads in flight as if it had not been taken, and waits for the block just requested.
+    auto fetch = [&](f32x4_t(&kf)[NJ], f32x4_t(&vf)[4][NH], int k) __attribute__((always_inline)) {
+      const int at = block_of(k < mine_n ? k : mine_n - 1), vi = (int)((unsigned)at / (unsigned)bps), sub = at - vi * bps;
+      load(kf, vf, vi, sub);
+      return p.T - sub * F_K;  // keys of the block (16 or more: a whole one)
+    };
+    int keys_a = fetch(ka, va, 0);
     for (int k = 1;; k += 2) {
-      if (k < mine_n) {
-        at = block_of(k); vi = (int)((unsigned)at / (unsigned)bps); sub = at - vi * bps;
-        load(kb, vb, vi, sub);
-        keys_b = p.T - sub * F_K;
-      }
+      const int keys_b = fetch(kb, vb, k);
+      __builtin_amdgcn_sched_barrier(0);
       block(ka, va, keys_a);
       if (k >= mine_n) break;
-      if (k + 1 < mine_n) {
-        at = block_of(k + 1); vi = (int)((unsigned)at / (unsigned)bps); sub = at - vi * bps;
-        load(ka, va, vi, sub);
-        keys_a = p.T - sub * F_K;
-      }
+      keys_a = fetch(ka, va, k + 1);
+      __builtin_amdgcn_sched_barrier(0);
       block(kb, vb, keys_b);
       if (k + 1 >= mine_n) break;
     }
