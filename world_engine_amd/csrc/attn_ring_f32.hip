@@ -15,10 +15,9 @@
 //
 // Bound by the matrix cores (64 MFMAs of 32 cycles per block of 16 keys at Dh = 128, against 16 loads
 // and some 40 vector instructions) and, at 16 queries a workgroup, by the loads' way through the CU's
-// address path beside them: 16 heads of 128, 256 queries, 2048 keys take 54 us = 79 TFLOP/s (a large
-// fp32 matrix product reaches 153 here), 42 us without the loads; 8 heads, 1024 queries and 4096 keys
-// 184 us = 93 TFLOP/s.  The kernel before it (vector ALUs, K and V read from LDS four bytes at a
-// time) took 775 us = 5.5 TFLOP/s for the first; 8 heads of 64, 64 queries, 256 keys: 53 us, now 8.
+// address path beside them: 16 heads of 128, 256 queries, 2048 keys take 45.5 us = 94 TFLOP/s (a large
+// fp32 matrix product reaches 153 here), 37 us without the loads; 8 heads, 1024 queries and 4096 keys
+// 151 us = 114 TFLOP/s.  (54 and 185 us while the next block's loads stood behind a branch, below.)
 #include "attn_mma.h"
 #include "we_kernels.h"
 #include "../../include/we_attn.h"
@@ -156,6 +155,13 @@ attn_ring_f32_kernel(AttnParams p) {
         s0 = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[j][i], qf[j][i], s0, 0, 0, 0);
         s1 = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[j + 1][i], qf[j + 1][i], s1, 0, 0, 0);
       }
+    // (the next block's loads go out between these products: together they keep a wavefront from issuing anything
+    // else while the CU's address path takes them, 47.0 against 45.5 us for the first shape above)
+#pragma unroll
+    for (int i = 0; i < NJ + 4 * NH; ++i) {
+      __builtin_amdgcn_sched_group_barrier(0x20, 1, 0);
+      __builtin_amdgcn_sched_group_barrier(0x8, 4 * NJ / (NJ + 4 * NH), 0);
+    }
     f32x4_t s = s0 + s1;
     if (keys < F_K) {  // missing keys: no weight, and nothing for a zero weight to meet but zeros
 #pragma unroll
@@ -200,11 +206,9 @@ attn_ring_f32_kernel(AttnParams p) {
     int keys_a = fetch(ka, va, 0);
     for (int k = 1;; k += 2) {
       const int keys_b = fetch(kb, vb, k);
-      __builtin_amdgcn_sched_barrier(0);
       block(ka, va, keys_a);
       if (k >= mine_n) break;
       keys_a = fetch(ka, va, k + 1);
-      __builtin_amdgcn_sched_barrier(0);
       block(kb, vb, keys_b);
       if (k + 1 >= mine_n) break;
     }
