@@ -241,8 +241,9 @@ int we_attn_ring_fwd_static(const void* q, const int64_t q_strides[3],
  *                {batch, token}), gate_w at gate_proj.weight [H, H] row-major (out, in).  The
  *                projection's output and the sigmoid's are rounded to the element type like the
  *                module's tensors.  Both NULL = off; not together with `gate`; bf16 / f16 only.
- * Results equal the separate torch operations up to the last bit of the norm's row reduction and of
- * the gate's dot product (1 ulp of the element type); the lerp and the gate multiply have their bits.
+ * Results equal the separate torch operations up to the last bit of the gate's dot product (1 ulp of the
+ * element type); the lerp, the gate multiply and, for half-precision rows, the norm have their bits (the
+ * norm's additions are in torch 2.10's order on the GPU: groups of four, then halves).
  */
 typedef struct we_attn_extras {
   float qk_norm_eps;

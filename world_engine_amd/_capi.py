@@ -158,7 +158,7 @@ class _Native:
             raise RuntimeError("the compiled binding world_engine_amd/_native.so is missing or cannot be loaded "
                                f"(run `python -m world_engine_amd.build`): {e}") from e
         for fn in ("rope_kv_store", "rope_apply", "attn_ring", "attn_ring_static", "rope_kv_attn", "qkv_rope_kv_attn", "linear",
-                   "plain", "blend_ready", "gate_ready"):
+                   "plain", "blend_ready", "gate_ready", "norm_ready"):
             setattr(self, fn, getattr(_native, fn))
         return object.__getattribute__(self, name)
 

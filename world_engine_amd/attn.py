@@ -7,9 +7,10 @@ cache update, masked attention, and with them the value-residual lerp and the he
 two HIP kernel launches (three with context splits) instead of the reference's eager/compiled op
 sequence.  Projections of small half-precision frames run on the library's own kernel (fp32 sums
 rounded once, in another order of additions than a BLAS routine's), others are ordinary torch ops.
-The weightless RMS norm is torch's by default and moves into the store kernel with
-``fuse_elementwise=True`` (1 ulp).  From the projections' rows on, the default module stores the
-bits that the reference's operations give on the same device.
+The weightless RMS norm of half-precision rows is done in the store kernel, in the order of additions
+of torch 2.10's own on the GPU; with another torch it stays torch's unless ``fuse_elementwise=True``.
+From the projections' rows on, the default module stores the bits that the reference's operations give
+on the same device.
 """
 from __future__ import annotations
 
@@ -140,6 +141,10 @@ def ring_attention(q: Tensor, k: Tensor, v: Tensor, block_mask: RingMask, enable
 
 _LINEAR_FORWARD = nn.Linear.forward
 
+# The store kernel's norm adds its squares in the order that torch 2.10 does on the GPU; with any other torch the
+# default module keeps torch's own norm, for its bits.
+_NORM_BITS_KNOWN = torch.__version__.startswith("2.10.") and torch.version.hip is not None
+
 
 def _plain_weight(lin: nn.Module) -> Optional[Tensor]:
     """The weight of a linear layer that is nothing else, so that the product alone stands for a call of it; None for
@@ -187,13 +192,13 @@ class RingAttn(nn.Module):
     ``merged_qkv`` the three projections are one ``qkv_proj`` as after the reference's inference
     patch (``src/patch_model.py:102-114``); otherwise the keys are ``q_proj/k_proj/v_proj``.
 
-    In eager mode the value-residual lerp (torch's bits) and the head gate incl. its H x H projection and
-    sigmoid (projection sums in another order, then the module's own roundings) are done inside the
-    two kernels, unless a gradient is recorded, a type or layout is not theirs, or a layer is more than its
-    weight; ``torch.compile`` fuses the torch operations itself and rounds between them where it
-    chooses to.  ``fuse_elementwise`` moves the QK RMS norm there too: one launch and one pass over
-    q, k and v fewer per layer, rows within 1 ulp of torch's norm instead of bit-identical, which is
-    why it is off unless asked for.
+    In eager mode the QK RMS norm and the value-residual lerp (torch's bits) and the head gate incl. its
+    H x H projection and sigmoid (projection sums in another order, then the module's own roundings) are
+    done inside the two kernels, unless a gradient is recorded, a type or layout is not theirs, or a layer is
+    more than its weight; ``torch.compile`` fuses the torch operations itself and rounds between them where
+    it chooses to.  The norm as a launch of its own took 8.5 of a layer's 58 us (16 + 2 x 8 heads of 128, 256
+    tokens).  ``fuse_elementwise`` has all of it done there whatever torch is installed (the norm's bits are
+    torch 2.10's) and under ``torch.compile`` too.
 
     ``fuse_projection`` (on top of ``merged_qkv`` and ``fuse_elementwise``) also runs the merged
     q/k/v projection in the library, in one kernel with the cache write: x goes in, the rotated q
@@ -321,25 +326,27 @@ class RingAttn(nn.Module):
             return self._forward_fused_projection(x, pos_ids, v1, kv_cache)
         one_call = hasattr(kv_cache, "rope_upsert_attend")
         fuse = self.fuse_elementwise and one_call and x.dtype != torch.float32
+        # The neighbours belong into the kernels (torch.compile has fusions of its own for them).
+        inside = one_call and (fuse or not torch.compiler.is_compiling())
         H, Hkv, Dh = self.n_heads, self.n_kv_heads, self.d_head
         if self.merged_qkv:
             qkv_proj = self.qkv_proj
             rows = _project(qkv_proj, x, _plain_weight(qkv_proj)).view(B, T, H + 2 * Hkv, Dh)
-            heads = rows.transpose(1, 2)
-            q, k, v = heads.split((H, Hkv, Hkv), dim=1)
-            if not fuse:
-                # The norm is per row, so q and k take it together, as the rows lie in memory: one launch over
-                # the projection's output (the v rows it also covers are not used) where two launches over the
-                # strided q and k views each made a copy first.
-                q, k, _ = F.rms_norm(rows, (Dh,)).transpose(1, 2).split((H, Hkv, Hkv), dim=1)
+            q, k, v = rows.transpose(1, 2).split((H, Hkv, Hkv), dim=1)
         else:
-            q, k, v = (_project(proj, x, _plain_weight(proj)).reshape(B, T, -1, Dh) for proj in (self.q_proj, self.k_proj, self.v_proj))
-            if not fuse:
-                q, k = F.rms_norm(q, (Dh,)), F.rms_norm(k, (Dh,))
-            q, k, v = q.transpose(1, 2), k.transpose(1, 2), v.transpose(1, 2)
+            rows = None
+            q, k, v = (_project(proj, x, _plain_weight(proj)).reshape(B, T, -1, Dh).transpose(1, 2)
+                       for proj in (self.q_proj, self.k_proj, self.v_proj))
+        # The norm: in the store kernel with torch's bits, where torch's order of additions is known
+        norm = fuse or (inside and _NORM_BITS_KNOWN and not torch.is_autocast_enabled() and native.norm_ready(q, k))
+        if not norm and rows is not None:
+            # It is per row, so q and k take it together, as the rows lie in memory: one launch over the
+            # projection's output (the v rows it also covers are not used) where two launches over the strided
+            # q and k views each made a copy first.
+            q, k, _ = F.rms_norm(rows, (Dh,)).transpose(1, 2).split((H, Hkv, Hkv), dim=1)
+        elif not norm:
+            q, k = (F.rms_norm(r.transpose(1, 2), (Dh,)).transpose(1, 2) for r in (q, k))
 
-        # The blend and the gate belong into the kernels (torch.compile has fusions of its own for them).
-        inside = one_call and (fuse or not torch.compiler.is_compiling())
         records = self._records(x)
         extras = {}
         if self.value_residual and v1 is None:
@@ -365,7 +372,7 @@ class RingAttn(nn.Module):
                 if inside and not records and native.plain(gates, q):
                     extras["gate"] = gates       # the epilogue multiplies the rounded output, as `y * gates` would
                     gates = None
-        if fuse:
+        if norm:
             extras["qk_norm_eps"] = torch.finfo(torch.float32).eps     # F.rms_norm's epsilon for these inputs
 
         # RoPE(q), RoPE(k), cache write (one launch) and attention over the ring (one or two), all

@@ -725,6 +725,22 @@ PyObject* gate_ready(PyObject* self, PyObject* const* argv, Py_ssize_t n) {
   });
 }
 
+// And for the norm of the query and key rows in the store kernel: half-precision rows of 64 or 128 on 16-byte
+// boundaries, on a GPU.
+PyObject* norm_ready(PyObject* self, PyObject* const* argv, Py_ssize_t n) {
+  return guarded([&]() -> PyObject* {
+    Args a("norm_ready", argv, n, 2);
+    for (int i = 0; i < 2; ++i) {
+      const Tensor& t = a.tensor();
+      if (!t.is_cuda() || (t.scalar_type() != at::kBFloat16 && t.scalar_type() != at::kHalf) || t.dim() != 4 ||
+          (t.size(3) != 64 && t.size(3) != 128) || t.stride(3) != 1 || t.stride(0) % 8 != 0 || t.stride(1) % 8 != 0 ||
+          t.stride(2) % 8 != 0 || !t.has_storage() || (reinterpret_cast<uintptr_t>(t.const_data_ptr()) & 15u) != 0)
+        Py_RETURN_FALSE;
+    }
+    return plain(self, argv, n);
+  });
+}
+
 // x [..., K] times w [N, K] transposed; None where the kernel is not the one to use (shape, layout,
 // element type, a gradient to record, somebody who watches torch's operations): the caller then takes
 // its linear layer.
@@ -766,6 +782,7 @@ PyMethodDef methods[] = {
     {"plain", (PyCFunction)(void (*)(void))plain, METH_FASTCALL, nullptr},
     {"blend_ready", (PyCFunction)(void (*)(void))blend_ready, METH_FASTCALL, nullptr},
     {"gate_ready", (PyCFunction)(void (*)(void))gate_ready, METH_FASTCALL, nullptr},
+    {"norm_ready", (PyCFunction)(void (*)(void))norm_ready, METH_FASTCALL, nullptr},
     {"linear", (PyCFunction)(void (*)(void))linear, METH_FASTCALL, nullptr},
     {"rope_kv_store", (PyCFunction)(void (*)(void))rope_kv_store, METH_FASTCALL, nullptr},
     {"rope_apply", (PyCFunction)(void (*)(void))rope_apply, METH_FASTCALL, nullptr},

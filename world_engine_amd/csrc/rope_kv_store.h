@@ -67,20 +67,33 @@ __device__ __forceinline__ void store8(void* p, const Chunk8<Tag>& c) {
 
 // Weightless RMS norm of a row held 16 elements per lane by `cpr` consecutive lanes (a power of
 // two, at most 64): x * rsqrt(mean(x^2) + eps) in fp32, rounded to the element type, as
-// F.rms_norm on a low-precision tensor does (src/model/nn.py:55-56).
+// F.rms_norm on a low-precision tensor does (src/model/nn.py:55-56).  The squares are added in the order
+// that torch 2.10's norm shows on this GPU - four neighbours one after the other, then halves onto halves:
+// half-precision squares are exact in fp32, so the order is all that decides a sum's bits, and of the orders
+// tried (groups of 1 to 16, neighbouring or strided, sequential or as trees) this one, with this reciprocal
+// root, gives every bit of 2*10^5 rows of 64 and of 128.
 template <typename Tag>
 __device__ __forceinline__ void rms_norm_chunk(Chunk16<Tag>& c, int cpr, int Dh, float eps) {
-  float x[16];
-  float ss = 0.f;
+  float x[16], part[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    part[j] = 0.f;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      x[4 * j + i] = Tag::to_f32(c.e[4 * j + i]);
+      part[j] += x[4 * j + i] * x[4 * j + i];
+    }
+  }
+  for (int m = cpr >> 1; m > 0; m >>= 1)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) part[j] += __shfl_xor(part[j], m);
+  const float r = rsqrtf(((part[0] + part[2]) + (part[1] + part[3])) / (float)Dh + eps);
 #pragma unroll
   for (int i = 0; i < 16; ++i) {
-    x[i] = Tag::to_f32(c.e[i]);
-    ss += x[i] * x[i];
+    float y = x[i] * r;
+    asm("" : "+v"(y));  // (fused with the conversion to f16 the product of a negative value and 0 loses its sign)
+    c.e[i] = Tag::from_f32(y);
   }
-  for (int m = 1; m < cpr; m <<= 1) ss += __shfl_xor(ss, m);
-  const float r = rsqrtf(ss / (float)Dh + eps);
-#pragma unroll
-  for (int i = 0; i < 16; ++i) c.e[i] = Tag::from_f32(x[i] * r);
 }
 
 // torch.lerp(v, v1, w) on 16 elements: fp32 arithmetic, the formula switches at |w| = 0.5

@@ -219,9 +219,9 @@ def rope_kv_attn(q: Tensor, k: Tensor, v: Tensor, pos_ids: Mapping[str, Tensor],
     epsilon for low-precision inputs is ``torch.finfo(torch.float32).eps``); ``v1`` ``[B,Hkv,T,Dh]``
     with the one-element ``v_lamb`` stores ``lerp(v, v1, v_lamb)``; ``gate`` ``[B,H,T]`` (any
     strides, sigmoid applied) multiplies the output rows; ``gate_x`` ``[B,T,H]`` and ``gate_w``
-    ``[H,H]`` have it computed there, ``sigmoid(gate_x @ gate_w.T)``.  The blend and the multiply have
-    torch's bits; the norm (row reduction order) and the gate's projection (order of additions) match
-    the separate torch operations to 1 ulp of the element type."""
+    ``[H,H]`` have it computed there, ``sigmoid(gate_x @ gate_w.T)``.  The blend, the multiply and (for
+    half-precision rows, against torch 2.10) the norm have torch's bits; the gate's projection (order of
+    additions) matches the separate torch operation to 1 ulp of the element type."""
     return native.rope_kv_attn(q, k, v, pos_ids["t_pos"], pos_ids["y_pos"], pos_ids["x_pos"], cos_table, sin_table, grid_h,
                                grid_w, kv, written, L, dilation, is_frozen, scale, n_splits, q_tile, out, workspace, q_rot,
                                token_major_out, qk_norm_eps, v1, v_lamb, gate, gate_x, gate_w, 0, 0)
