@@ -53,6 +53,7 @@
 // Roofline: 4*T*N_vis*Dh flops and 4*N_vis*Dh bytes of K/V per (batch, kv head).
 #include "attn_mma.h"
 #include "device_state.h"
+#include "ring_tiles.h"
 #include "we_kernels.h"
 #include "../../include/we_attn.h"
 
@@ -279,17 +280,12 @@ attn_ring_kernel(AttnParams p) {
   // keys does not matter to a softmax.
   int rot_g = 1;
   while (rot_g * 2 <= p.members && rot_g < 4) rot_g *= 2;
-  const unsigned rot_m = (unsigned)(qtile * p.q_heads + hq_in) & (unsigned)(rot_g - 1);
-  const unsigned rot_end = (unsigned)(ntile - (shorted ? 1 : 0)) & ~(unsigned)(rot_g - 1);
+  const SplitTiles split_tiles = {(unsigned)t_begin, (unsigned)t_end, shorted, (unsigned)rot_g,
+                                  (unsigned)(qtile * p.q_heads + hq_in) & (unsigned)(rot_g - 1)};
   uint32_t toff = 0, tgap = 0;
   struct TileAt { uint32_t off, gap; };
   auto load_offsets = [&](int first) __attribute__((always_inline)) {
-    unsigned kk = (unsigned)(first + lane);
-    const bool head = shorted && kk == 0;
-    if (shorted && kk > 0) --kk;  // (the short tile stands in front of the others)
-    if (kk < rot_end) kk = (kk & ~(unsigned)(rot_g - 1)) | ((kk + rot_m) & (unsigned)(rot_g - 1));
-    unsigned ti = (unsigned)t_begin + kk;
-    if (head || ti > (unsigned)(t_end - 1)) ti = (unsigned)(t_end - 1);
+    const unsigned ti = split_tiles.at((unsigned)(first + lane));
     if (RUN) {
       const unsigned v0 = ti * BN, T = (unsigned)p.T;
       const unsigned sidx = v0 / T, in = v0 - sidx * T;
@@ -310,7 +306,7 @@ attn_ring_kernel(AttnParams p) {
     TileAt t;
     t.off = (uint32_t)__builtin_amdgcn_readlane((int)toff, kc & 63);
     t.gap = RUN ? (uint32_t)__builtin_amdgcn_readlane((int)tgap, kc & 63) : 0u;
-    if (kc < ntile - 1) ++kc;
+    kc = split_tiles.next(kc);
     return t;
   };
   const uint64_t kplane = uniform64(kbase), vplane = uniform64(vbase);
