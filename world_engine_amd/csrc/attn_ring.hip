@@ -542,6 +542,13 @@ attn_ring_kernel(AttnParams p) {
     s_cur = s_next;
   };
 
+  // A wavefront whose 32 rows all lie behind the last token only fetches: its products would be thrown away, and they
+  // cost the others clock (the board runs these kernels at its power limit).  24 heads, 3600 tokens, 8 slots (15 tiles
+  // of 256 rows, the last with 16 of them) 1102 -> 1074 us; 12 heads on 6, 920 tokens 50.9 -> 49.5; 32 heads, 130
+  // tokens, 16 slots 20.0 -> 19.3.  Not in the 128-query shape of whole tiles, whose frames leave no wavefront idle or
+  // half of them: there the branch cost 256-token frames 1 to 2 % (32 slots 28.6 -> 29.1).
+  constexpr bool MAY_IDLE = RUN || KSPLIT == 1;
+  const bool idle = MAY_IDLE && __builtin_amdgcn_readfirstlane(row0 + qb * 32) >= (SHARED ? p.group * p.T : p.T);
   if (ntile > 0) {
     // 256-query shape: zero V slot 3, which stands in for "tile -1", and P, so that the first
     // product adds zeros (the 128-query shape skips the product of its first step instead)
@@ -588,6 +595,22 @@ attn_ring_kernel(AttnParams p) {
     dma_wait<(KA + 1) * NDMA>();
     __syncthreads();  // K(0) and the zeroed V slot (128-query shape: the Q tile, requested long before K(0)) are in LDS
     stamp(1);  // first K tile landed
+    if (idle) {
+      // (the same requests and barriers as the wavefronts that have queries)
+      dma_wait<2 * NDMA>();
+      __syncthreads();
+      for (int j = 0; j < ntile; ++j) {
+        const TileAt o = next_off();
+        dma_k(o, (j + KA) % NST);
+        dma_v(KA == 3 ? off1 : off2, (j + 2) % NST);
+        off2 = off1;
+        off1 = o;
+        dma_wait<2 * NDMA>();
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+      }
+      m_ref = 0.f;
+    } else {
     if (KSPLIT == 2 && q_dma) {
       // row qb*32 + l32 of the tile, logical chunk 2*ks + hh: the K fragment's address arithmetic
       const int x = k_swz<DH>(l32);
@@ -702,6 +725,7 @@ attn_ring_kernel(AttnParams p) {
           o[db] = M::mma(__builtin_bit_cast(frag_t, a8), p_prev[m], o[db]);
         }
       }
+    }
     }
     dma_wait<0>();  // no DMA may still be writing LDS when the rings are reused or the CU is freed
   } else if (q_dma) {
