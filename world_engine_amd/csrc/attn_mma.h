@@ -15,6 +15,9 @@ struct Bf16Mma {
   __device__ static __forceinline__ f32x16_t mma(frag_t a, frag_t b, f32x16_t c) {
     return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
   }
+  __device__ static __forceinline__ f32x4_t mma16(frag_t a, frag_t b, f32x4_t c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
+  }
   __device__ static __forceinline__ frag_t pack8(float v0, float v1, float v2, float v3, float v4,
                                                  float v5, float v6, float v7) {
     frag_t r;
@@ -34,6 +37,9 @@ struct F16Mma {
   typedef _Float16 elem_t;
   __device__ static __forceinline__ f32x16_t mma(frag_t a, frag_t b, f32x16_t c) {
     return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
+  }
+  __device__ static __forceinline__ f32x4_t mma16(frag_t a, frag_t b, f32x4_t c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
   }
   __device__ static __forceinline__ frag_t pack8(float v0, float v1, float v2, float v3, float v4,
                                                  float v5, float v6, float v7) {

@@ -377,6 +377,19 @@ attn_ring_kernel(AttnParams p) {
   // the running reference m_ref of this lane's query (every lane owns one query column of the
   // transposed scores) are applied by one fused multiply-add per logit in front of its
   // exponential: p = 2^(s * c + msc), msc = -m_ref * c.
+  // Row sums of P (of the rounded values).  256-query shape: on the matrix cores; a 16x16x32 product reads P's registers
+  // as 32 keys by 16 columns whose contraction groups are the lane groups, so rows of ones on the even groups, or on the
+  // odd ones, leave every lane its own query's sum, both half-waves' keys in it.  (What is not finite in another
+  // query's P meets a zero there and makes the sum NaN: that takes the rare path, which adds lane by lane.)  A
+  // v_dot2c_f32_bf16 behind another wavefront's products waits for them (16 products and a block's softmax on two
+  // wavefronts of a SIMD: 722 cycles each with eight of them, 606 with two 16x16x32, 556 without); in the kernel, at its
+  // power limit, 24 heads of 64 on 8, 720 tokens 42.9 -> 41.9 us, 4 x 24 heads, 1024 tokens 352 -> 349, 10 heads of 64,
+  // 1500 tokens 55.2 -> 54.4, 24 heads, 3600 tokens 1074 -> 1071.  The 128-query shape keeps the dot products: 16 heads,
+  // 256 tokens 19.9 either way, 32 heads on 8, 64 slots 68.6 -> 68.9.
+  constexpr bool SUMS_MMA = KSPLIT == 1;
+  frag_t sum_rows;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) sum_rows[i] = (typename M::elem_t)((((lane >> 2) ^ (lane >> 4)) & 1) == 0 ? 1.f : 0.f);
   const float lmul = p.scale_log2;
   float msc = 0.f;
   auto set_shift = [&]() __attribute__((always_inline)) { msc = -m_ref * lmul; };
@@ -465,6 +478,7 @@ attn_ring_kernel(AttnParams p) {
     frag_t p_cur[2];
     float e[16];
     float rs = 0.f;
+    f32x4_t sums;  // (SUMS_MMA)
     // VALU slices: the 16 exponentials of the current block are spread evenly over the MFMAs of
     // the step.  The two wavefronts of a SIMD run in phase, so bunching them under the logits
     // would saturate the quarter-rate unit there and leave it idle under the product.
@@ -510,14 +524,22 @@ attn_ring_kernel(AttnParams p) {
       exp_slot(KS + i);
       if (i == 1) p_cur[0] = M::pack8(e[0], e[1], e[2], e[3], e[4], e[5], e[6], e[7]);
       if (i == 2) {
+        if (SUMS_MMA) {
+          sums = M::mma16(sum_rows, p_cur[0], f32x4_t{0.f, 0.f, 0.f, 0.f});
+        } else {
 #pragma unroll
-        for (int t = 0; t < 4; ++t) rs = M::add_pair(rs, p_cur[0], t);
+          for (int t = 0; t < 4; ++t) rs = M::add_pair(rs, p_cur[0], t);
+        }
       }
       if (i == NV - 1) p_cur[1] = M::pack8(e[8], e[9], e[10], e[11], e[12], e[13], e[14], e[15]);
       __builtin_amdgcn_sched_barrier(0);
     }
+    if (SUMS_MMA) {
+      rs = M::mma16(sum_rows, p_cur[1], sums)[0];
+    } else {
 #pragma unroll
-    for (int t = 0; t < 4; ++t) rs = M::add_pair(rs, p_cur[1], t);
+      for (int t = 0; t < 4; ++t) rs = M::add_pair(rs, p_cur[1], t);
+    }
 
     if (__ballot(!(rs <= 256.f)) != 0ull) {
       // Rare: some probability of this block may exceed 2^8.  Raise the reference of the rows
@@ -527,6 +549,11 @@ attn_ring_kernel(AttnParams p) {
       const float m_new = mx > m_ref ? mx : m_ref;
       const float alpha = __builtin_amdgcn_exp2f((m_ref - m_new) * lmul);
       rs = probabilities(p_cur, s_cur, m_new);
+      if (SUMS_MMA) {
+        float lo, up;
+        half_wave_pair(rs, lo, up);
+        rs = lo + up;
+      }
       l_run *= alpha;
       m_ref = m_new;
       set_shift();
@@ -732,9 +759,12 @@ attn_ring_kernel(AttnParams p) {
     dma_wait<0>();  // (a split without visible keys: the Q tile it asked for must not land after the merge below)
   }
 
-  float lo, up;
-  half_wave_pair(l_run, lo, up);
-  float l_tot = lo + up;
+  float l_tot = l_run;
+  if (!SUMS_MMA) {
+    float lo, up;
+    half_wave_pair(l_run, lo, up);
+    l_tot = lo + up;
+  }
   m_ref *= lmul;  // from raw logits to the log2 domain the merges work in
 
   if (KSPLIT == 2) {
