@@ -12,6 +12,7 @@ namespace we {
 // start-up code has one 32-bit division in it (the kernel is short enough for that to show).
 template <typename M, int DH, bool F32>
 __global__ void __launch_bounds__(256) attn_combine_kernel(AttnParams p) {
+  touch_args<AttnParams>();
   const int64_t rows = (int64_t)p.B * p.H * p.T - p.ws_row0;  // rows that were split
   const int item = blockIdx.x * 256 + threadIdx.x;
   if (item >= p.T * (DH / 8)) return;

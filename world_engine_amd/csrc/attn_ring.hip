@@ -123,6 +123,7 @@ constexpr int KEYS_SHARED = 3;  // as KEYS_PACKED, any T > 64, and grouped heads
 template <typename M, int DH, int KSPLIT, int KEYS, bool CLOCKED>
 __global__ void __attribute__((amdgpu_flat_work_group_size(512, 512), amdgpu_waves_per_eu(2, 2)))
 attn_ring_kernel(AttnParams p) {
+  touch_args<AttnParams>();
   constexpr bool SHARED = KEYS == KEYS_SHARED, RUN = KEYS == KEYS_PACKED || SHARED;
   constexpr bool PARTS_F32 = std::is_same<M, F16Mma>::value;
   typedef typename M::frag_t frag_t;

@@ -37,6 +37,7 @@ struct LinLds {
 template <typename M, int BN>
 __global__ void __attribute__((amdgpu_flat_work_group_size(512, 512), amdgpu_waves_per_eu(2, 2)))
 linear_skinny_kernel(LinearParams p) {
+  touch_args<LinearParams>();
   typedef typename M::frag_t frag_t;
   typedef LinLds<BN> L;
   constexpr int NF = BN / 32;              // feature blocks of the tile

@@ -50,6 +50,7 @@ static_assert(2 * 4 * 4 * (32 * 32 * 4) <= IDS_OFF, "the exchange area (4 shares
 template <typename M, typename Tag>
 __global__ void __attribute__((amdgpu_flat_work_group_size(512, 512), amdgpu_waves_per_eu(2, 2)))
 qkv_rope_store_kernel(ProjParams p) {
+  touch_args<ProjParams>();
   typedef typename M::frag_t frag_t;
   typedef typename Tag::store_t st_t;
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];

@@ -19,6 +19,7 @@ namespace we {
 // stores costs an unchecked call 0.5 us).
 template <typename Tag, bool CHECK>
 __global__ void __launch_bounds__(256) rope_kv_store_kernel(StoreParams p) {
+  touch_args<StoreParams>();
   typedef typename Tag::store_t st_t;
   // grid: x = 256-thread slices of the (token, chunk) pairs of one row block, y = head among
   // [q heads | k heads | v heads], z = batch; everything below the block level is 32-bit math
