@@ -84,11 +84,6 @@ template <int N>
 __device__ __forceinline__ void dma_wait() {
   asm volatile("s_waitcnt vmcnt(%0)" : : "n"(N) : "memory");
 }
-__device__ __forceinline__ uint64_t uniform64(uint64_t x) {
-  const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)x);
-  const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(x >> 32));
-  return ((uint64_t)hi << 32) | lo;
-}
 
 // Head gate of output row (b, h, t): the given value, or sigmoid(gate_proj(x[b, t, :H]))[h] with
 // the module's rounding steps (src/model/attn.py:117-118: the projection's output and the sigmoid's

@@ -85,7 +85,7 @@ qkv_rope_store_kernel(ProjParams p) {
   const int dh_shift = s.Dh == 128 ? 7 : 6;
   const int e_h = f_in >> dh_shift;
   const int e_chunk = (f_in & (s.Dh - 1)) >> 4;
-  const int64_t frame_t = s.t_pos[0];
+  int64_t frame_t = s.t_pos[0];
 
   // ---- DMA plumbing: instruction q of a tile moves its rows 4q .. 4q+3 ----
   uint32_t xvo[2], wvo[4];
@@ -245,6 +245,9 @@ qkv_rope_store_kernel(ProjParams p) {
   }
 
   // ---- epilogue: the store kernel's work on this thread's item ----
+  // (the slot's arithmetic belongs here: the compiler puts it, and the wait for the frame index, in front of the first
+  // slot's requests otherwise: 8 layers of 256 tokens 812 against 805 us)
+  asm volatile("" : "+v"(frame_t));
   if (!e_live || (s.guard != nullptr && guard != 0u)) return;  // (refused position ids: nothing is written)
   if (blend) {
     *reinterpret_cast<u32x4_t*>(side.res.e) = res_raw[0];
@@ -256,7 +259,7 @@ qkv_rope_store_kernel(ProjParams p) {
   } else {
     if (which == 2 && p.v_out != nullptr)
       store16<Tag>((st_t*)p.v_out + b * p.vo_b + e_h * p.vo_h + e_t * p.vo_t + e_chunk * 16, in);
-    const SlotInfo si = ring_slot(frame_t, s.dilation, s.num_buckets);
+    const SlotInfo si = ring_slot((int64_t)uniform64((uint64_t)frame_t), s.dilation, s.num_buckets);
     finish_kv_chunk<Tag>(s, which, b, e_h, e_t, e_chunk, si, in, side.rotate, side.c, side.s, side.res, side.lamb);
   }
 }

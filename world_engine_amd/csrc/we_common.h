@@ -29,6 +29,13 @@ __device__ __forceinline__ void touch_args() {
                "s"(word(7)));
 }
 
+// A value that is the same in every lane, as a scalar.
+__device__ __forceinline__ uint64_t uniform64(uint64_t x) {
+  const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)x);
+  const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(x >> 32));
+  return ((uint64_t)hi << 32) | lo;
+}
+
 // Floor division / modulo on int64, the semantics of `//` and `%` on torch int64 tensors
 // (src/model/kv_cache.py:129-130,140).
 __device__ __forceinline__ int64_t floor_div(int64_t a, int64_t b) {
