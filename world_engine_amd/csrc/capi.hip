@@ -458,7 +458,7 @@ int we_qkv_rope_kv_store(const we_qkv_proj* proj, void* q_out, const float* cos_
   hipStream_t st = static_cast<hipStream_t>(stream);
   const Dev dev = dev_for(st);  // (the kernel's LDS limit is raised by the device's set-up)
   if (dev.rc != WE_OK) return dev.rc;
-  return we::launch_qkv_rope_store(pp, dtype, st) == hipSuccess ? WE_OK : WE_ERR_LAUNCH;
+  return we::launch_qkv_rope_store(pp, dtype, dev.state.cus, st) == hipSuccess ? WE_OK : WE_ERR_LAUNCH;
 }
 
 int we_qkv_rope_kv_attn_fwd(const we_qkv_proj* proj, void* q_out, const float* cos_table, const float* sin_table,
@@ -500,7 +500,7 @@ int we_qkv_rope_kv_attn_fwd_checked(const we_qkv_proj* proj, void* q_out, const 
   if (dev.rc != WE_OK) return dev.rc;
   rc = apply_check(check, true, pp.s, st);
   if (rc != WE_OK) return rc;
-  if (we::launch_qkv_rope_store(pp, dtype, st) != hipSuccess) return WE_ERR_LAUNCH;
+  if (we::launch_qkv_rope_store(pp, dtype, dev.state.cus, st) != hipSuccess) return WE_ERR_LAUNCH;
   return launch_attn(p, pl, Dh, dtype, st);
 }
 
@@ -530,7 +530,7 @@ int we_linear(const void* x, int64_t x_row_stride, const void* w, int64_t w_row_
   int bn = linear_tile(M, N, K, dev.state.cus);
   if (bn == 0) bn = N % 128 == 0 ? 128 : (N % 64 == 0 ? 64 : 32);
   if ((((int64_t)M + 63) / 64) * 8 * ((N / bn + 7) / 8) >= (1ll << 31)) return WE_ERR_UNSUPPORTED;
-  return we::launch_linear_skinny(p, bn, dtype, st) == hipSuccess ? WE_OK : WE_ERR_LAUNCH;
+  return we::launch_linear_skinny(p, bn, dtype, dev.state.cus, st) == hipSuccess ? WE_OK : WE_ERR_LAUNCH;
 }
 
 }  // extern "C"

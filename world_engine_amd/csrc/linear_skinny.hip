@@ -9,7 +9,7 @@
 // steps of every slot (A = W rows, B = x rows); the shares are added through LDS in a fixed order and
 // rounded once.  Workgroup id % 8 is the XCD, the row tiles of one weight slab follow each other on
 // one XCD and take the contraction chunks in rotated order (see qkv_proj_store.hip): a slab comes
-// from HBM once and its lines are L2 hits for the other tiles.
+// from HBM once and its lines are L2 hits for the other tiles; CUs without a tile fetch slabs into their L2 (fetch_ahead).
 //
 // Bound by what a CU takes in, (64 + BN) rows of K elements at some 90 GB/s, behind 3.5 us of launch,
 // first slot and reduction.  Against the BLAS routine, us in a graph with weights out of HBM (256 rows):
@@ -56,7 +56,11 @@ linear_skinny_kernel(LinearParams p) {
 
   // ---- which tile ----
   const int xcd = blockIdx.x & 7;
-  const unsigned j = blockIdx.x >> 3;
+  const unsigned j = blockIdx.x >> 3, own = (unsigned)(p.n_tiles + 7) / 8u * (unsigned)p.m_tiles;
+  if (j >= own) {
+    fetch_ahead<BN>(p.w, p.ws, p.n_tiles, p.K, xcd, (int)(j - own), p.helpers, wave, lane, lds0);
+    return;
+  }
   const int ng = (int)(j / (unsigned)p.m_tiles);
   const int mi = (int)j - ng * p.m_tiles;
   const int nt = ng * 8 + xcd;
@@ -174,17 +178,19 @@ linear_skinny_kernel(LinearParams p) {
 }
 
 template <typename M, int BN>
-static hipError_t launch_lin(LinearParams p, hipStream_t stream) {
+static hipError_t launch_lin(LinearParams p, int cus, hipStream_t stream) {
   p.m_tiles = (p.M + LM - 1) / LM;
   p.n_tiles = p.N / BN;
-  const dim3 grid(8u * (unsigned)((p.n_tiles + 7) / 8) * (unsigned)p.m_tiles);
+  const unsigned per_xcd = (unsigned)((p.n_tiles + 7) / 8) * (unsigned)p.m_tiles;
+  p.helpers = helpers_of((int)per_xcd, cus, p.K / LK, LinLds<BN>::NSLOT - 1);
+  const dim3 grid(8u * (per_xcd + (unsigned)p.helpers));
   hipLaunchKernelGGL((linear_skinny_kernel<M, BN>), grid, dim3(512), LinLds<BN>::kBytes, stream, p);
   return hipGetLastError();
 }
 
-hipError_t launch_linear_skinny(const LinearParams& p, int bn, int dtype, hipStream_t stream) {
-  if (dtype == 0) return bn == 32 ? launch_lin<Bf16Mma, 32>(p, stream) : bn == 64 ? launch_lin<Bf16Mma, 64>(p, stream) : launch_lin<Bf16Mma, 128>(p, stream);
-  return bn == 32 ? launch_lin<F16Mma, 32>(p, stream) : bn == 64 ? launch_lin<F16Mma, 64>(p, stream) : launch_lin<F16Mma, 128>(p, stream);
+hipError_t launch_linear_skinny(const LinearParams& p, int bn, int dtype, int cus, hipStream_t stream) {
+  if (dtype == 0) return bn == 32 ? launch_lin<Bf16Mma, 32>(p, cus, stream) : bn == 64 ? launch_lin<Bf16Mma, 64>(p, cus, stream) : launch_lin<Bf16Mma, 128>(p, cus, stream);
+  return bn == 32 ? launch_lin<F16Mma, 32>(p, cus, stream) : bn == 64 ? launch_lin<F16Mma, 64>(p, cus, stream) : launch_lin<F16Mma, 128>(p, cus, stream);
 }
 
 template <typename M, int BN>

@@ -24,7 +24,8 @@
 // x 2048, weights out of HBM: 18.96 -> 18.36 us; 11.2 of it is the tiles' intake alone).
 //
 // The grid is 1-D: workgroup id % 8 is the XCD, and the token tiles of one feature tile follow
-// each other on one XCD, so a weight slab is fetched from HBM once and re-read from that L2.
+// each other on one XCD, so a weight slab is fetched from HBM once and re-read from that L2; the CUs left without a
+// tile fetch weights into it as well (fetch_ahead).
 // Roofline: the weight matrix once (2 K N bytes) + x once; 2 T N K flops.
 #include "attn_mma.h"
 #include "rope_kv_store.h"
@@ -65,6 +66,11 @@ qkv_rope_store_kernel(ProjParams p) {
   // ---- which tile ----
   const int xcd = blockIdx.x & 7, j = blockIdx.x >> 3;
   const int mt_all = p.m_tiles * s.B;
+  const int own = (int)((unsigned)(p.n_tiles + 7) / 8u) * mt_all;
+  if (j >= own) {
+    fetch_ahead<PN>(p.w, p.ws_n, p.n_tiles, p.K, xcd, j - own, p.helpers, wave, lane, lds0);
+    return;
+  }
   const int ng = j / mt_all;
   const int mi = j - ng * mt_all;
   const int nt = ng * 8 + xcd;
@@ -265,16 +271,17 @@ qkv_rope_store_kernel(ProjParams p) {
 }
 
 template <typename M, typename Tag>
-static hipError_t launch_proj(const ProjParams& p, hipStream_t stream) {
-  const unsigned groups = (unsigned)((p.n_tiles + 7) / 8);
-  const dim3 grid(8u * groups * (unsigned)(p.m_tiles * p.s.B));
+static hipError_t launch_proj(ProjParams p, int cus, hipStream_t stream) {
+  const unsigned groups = (unsigned)((p.n_tiles + 7) / 8), per_xcd = groups * (unsigned)(p.m_tiles * p.s.B);
+  p.helpers = helpers_of((int)per_xcd, cus, p.K / PK, NSLOT - 1);
+  const dim3 grid(8u * (per_xcd + (unsigned)p.helpers));
   hipLaunchKernelGGL((qkv_rope_store_kernel<M, Tag>), grid, dim3(512), PROJ_LDS_B, stream, p);
   return hipGetLastError();
 }
 
-hipError_t launch_qkv_rope_store(const ProjParams& p, int dtype, hipStream_t stream) {
-  if (dtype == 0) return launch_proj<Bf16Mma, Bf16Tag>(p, stream);
-  return launch_proj<F16Mma, F16Tag>(p, stream);
+hipError_t launch_qkv_rope_store(const ProjParams& p, int dtype, int cus, hipStream_t stream) {
+  if (dtype == 0) return launch_proj<Bf16Mma, Bf16Tag>(p, cus, stream);
+  return launch_proj<F16Mma, F16Tag>(p, cus, stream);
 }
 
 // The kernel's LDS ring exceeds the default per-launch limit: raised once per device by the

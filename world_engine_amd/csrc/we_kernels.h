@@ -91,6 +91,7 @@ struct ProjParams {
   int64_t vo_b, vo_h, vo_t;
   int m_tiles;          // ceil(T / 64)
   int n_tiles;          // (H + 2 Hkv) Dh / 128
+  int helpers;          // workgroups per XCD without a tile (fetch_ahead)
 };
 
 // y [M, N] = x [M, K] W [N, K]^T (linear_skinny.hip)
@@ -100,15 +101,15 @@ struct LinearParams {
   void* y;
   int64_t xs, ws, ys;   // element strides between rows
   int M, N, K;
-  int m_tiles, n_tiles;
+  int m_tiles, n_tiles, helpers;
 };
 // bn: features per workgroup, 32, 64 or 128
-hipError_t launch_linear_skinny(const LinearParams& p, int bn, int dtype, hipStream_t stream);
+hipError_t launch_linear_skinny(const LinearParams& p, int bn, int dtype, int cus, hipStream_t stream);
 
 hipError_t launch_rope_kv_store(const StoreParams& p, int dtype, hipStream_t stream);
 // the check of p's position ids as a kernel of its own: verdict to p.report and *guard
 hipError_t launch_pos_check(const StoreParams& p, uint32_t* guard, hipStream_t stream);
-hipError_t launch_qkv_rope_store(const ProjParams& p, int dtype, hipStream_t stream);
+hipError_t launch_qkv_rope_store(const ProjParams& p, int dtype, int cus, hipStream_t stream);
 
 // main kernel, one launcher per (element type, head dim) family: ksplit = 2 -> 128 queries per
 // workgroup, 1 -> 256
