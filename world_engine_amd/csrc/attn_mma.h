@@ -1,6 +1,7 @@
 // MFMA wrappers and small wave-level helpers shared by the attention kernels (gfx950).
 #pragma once
 #include "we_common.h"
+#include "fetch_ahead.h"
 
 namespace we {
 
@@ -85,34 +86,18 @@ __device__ __forceinline__ void dma_wait() {
   asm volatile("s_waitcnt vmcnt(%0)" : : "n"(N) : "memory");
 }
 
-// The work of helper workgroup `k` of an XCD in a projection x W^T: it asks for the weights of that XCD's tiles - rows of
-// K elements, tile t (ROWS of them) on XCD t % 8, in steps of 128 elements as the tiles take them - and has no
-// use for them: they are in the XCD's L2 when the tiles get there.  A CU takes 50 to 60 GB/s out of HBM whatever it has
-// in flight, 120 out of L2, and a weight's tile count is given by the product: the CUs that have none do the fetching.
-// The first step is left to the tiles themselves.  Weights out of HBM, a layer of projection + store, attention and second
-// pass (16 heads of 128, d_model 2048, 4 slots): 256 tokens 30.6 -> 29.4 us, 64 tokens 26.6 -> 22.1, 16 heads on 8, 256
-// tokens 29.5 -> 28.4; linear of 128 x 2048 x 2048 8.8 -> 7.65, 192 x 3072 x 3072
-// 15.0 -> 13.15.  Asking for x too, or for 1 KB of a row at a time: no better.
+// The work of helper workgroup `k` of an XCD in a projection x W^T (AheadOrder): DMA into a corner of LDS that nobody reads.
 template <int ROWS>
 __device__ __forceinline__ void fetch_ahead(const void* w, int64_t row_elems, int n_tiles, int K, int xcd, int k, int helpers,
                                             int wave, int lane, uint32_t lds0) {
-  const int quads = ((n_tiles - xcd + 7) >> 3) * (ROWS / 4);  // groups of four rows: one DMA instruction each
+  const AheadOrder order(n_tiles, xcd, helpers, ROWS);
   const uint32_t junk = (uint32_t)__builtin_amdgcn_readfirstlane((int)(lds0 + wave * 1024));
   const int first = __builtin_amdgcn_readfirstlane(k * 8 + wave);
   const uint32_t voff = (uint32_t)(lane >> 4) * (uint32_t)(row_elems * 2) + (uint32_t)((lane & 15) << 4);
-  for (int c = 1; c < K / 128; ++c)
-    for (int q = first; q < quads; q += helpers * 8) {
-      const int row = ((q / (ROWS / 4)) * 8 + xcd) * ROWS + (q % (ROWS / 4)) * 4;
-      dma16(uniform64((uint64_t)(uintptr_t)w + (uint64_t)row * (uint64_t)(row_elems * 2) + (uint64_t)c * 256), voff, junk);
-    }
+  for (int c = 1; c < K / 128; c += order.every)
+    for (int q = first; q < order.quads; q += helpers * 8)
+      dma16(uniform64((uint64_t)(uintptr_t)w + (uint64_t)order.row(q) * (uint64_t)(row_elems * 2) + (uint64_t)c * 256), voff, junk);
   dma_wait<0>();
-}
-// Helpers per XCD: the CUs that tiles leave idle, up to eight (16 and more ask for the same lines no sooner and
-// get in the tiles' way: the layer of 64 tokens above with 8 / 16 / 32: 22.1 / 23.0 / 24.1 us); none where the tiles ask for half of the
-// contraction's steps before their first wait (64 x 1536 x 512 4.04 -> 4.09 us with helpers).
-inline int helpers_of(int tiles_per_xcd, int cus, int steps, int in_flight) {
-  const int idle = cus / 8 - tiles_per_xcd;
-  return idle <= 0 || steps < 2 * in_flight ? 0 : (idle < 8 ? idle : 8);
 }
 
 // Head gate of output row (b, h, t): the given value, or sigmoid(gate_proj(x[b, t, :H]))[h] with
