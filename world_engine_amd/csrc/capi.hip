@@ -190,17 +190,21 @@ int apply_gate_extras(const we_attn_extras* extras, int dtype, we::AttnParams& p
 }
 
 // Features per workgroup of the skinny projection kernel: the narrowest tile whose workgroups still
-// fit the CUs in one round; 0 where a GEMM library is the better choice.  Over 300 shapes (64 to 4096
-// rows, 128 to 8192 features, 128 to 4096 contraction elements, MI355X) the library won where no tile
-// fits one round, where a workgroup's stream gets long while many rows could share a larger tile
-// (4096 x 512 x 1024: 10.0 against 17.8 us), and where a long contraction leaves most CUs idle that
-// it can split (128 x 256 x 4096: 7.9 against 10.6 us).
+// fit the CUs in one round; 0 where a GEMM library is the better choice.  Over 2200 shapes of up to 1024
+// rows (128 to 9216 features, 128 to 8192 contraction elements, MI355X, weights out of HBM) that is where no tile fits one
+// round; where a long contraction leaves CUs idle that the library splits it over (192 x 512 x 5120: 10.1 against 12.4 us;
+// 64 x 2048 x 2048, 64 workgroups: 11.9 against 7.6 here, with the idle CUs fetching weights); for a handful of rows of a
+// long contraction (1 x 3072 x 5120: 10.7 against 15.6); and where the widest tile has a long stream (300 x 6144 x 4096:
+// 30.6 against 38.7).  Against the better of the two everywhere the choice is 2.6 % behind, 1.3 % where there are
+// 48 rows and a quarter as many features as contraction elements or more.
 int linear_tile(int M, int N, int K, int cus) {
   const int64_t m_tiles = ((int64_t)M + 63) / 64;
-  if (K % 128 != 0 || M > 1024 || (int64_t)M * K > (1 << 20) || (K > 2048 && M < 128)) return 0;
+  if (K % 128 != 0 || M > 1024 || (K > 2048 && M < 32) || (K > 6144 && M < 128)) return 0;
   for (int bn = 32; bn <= 128; bn *= 2) {
     const int64_t wgs = m_tiles * (N / bn);
-    if (N % bn == 0 && wgs <= cus) return K > 1024 && wgs * 2 < cus ? 0 : bn;
+    if (N % bn != 0 || wgs > cus) continue;
+    if (K > 1024 && wgs * 2 < cus && wgs * 48 < K) return 0;
+    return bn == 128 && (int64_t)M * K > (1 << 20) ? 0 : bn;
   }
   return 0;
 }
