@@ -9,16 +9,18 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("value", [float("nan"), float("inf"), -float("inf")])
-@pytest.mark.parametrize("q_tile,Dh,dtype,n_splits", [(256, 128, torch.bfloat16, 1), (256, 64, torch.float16, 2), (128, 128, torch.float16, 2)])
-def test_a_row_that_is_not_finite_stays_alone(gpu_device, value, q_tile, Dh, dtype, n_splits):
-    B, H, T, n = 1, 2, 256, 3
+@pytest.mark.parametrize("q_tile,Dh,dtype,n_splits,T", [
+    (256, 128, torch.bfloat16, 1, 256), (256, 64, torch.float16, 2, 256), (128, 128, torch.float16, 2, 256),
+    (128, 64, torch.bfloat16, 1, 250), (128, 64, torch.float16, 2, 250), (128, 64, torch.bfloat16, 1, 131)])
+def test_a_row_that_is_not_finite_stays_alone(gpu_device, value, q_tile, Dh, dtype, n_splits, T):
+    B, H, n = 1, 2, 3
     g = torch.Generator(gpu_device).manual_seed(11)
     q = torch.randn(B, H, T, Dh, device=gpu_device, generator=g).to(dtype)
     kv = torch.randn(2, B, H, (n + 1) * T, Dh, device=gpu_device, generator=g).to(dtype)
     written = torch.ones((n + 1) * T, dtype=torch.bool, device=gpu_device)
     t_pos = torch.zeros(B, T, dtype=torch.long, device=gpu_device)
     want = ops.attn_ring(q, kv, written, t_pos, n * T, 1, None, n_splits, q_tile).clone()
-    odd = [0, 5, 47, 130, 255]
+    odd = [0, 5, 47, 130, T - 1]
     bad = q.clone()
     bad[:, 0, odd, 3] = value
     got = ops.attn_ring(bad, kv, written, t_pos, n * T, 1, None, n_splits, q_tile)

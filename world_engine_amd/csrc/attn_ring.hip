@@ -385,9 +385,11 @@ attn_ring_kernel(AttnParams p) {
   // v_dot2c_f32_bf16 behind another wavefront's products waits for them (16 products and a block's softmax on two
   // wavefronts of a SIMD: 722 cycles each with eight of them, 606 with two 16x16x32, 556 without); in the kernel, at its
   // power limit, 24 heads of 64 on 8, 720 tokens 42.9 -> 41.9 us, 4 x 24 heads, 1024 tokens 352 -> 349, 10 heads of 64,
-  // 1500 tokens 55.2 -> 54.4, 24 heads, 3600 tokens 1074 -> 1071.  The 128-query shape keeps the dot products: 16 heads,
-  // 256 tokens 19.9 either way, 32 heads on 8, 64 slots 68.6 -> 68.9.
-  constexpr bool SUMS_MMA = KSPLIT == 1;
+  // 1500 tokens 55.2 -> 54.4, 24 heads, 3600 tokens 1074 -> 1071.  128-query shape: heads of 64 off the 64-key tile, where
+  // the softmax outweighs the products (60 heads on 15, 304 tokens 18.2 -> 17.9; 16 heads, 2 x 1000 tokens 82.0 -> 81.0;
+  // 1540 tokens 68.9 -> 68.3).  The others keep the dot products: 16 heads of 128, 256 tokens 19.9 either way, 32 on 8, 64
+  // slots 68.6 -> 68.9; 16 heads of 64, 256 tokens, 64 slots 32.9 -> 33.1.
+  constexpr bool SUMS_MMA = KSPLIT == 1 || (DH == 64 && KEYS != KEYS_TILED);
   frag_t sum_rows;
 #pragma unroll
   for (int i = 0; i < 8; ++i) sum_rows[i] = (typename M::elem_t)((((lane >> 2) ^ (lane >> 4)) & 1) == 0 ? 1.f : 0.f);
