@@ -24,15 +24,17 @@ struct SplitTiles {
     const bool head = shorted && k == 0;
     if (shorted && k > 0) --k;  // (the short tile stands in front of the others)
     if (k < rot_end) k = (k & ~(rot_g - 1u)) | ((k + rot_m) & (rot_g - 1u));
-    unsigned t = begin + k;
-    if (head || t > end - 1) t = end - 1;
     // Only the first request keeps to the keys that the short tile has: the rows behind the last one are nobody's.
     // Where it is all there is, the requests that follow it go to the whole tile in front of it.
-    if (shorted && count() == 1 && !head) t = begin - 1;
-    return t;
+    const unsigned top = end - (shorted && count() == 1 ? 2u : 1u), t = begin + k;
+    return head ? end - 1 : (t < top ? t : top);
   }
-  // place that the request after the one for place k is for: the last one again once there
-  WE_TILES_FN int next(int k) const { return k < (int)count() - 1 || (shorted && k == 0) ? k + 1 : k; }
+  // place that the request after the one for place k is for: the last one again once there (a short tile alone is
+  // followed by the whole one in front of it; the bound is the same for every k)
+  WE_TILES_FN int next(int k) const {
+    const int last = shorted && count() == 1 ? 1 : (int)count() - 1;
+    return k < last ? k + 1 : k;
+  }
 };
 
 }  // namespace we
