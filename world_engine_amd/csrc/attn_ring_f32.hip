@@ -119,7 +119,7 @@ attn_ring_f32_kernel(AttnParams p) {
   // Blocks go round the wavefronts in rounds of NW.  The workgroups that share a K/V stream take the
   // rounds in groups of rot_g, member m starting at round m of every group: they then ask for
   // different lines at any one time, and each line comes from memory at one member's request (184
-  // against 192 us for the 1024-query shape above; groups of 8 or 16: the same).
+  // against 192 us for the 1024-query shape above when it took 184; groups of 8 or 16: the same, then and now).
   const int bps = (p.T + F_K - 1) / F_K;  // blocks per slot; the last one may be short
   const int nblk = nvis * bps, rounds = (nblk + NW - 1) / NW;
   int rot_g = 1;

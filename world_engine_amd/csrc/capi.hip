@@ -195,7 +195,7 @@ int apply_gate_extras(const we_attn_extras* extras, int dtype, we::AttnParams& p
 // round; where a long contraction leaves CUs idle that the library splits it over (192 x 512 x 5120: 10.1 against 12.4 us;
 // 64 x 2048 x 2048, 64 workgroups: 11.9 against 7.6 here, with the idle CUs fetching weights); for a handful of rows of a
 // long contraction (1 x 3072 x 5120: 10.7 against 15.6); and where the widest tile has a long stream (300 x 6144 x 4096:
-// 30.6 against 38.7).  Against the better of the two everywhere the choice is 2.6 % behind, 1.3 % where there are
+// 30.6 against 38.7).  Against the better of the two everywhere the choice is 2.7 % behind, 1.4 % where there are
 // 48 rows and a quarter as many features as contraction elements or more.
 int linear_tile(int M, int N, int K, int cus) {
   const int64_t m_tiles = ((int64_t)M + 63) / 64;

@@ -14,7 +14,7 @@
 // Bound by what a CU takes in, (64 + BN) rows of K elements at some 90 GB/s, behind 3.5 us of launch,
 // first slot and reduction.  Against the BLAS routine, us in a graph with weights out of HBM (256 rows):
 // 2048 x 2048 8.2 / 9.6, 4096 x 2048 12.0 / 13.4, 6144 x 2048 16.9 / 24.2, 3072 x 3072 15.0 / 17.7;
-// 64 rows, 1536 x 512 4.3 / 7.0.
+// 64 rows, 1536 x 512 4.1 / 7.0, 2048 x 2048 7.6 / 11.9, 3072 x 3072 11.5 / 16.1.
 #include "attn_mma.h"
 #include "device_state.h"
 #include "we_kernels.h"
