@@ -22,3 +22,15 @@ def test_f32_attention_block_edges(gpu_device, B, H, Hkv, T, Dh, n, d):
         (q_o, k_all, v_all, mask), (q_h, ring) = p.store(q, k, v, pos)
         out = p.attend(q_h, ring)
         assert (out.cpu() - ro.attention_fp32(q_o, k_all, v_all, mask)).abs().max().item() <= 1e-5, f"t={t}"
+
+
+@pytest.mark.parametrize("B,H,T,Dh,n", [(1, 2, 64, 64, 9), (1, 2, 64, 128, 9), (3, 6, 240, 128, 2)])
+def test_f32_attention_every_number_of_blocks_a_wavefront(gpu_device, B, H, T, Dh, n):
+    """A ring that fills: wavefronts take none, one, two, three, ... blocks of keys, the last ones behind the loop (four
+    key blocks per slot for eight wavefronts; 15 per slot for four, with more workgroups than CUs)."""
+    p = Pair(gpu_device, torch.float32, B=B, H=H, Hkv=H, T=T, Dh=Dh, n_slots=n, d=1, cfg_id=92)
+    for t in range(n + 1):
+        q, k, v, pos = p.inputs(t)
+        (q_o, k_all, v_all, mask), (q_h, ring) = p.store(q, k, v, pos)
+        out = p.attend(q_h, ring)
+        assert (out.cpu() - ro.attention_fp32(q_o, k_all, v_all, mask)).abs().max().item() <= 1e-5, f"t={t}"

@@ -15,9 +15,9 @@
 //
 // Bound by the matrix cores (64 MFMAs of 32 cycles per block of 16 keys at Dh = 128, against 16 loads
 // and some 40 vector instructions) and, at 16 queries a workgroup, by the loads' way through the CU's
-// address path beside them: 16 heads of 128, 256 queries, 2048 keys take 45.5 us = 94 TFLOP/s (a large
+// address path beside them: 16 heads of 128, 256 queries, 2048 keys take 44.4 us = 97 TFLOP/s (a large
 // fp32 matrix product reaches 153 here), 37 us without the loads; 8 heads, 1024 queries and 4096 keys
-// 151 us = 114 TFLOP/s.  (54 and 185 us while the next block's loads stood behind a branch, below.)
+// 149 us = 115 TFLOP/s.  (54 and 185 us while the next block's loads stood behind a branch, below.)
 #include "attn_mma.h"
 #include "we_kernels.h"
 #include "../../include/we_attn.h"
@@ -192,25 +192,35 @@ attn_ring_f32_kernel(AttnParams p) {
       for (int hh = 0; hh < NH; ++hh)
 #pragma unroll
         for (int e = 0; e < 4; ++e) o[hh][e] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[i][hh][e], pr[i], o[hh][e], 0, 0, 0);
+    // (two blocks in a row are not scheduled as one: 44.4 against 46.8 us for the first shape above)
+    __builtin_amdgcn_sched_barrier(0);
   };
   const int mine_n = rounds - (nblk - (rounds - 1) * NW > wave ? 0 : 1);  // rounds this wavefront takes part in
   if (mine_n > 0) {
     f32x4_t ka[NJ], va[4][NH], kb[NJ], vb[4][NH];
-    // The next block is requested whether there is one or not (the last one again then): behind a branch the
-    // compiler counts the loads in flight as if it had not been taken, and waits for the block just requested.
+    // The loop always requests the next block - behind a branch the compiler counts the loads in flight as if it had
+    // not been taken, and waits for the block just requested - and the last one or two blocks follow it.  (A last block
+    // requested a second time, for nothing, costs wavefronts with one or two of them most: attention alone, 4 heads of 128,
+    // 64 queries, 128 keys 9.8 -> 8.75 us, 8 heads, 256 keys 12.25 -> 11.4, 8 heads of 64, 256 keys 7.64 -> 7.40, 128 keys
+    // 6.43 -> 6.11.)
     auto fetch = [&](f32x4_t(&kf)[NJ], f32x4_t(&vf)[4][NH], int k) __attribute__((always_inline)) {
-      const int at = block_of(k < mine_n ? k : mine_n - 1), vi = (int)((unsigned)at / (unsigned)bps), sub = at - vi * bps;
+      const int at = block_of(k), vi = (int)((unsigned)at / (unsigned)bps), sub = at - vi * bps;
       load(kf, vf, vi, sub);
       return p.T - sub * F_K;  // keys of the block (16 or more: a whole one)
     };
-    int keys_a = fetch(ka, va, 0);
-    for (int k = 1;; k += 2) {
+    int keys_a = fetch(ka, va, 0), k = 1;
+    for (; k + 1 < mine_n; k += 2) {
       const int keys_b = fetch(kb, vb, k);
       block(ka, va, keys_a);
-      if (k >= mine_n) break;
       keys_a = fetch(ka, va, k + 1);
       block(kb, vb, keys_b);
-      if (k + 1 >= mine_n) break;
+    }
+    if (k < mine_n) {
+      const int keys_b = fetch(kb, vb, k);
+      block(ka, va, keys_a);
+      block(kb, vb, keys_b);
+    } else {
+      block(ka, va, keys_a);
     }
   }
 
