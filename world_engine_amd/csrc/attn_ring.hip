@@ -24,8 +24,8 @@
 //   S^T = K Q^T        v_mfma_f32_32x32x16, A = K rows (ds_read_b128), B = Q in registers as
 //                      loaded (no scaling, so nothing is rounded in front of the matrix core).
 //   P = 2^((S-m) c)    one fused multiply-add per logit applies the softmax scale (c = scale *
-//                      log2 e) and the running reference m, then v_exp_f32 + v_cvt_pk +
-//                      v_dot2c row sum; each lane owns one query column.
+//                      log2 e) and the running reference m, then v_exp_f32 + v_cvt_pk and the row sum
+//                      (v_dot2c, or a small product); each lane owns one query column.
 //   O^T += V^T P^T     A = V^T via ds_read_b64_tr_b16, B = P straight from registers.
 // The three are software-pipelined across blocks (logits of block i+1 and product of block i-1
 // run on the matrix cores while the VALU handles block i); LDS fragment reads are stated up to 15
@@ -385,11 +385,12 @@ attn_ring_kernel(AttnParams p) {
   // v_dot2c_f32_bf16 behind another wavefront's products waits for them (16 products and a block's softmax on two
   // wavefronts of a SIMD: 722 cycles each with eight of them, 606 with two 16x16x32, 556 without); in the kernel, at its
   // power limit, 24 heads of 64 on 8, 720 tokens 42.9 -> 41.9 us, 4 x 24 heads, 1024 tokens 352 -> 349, 10 heads of 64,
-  // 1500 tokens 55.2 -> 54.4, 24 heads, 3600 tokens 1074 -> 1071.  128-query shape: heads of 64 off the 64-key tile, where
-  // the softmax outweighs the products (60 heads on 15, 304 tokens 18.2 -> 17.9; 16 heads, 2 x 1000 tokens 82.0 -> 81.0;
-  // 1540 tokens 68.9 -> 68.3).  The others keep the dot products: 16 heads of 128, 256 tokens 19.9 either way, 32 on 8, 64
-  // slots 68.6 -> 68.9; 16 heads of 64, 256 tokens, 64 slots 32.9 -> 33.1.
-  constexpr bool SUMS_MMA = KSPLIT == 1 || (DH == 64 && KEYS != KEYS_TILED);
+  // 1500 tokens 55.2 -> 54.4, 24 heads, 3600 tokens 1074 -> 1071 (once more with the present loops: 1600 tokens, 24 heads
+  // of 64 140.0 against 136.7, 4 x 40 heads, 256 tokens 32.4 / 30.4).  The 128-query shape keeps the dot products, whose
+  // result a step has sooner: 2 x 16 heads of 64, 1000 tokens 0.6 to 1.4 % faster with them (8 slots 74.4 against 75.3 us),
+  // 13 heads of 64, 209 tokens, 2 slots 8.83 / 8.97, 56 shapes of heads of 64 off the key tile 0.25 % in the mean; 16 heads
+  // of 128, 256 tokens 19.9 either way, 32 on 8, 64 slots 68.6 / 68.9.
+  constexpr bool SUMS_MMA = KSPLIT == 1;
   frag_t sum_rows;
 #pragma unroll
   for (int i = 0; i < 8; ++i) sum_rows[i] = (typename M::elem_t)((((lane >> 2) ^ (lane >> 4)) & 1) == 0 ? 1.f : 0.f);
@@ -640,9 +641,10 @@ attn_ring_kernel(AttnParams p) {
         asm volatile("" ::: "memory");
       }
       if (KSPLIT == 2 && DH == 64) {
-        // Nothing of it is merged, stored or kept, and the two ways need not meet again: 8 heads, 100 tokens, 2 slots
-        // 7.73 -> 7.61 us, 13 heads, 209 tokens, 2 slots 9.05 -> 8.96.  The other shapes are better off where they meet (16
-        // heads of 128, 225 tokens, 2 slots 12.54 against 12.69; 256 queries: 24 heads of 64 on 8, 720 tokens 43.8 / 44.1).
+        // Nothing of it is merged, stored or kept, and the two ways need not meet again: bf16, 8 heads, 100 tokens, 2
+        // slots 7.70 -> 7.57 us, 13 heads, 209 tokens 8.97 -> 8.88, 2 x 24 heads, 150 tokens 8.15 -> 8.03; f16 the same to 1 %
+        // slower (7.71 / 7.72, 9.00 / 9.01, 8.10 / 8.19).  The other shapes gain nothing (16 heads of 128, 225 tokens, 2 slots
+        // 12.72 / 12.74, 6 heads, 150 tokens 9.91 / 9.99; 256 queries: 24 heads of 64 on 8, 720 tokens 42.9 / 43.2).
         dma_wait<0>();
         __syncthreads();
         __syncthreads();
