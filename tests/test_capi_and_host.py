@@ -501,3 +501,14 @@ def test_rope_position_ids_are_bounds_checked_in_eager_mode():
     cos, sin = ro.rope_table_1d(4 * 16, 32)
     with pytest.raises((IndexError, RuntimeError)):
         ro.rope_angles(ro.synth_pos_ids(4, 1, 16, 4), cos, sin, 4, 4)
+
+
+@pytest.mark.parametrize("version,commit", [
+    ("2.10.0+rocm7.0", "0" * 40), ("2.10.1+rocm7.0", None), ("2.10.0", None), ("2.10.0+cu130", None), ("2.11.0+rocm7.0", None),
+    ("2.10.0a0+local", "449b1768410104d3ed79d3bcfe4ba1d65c7f22c0")])
+def test_the_kernels_norm_stands_for_one_build_of_torchs(version, commit):
+    """The default module has its norm in the store kernel only with the build whose bits were compared: another version,
+    variant or source commit keeps torch's norm."""
+    from world_engine_amd import attn
+    assert attn._norm_bits_known(*attn._NORM_BITS_BUILD)
+    assert not attn._norm_bits_known(version, commit)

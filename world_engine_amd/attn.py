@@ -7,8 +7,8 @@ cache update, masked attention, and with them the value-residual lerp and the he
 two HIP kernel launches (three with context splits) instead of the reference's eager/compiled op
 sequence.  Projections of small half-precision frames run on the library's own kernel (fp32 sums
 rounded once, in another order of additions than a BLAS routine's), others are ordinary torch ops.
-The weightless RMS norm of half-precision rows is done in the store kernel, in the order of additions
-of torch 2.10's own on the GPU; with another torch it stays torch's unless ``fuse_elementwise=True``.
+The weightless RMS norm of half-precision rows is done in the store kernel, in the order of additions of
+torch 2.10.0+rocm7.0's own on the GPU; with any other build it stays torch's unless ``fuse_elementwise=True``.
 From the projections' rows on, the default module stores the bits that the reference's operations give
 on the same device.
 """
@@ -141,9 +141,17 @@ def ring_attention(q: Tensor, k: Tensor, v: Tensor, block_mask: RingMask, enable
 
 _LINEAR_FORWARD = nn.Linear.forward
 
-# The store kernel's norm adds its squares in the order that torch 2.10 does on the GPU; with any other torch the
-# default module keeps torch's own norm, for its bits.
-_NORM_BITS_KNOWN = torch.__version__.startswith("2.10.") and torch.version.hip is not None
+# The store kernel's norm adds its squares in the order of this build of torch's own norm on the GPU (found by comparing
+# outputs, and held by a test on it); a build of other sources may add in another, so with any other the default module
+# keeps torch's own norm, for its bits.
+_NORM_BITS_BUILD = ("2.10.0+rocm7.0", "449b1768410104d3ed79d3bcfe4ba1d65c7f22c0")
+
+
+def _norm_bits_known(version: str, git_version: Optional[str]) -> bool:
+    return (version, git_version) == _NORM_BITS_BUILD
+
+
+_NORM_BITS_KNOWN = _norm_bits_known(str(torch.__version__), torch.version.git_version)
 
 
 def _plain_weight(lin: nn.Module) -> Optional[Tensor]:
@@ -198,7 +206,7 @@ class RingAttn(nn.Module):
     more than its weight; ``torch.compile`` fuses the torch operations itself and rounds between them where
     it chooses to.  The norm as a launch of its own took 8.5 of a layer's 58 us (16 + 2 x 8 heads of 128, 256
     tokens).  ``fuse_elementwise`` has all of it done there whatever torch is installed (the norm's bits are
-    torch 2.10's) and under ``torch.compile`` too.
+    torch 2.10.0+rocm7.0's) and under ``torch.compile`` too.
 
     ``fuse_projection`` (on top of ``merged_qkv`` and ``fuse_elementwise``) also runs the merged
     q/k/v projection in the library, in one kernel with the cache write: x goes in, the rotated q
