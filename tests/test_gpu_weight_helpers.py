@@ -31,3 +31,18 @@ def test_product_is_exact_beside_helpers(gpu_device, M, N, K, dtype):
 def test_long_contractions_of_few_workgroups_are_left_to_the_library(gpu_device, M, N, K):
     x = torch.zeros(M, K, device=gpu_device, dtype=torch.bfloat16)
     assert native.linear(x, torch.zeros(N, K, device=gpu_device, dtype=torch.bfloat16)) is None
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [
+    (1024, 512, 8192), (961, 512, 16384),    # 256 tiles of 32 features, one round to the last CU
+    (1000, 1024, 4096), (900, 1088, 8192),   # tiles of 64, the last row tile short; 255 workgroups
+    (1024, 96, 2304)])                       # the longest contraction that 48 workgroups are taken for
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_product_is_exact_for_many_rows_of_a_long_contraction(gpu_device, M, N, K, dtype):
+    print(f"M={M} N={N} K={K} {dtype}", flush=True)
+    g = torch.Generator(gpu_device).manual_seed(K)
+    x = torch.randint(-3, 4, (M, K), device=gpu_device, generator=g).to(dtype)
+    w = torch.randint(-3, 4, (N, K), device=gpu_device, generator=g).to(dtype)
+    # (sums of at most 16384 products of at most 9 - whole numbers below 2^24 - of a spread of 512, far inside f16's range)
+    assert torch.equal(native.linear(x, w), (x.float() @ w.float().t()).to(dtype))
