@@ -177,8 +177,8 @@ def _kernel_covers(rows: int, features: int, contraction: int, half: bool) -> bo
 
 def _project(lin: nn.Module, x: Tensor, w: Optional[Tensor]) -> Tensor:
     """``lin(x)``, on the library's own kernel where the frame is small enough for it to be the faster one
-    (one round of workgroups; 256 x 2048 x 2048: 8.2 us against 9.6 on the GPU, and 4 against 19 us of the
-    host's time, most of it the BLAS routine's choice of a kernel).  fp32 sums rounded once, as there.  ``w`` is the
+    (one round of workgroups; 256 x 2048 x 2048, weights out of HBM: 10.0 us against 14.1 on the GPU, and 4 against 19 us
+    of the host's time, most of it the BLAS routine's choice of a kernel).  fp32 sums rounded once, as there.  ``w`` is the
     layer's ``_plain_weight``."""
     if w is not None and type(x) is Tensor and not torch.is_autocast_enabled():
         if torch.compiler.is_compiling():        # the opaque op where the kernel covers the shape, for the same bits as eager
@@ -215,10 +215,10 @@ class RingAttn(nn.Module):
     That kernel is built for the frames this path is slow on - a few hundred tokens, where the
     projection streams its weights once and is bound by memory latency: 64 tokens x 128 features
     per workgroup, one workgroup per CU.  Where the shape needs more workgroups than the 256 CUs
-    (``fused_projection_max_workgroups``) the projection is a matrix-core-bound GEMM, the BLAS
-    routine is the faster one (measured at 16 heads of 128, d_model 2048, per call: 256 tokens
-    16.5 us against 23.4 us for linear layer + store kernel; 1024 tokens 45 against 36; 4096
-    tokens of 24 heads, d_model 3072: 356 against 214), and ``forward`` takes the linear layer
+    (``fused_projection_max_workgroups``) the projection is a matrix-core-bound GEMM and the BLAS
+    routine the faster one (16 heads of 128, d_model 2048, per call with weights out of HBM, against linear
+    layer + store kernel: 256 tokens 17.2 us against 20.6, with the BLAS routine 30.7; 1024 tokens 46.8
+    against 39.6; 4096 tokens of 24 heads, d_model 3072: 365 against 224), and ``forward`` takes the linear layer
     followed by the ``fuse_elementwise`` call instead.
     """
 

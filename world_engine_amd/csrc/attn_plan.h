@@ -130,9 +130,10 @@ inline AttnPlan plan_basic(int B, int H, int Hkv, int T, int64_t L, int n_splits
 // - a unit's workgroups all run on one - in rounds of a workgroup per CU; then the second pass over the
 // partial rows.  Per 64-key tile, per round and per call, with the partial rows' traffic at 3 to 5 TB/s;
 // fitted to 860 timings over 46 shapes (2 to 124 heads, 153 to 3600 tokens, 2 to 64 slots, both tile
-// sizes, 1 to 24 parts), which it meets to 3 to 7 %.  The rows counted are 16-bit ones; an f16 call's are
-// fp32, and its best plan differs little: over 30 shapes the choice is 1.1 % behind the best uniform
-// split on average for bf16, 1.7 % for f16.
+// sizes, 1 to 24 parts), which it met to 3 to 7 %.  The kernels have become faster since: over 1322 timings
+// of 30 shapes the estimate is 3 to 4.5 % high for either tile size and head dim alike, and the choices, which hang
+// on its ratios, are as good as they were: 0.8 to 1 % behind the best uniform split on average for bf16.  The
+// rows counted are 16-bit ones; an f16 call's are fp32, and its best plan differs little: 1.3 to 1.6 % behind.
 inline double plan_cost(const AttnPlan& pl, int B, int H, int Hkv, int T, int Dh, int64_t L) {
   struct Fit { double tile, round, call, comb, comb_mb; };
   static constexpr Fit kFit[2][2] = {{{0.484, 3.94, 2.21, 2.79, 0.215}, {0.733, 3.01, 2.39, 3.39, 0.331}},

@@ -190,13 +190,15 @@ int apply_gate_extras(const we_attn_extras* extras, int dtype, we::AttnParams& p
 }
 
 // Features per workgroup of the skinny projection kernel: the narrowest tile whose workgroups still
-// fit the CUs in one round; 0 where a GEMM library is the better choice.  Over 2200 shapes of up to 1024
-// rows (128 to 9216 features, 128 to 8192 contraction elements, MI355X, weights out of HBM) that is where no tile fits one
-// round; where a long contraction leaves CUs idle that the library splits it over (192 x 512 x 5120: 10.1 against 12.4 us;
-// 64 x 2048 x 2048, 64 workgroups: 11.9 against 7.6 here, with the idle CUs fetching weights); for a handful of rows of a
-// long contraction (1 x 3072 x 5120: 10.7 against 15.6); and where the widest tile has a long stream (300 x 6144 x 4096:
-// 30.6 against 38.7).  Against the better of the two everywhere the choice is 2.7 % behind, 1.4 % where there are
-// 48 rows and a quarter as many features as contraction elements or more.
+// fit the CUs in one round; 0 where a GEMM library is the better choice.  Over 2000 shapes of up to 1024 rows (128 to
+// 9216 features, 128 to 8192 contraction elements, MI355X) the kernel takes 0.69 of the library's time where it is chosen
+// with weights out of HBM, 0.80 with weights in the last-level cache.  The lines were drawn for the latter: where no tile fits
+// one round; where a long contraction leaves CUs idle that the library splits it over (192 x 512 x 5120: 10.1 us there
+// against 12.8); for a handful of rows of a long contraction (1 x 3072 x 5120: 8.1 against 12.6); and where the widest tile
+// has a long stream.  Against the better of the two the choice is 3.9 % behind there, 0.9 % where there are 48 rows and a
+// quarter as many features as contraction elements or more.  With weights out of HBM that is 9.2 and 1.4 %: a long
+// contraction of few rows or features would be the kernel's then (2 x 1248 x 2688: 9.2 against 16.7 us, 8.2 against 12.4
+// from the cache).
 int linear_tile(int M, int N, int K, int cus) {
   const int64_t m_tiles = ((int64_t)M + 63) / 64;
   if (K % 128 != 0 || M > 1024 || (K > 2048 && M < 32) || (K > 6144 && M < 128)) return 0;

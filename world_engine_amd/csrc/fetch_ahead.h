@@ -4,10 +4,12 @@
 // A projection x W^T of a small frame is bound by what the CUs with a tile take in: 50 to 60 GB/s out of HBM whatever a CU
 // has in flight, 120 out of L2.  The CUs that have no tile run a workgroup that asks for the weights of their XCD's tiles
 // in steps of 128 contraction elements, as the tiles take them, and has no use for them: they are in the XCD's L2 when the
-// tiles get there.  The first step is left to the tiles themselves.  Weights out of HBM, a layer of projection + store,
-// attention and second pass (16 heads of 128, d_model 2048, 4 slots): 256 tokens 30.6 -> 29.4 us, 64 tokens 26.6 -> 22.1,
-// 16 heads on 8, 256 tokens 29.5 -> 28.4; linear of 128 x 2048 x 2048 8.8 -> 7.65, 192 x 3072 x 3072 15.0 -> 13.15.
-// Asking for x too, or for 1 KB of a row at a time: no better.
+// tiles get there.  The first step is left to the tiles themselves.  us without / with them, weights out of HBM: linear of
+// 64 x 2048 x 2048 11.2 / 8.7, 192 x 3072 x 3072 17.1 / 14.7; a layer of projection + store, attention and second pass (16
+// heads of 128, d_model 2048, 4 slots) of 256 tokens 34.9 / 33.1, 64 tokens 33.6 / 27.4, 16 heads on 8, 256 tokens 33.7 /
+// 31.6, 40 heads (5120), 64 tokens 62.5 / 59.3.  Weights that are in the last-level cache anyway gain nothing (7.24 / 7.28,
+// 29.2 / 29.2), and the layer of 64 tokens loses 0.4 us (22.7 / 23.1).  Asking for x too, or for 1 KB of a row at a time: no
+// better.
 #pragma once
 
 #ifdef __HIPCC__
@@ -19,9 +21,9 @@
 namespace we {
 
 // Helpers per XCD: eight where tiles leave that many CUs idle (16 and more ask for the same lines no sooner and get in the
-// tiles' way: the layer of 64 tokens above with 8 / 16 / 32: 22.1 / 23.0 / 24.1 us; fewer beside more tiles are no help, 52
-// heads on 26, d_model 6656, 81 tokens with six: 49.4 -> 51.7); none where the tiles ask for half of the contraction's
-// steps before their first wait (64 x 1536 x 512 4.04 -> 4.09 us with helpers).
+// tiles' way: the layer of 64 tokens above, its weights partly in that cache, with 8 / 16 / 32: 22.1 / 23.0 / 24.1 us; fewer
+// beside more tiles are no help, 52 heads on 26, d_model 6656, 81 tokens with six: 49.4 -> 51.7); none where the tiles ask
+// for half of the contraction's steps before their first wait (64 x 1536 x 512 4.04 -> 4.09 us with helpers).
 inline int helpers_of(int tiles_per_xcd, int cus, int steps, int in_flight) {
   return cus / 8 - tiles_per_xcd < 8 || steps < 2 * in_flight ? 0 : 8;
 }

@@ -12,9 +12,10 @@
 // from HBM once and its lines are L2 hits for the other tiles; CUs without a tile fetch slabs into their L2 (fetch_ahead).
 //
 // Bound by what a CU takes in, (64 + BN) rows of K elements at some 90 GB/s, behind 3.5 us of launch,
-// first slot and reduction.  Against the BLAS routine, us in a graph with weights out of HBM (256 rows):
-// 2048 x 2048 8.2 / 9.6, 4096 x 2048 12.0 / 13.4, 6144 x 2048 16.9 / 24.2, 3072 x 3072 15.0 / 17.7;
-// 64 rows, 1536 x 512 4.1 / 7.0, 2048 x 2048 7.6 / 11.9, 3072 x 3072 11.5 / 16.1.
+// first slot and reduction.  Against the BLAS routine, us in a graph, 24 weight matrices with the last-level cache
+// emptied in between (in brackets: eight matrices that stay in it), 256 rows: 2048 x 2048 10.0 / 14.1 (8.2 / 9.8), 4096
+// x 2048 12.6 / 15.4 (10.5 / 11.3), 6144 x 2048 16.3 / 26.6 (14.3 / 19.3), 3072 x 3072 14.8 / 20.0 (12.3 / 14.2); 64 rows,
+// 1536 x 512 5.4 / 9.5 (4.1 / 6.1), 2048 x 2048 8.6 / 13.9 (7.2 / 8.9), 3072 x 3072 13.0 / 18.4 (9.2 / 11.6).
 #include "attn_mma.h"
 #include "device_state.h"
 #include "we_kernels.h"
