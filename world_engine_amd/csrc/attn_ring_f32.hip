@@ -5,20 +5,36 @@
 // One workgroup = 16 queries of one (batch, head) and NW wavefronts that share out its keys: blocks
 // of 16 keys go round the wavefronts, each keeps its own running (reference, sum, O) and they merge
 // through LDS at the end.  A wavefront's keys are nobody else's, so K and V go from memory straight
-// into the matrix operands' registers, one block ahead, without LDS and without a barrier in the loop:
-//   S^T = K Q^T      v_mfma_f32_16x16x4_f32; the contraction is taken in an order that lets a lane
-//                    load four of its head-dim values at once (lane group g of step (j, i) has value
-//                    16 j + 4 g + i of both operands);
-//   O^T += V^T P^T   the S^T accumulators are the B operand as they are (lane group g, register i =
-//                    key 4 g + i), and output rows are numbered so that a lane's four values of V are
-//                    consecutive: one 16-byte load per key and 64 head-dim values, 256 bytes a row.
+// into registers, one block ahead, without a barrier in the loop.
 //
-// Bound by the matrix cores (64 MFMAs of 32 cycles per block of 16 keys at Dh = 128, against 16 loads
-// and some 40 vector instructions) and, at 16 queries a workgroup, by the loads' way through the CU's
-// address path beside them: 16 heads of 128, 256 queries, 2048 keys take 44.4 us = 97 TFLOP/s (a large
-// fp32 matrix product reaches 153 here), 37 us without the loads; 8 heads, 1024 queries and 4096 keys
-// 149 us = 115 TFLOP/s.  (54 and 185 us while the next block's loads stood behind a branch, below.)
+// Most blocks go through the f16 matrix instructions, sixteen times the fp32 ones' rate, as sums of two
+// halves (x = hi + lo, 22 bits; four products per pair).  S^T = K Q^T: K comes row by row - whole lines; read
+// in the operands' layout every request touches 64 of them - and changes places between the lanes through the
+// wavefront's own 8 KB of LDS, halved.  O^T += V^T P^T: the S^T accumulators are the B operand as they are (lane
+// group g, register i = key 4 g + i), and one instruction's 32 places take 16 keys' hi and lo of V.  What a
+// product of these instructions adds is cut off at the last bit of the largest one in its group of eight, and
+// so is the sum it is carried into where that is smaller: the large products of S start from zero each and
+// O's are added by the vector unit, so that no chain of products loses more than its own size.  Relative
+// error against 64 bits, fp32 products / halves: 16 heads of 128, 2048 keys 3.9e-7 / 3.0e-7, 8 heads, 4096
+// keys 6.3e-7 / 3.4e-7, 4 heads, 128 keys 2.3e-7 / 2.2e-7; heads of 64, 2880 keys 5.2e-7 / 3.2e-7, 1024 keys
+// 2.9e-7 / 2.8e-7, but 512 keys 2.4e-7 / 2.6e-7: their short contexts stay with fp32 products (split_rounds).
+// Halves hold values of a certain size only; each wavefront looks at its own as they come and goes on with fp32
+// products where they do not (a block in front of which it notices costs it one round trip).
+//
+// Blocks through v_mfma_f32_16x16x4_f32: the contraction of S is taken in an order that lets a lane load four of its
+// head-dim values at once (lane group g of step (j, i) has value 16 j + 4 g + i of both operands), and output rows
+// are numbered so that a lane's four values of V are consecutive: one 16-byte load per key and 64 head-dim values.
+//
+// Bound by the vector unit: at 16 queries a workgroup every CU halves all of its unit's keys and values itself, 128 of
+// some 270 vector instructions per block and wavefront (32 f16 MFMAs of 16 cycles beside them, 33 us without any load
+// behind the first).  us, fp32 products / halves: 16 heads of 128, 256 queries, 2048 keys 49.5 / 42.4 (101 TFLOP/s),
+// 8 heads, 1024 queries, 4096 keys 156 / 133, 24 heads of 64 on 8, 720 queries, 2880 keys 140 / 118, 8 heads of
+// 128, 64 queries, 512 keys 17.0 / 13.2, 4 heads, 128 keys 9.0 / 8.0.  Values that halves do not hold: 49 -> 52 for the first
+// shape.
+#include <type_traits>
+
 #include "attn_mma.h"
+#include "device_state.h"
 #include "we_kernels.h"
 #include "../../include/we_attn.h"
 
@@ -27,6 +43,21 @@ namespace we {
 namespace {
 constexpr int F_Q = 16;   // queries per workgroup
 constexpr int F_K = 16;   // keys per block
+constexpr float P_LOW = 10.f, P_HIGH = 15.f;   // exponents of split probabilities
+
+// Key blocks per wavefront from which on the split products are as exact as the fp32 ones (below).
+constexpr int split_rounds(int dh) { return dh == 64 ? 8 : 1; }
+
+template <int DH, int NW, bool SPLIT>
+struct F32Lds {
+  static constexpr int OROW = DH + 4;   // floats per row of a wavefront's O (the odd 16 bytes spread the banks)
+  static constexpr int NOUT = NW / 2;   // wavefronts whose O is there at a time
+  static constexpr int KROW = DH * 2 + 16;                  // bytes per key, halved (the odd 16 spread the banks)
+  static constexpr int kWave = SPLIT ? 2 * F_K * KROW : 0;  // a wavefront's block of keys: [hi, lo][key][value]
+  static constexpr int kOut = NOUT * F_Q * OROW * 4;
+  static constexpr int kKeys = NW * kWave > kOut ? NW * kWave : kOut;
+  static constexpr int kBytes = kKeys + 2 * NW * F_Q * 4 + (WE_MAX_SLOTS + 2) * 4;
+};
 }  // namespace
 
 // maximum / sum over the four 16-lane groups of a wavefront, for each lane position in a group
@@ -45,16 +76,38 @@ __device__ __forceinline__ float groups_sum(float x) {
   return lo + up;
 }
 
-template <int DH, int NW>
+typedef float float2_t __attribute__((ext_vector_type(2)));
+typedef _Float16 f16x4_t __attribute__((ext_vector_type(4)));
+
+// fp32 values as sums of two f16 ones: the value rounded, and what that leaves, rounded.
+struct Halves {
+  f16x8_t hi, lo;
+  // (minus_one: -1 that the compiler does not know, so that the rest stays one v_fma_mix)
+  __device__ __forceinline__ void set(int i, float a, float b, float minus_one) {
+    const f16x2_t h = __builtin_convertvector((float2_t{a, b}), f16x2_t);
+    hi[i] = h[0];
+    hi[i + 1] = h[1];
+    lo[i] = (_Float16)__builtin_fmaf((float)h[0], minus_one, a);
+    lo[i + 1] = (_Float16)__builtin_fmaf((float)h[1], minus_one, b);
+  }
+};
+__device__ __forceinline__ float max_abs3(float m, float a, float b) {
+  asm("v_max3_f32 %0, %0, |%1|, |%2|" : "+v"(m) : "v"(a), "v"(b));
+  return m;
+}
+
+template <int DH, int NW, bool SPLIT>
 __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2)))
 attn_ring_f32_kernel(AttnParams p) {
   constexpr int NJ = DH / 16;    // 16-byte loads of K per lane and block
   constexpr int NH = DH / 64;    // 16-byte loads of V per lane and key
-  constexpr int OROW = DH + 4;   // floats per row of a wavefront's O in LDS (the odd 16 bytes spread the banks)
-  constexpr int NOUT = NW / 2;   // wavefronts whose O is in LDS at a time
-  __shared__ __attribute__((aligned(16))) float osh[NOUT][F_Q][OROW];
-  __shared__ float msh[NW][F_Q], lsh[NW][F_Q];
-  __shared__ int vis[WE_MAX_SLOTS + 2];
+  constexpr int OROW = F32Lds<DH, NW, SPLIT>::OROW, NOUT = F32Lds<DH, NW, SPLIT>::NOUT;
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  typedef F32Lds<DH, NW, SPLIT> Lds;
+  float(*osh)[F_Q][OROW] = reinterpret_cast<float(*)[F_Q][OROW]>(smem);   // (behind the loops: where the wavefronts' keys were)
+  float(*msh)[F_Q] = reinterpret_cast<float(*)[F_Q]>(smem + Lds::kKeys);
+  float(*lsh)[F_Q] = msh + NW;
+  int* vis = reinterpret_cast<int*>(lsh + NW);
 
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int c = lane & 15, g = lane >> 4;
@@ -94,13 +147,39 @@ attn_ring_f32_kernel(AttnParams p) {
     }
   }
 
+  const int qr = q0 + c < p.T ? q0 + c : p.T - 1;
+  const float* q_row = reinterpret_cast<const float*>(p.q) + b * p.qs_b + h * p.qs_h + (int64_t)qr * p.qs_t;
+  float minus_one = -1.f;
+  asm volatile("" : "+s"(minus_one));
   // ---- query c, values 16 j + 4 g + i, pre-multiplied by scale * log2(e) ----
   f32x4_t qf[NJ];
-  {
-    const int qr = q0 + c < p.T ? q0 + c : p.T - 1;
-    const float* src = reinterpret_cast<const float*>(p.q) + b * p.qs_b + h * p.qs_h + (int64_t)qr * p.qs_t + 4 * g;
+  auto load_q = [&]() __attribute__((always_inline)) {
 #pragma unroll
-    for (int j = 0; j < NJ; ++j) qf[j] = *reinterpret_cast<const f32x4_t*>(src + 16 * j) * p.scale_log2;
+    for (int j = 0; j < NJ; ++j) qf[j] = *reinterpret_cast<const f32x4_t*>(q_row + 16 * j + 4 * g) * p.scale_log2;
+  };
+  if (!SPLIT) load_q();
+  // ---- or in halves, values 32 j + 8 g + i, and by a power of two that brings the row's largest value to 2^10 .. 2^11 ----
+  Halves qs[NJ / 2];
+  float q_back = 0.f, k_low = 0.f;   // the power's inverse; smallest key value (below) that halves stand for
+  bool split = false;
+  if (SPLIT) {
+    float top = 0.f;
+#pragma unroll
+    for (int j = 0; j < NJ; ++j)
+      qf[j] = *reinterpret_cast<const f32x4_t*>(q_row + 32 * (j / 2) + 8 * g + 4 * (j & 1)) * p.scale_log2;
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) top = max_abs3(max_abs3(top, qf[j][0], qf[j][1]), qf[j][2], qf[j][3]);
+    top = groups_max(top);
+    split = __ballot(!(top < 0x1p100f)) == 0ull;
+    k_low = __ballot(top > 1.5f) == 0ull ? 0.f : 0.25f;
+    int e = 11 - __builtin_amdgcn_frexp_expf(top);
+    e = e < 100 ? e : 100;
+    q_back = __builtin_amdgcn_ldexpf(1.f, -e);
+#pragma unroll
+    for (int j = 0; j < NJ; ++j)
+#pragma unroll
+      for (int i = 0; i < 4; i += 2)
+        qs[j / 2].set(4 * (j & 1) + i, __builtin_amdgcn_ldexpf(qf[j][i], e), __builtin_amdgcn_ldexpf(qf[j][i + 1], e), minus_one);
   }
   __syncthreads();
   const int nvis = vis[WE_MAX_SLOTS + 1];
@@ -131,22 +210,30 @@ attn_ring_f32_kernel(AttnParams p) {
   };
 
   // (uniform base and 32-bit lane offsets; rows past the frame repeat its last one)
-  auto load = [&](f32x4_t(&kf)[NJ], f32x4_t(&vf)[4][NH], int vi_, int sub_) __attribute__((always_inline)) {
-    const int64_t row0 = (int64_t)__builtin_amdgcn_readfirstlane(vis[vi_]) * p.T + sub_ * F_K;
-    const int last = p.T - 1 - sub_ * F_K;
-    const char* kb = reinterpret_cast<const char*>(kplane + row0 * DH);
-    const char* vb = reinterpret_cast<const char*>(vplane + row0 * DH);
-    const uint32_t ko = (uint32_t)((c < last ? c : last) * DH + 4 * g) * 4u;
+  struct Place {
+    int64_t row0;
+    int last;   // its last key
+  };
+  auto place = [&](int k) __attribute__((always_inline)) {
+    const int at = block_of(k), vi = (int)((unsigned)at / (unsigned)bps), sub = at - vi * bps;
+    return Place{(int64_t)__builtin_amdgcn_readfirstlane(vis[vi]) * p.T + sub * F_K, p.T - 1 - sub * F_K};
+  };
+  auto load_k = [&](f32x4_t(&kf)[NJ], Place at) __attribute__((always_inline)) {
+    const char* kb = reinterpret_cast<const char*>(kplane + at.row0 * DH);
+    const uint32_t ko = (uint32_t)((c < at.last ? c : at.last) * DH + 4 * g) * 4u;
 #pragma unroll
     for (int j = 0; j < NJ; ++j) kf[j] = *reinterpret_cast<const f32x4_t*>(kb + ko + 64 * j);
+  };
+  auto load_v = [&](f32x4_t(&vf)[4][NH], Place at) __attribute__((always_inline)) {
+    const char* vb = reinterpret_cast<const char*>(vplane + at.row0 * DH);
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const uint32_t vo = (uint32_t)((4 * g + i < last ? 4 * g + i : last) * DH + 4 * c) * 4u;
+      const uint32_t vo = (uint32_t)((4 * g + i < at.last ? 4 * g + i : at.last) * DH + 4 * c) * 4u;
 #pragma unroll
       for (int hh = 0; hh < NH; ++hh) vf[i][hh] = *reinterpret_cast<const f32x4_t*>(vb + vo + 256 * hh);
     }
   };
-  auto block = [&](const f32x4_t(&kf)[NJ], f32x4_t(&vf)[4][NH], int keys) __attribute__((always_inline)) {
+  auto block = [&](const f32x4_t(&qf)[NJ], const f32x4_t(&kf)[NJ], f32x4_t(&vf)[4][NH], int keys) __attribute__((always_inline)) {
     f32x4_t s0 = {0.f, 0.f, 0.f, 0.f}, s1 = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int j = 0; j < NJ; j += 2)
@@ -196,31 +283,206 @@ attn_ring_f32_kernel(AttnParams p) {
     __builtin_amdgcn_sched_barrier(0);
   };
   const int mine_n = rounds - (nblk - (rounds - 1) * NW > wave ? 0 : 1);  // rounds this wavefront takes part in
-  if (mine_n > 0) {
+  auto fetch = [&](f32x4_t(&kf)[NJ], f32x4_t(&vf)[4][NH], int k) __attribute__((always_inline)) {
+    const Place at = place(k);
+    load_k(kf, at);
+    load_v(vf, at);
+    return at.last + 1;  // keys of the block (16 or more: a whole one)
+  };
+
+  // ---- blocks whose values two f16 halves hold ----
+  int k = 0;
+  if (SPLIT && split && rounds >= split_rounds(DH) && mine_n > 0) {
+    // The keys come row by row, whole cache lines a request, and change places with the other lanes' through LDS, halved.
+    constexpr int CPR = DH / 4, RPL = 64 / CPR;   // 16-byte chunks per row, rows per request
+    unsigned char* const k_to = smem + wave * Lds::kWave + (lane / CPR) * Lds::KROW + (lane % CPR) * 8;
+    const unsigned char* const k_from = smem + wave * Lds::kWave + c * Lds::KROW + g * 16;
+    f32x4_t kf[NJ], vf[4][NH];
+    auto load_rows = [&](Place at) __attribute__((always_inline)) {
+      const char* kb = reinterpret_cast<const char*>(kplane + at.row0 * DH);
+      if (at.last >= F_K - 1) {
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) kf[j] = *reinterpret_cast<const f32x4_t*>(kb + 1024 * j + (uint32_t)lane * 16u);
+      } else {
+        int l = lane;   // (worked out where it is wanted: no registers to keep it in)
+        asm volatile("" : "+v"(l));
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) {
+          const int r = RPL * j + l / CPR;
+          kf[j] = *reinterpret_cast<const f32x4_t*>(kb + (uint32_t)((r < at.last ? r : at.last) * DH + 4 * (l % CPR)) * 4u);
+        }
+      }
+    };
+    auto load_values = [&](Place at) __attribute__((always_inline)) {
+      const char* vb = reinterpret_cast<const char*>(vplane + at.row0 * DH);
+      if (at.last >= F_K - 1) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+          for (int hh = 0; hh < NH; ++hh)
+            vf[i][hh] = *reinterpret_cast<const f32x4_t*>(vb + (uint32_t)(g * (DH * 16) + c * 16) + DH * 4 * i + 256 * hh);
+      } else {
+        int l = lane;
+        asm volatile("" : "+v"(l));
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int r = 4 * (l >> 4) + i;
+#pragma unroll
+          for (int hh = 0; hh < NH; ++hh)
+            vf[i][hh] = *reinterpret_cast<const f32x4_t*>(vb + (uint32_t)((r < at.last ? r : at.last) * (DH * 4) + (l & 15) * 16) + 256 * hh);
+        }
+      }
+    };
+    Place at = place(0);
+    load_rows(at);
+    load_values(at);
+    // The rest of a rounded value is off by up to 2^-22 of it and by up to 2^-25 (the smallest f16 numbers): next to values
+    // of 1/8 and more that is less than what an fp32 sum over them loses, for the keys so long as the queries are not large.
+    auto fits = [&]() __attribute__((always_inline)) {
+      float kt = 0.f, vt = 0.f;
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) kt = max_abs3(max_abs3(kt, kf[j][0], kf[j][1]), kf[j][2], kf[j][3]);
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int hh = 0; hh < NH; ++hh) vt = max_abs3(max_abs3(vt, vf[i][hh][0], vf[i][hh][1]), vf[i][hh][2], vf[i][hh][3]);
+      return __ballot(kt < k_low || vt < 0.125f || fmaxf(kt, vt) > 0x1p15f) == 0ull;
+    };
+    auto step = [&](auto more) __attribute__((always_inline)) {
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) {
+        Halves x;
+        x.set(0, kf[j][0], kf[j][1], minus_one);
+        x.set(2, kf[j][2], kf[j][3], minus_one);
+        *reinterpret_cast<f16x4_t*>(k_to + RPL * j * Lds::KROW) = f16x4_t{x.hi[0], x.hi[1], x.hi[2], x.hi[3]};
+        *reinterpret_cast<f16x4_t*>(k_to + (F_K + RPL * j) * Lds::KROW) = f16x4_t{x.lo[0], x.lo[1], x.lo[2], x.lo[3]};
+      }
+      asm volatile("" ::: "memory");
+      const int keys = at.last + 1;   // (16 or more: a whole block)
+      // (the large products one by one, the others on top of each other: a sum that is carried from product to product
+      // loses the bits that hang over the products')
+      f32x4_t sh[NJ / 2], sl = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int j = 0; j < NJ / 2; ++j) {
+        Halves x;
+        x.hi = *reinterpret_cast<const f16x8_t*>(k_from + 64 * j);
+        x.lo = *reinterpret_cast<const f16x8_t*>(k_from + F_K * Lds::KROW + 64 * j);
+        sh[j] = F16Mma::mma16(x.hi, qs[j].hi, f32x4_t{0.f, 0.f, 0.f, 0.f});
+        sl = F16Mma::mma16(x.lo, qs[j].lo, sl);
+        sl = F16Mma::mma16(x.lo, qs[j].hi, sl);
+        sl = F16Mma::mma16(x.hi, qs[j].lo, sl);
+      }
+      asm volatile("" ::: "memory");
+      if (decltype(more)::value) {
+        at = place(k + 1);
+        load_rows(at);
+      }
+      float undo = q_back;
+      asm volatile("" : "+v"(undo));
+      __builtin_amdgcn_sched_barrier(0);
+      f32x4_t s;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        s[i] = sh[0][i] + sh[1][i];
+        if (NJ == 8) s[i] += sh[NJ / 2 - 2][i] + sh[NJ / 2 - 1][i];
+        s[i] = (s[i] + sl[i]) * undo;
+      }
+      if (keys < F_K) {  // missing keys: no weight, and nothing for a zero weight to meet but zeros
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          if (4 * g + i >= keys) {
+            s[i] = -INFINITY;
+#pragma unroll
+            for (int hh = 0; hh < NH; ++hh) vf[i][hh] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+          }
+      }
+      // (o and l_run are relative to m_run, P_LOW to P_HIGH below the largest logit: probabilities are up to 2^15)
+      const float top = groups_max(fmaxf(fmaxf(s[0], s[1]), fmaxf(s[2], s[3])));
+      if (__ballot(top > m_run + P_HIGH) != 0ull) {
+        const float mx = fmaxf(m_run, top - P_LOW), alpha = __builtin_amdgcn_exp2f(m_run - mx);  // 0 on the first block
+        l_run *= alpha;
+#pragma unroll
+        for (int hh = 0; hh < NH; ++hh)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) o[hh][e] *= alpha;
+        m_run = mx;
+      }
+      f32x4_t pr;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) pr[i] = __builtin_amdgcn_exp2f(s[i] - m_run);
+      l_run += (pr[0] + pr[1]) + (pr[2] + pr[3]);
+      Halves ps;
+      ps.set(0, pr[0], pr[1], minus_one);
+      ps.set(2, pr[2], pr[3], minus_one);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        ps.hi[4 + i] = ps.hi[i];
+        ps.lo[4 + i] = ps.lo[i];
+      }
+      // (the large products first: what is added to a large sum is rounded, what a large product meets is cut off)
+#pragma unroll
+      for (int hh = 0; hh < NH; ++hh) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          f16x8_t v;   // value 64 hh + 4 c + e of the lane's four keys: rounded, and the rest
+#pragma unroll
+          for (int i = 0; i < 4; i += 2) {
+            Halves x;
+            x.set(0, vf[i][hh][e], vf[i + 1][hh][e], minus_one);
+            v[i] = x.hi[0];
+            v[i + 1] = x.hi[1];
+            v[4 + i] = x.lo[0];
+            v[5 + i] = x.lo[1];
+          }
+          f32x4_t d = F16Mma::mma16(v, ps.hi, F16Mma::mma16(v, ps.lo, f32x4_t{0.f, 0.f, 0.f, 0.f}));
+#pragma unroll
+          for (int i = 0; i < 4; ++i) o[hh][e][i] += d[i];
+        }
+      }
+      if (decltype(more)::value) load_values(at);
+      // (the next block is not looked at, and waited for, in front of these products)
+      __builtin_amdgcn_sched_barrier(0);
+      ++k;
+    };
+    bool good = fits();
+    while (good && k + 1 < mine_n) {
+      step(std::true_type());
+      good = fits();
+    }
+    if (good) step(std::false_type());
+    if (k < mine_n) {  // (the blocks below may have values that 2^15 times as much of would be too much)
+      m_run += P_LOW;
+      l_run *= __builtin_amdgcn_exp2f(-P_LOW);
+#pragma unroll
+      for (int hh = 0; hh < NH; ++hh)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) o[hh][e] *= __builtin_amdgcn_exp2f(-P_LOW);
+    }
+  }
+
+  // ---- the others ----
+  if (k < mine_n) {
+    if (SPLIT) load_q();
     f32x4_t ka[NJ], va[4][NH], kb[NJ], vb[4][NH];
     // The loop always requests the next block - behind a branch the compiler counts the loads in flight as if it had
     // not been taken, and waits for the block just requested - and the last one or two blocks follow it.  (A last block
     // requested a second time, for nothing, costs wavefronts with one or two of them most: attention alone, 4 heads of 128,
     // 64 queries, 128 keys 9.8 -> 8.75 us, 8 heads, 256 keys 12.25 -> 11.4, 8 heads of 64, 256 keys 7.64 -> 7.40, 128 keys
     // 6.43 -> 6.11.)
-    auto fetch = [&](f32x4_t(&kf)[NJ], f32x4_t(&vf)[4][NH], int k) __attribute__((always_inline)) {
-      const int at = block_of(k), vi = (int)((unsigned)at / (unsigned)bps), sub = at - vi * bps;
-      load(kf, vf, vi, sub);
-      return p.T - sub * F_K;  // keys of the block (16 or more: a whole one)
-    };
-    int keys_a = fetch(ka, va, 0), k = 1;
+    int keys_a = fetch(ka, va, k);
+    ++k;
     for (; k + 1 < mine_n; k += 2) {
       const int keys_b = fetch(kb, vb, k);
-      block(ka, va, keys_a);
+      block(qf, ka, va, keys_a);
       keys_a = fetch(ka, va, k + 1);
-      block(kb, vb, keys_b);
+      block(qf, kb, vb, keys_b);
     }
     if (k < mine_n) {
       const int keys_b = fetch(kb, vb, k);
-      block(ka, va, keys_a);
-      block(kb, vb, keys_b);
+      block(qf, ka, va, keys_a);
+      block(qf, kb, vb, keys_b);
     } else {
-      block(ka, va, keys_a);
+      block(qf, ka, va, keys_a);
     }
   }
 
@@ -230,7 +492,7 @@ attn_ring_f32_kernel(AttnParams p) {
     msh[wave][c] = m_run;
     lsh[wave][c] = l_run;
   }
-  __syncthreads();
+  __syncthreads();   // (and everybody is done with the keys)
   float mm = -INFINITY, lt = 0.f;
 #pragma unroll
   for (int w = 0; w < NW; ++w)
@@ -284,9 +546,23 @@ static hipError_t launch_f32(AttnParams p, int cus, hipStream_t stream) {
   if (wgs > 0x7fffffff) return hipErrorInvalidValue;
   // eight wavefronts per workgroup (two per SIMD of a CU) while a CU gets one workgroup; two
   // workgroups of four beyond, which leave a smaller last round
-  if (wgs <= cus) hipLaunchKernelGGL((attn_ring_f32_kernel<DH, 8>), dim3((unsigned)wgs), dim3(512), 0, stream, p);
-  else hipLaunchKernelGGL((attn_ring_f32_kernel<DH, 4>), dim3((unsigned)wgs), dim3(256), 0, stream, p);
-  return hipGetLastError();
+  const int nw = wgs <= cus ? 8 : 4;
+  const int64_t blocks = (int64_t)p.num_buckets * ((p.T + F_K - 1) / F_K);   // of a full ring
+  const bool split = (blocks + nw - 1) / nw >= split_rounds(DH);
+  const void* kernel = nw == 8 ? (split ? reinterpret_cast<const void*>(&attn_ring_f32_kernel<DH, 8, true>)
+                                        : reinterpret_cast<const void*>(&attn_ring_f32_kernel<DH, 8, false>))
+                               : (split ? reinterpret_cast<const void*>(&attn_ring_f32_kernel<DH, 4, true>)
+                                        : reinterpret_cast<const void*>(&attn_ring_f32_kernel<DH, 4, false>));
+  const int lds = nw == 8 ? (split ? F32Lds<DH, 8, true>::kBytes : F32Lds<DH, 8, false>::kBytes)
+                          : (split ? F32Lds<DH, 4, true>::kBytes : F32Lds<DH, 4, false>::kBytes);
+  void* args[] = {&p};
+  return hipLaunchKernel(kernel, dim3((unsigned)wgs), dim3(64 * nw), args, lds, stream);
+}
+
+// The dynamic-LDS limit of the one instance that needs more than the default.
+hipError_t configure_attn_ring_f32() {
+  return hipFuncSetAttribute(reinterpret_cast<const void*>(&attn_ring_f32_kernel<128, 8, true>),
+                             hipFuncAttributeMaxDynamicSharedMemorySize, F32Lds<128, 8, true>::kBytes);
 }
 
 hipError_t launch_attn_ring_f32(const AttnParams& p, int Dh, int cus, hipStream_t stream) {

@@ -34,6 +34,7 @@ hipError_t configure_attn_ring_short_bf16();
 hipError_t configure_attn_ring_short_f16();
 hipError_t configure_attn_ring_shared_bf16();
 hipError_t configure_attn_ring_shared_f16();
+hipError_t configure_attn_ring_f32();
 hipError_t configure_qkv_rope_store();
 hipError_t configure_linear_skinny();
 

@@ -54,7 +54,8 @@ int init_current_device() {
       configure_attn_ring_f16_128() != hipSuccess || configure_attn_ring_f16_64() != hipSuccess ||
       configure_attn_ring_short_bf16() != hipSuccess || configure_attn_ring_short_f16() != hipSuccess ||
       configure_attn_ring_shared_bf16() != hipSuccess || configure_attn_ring_shared_f16() != hipSuccess ||
-      configure_qkv_rope_store() != hipSuccess || configure_linear_skinny() != hipSuccess)
+      configure_attn_ring_f32() != hipSuccess || configure_qkv_rope_store() != hipSuccess ||
+      configure_linear_skinny() != hipSuccess)
     return WE_ERR_LAUNCH;
   void* p = nullptr;
   if (hipGetSymbolAddress(&p, HIP_SYMBOL(scratch)) != hipSuccess || p == nullptr) return WE_ERR_LAUNCH;
