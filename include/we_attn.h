@@ -148,7 +148,8 @@ size_t we_attn_workspace_bytes_for(int32_t B, int32_t H, int32_t Hkv, int32_t T,
  * counterpart in the reference; launches nothing): plan[0] = queries per workgroup, [1] = context
  * parts of the units that are split, [2] = leading (batch, kv head) units left whole, [3] =
  * workgroups of the main launch, [4] = compute units planned for.  compute_units = 0 asks the
- * current device (256 without one).
+ * current device (256 without one).  A call may take fewer parts: of a dilated ring, and of a frame of up to
+ * 256 tokens where its element type's partial rows cost more than they save.
  */
 #define WE_PLAN_FIELDS 5
 int we_attn_plan(int32_t B, int32_t H, int32_t Hkv, int32_t T, int32_t Dh, int64_t L, int32_t n_splits,

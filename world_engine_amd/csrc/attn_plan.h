@@ -3,6 +3,7 @@
 // measurement library's entry points (probe_capi.hip), so that both plan a call identically.
 #pragma once
 #include "../../include/we_attn.h"
+#include "short_parts.h"
 #include "we_kernels.h"
 
 namespace we {
@@ -195,18 +196,27 @@ inline AttnPlan plan_attn(int B, int H, int Hkv, int T, int Dh, int64_t L, int n
 }
 
 // plan_attn for callers that ask again and again: a thread keeps its last plans (each layer and frame of
-// a model asks twice, and a plan is some fifty cost estimates).
-inline AttnPlan plan_cached(int B, int H, int Hkv, int T, int Dh, int64_t L, int n_splits, int variant, int cus) {
-  struct Entry { int64_t key[9]; AttnPlan plan; };
+// a model asks twice, and a plan is some fifty cost estimates).  row_bytes: of a partial row, for a call that takes fewer
+// parts where that is the faster plan (short_parts.h; it needs less workspace than the plan without, which the sizing
+// helpers go by); 0: the plan without.
+inline AttnPlan plan_cached(int B, int H, int Hkv, int T, int Dh, int64_t L, int n_splits, int variant, int cus, int row_bytes = 0) {
+  struct Entry { int64_t key[10]; AttnPlan plan; };
   static thread_local Entry kept[16] = {};
-  const int64_t key[9] = {B, H, Hkv, T, Dh, L, n_splits, variant, cus};
+  const int64_t key[10] = {B, H, Hkv, T, Dh, L, n_splits, variant, cus, row_bytes};
   uint64_t h = 0;
   for (int64_t k : key) h = (h ^ (uint64_t)k) * 0x9e3779b97f4a7c15ull;
   Entry& e = kept[h >> 60];
-  for (int i = 0; i < 9; ++i)
+  for (int i = 0; i < 10; ++i)
     if (e.key[i] != key[i]) {
       e.plan = plan_attn(B, H, Hkv, T, Dh, L, n_splits, variant, cus);
-      for (int j = 0; j < 9; ++j) e.key[j] = key[j];
+      AttnPlan& pl = e.plan;
+      if (row_bytes > 0 && n_splits == 0 && T >= 64 && T <= 256 && pl.variant == 1 && pl.units_whole == 0 && pl.n_splits > 1) {
+        const ShortCall call = {(int64_t)B * Hkv, members_of(B * Hkv, H / Hkv, T, pl.block_m, pl.cus), (L + 63) / 64,
+                                (int64_t)B * H * T, row_bytes, Dh > 64, pl.cus};
+        pl.n_splits = call.parts(pl.n_splits);
+        if (pl.n_splits == 1) pl.ws_rows = 0;
+      }
+      for (int j = 0; j < 10; ++j) e.key[j] = key[j];
       break;
     }
   return e.plan;
@@ -244,21 +254,28 @@ inline int prepare_attn(const void* q, const int64_t* q_strides, const void* kv,
     return WE_ERR_ALIGNMENT;
 
   pl = plan_cached(B, H, Hkv, T, Dh, L, n_splits, variant_of(q_tile), cus);
+  int64_t keys = L;   // that the plan is for
   if (dilation > 1 && n_splits == 0) {
     // a dilated ring holds frames in one of `dilation` slots only; the sizing helpers do not know of it,
     // so the plan for the keys there are is taken where it needs no more workspace
     const AttnPlan short_ring = plan_cached(B, H, Hkv, T, Dh, L / dilation, 0, variant_of(q_tile), cus);
-    if (workspace_bytes_of(short_ring, Dh) <= workspace_bytes_of(pl, Dh)) pl = short_ring;
+    if (workspace_bytes_of(short_ring, Dh) <= workspace_bytes_of(pl, Dh)) {
+      pl = short_ring;
+      keys = L / dilation;
+    }
   }
+  const size_t given = workspace_bytes < workspace_limit ? workspace_bytes : workspace_limit;
   if (n_splits == 0 && workspace_bytes_of(pl, Dh) > workspace_limit)
     pl = plan_basic(B, H, Hkv, T, L, 0, variant_of(q_tile), cus);
+  else if (n_splits == 0 && workspace && aligned16(workspace) && workspace_bytes_of(pl, Dh) <= given)
+    // (a workspace that is too short for the plan of the sizing helpers stays too short)
+    pl = plan_cached(B, H, Hkv, T, Dh, keys, 0, variant_of(q_tile), cus, Dh * (dtype == WE_DTYPE_F16 ? 4 : 2) + 4 * (int)sizeof(float));
   // An f16 output has the 11 significant bits of a 16-bit partial row itself, which would round it once
   // more: its partial rows are fp32.  (24 heads of 64 on 8, 720 tokens, 16 slots, dilation 2, relative
   // error against 64 bits: one pass 2.93e-4; three parts with fp16 rows 3.50e-4, with fp32 rows 2.93e-4.
   // A bf16 output has 8 bits: 2.347e-3 in one pass, 2.352e-3 with fp16 rows.)  A workspace that holds
   // 16-bit rows only gets the basic plan, which splits less, where it holds that one's.
   bool wide = false;
-  const size_t given = workspace_bytes < workspace_limit ? workspace_bytes : workspace_limit;
   if (dtype == WE_DTYPE_F16 && workspace_bytes_of(pl, Dh) > 0 && workspace_bytes_of(pl, Dh) <= given) {
     wide = workspace_bytes_of(pl, Dh, true) <= given;
     if (!wide) {
