@@ -25,12 +25,13 @@
 // head-dim values at once (lane group g of step (j, i) has value 16 j + 4 g + i of both operands), and output rows
 // are numbered so that a lane's four values of V are consecutive: one 16-byte load per key and 64 head-dim values.
 //
-// Bound by the vector unit: at 16 queries a workgroup every CU halves all of its unit's keys and values itself, 128 of
-// some 270 vector instructions per block and wavefront (32 f16 MFMAs of 16 cycles beside them, 33 us without any load
-// behind the first).  us, fp32 products / halves: 16 heads of 128, 256 queries, 2048 keys 49.5 / 42.4 (101 TFLOP/s),
-// 8 heads, 1024 queries, 4096 keys 156 / 133, 24 heads of 64 on 8, 720 queries, 2880 keys 140 / 118, 8 heads of
-// 128, 64 queries, 512 keys 17.0 / 13.2, 4 heads, 128 keys 9.0 / 8.0.  Values that halves do not hold: 49 -> 52 for the first
-// shape.
+// Bound by the vector unit and the trips through LDS: at 16 queries a workgroup every CU halves all of its unit's keys and
+// values itself, 128 of some 270 vector instructions per block and wavefront (57 % of the time they issue, 32 f16 MFMAs of 16
+// cycles beside them; a request for V a whole block ahead, into registers of its own, changes nothing).  us, fp32 products /
+// halves: 16 heads of 128, 256 queries, 2048 keys 49.5 / 40.4 (106 TFLOP/s), 8 heads, 1024 queries, 4096 keys 156 / 126, 24 heads
+// of 64 on 8, 720 queries, 2880 keys 140 / 108, 8 heads of 128, 64 queries, 512 keys 17.0 / 12.5, 4 heads, 128 keys 9.0 / 7.9
+// (the loads' addresses in vector registers, o copied at a way out in mid-block and a check of every key's size cost
+// another 44.3, 133, 120, 13.2, 8.0).  Values that halves do not hold: 49 -> 52 for the first shape.
 #include <type_traits>
 
 #include "attn_mma.h"
@@ -96,7 +97,9 @@ __device__ __forceinline__ float max_abs3(float m, float a, float b) {
   return m;
 }
 
-template <int DH, int NW, bool SPLIT>
+// WHOLE: T % 16 == 0, every block has 16 keys (a separate instance: what the others work out per request is a tenth of a
+// block's vector instructions).
+template <int DH, int NW, bool SPLIT, bool WHOLE>
 __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2)))
 attn_ring_f32_kernel(AttnParams p) {
   constexpr int NJ = DH / 16;    // 16-byte loads of K per lane and block
@@ -298,38 +301,33 @@ attn_ring_f32_kernel(AttnParams p) {
     unsigned char* const k_to = smem + wave * Lds::kWave + (lane / CPR) * Lds::KROW + (lane % CPR) * 8;
     const unsigned char* const k_from = smem + wave * Lds::kWave + c * Lds::KROW + g * 16;
     f32x4_t kf[NJ], vf[4][NH];
+    // (offsets of the lanes that are known here only: a uniform base and these, no vector addresses kept)
     auto load_rows = [&](Place at) __attribute__((always_inline)) {
-      const char* kb = reinterpret_cast<const char*>(kplane + at.row0 * DH);
-      if (at.last >= F_K - 1) {
+      typedef const __attribute__((address_space(1))) char* bytes_t;
+      bytes_t kb = (bytes_t)(kplane + at.row0 * DH), kb4 = kb + 4096;
+      uint32_t l = (uint32_t)lane;
+      asm volatile("" : "+v"(l), "+s"(kb4));
 #pragma unroll
-        for (int j = 0; j < NJ; ++j) kf[j] = *reinterpret_cast<const f32x4_t*>(kb + 1024 * j + (uint32_t)lane * 16u);
-      } else {
-        int l = lane;   // (worked out where it is wanted: no registers to keep it in)
-        asm volatile("" : "+v"(l));
-#pragma unroll
-        for (int j = 0; j < NJ; ++j) {
-          const int r = RPL * j + l / CPR;
-          kf[j] = *reinterpret_cast<const f32x4_t*>(kb + (uint32_t)((r < at.last ? r : at.last) * DH + 4 * (l % CPR)) * 4u);
+      for (int j = 0; j < NJ; ++j) {
+        if (WHOLE) {
+          kf[j] = *reinterpret_cast<const __attribute__((address_space(1))) f32x4_t*>((j < 4 ? kb + 1024 * j : kb4 + 1024 * (j - 4)) + l * 16u);
+        } else {
+          const int r = RPL * j + (int)(l / CPR);
+          kf[j] = *reinterpret_cast<const __attribute__((address_space(1))) f32x4_t*>(kb + (uint32_t)((r < at.last ? r : at.last) * DH + 4 * (int)(l % CPR)) * 4u);
         }
       }
     };
     auto load_values = [&](Place at) __attribute__((always_inline)) {
       const char* vb = reinterpret_cast<const char*>(vplane + at.row0 * DH);
-      if (at.last >= F_K - 1) {
+      uint32_t l = (uint32_t)lane;
+      asm volatile("" : "+v"(l));
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
+      for (int i = 0; i < 4; ++i) {
+        const int r = 4 * (int)(l >> 4) + i;
 #pragma unroll
-          for (int hh = 0; hh < NH; ++hh)
-            vf[i][hh] = *reinterpret_cast<const f32x4_t*>(vb + (uint32_t)(g * (DH * 16) + c * 16) + DH * 4 * i + 256 * hh);
-      } else {
-        int l = lane;
-        asm volatile("" : "+v"(l));
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const int r = 4 * (l >> 4) + i;
-#pragma unroll
-          for (int hh = 0; hh < NH; ++hh)
-            vf[i][hh] = *reinterpret_cast<const f32x4_t*>(vb + (uint32_t)((r < at.last ? r : at.last) * (DH * 4) + (l & 15) * 16) + 256 * hh);
+        for (int hh = 0; hh < NH; ++hh) {
+          if (WHOLE) vf[i][hh] = *reinterpret_cast<const f32x4_t*>(vb + DH * 4 * i + 256 * hh + ((l >> 4) * (DH * 16) + (l & 15) * 16));
+          else vf[i][hh] = *reinterpret_cast<const f32x4_t*>(vb + (uint32_t)((r < at.last ? r : at.last) * (DH * 4) + (int)(l & 15) * 16) + 256 * hh);
         }
       }
     };
@@ -338,17 +336,25 @@ attn_ring_f32_kernel(AttnParams p) {
     load_values(at);
     // The rest of a rounded value is off by up to 2^-22 of it and by up to 2^-25 (the smallest f16 numbers): next to values
     // of 1/8 and more that is less than what an fp32 sum over them loses, for the keys so long as the queries are not large.
-    auto fits = [&]() __attribute__((always_inline)) {
-      float kt = 0.f, vt = 0.f;
+    // (Values too large for f16 are infinite and their rest the other infinity: what they meet is no number, at the end.)
+    auto keys_fit = [&]() __attribute__((always_inline)) {
+      if (k_low == 0.f) return true;
+      float top = 0.f;
 #pragma unroll
-      for (int j = 0; j < NJ; ++j) kt = max_abs3(max_abs3(kt, kf[j][0], kf[j][1]), kf[j][2], kf[j][3]);
+      for (int j = 0; j < NJ; ++j) top = max_abs3(max_abs3(top, kf[j][0], kf[j][1]), kf[j][2], kf[j][3]);
+      return __ballot(top < k_low) == 0ull;
+    };
+    auto values_fit = [&]() __attribute__((always_inline)) {
+      float top = 0.f;
 #pragma unroll
       for (int i = 0; i < 4; ++i)
 #pragma unroll
-        for (int hh = 0; hh < NH; ++hh) vt = max_abs3(max_abs3(vt, vf[i][hh][0], vf[i][hh][1]), vf[i][hh][2], vf[i][hh][3]);
-      return __ballot(kt < k_low || vt < 0.125f || fmaxf(kt, vt) > 0x1p15f) == 0ull;
+        for (int hh = 0; hh < NH; ++hh) top = max_abs3(max_abs3(top, vf[i][hh][0], vf[i][hh][1]), vf[i][hh][2], vf[i][hh][3]);
+      return __ballot(top < 0.125f) == 0ull;
     };
-    auto step = [&](auto more) __attribute__((always_inline)) {
+    f32x4_t s;
+    int keys = 0;
+    auto logits = [&](auto more) __attribute__((always_inline)) {
 #pragma unroll
       for (int j = 0; j < NJ; ++j) {
         Halves x;
@@ -358,7 +364,7 @@ attn_ring_f32_kernel(AttnParams p) {
         *reinterpret_cast<f16x4_t*>(k_to + (F_K + RPL * j) * Lds::KROW) = f16x4_t{x.lo[0], x.lo[1], x.lo[2], x.lo[3]};
       }
       asm volatile("" ::: "memory");
-      const int keys = at.last + 1;   // (16 or more: a whole block)
+      keys = at.last + 1;   // (16 or more: a whole block)
       // (the large products one by one, the others on top of each other: a sum that is carried from product to product
       // loses the bits that hang over the products')
       f32x4_t sh[NJ / 2], sl = {0.f, 0.f, 0.f, 0.f};
@@ -380,14 +386,15 @@ attn_ring_f32_kernel(AttnParams p) {
       float undo = q_back;
       asm volatile("" : "+v"(undo));
       __builtin_amdgcn_sched_barrier(0);
-      f32x4_t s;
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         s[i] = sh[0][i] + sh[1][i];
         if (NJ == 8) s[i] += sh[NJ / 2 - 2][i] + sh[NJ / 2 - 1][i];
         s[i] = (s[i] + sl[i]) * undo;
       }
-      if (keys < F_K) {  // missing keys: no weight, and nothing for a zero weight to meet but zeros
+    };
+    auto outputs = [&](auto more) __attribute__((always_inline)) {
+      if (!WHOLE && keys < F_K) {  // missing keys: no weight, and nothing for a zero weight to meet but zeros
 #pragma unroll
         for (int i = 0; i < 4; ++i)
           if (4 * g + i >= keys) {
@@ -439,18 +446,36 @@ attn_ring_f32_kernel(AttnParams p) {
           for (int i = 0; i < 4; ++i) o[hh][e][i] += d[i];
         }
       }
-      if (decltype(more)::value) load_values(at);
       // (the next block is not looked at, and waited for, in front of these products)
       __builtin_amdgcn_sched_barrier(0);
       ++k;
     };
-    bool good = fits();
-    while (good && k + 1 < mine_n) {
-      step(std::true_type());
-      good = fits();
-    }
-    if (good) step(std::false_type());
-    if (k < mine_n) {  // (the blocks below may have values that 2^15 times as much of would be too much)
+    // (one way out, at the end: with two the compiler copies o from one set of registers to another in every block)
+    auto block_of_halves = [&](auto more) __attribute__((always_inline)) {
+      const bool fit = keys_fit();
+      logits(more);
+      const bool good = fit && values_fit();
+      if (good) outputs(more);
+      if (decltype(more)::value) load_values(at);   // (either way: the keys' requests are counted from here)
+      return good;
+    };
+    bool good = true;
+    while (good && k + 1 < mine_n) good = block_of_halves(std::true_type());
+    if (good) block_of_halves(std::false_type());
+    float all = l_run;
+#pragma unroll
+    for (int hh = 0; hh < NH; ++hh)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) all += (o[hh][e][0] + o[hh][e][1]) + (o[hh][e][2] + o[hh][e][3]);
+    if (__ballot(!(__builtin_fabsf(all) < INFINITY)) != 0ull) {  // all of it once more
+      k = 0;
+      m_run = -INFINITY;
+      l_run = 0.f;
+#pragma unroll
+      for (int hh = 0; hh < NH; ++hh)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) o[hh][e] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    } else if (k < mine_n) {  // (the blocks below may have values that 2^15 times as much of would be too much)
       m_run += P_LOW;
       l_run *= __builtin_amdgcn_exp2f(-P_LOW);
 #pragma unroll
@@ -549,20 +574,29 @@ static hipError_t launch_f32(AttnParams p, int cus, hipStream_t stream) {
   const int nw = wgs <= cus ? 8 : 4;
   const int64_t blocks = (int64_t)p.num_buckets * ((p.T + F_K - 1) / F_K);   // of a full ring
   const bool split = (blocks + nw - 1) / nw >= split_rounds(DH);
-  const void* kernel = nw == 8 ? (split ? reinterpret_cast<const void*>(&attn_ring_f32_kernel<DH, 8, true>)
-                                        : reinterpret_cast<const void*>(&attn_ring_f32_kernel<DH, 8, false>))
-                               : (split ? reinterpret_cast<const void*>(&attn_ring_f32_kernel<DH, 4, true>)
-                                        : reinterpret_cast<const void*>(&attn_ring_f32_kernel<DH, 4, false>));
+  const bool whole = p.T % F_K == 0;
+  auto pick = [&](auto waves) {
+    constexpr int NW = decltype(waves)::value;
+    return !split  ? reinterpret_cast<const void*>(&attn_ring_f32_kernel<DH, NW, false, false>)
+           : whole ? reinterpret_cast<const void*>(&attn_ring_f32_kernel<DH, NW, true, true>)
+                   : reinterpret_cast<const void*>(&attn_ring_f32_kernel<DH, NW, true, false>);
+  };
+  const void* kernel = nw == 8 ? pick(std::integral_constant<int, 8>()) : pick(std::integral_constant<int, 4>());
   const int lds = nw == 8 ? (split ? F32Lds<DH, 8, true>::kBytes : F32Lds<DH, 8, false>::kBytes)
                           : (split ? F32Lds<DH, 4, true>::kBytes : F32Lds<DH, 4, false>::kBytes);
   void* args[] = {&p};
   return hipLaunchKernel(kernel, dim3((unsigned)wgs), dim3(64 * nw), args, lds, stream);
 }
 
-// The dynamic-LDS limit of the one instance that needs more than the default.
-hipError_t configure_attn_ring_f32() {
-  return hipFuncSetAttribute(reinterpret_cast<const void*>(&attn_ring_f32_kernel<128, 8, true>),
+// The dynamic-LDS limit of the instances that need more than the default.
+template <bool WHOLE>
+static hipError_t configure_f32() {
+  return hipFuncSetAttribute(reinterpret_cast<const void*>(&attn_ring_f32_kernel<128, 8, true, WHOLE>),
                              hipFuncAttributeMaxDynamicSharedMemorySize, F32Lds<128, 8, true>::kBytes);
+}
+hipError_t configure_attn_ring_f32() {
+  const hipError_t e = configure_f32<true>();
+  return e == hipSuccess ? configure_f32<false>() : e;
 }
 
 hipError_t launch_attn_ring_f32(const AttnParams& p, int Dh, int cus, hipStream_t stream) {
