@@ -55,6 +55,45 @@ def test_f32_values_that_halves_do_not_hold(gpu_device, Dh, what, frame, factor)
     assert err <= REL * max(1.0, factor if what == "q" else 1.0)   # (larger logits: REL's comment)
 
 
+@pytest.mark.parametrize("B,H,Hkv,T,Dh,n", [
+    (3, 24, 24, 49, 128, 2), (3, 24, 12, 64, 128, 3), (4, 30, 30, 33, 128, 1), (5, 52, 52, 16, 128, 4), (2, 30, 6, 81, 64, 11),
+    (3, 30, 30, 48, 64, 22), (1, 17, 17, 250, 128, 3), (2, 10, 10, 224, 64, 5), (5, 60, 20, 31, 64, 33)])
+def test_f32_halves_of_two_groups_of_queries(gpu_device, B, H, Hkv, T, Dh, n):
+    """More than one workgroup of 16 queries a CU: tiles of 32, whole, short and with a second group that is all padding."""
+    out, ref = _ring(gpu_device, B, H, Hkv, T, Dh, n)
+    err = _rel(out, ref)
+    print(f"f32 halves, two groups B={B} H={H}/{Hkv} T={T} Dh={Dh} n={n}: rel {err:.2e}", flush=True)
+    assert err <= REL
+
+
+@pytest.mark.parametrize("Dh,n", [(128, 4), (64, 22)])
+@pytest.mark.parametrize("what,frame,factor", [("v", 2, 1e-4), ("v", None, 1e-20), ("v", 3, 1e30), ("k", 2, 1e6), ("q", None, 1e-30)])
+def test_f32_two_groups_without_halves(gpu_device, Dh, n, what, frame, factor):
+    """Both groups go on with fp32 products from the same block on, or start over."""
+    def change(t, q, k, v):
+        if frame is None or t == frame:
+            {"q": q, "k": k, "v": v}[what].mul_(factor)
+
+    out, ref = _ring(gpu_device, 3, 30, 30, 49, Dh, n, change)
+    err = _rel(out, ref)
+    print(f"f32 halves, two groups Dh={Dh} {what} x {factor:g} in {frame}: rel {err:.2e}", flush=True)
+    assert err <= REL * max(1.0, factor * 1e-2 if what == "k" else 1.0)   # (larger logits: REL's comment)
+
+
+@pytest.mark.parametrize("Dh,n", [(128, 4), (64, 22)])
+def test_f32_two_groups_and_missing_numbers(gpu_device, Dh, n):
+    """A query that is not a number, in either group: its row and nothing else."""
+    def change(t, q, k, v):
+        if t == n:
+            q[0, 0, 11, 2] = float("nan")
+            q[1, 3, 20, 7] = float("nan")
+
+    out, ref = _ring(gpu_device, 3, 30, 30, 49, Dh, n, change)
+    assert torch.equal(out.isnan(), ref.isnan())
+    good = ref.isfinite()
+    assert _rel(out[good], ref[good]) <= REL
+
+
 def test_f32_large_keys_meet_small_queries(gpu_device):
     """Logits of the usual size from keys above the halves' range."""
     out, ref = _ring(gpu_device, 1, 2, 2, 144, 128, 8, lambda t, q, k, v: (q.mul_(1e-5), k.mul_(1e5)))

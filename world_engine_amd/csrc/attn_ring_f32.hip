@@ -2,7 +2,7 @@
 // half-precision kernel (attn_ring.hip), fp32 throughout (fp32 scores, softmax and P V,
 // src/model/attn.py:116 in eager mode) on the fp32 matrix instructions.
 //
-// One workgroup = 16 queries of one (batch, head) and NW wavefronts that share out its keys: blocks
+// One workgroup = one or two groups of 16 queries of one (batch, head) and NW wavefronts that share out its keys: blocks
 // of 16 keys go round the wavefronts, each keeps its own running (reference, sum, O) and they merge
 // through LDS at the end.  A wavefront's keys are nobody else's, so K and V go from memory straight
 // into registers, one block ahead, without a barrier in the loop.
@@ -27,11 +27,13 @@
 //
 // Bound by the vector unit and the trips through LDS: at 16 queries a workgroup every CU halves all of its unit's keys and
 // values itself, 128 of some 270 vector instructions per block and wavefront (57 % of the time they issue, 32 f16 MFMAs of 16
-// cycles beside them; a request for V a whole block ahead, into registers of its own, changes nothing).  us, fp32 products /
-// halves: 16 heads of 128, 256 queries, 2048 keys 49.5 / 40.4 (106 TFLOP/s), 8 heads, 1024 queries, 4096 keys 156 / 126, 24 heads
-// of 64 on 8, 720 queries, 2880 keys 140 / 108, 8 heads of 128, 64 queries, 512 keys 17.0 / 12.5, 4 heads, 128 keys 9.0 / 7.9
-// (the loads' addresses in vector registers, o copied at a way out in mid-block and a check of every key's size cost
-// another 44.3, 133, 120, 13.2, 8.0).  Values that halves do not hold: 49 -> 52 for the first shape.
+// cycles beside them; a request for V a whole block ahead, into registers of its own, changes nothing).  Where that is more
+// than a workgroup a CU, two groups share what is halved (some 340 instructions for both; the queries' halves in LDS then).
+// us, fp32 products / halves / of two groups: 16 heads of 128, 256 queries, 2048 keys 49.5 / 40.4 (106 TFLOP/s), 8 heads, 1024
+// queries, 4096 keys 156 / 126 / 103 (167 TFLOP/s, where a large fp32 matrix product reaches 153), 24 heads of 64 on 8, 720
+// queries, 2880 keys 140 / 107 / 99.7, 16 heads, 272 queries, 2176 keys - / 63.5 / 52.8, 8 heads of 128, 64 queries, 512 keys 17.0 /
+// 12.5, 4 heads, 128 keys 9.0 / 7.9 (the loads' addresses in vector registers, o copied at a way out in mid-block and
+// a check of every key's size cost another 44.3, 133, 120, -, 13.2, 8.0).  Values that halves do not hold: 49 -> 52 for the first shape.
 #include <type_traits>
 
 #include "attn_mma.h"
@@ -42,22 +44,26 @@
 namespace we {
 
 namespace {
-constexpr int F_Q = 16;   // queries per workgroup
+constexpr int F_Q = 16;   // queries of a group
 constexpr int F_K = 16;   // keys per block
 constexpr float P_LOW = 10.f, P_HIGH = 15.f;   // exponents of split probabilities
 
 // Key blocks per wavefront from which on the split products are as exact as the fp32 ones (below).
 constexpr int split_rounds(int dh) { return dh == 64 ? 8 : 1; }
 
-template <int DH, int NW, bool SPLIT>
+// NQ: groups of queries per workgroup
+template <int DH, int NW, int NQ, bool SPLIT>
 struct F32Lds {
   static constexpr int OROW = DH + 4;   // floats per row of a wavefront's O (the odd 16 bytes spread the banks)
   static constexpr int NOUT = NW / 2;   // wavefronts whose O is there at a time
   static constexpr int KROW = DH * 2 + 16;                  // bytes per key, halved (the odd 16 spread the banks)
   static constexpr int kWave = SPLIT ? 2 * F_K * KROW : 0;  // a wavefront's block of keys: [hi, lo][key][value]
-  static constexpr int kOut = NOUT * F_Q * OROW * 4;
-  static constexpr int kKeys = NW * kWave > kOut ? NW * kWave : kOut;
-  static constexpr int kBytes = kKeys + 2 * NW * F_Q * 4 + (WE_MAX_SLOTS + 2) * 4;
+  static constexpr int kOut = NOUT * NQ * F_Q * OROW * 4;
+  static constexpr int kMl = NW * kWave > kOut ? NW * kWave : kOut;                        // references, sums
+  static constexpr int kQ = kMl + 2 * NW * NQ * F_Q * 4;                                   // queries: [group][hi, lo][step][lane] 16 bytes,
+  static constexpr int kBack = kQ + (SPLIT && NQ > 1 ? NQ * F_Q * DH * 4 : 0);             // what undoes their scaling
+  static constexpr int kVis = kBack + (SPLIT && NQ > 1 ? NQ * F_Q * 4 : 0);
+  static constexpr int kBytes = kVis + (WE_MAX_SLOTS + 2) * 4;
 };
 }  // namespace
 
@@ -99,25 +105,28 @@ __device__ __forceinline__ float max_abs3(float m, float a, float b) {
 
 // WHOLE: T % 16 == 0, every block has 16 keys (a separate instance: what the others work out per request is a tenth of a
 // block's vector instructions).
-template <int DH, int NW, bool SPLIT, bool WHOLE>
+template <int DH, int NW, int NQ, bool SPLIT, bool WHOLE>
 __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2)))
 attn_ring_f32_kernel(AttnParams p) {
   constexpr int NJ = DH / 16;    // 16-byte loads of K per lane and block
   constexpr int NH = DH / 64;    // 16-byte loads of V per lane and key
-  constexpr int OROW = F32Lds<DH, NW, SPLIT>::OROW, NOUT = F32Lds<DH, NW, SPLIT>::NOUT;
+  constexpr int OROW = F32Lds<DH, NW, NQ, SPLIT>::OROW, NOUT = F32Lds<DH, NW, NQ, SPLIT>::NOUT;
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-  typedef F32Lds<DH, NW, SPLIT> Lds;
-  float(*osh)[F_Q][OROW] = reinterpret_cast<float(*)[F_Q][OROW]>(smem);   // (behind the loops: where the wavefronts' keys were)
-  float(*msh)[F_Q] = reinterpret_cast<float(*)[F_Q]>(smem + Lds::kKeys);
-  float(*lsh)[F_Q] = msh + NW;
-  int* vis = reinterpret_cast<int*>(lsh + NW);
+  typedef F32Lds<DH, NW, NQ, SPLIT> Lds;
+  constexpr int BQ = NQ * F_Q;   // queries per workgroup
+  float(*osh)[BQ][OROW] = reinterpret_cast<float(*)[BQ][OROW]>(smem);   // (behind the loops: where the wavefronts' keys were)
+  float(*msh)[BQ] = reinterpret_cast<float(*)[BQ]>(smem + Lds::kMl);
+  float(*lsh)[BQ] = msh + NW;
+  f16x8_t* qsh = reinterpret_cast<f16x8_t*>(smem + Lds::kQ);
+  float* back = reinterpret_cast<float*>(smem + Lds::kBack);
+  int* vis = reinterpret_cast<int*>(smem + Lds::kVis);
 
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int c = lane & 15, g = lane >> 4;
 
   // ---- which queries ----
   // (spread over the XCDs by unit where every XCD gets the same number: a unit's workgroups share an L2)
-  const int units = p.B * p.Hkv, q_tiles = (p.T + F_Q - 1) / F_Q;
+  const int units = p.B * p.Hkv, q_tiles = (p.T + BQ - 1) / BQ;
   int unit, member;
   if ((units & 7) == 0) {
     const unsigned j = blockIdx.x >> 3;
@@ -130,7 +139,7 @@ attn_ring_f32_kernel(AttnParams p) {
   }
   const int b = unit / p.Hkv, hkv = unit - b * p.Hkv;
   const int hq_in = member / q_tiles, h = hkv * p.group + hq_in;
-  const int q0 = (member - hq_in * q_tiles) * F_Q;
+  const int q0 = (member - hq_in * q_tiles) * BQ;
 
   // ---- list of visible slots; the tail is pseudo-slot n_slots ----
   if (wave == 0) {
@@ -150,49 +159,81 @@ attn_ring_f32_kernel(AttnParams p) {
     }
   }
 
-  const int qr = q0 + c < p.T ? q0 + c : p.T - 1;
-  const float* q_row = reinterpret_cast<const float*>(p.q) + b * p.qs_b + h * p.qs_h + (int64_t)qr * p.qs_t;
+  auto query = [&](int qi) __attribute__((always_inline)) {
+    const int qr = q0 + qi * F_Q + c < p.T ? q0 + qi * F_Q + c : p.T - 1;
+    return reinterpret_cast<const float*>(p.q) + b * p.qs_b + h * p.qs_h + (int64_t)qr * p.qs_t;
+  };
   float minus_one = -1.f;
   asm volatile("" : "+s"(minus_one));
-  // ---- query c, values 16 j + 4 g + i, pre-multiplied by scale * log2(e) ----
+  // ---- query c of a group, values 16 j + 4 g + i, pre-multiplied by scale * log2(e) ----
   f32x4_t qf[NJ];
-  auto load_q = [&]() __attribute__((always_inline)) {
+  auto load_q = [&](int qi) __attribute__((always_inline)) {
+    const float* row = query(qi);
 #pragma unroll
-    for (int j = 0; j < NJ; ++j) qf[j] = *reinterpret_cast<const f32x4_t*>(q_row + 16 * j + 4 * g) * p.scale_log2;
+    for (int j = 0; j < NJ; ++j) qf[j] = *reinterpret_cast<const f32x4_t*>(row + 16 * j + 4 * g) * p.scale_log2;
   };
-  if (!SPLIT) load_q();
-  // ---- or in halves, values 32 j + 8 g + i, and by a power of two that brings the row's largest value to 2^10 .. 2^11 ----
+  if (!SPLIT) load_q(0);
+  // ---- or in halves, values 32 j + 8 g + i, and by a power of two that brings the row's largest value to 2^10 .. 2^11; in
+  // registers, or where there are several groups in LDS ----
   Halves qs[NJ / 2];
-  float q_back = 0.f, k_low = 0.f;   // the power's inverse; smallest key value (below) that halves stand for
+  float q_back[NQ];    // the power's inverse
+  float k_low = 0.f;   // smallest key value (below) that halves stand for
   bool split = false;
-  if (SPLIT) {
+  auto halve_q = [&](int qi, float& undo) __attribute__((always_inline)) {
+    const float* row = query(qi);
     float top = 0.f;
 #pragma unroll
-    for (int j = 0; j < NJ; ++j)
-      qf[j] = *reinterpret_cast<const f32x4_t*>(q_row + 32 * (j / 2) + 8 * g + 4 * (j & 1)) * p.scale_log2;
+    for (int j = 0; j < NJ; ++j) qf[j] = *reinterpret_cast<const f32x4_t*>(row + 32 * (j / 2) + 8 * g + 4 * (j & 1)) * p.scale_log2;
 #pragma unroll
     for (int j = 0; j < NJ; ++j) top = max_abs3(max_abs3(top, qf[j][0], qf[j][1]), qf[j][2], qf[j][3]);
     top = groups_max(top);
-    split = __ballot(!(top < 0x1p100f)) == 0ull;
-    k_low = __ballot(top > 1.5f) == 0ull ? 0.f : 0.25f;
     int e = 11 - __builtin_amdgcn_frexp_expf(top);
     e = e < 100 ? e : 100;
-    q_back = __builtin_amdgcn_ldexpf(1.f, -e);
+    undo = top < 0x1p100f ? __builtin_amdgcn_ldexpf(1.f, -e) : INFINITY;
 #pragma unroll
     for (int j = 0; j < NJ; ++j)
 #pragma unroll
       for (int i = 0; i < 4; i += 2)
         qs[j / 2].set(4 * (j & 1) + i, __builtin_amdgcn_ldexpf(qf[j][i], e), __builtin_amdgcn_ldexpf(qf[j][i + 1], e), minus_one);
+  };
+  if (SPLIT && NQ == 1) halve_q(0, q_back[0]);
+  if (SPLIT && NQ > 1 && wave >= 1 && wave <= NQ) {
+    float undo;
+    halve_q(wave - 1, undo);
+    if (g == 0) back[(wave - 1) * F_Q + c] = undo;
+#pragma unroll
+    for (int j = 0; j < NJ / 2; ++j) {
+      qsh[((wave - 1) * NJ + j) * 64 + lane] = qs[j].hi;
+      qsh[((wave - 1) * NJ + NJ / 2 + j) * 64 + lane] = qs[j].lo;
+    }
   }
   __syncthreads();
   const int nvis = vis[WE_MAX_SLOTS + 1];
+  if (SPLIT) {
+    float most = 0.f;
+#pragma unroll
+    for (int qi = 0; qi < NQ; ++qi) {
+      if (NQ > 1) q_back[qi] = back[qi * F_Q + c];
+      most = fmaxf(most, q_back[qi]);
+    }
+    split = __ballot(!(most < INFINITY)) == 0ull;
+    k_low = __ballot(most > 0x1p-10f) == 0ull ? 0.f : 0.25f;   // (a row's largest value below 2, 1 on average)
+  }
 
-  f32x4_t o[NH][4];  // o[hh][e] register i: query c, value 64 hh + 16 g + 4 i + e
+  f32x4_t o[NQ][NH][4];  // o[qi][hh][e] register i: query c of group qi, value 64 hh + 16 g + 4 i + e
+  float m_run[NQ], l_run[NQ];  // (l_run: this lane group's keys only)
+  auto nothing_yet = [&]() __attribute__((always_inline)) {
 #pragma unroll
-  for (int hh = 0; hh < NH; ++hh)
+    for (int qi = 0; qi < NQ; ++qi) {
+      m_run[qi] = -INFINITY;
+      l_run[qi] = 0.f;
 #pragma unroll
-    for (int e = 0; e < 4; ++e) o[hh][e] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-  float m_run = -INFINITY, l_run = 0.f;  // (l_run: this lane group's keys only)
+      for (int hh = 0; hh < NH; ++hh)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) o[qi][hh][e] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    }
+  };
+  nothing_yet();
 
   const int64_t cap = p.L + p.T;
   const float* kplane = reinterpret_cast<const float*>(p.kv) + (((int64_t)b * p.Hkv + hkv) * cap) * DH;
@@ -236,7 +277,8 @@ attn_ring_f32_kernel(AttnParams p) {
       for (int hh = 0; hh < NH; ++hh) vf[i][hh] = *reinterpret_cast<const f32x4_t*>(vb + vo + 256 * hh);
     }
   };
-  auto block = [&](const f32x4_t(&qf)[NJ], const f32x4_t(&kf)[NJ], f32x4_t(&vf)[4][NH], int keys) __attribute__((always_inline)) {
+  auto block = [&](auto group, const f32x4_t(&kf)[NJ], f32x4_t(&vf)[4][NH], int keys) __attribute__((always_inline)) {
+    constexpr int qi = decltype(group)::value;
     f32x4_t s0 = {0.f, 0.f, 0.f, 0.f}, s1 = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int j = 0; j < NJ; j += 2)
@@ -262,26 +304,26 @@ attn_ring_f32_kernel(AttnParams p) {
           for (int hh = 0; hh < NH; ++hh) vf[i][hh] = f32x4_t{0.f, 0.f, 0.f, 0.f};
         }
     }
-    const float mx = fmaxf(m_run, groups_max(fmaxf(fmaxf(s[0], s[1]), fmaxf(s[2], s[3]))));
-    if (__ballot(mx != m_run) != 0ull) {
-      const float alpha = __builtin_amdgcn_exp2f(m_run - mx);  // 0 on the first block
-      l_run *= alpha;
+    const float mx = fmaxf(m_run[qi], groups_max(fmaxf(fmaxf(s[0], s[1]), fmaxf(s[2], s[3]))));
+    if (__ballot(mx != m_run[qi]) != 0ull) {
+      const float alpha = __builtin_amdgcn_exp2f(m_run[qi] - mx);  // 0 on the first block
+      l_run[qi] *= alpha;
 #pragma unroll
       for (int hh = 0; hh < NH; ++hh)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) o[hh][e] *= alpha;
-      m_run = mx;
+        for (int e = 0; e < 4; ++e) o[qi][hh][e] *= alpha;
+      m_run[qi] = mx;
     }
     f32x4_t pr;
 #pragma unroll
     for (int i = 0; i < 4; ++i) pr[i] = __builtin_amdgcn_exp2f(s[i] - mx);
-    l_run += (pr[0] + pr[1]) + (pr[2] + pr[3]);
+    l_run[qi] += (pr[0] + pr[1]) + (pr[2] + pr[3]);
 #pragma unroll
     for (int i = 0; i < 4; ++i)
 #pragma unroll
       for (int hh = 0; hh < NH; ++hh)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) o[hh][e] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[i][hh][e], pr[i], o[hh][e], 0, 0, 0);
+        for (int e = 0; e < 4; ++e) o[qi][hh][e] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[i][hh][e], pr[i], o[qi][hh][e], 0, 0, 0);
     // (two blocks in a row are not scheduled as one: 44.4 against 46.8 us for the first shape above)
     __builtin_amdgcn_sched_barrier(0);
   };
@@ -352,7 +394,7 @@ attn_ring_f32_kernel(AttnParams p) {
         for (int hh = 0; hh < NH; ++hh) top = max_abs3(max_abs3(top, vf[i][hh][0], vf[i][hh][1]), vf[i][hh][2], vf[i][hh][3]);
       return __ballot(top < 0.125f) == 0ull;
     };
-    f32x4_t s;
+    f32x4_t s[NQ];
     int keys = 0;
     auto logits = [&](auto more) __attribute__((always_inline)) {
 #pragma unroll
@@ -367,66 +409,82 @@ attn_ring_f32_kernel(AttnParams p) {
       keys = at.last + 1;   // (16 or more: a whole block)
       // (the large products one by one, the others on top of each other: a sum that is carried from product to product
       // loses the bits that hang over the products')
-      f32x4_t sh[NJ / 2], sl = {0.f, 0.f, 0.f, 0.f};
+      f32x4_t sh[NQ][NJ / 2], sl[NQ];
+      int lane_q = lane;   // (the queries are read anew for every block: no registers to keep them in)
+      if (NQ > 1) asm volatile("" : "+v"(lane_q));
+#pragma unroll
+      for (int qi = 0; qi < NQ; ++qi) sl[qi] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int j = 0; j < NJ / 2; ++j) {
         Halves x;
         x.hi = *reinterpret_cast<const f16x8_t*>(k_from + 64 * j);
         x.lo = *reinterpret_cast<const f16x8_t*>(k_from + F_K * Lds::KROW + 64 * j);
-        sh[j] = F16Mma::mma16(x.hi, qs[j].hi, f32x4_t{0.f, 0.f, 0.f, 0.f});
-        sl = F16Mma::mma16(x.lo, qs[j].lo, sl);
-        sl = F16Mma::mma16(x.lo, qs[j].hi, sl);
-        sl = F16Mma::mma16(x.hi, qs[j].lo, sl);
+#pragma unroll
+        for (int qi = 0; qi < NQ; ++qi) {
+          const f16x8_t q_hi = NQ > 1 ? qsh[(qi * NJ + j) * 64 + lane_q] : qs[j].hi;
+          const f16x8_t q_lo = NQ > 1 ? qsh[(qi * NJ + NJ / 2 + j) * 64 + lane_q] : qs[j].lo;
+          sh[qi][j] = F16Mma::mma16(x.hi, q_hi, f32x4_t{0.f, 0.f, 0.f, 0.f});
+          sl[qi] = F16Mma::mma16(x.lo, q_lo, sl[qi]);
+          sl[qi] = F16Mma::mma16(x.lo, q_hi, sl[qi]);
+          sl[qi] = F16Mma::mma16(x.hi, q_lo, sl[qi]);
+        }
+        if (NQ > 1) __builtin_amdgcn_sched_barrier(0);
       }
       asm volatile("" ::: "memory");
       if (decltype(more)::value) {
         at = place(k + 1);
         load_rows(at);
       }
-      float undo = q_back;
-      asm volatile("" : "+v"(undo));
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        s[i] = sh[0][i] + sh[1][i];
-        if (NJ == 8) s[i] += sh[NJ / 2 - 2][i] + sh[NJ / 2 - 1][i];
-        s[i] = (s[i] + sl[i]) * undo;
+      for (int qi = 0; qi < NQ; ++qi) {
+        float undo = q_back[qi];
+        asm volatile("" : "+v"(undo));
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          s[qi][i] = sh[qi][0][i] + sh[qi][1][i];
+          if (NJ == 8) s[qi][i] += sh[qi][NJ / 2 - 2][i] + sh[qi][NJ / 2 - 1][i];
+          s[qi][i] = (s[qi][i] + sl[qi][i]) * undo;
+        }
       }
     };
-    auto outputs = [&](auto more) __attribute__((always_inline)) {
+    auto outputs = [&]() __attribute__((always_inline)) {
       if (!WHOLE && keys < F_K) {  // missing keys: no weight, and nothing for a zero weight to meet but zeros
 #pragma unroll
         for (int i = 0; i < 4; ++i)
           if (4 * g + i >= keys) {
-            s[i] = -INFINITY;
+#pragma unroll
+            for (int qi = 0; qi < NQ; ++qi) s[qi][i] = -INFINITY;
 #pragma unroll
             for (int hh = 0; hh < NH; ++hh) vf[i][hh] = f32x4_t{0.f, 0.f, 0.f, 0.f};
           }
       }
-      // (o and l_run are relative to m_run, P_LOW to P_HIGH below the largest logit: probabilities are up to 2^15)
-      const float top = groups_max(fmaxf(fmaxf(s[0], s[1]), fmaxf(s[2], s[3])));
-      if (__ballot(top > m_run + P_HIGH) != 0ull) {
-        const float mx = fmaxf(m_run, top - P_LOW), alpha = __builtin_amdgcn_exp2f(m_run - mx);  // 0 on the first block
-        l_run *= alpha;
+      Halves ps[NQ];
 #pragma unroll
-        for (int hh = 0; hh < NH; ++hh)
+      for (int qi = 0; qi < NQ; ++qi) {
+        // (o and l_run are relative to m_run, P_LOW to P_HIGH below the largest logit: probabilities are up to 2^15)
+        const float top = groups_max(fmaxf(fmaxf(s[qi][0], s[qi][1]), fmaxf(s[qi][2], s[qi][3])));
+        if (__ballot(top > m_run[qi] + P_HIGH) != 0ull) {
+          const float mx = fmaxf(m_run[qi], top - P_LOW), alpha = __builtin_amdgcn_exp2f(m_run[qi] - mx);  // 0 on the first block
+          l_run[qi] *= alpha;
 #pragma unroll
-          for (int e = 0; e < 4; ++e) o[hh][e] *= alpha;
-        m_run = mx;
+          for (int hh = 0; hh < NH; ++hh)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) o[qi][hh][e] *= alpha;
+          m_run[qi] = mx;
+        }
+        f32x4_t pr;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) pr[i] = __builtin_amdgcn_exp2f(s[qi][i] - m_run[qi]);
+        l_run[qi] += (pr[0] + pr[1]) + (pr[2] + pr[3]);
+        ps[qi].set(0, pr[0], pr[1], minus_one);
+        ps[qi].set(2, pr[2], pr[3], minus_one);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          ps[qi].hi[4 + i] = ps[qi].hi[i];
+          ps[qi].lo[4 + i] = ps[qi].lo[i];
+        }
       }
-      f32x4_t pr;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) pr[i] = __builtin_amdgcn_exp2f(s[i] - m_run);
-      l_run += (pr[0] + pr[1]) + (pr[2] + pr[3]);
-      Halves ps;
-      ps.set(0, pr[0], pr[1], minus_one);
-      ps.set(2, pr[2], pr[3], minus_one);
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        ps.hi[4 + i] = ps.hi[i];
-        ps.lo[4 + i] = ps.lo[i];
-      }
-      // (the large products first: what is added to a large sum is rounded, what a large product meets is cut off)
 #pragma unroll
       for (int hh = 0; hh < NH; ++hh) {
 #pragma unroll
@@ -441,9 +499,12 @@ attn_ring_f32_kernel(AttnParams p) {
             v[4 + i] = x.lo[0];
             v[5 + i] = x.lo[1];
           }
-          f32x4_t d = F16Mma::mma16(v, ps.hi, F16Mma::mma16(v, ps.lo, f32x4_t{0.f, 0.f, 0.f, 0.f}));
 #pragma unroll
-          for (int i = 0; i < 4; ++i) o[hh][e][i] += d[i];
+          for (int qi = 0; qi < NQ; ++qi) {
+            const f32x4_t d = F16Mma::mma16(v, ps[qi].hi, F16Mma::mma16(v, ps[qi].lo, f32x4_t{0.f, 0.f, 0.f, 0.f}));
+#pragma unroll
+            for (int i = 0; i < 4; ++i) o[qi][hh][e][i] += d[i];
+          }
         }
       }
       // (the next block is not looked at, and waited for, in front of these products)
@@ -455,102 +516,126 @@ attn_ring_f32_kernel(AttnParams p) {
       const bool fit = keys_fit();
       logits(more);
       const bool good = fit && values_fit();
-      if (good) outputs(more);
+      if (good) outputs();
       if (decltype(more)::value) load_values(at);   // (either way: the keys' requests are counted from here)
       return good;
     };
     bool good = true;
     while (good && k + 1 < mine_n) good = block_of_halves(std::true_type());
     if (good) block_of_halves(std::false_type());
-    float all = l_run;
+    float all = 0.f;
 #pragma unroll
-    for (int hh = 0; hh < NH; ++hh)
+    for (int qi = 0; qi < NQ; ++qi) {
+      all += l_run[qi];
 #pragma unroll
-      for (int e = 0; e < 4; ++e) all += (o[hh][e][0] + o[hh][e][1]) + (o[hh][e][2] + o[hh][e][3]);
+      for (int hh = 0; hh < NH; ++hh)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) all += (o[qi][hh][e][0] + o[qi][hh][e][1]) + (o[qi][hh][e][2] + o[qi][hh][e][3]);
+    }
     if (__ballot(!(__builtin_fabsf(all) < INFINITY)) != 0ull) {  // all of it once more
       k = 0;
-      m_run = -INFINITY;
-      l_run = 0.f;
-#pragma unroll
-      for (int hh = 0; hh < NH; ++hh)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) o[hh][e] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+      nothing_yet();
     } else if (k < mine_n) {  // (the blocks below may have values that 2^15 times as much of would be too much)
-      m_run += P_LOW;
-      l_run *= __builtin_amdgcn_exp2f(-P_LOW);
+      const float less = __builtin_amdgcn_exp2f(-P_LOW);
 #pragma unroll
-      for (int hh = 0; hh < NH; ++hh)
+      for (int qi = 0; qi < NQ; ++qi) {
+        m_run[qi] += P_LOW;
+        l_run[qi] *= less;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) o[hh][e] *= __builtin_amdgcn_exp2f(-P_LOW);
+        for (int hh = 0; hh < NH; ++hh)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) o[qi][hh][e] *= less;
+      }
     }
   }
 
   // ---- the others ----
-  if (k < mine_n) {
-    if (SPLIT) load_q();
+  auto others = [&](auto group, int from) __attribute__((always_inline)) {
+    if (SPLIT) load_q(decltype(group)::value);
     f32x4_t ka[NJ], va[4][NH], kb[NJ], vb[4][NH];
     // The loop always requests the next block - behind a branch the compiler counts the loads in flight as if it had
     // not been taken, and waits for the block just requested - and the last one or two blocks follow it.  (A last block
     // requested a second time, for nothing, costs wavefronts with one or two of them most: attention alone, 4 heads of 128,
     // 64 queries, 128 keys 9.8 -> 8.75 us, 8 heads, 256 keys 12.25 -> 11.4, 8 heads of 64, 256 keys 7.64 -> 7.40, 128 keys
     // 6.43 -> 6.11.)
+    int k = from;
     int keys_a = fetch(ka, va, k);
     ++k;
     for (; k + 1 < mine_n; k += 2) {
       const int keys_b = fetch(kb, vb, k);
-      block(qf, ka, va, keys_a);
+      block(group, ka, va, keys_a);
       keys_a = fetch(ka, va, k + 1);
-      block(qf, kb, vb, keys_b);
+      block(group, kb, vb, keys_b);
     }
     if (k < mine_n) {
       const int keys_b = fetch(kb, vb, k);
-      block(qf, ka, va, keys_a);
-      block(qf, kb, vb, keys_b);
+      block(group, ka, va, keys_a);
+      block(group, kb, vb, keys_b);
     } else {
-      block(qf, ka, va, keys_a);
+      block(group, ka, va, keys_a);
     }
+  };
+  if (k < mine_n) {
+    others(std::integral_constant<int, 0>(), k);
+    if constexpr (NQ > 1) others(std::integral_constant<int, 1>(), k);
   }
 
   // ---- the wavefronts merge ----
-  l_run = groups_sum(l_run);
-  if (g == 0) {
-    msh[wave][c] = m_run;
-    lsh[wave][c] = l_run;
+#pragma unroll
+  for (int qi = 0; qi < NQ; ++qi) {
+    l_run[qi] = groups_sum(l_run[qi]);
+    if (g == 0) {
+      msh[wave][qi * F_Q + c] = m_run[qi];
+      lsh[wave][qi * F_Q + c] = l_run[qi];
+    }
   }
   __syncthreads();   // (and everybody is done with the keys)
-  float mm = -INFINITY, lt = 0.f;
+  float lt[NQ];
 #pragma unroll
-  for (int w = 0; w < NW; ++w)
-    if (lsh[w][c] != 0.f) mm = fmaxf(mm, msh[w][c]);  // (a wavefront without keys has no say)
+  for (int qi = 0; qi < NQ; ++qi) {
+    const int at = qi * F_Q + c;
+    float mm = -INFINITY;
+    lt[qi] = 0.f;
 #pragma unroll
-  for (int w = 0; w < NW; ++w)
-    if (lsh[w][c] != 0.f) lt += lsh[w][c] * __builtin_amdgcn_exp2f(msh[w][c] - mm);
-  const float mine = l_run != 0.f ? __builtin_amdgcn_exp2f(m_run - mm) : 0.f;
+    for (int w = 0; w < NW; ++w)
+      if (lsh[w][at] != 0.f) mm = fmaxf(mm, msh[w][at]);  // (a wavefront without keys has no say)
 #pragma unroll
-  for (int hh = 0; hh < NH; ++hh)
-#pragma unroll
-    for (int e = 0; e < 4; ++e) o[hh][e] *= mine;
-  auto row_of = [&](int w, int hh, int i) { return reinterpret_cast<f32x4_t*>(&osh[w][c][64 * hh + 16 * g + 4 * i]); };
-  if (wave >= NOUT) {
+    for (int w = 0; w < NW; ++w)
+      if (lsh[w][at] != 0.f) lt[qi] += lsh[w][at] * __builtin_amdgcn_exp2f(msh[w][at] - mm);
+    const float mine = l_run[qi] != 0.f ? __builtin_amdgcn_exp2f(m_run[qi] - mm) : 0.f;
 #pragma unroll
     for (int hh = 0; hh < NH; ++hh)
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
-        *row_of(wave - NOUT, hh, i) = f32x4_t{o[hh][0][i], o[hh][1][i], o[hh][2][i], o[hh][3][i]};
+      for (int e = 0; e < 4; ++e) o[qi][hh][e] *= mine;
+  }
+  auto row_of = [&](int w, int qi, int hh, int i) { return reinterpret_cast<f32x4_t*>(&osh[w][qi * F_Q + c][64 * hh + 16 * g + 4 * i]); };
+  if (wave >= NOUT) {
+#pragma unroll
+    for (int qi = 0; qi < NQ; ++qi)
+#pragma unroll
+      for (int hh = 0; hh < NH; ++hh)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          *row_of(wave - NOUT, qi, hh, i) = f32x4_t{o[qi][hh][0][i], o[qi][hh][1][i], o[qi][hh][2][i], o[qi][hh][3][i]};
   }
   __syncthreads();
   if (wave < NOUT) {
 #pragma unroll
-    for (int hh = 0; hh < NH; ++hh)
+    for (int qi = 0; qi < NQ; ++qi)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        f32x4_t* r = row_of(wave, hh, i);
-        *r = f32x4_t{o[hh][0][i], o[hh][1][i], o[hh][2][i], o[hh][3][i]} + *r;
-      }
+      for (int hh = 0; hh < NH; ++hh)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          f32x4_t* r = row_of(wave, qi, hh, i);
+          *r = f32x4_t{o[qi][hh][0][i], o[qi][hh][1][i], o[qi][hh][2][i], o[qi][hh][3][i]} + *r;
+        }
   }
-  if (wave == 0 && g == 0) lsh[0][c] = lt;  // (every wavefront has read the sums before the barrier above)
+  if (wave == 0 && g == 0) {  // (every wavefront has read the sums before the barrier above)
+#pragma unroll
+    for (int qi = 0; qi < NQ; ++qi) lsh[0][qi * F_Q + c] = lt[qi];
+  }
   __syncthreads();
-  for (int item = tid; item < F_Q * DH / 4; item += 64 * NW) {
+  for (int item = tid; item < BQ * DH / 4; item += 64 * NW) {
     const int qi = item / (DH / 4), d = (item % (DH / 4)) * 4;
     const int qrow = q0 + qi;
     if (qrow >= p.T) continue;
@@ -566,37 +651,48 @@ attn_ring_f32_kernel(AttnParams p) {
 
 template <int DH>
 static hipError_t launch_f32(AttnParams p, int cus, hipStream_t stream) {
-  p.members = p.group * ((p.T + F_Q - 1) / F_Q);
-  const int64_t wgs = (int64_t)p.B * p.Hkv * p.members;
+  const auto workgroups = [&](int queries) { return (int64_t)p.B * p.H * ((p.T + queries - 1) / queries); };
+  const int64_t blocks = (int64_t)p.num_buckets * ((p.T + F_K - 1) / F_K);   // of a full ring
+  // Two groups of queries share what is halved where one a workgroup would be more than one a CU.
+  const int nq = workgroups(F_Q) > cus && (blocks + 7) / 8 >= split_rounds(DH) ? 2 : 1;
+  const int64_t wgs = workgroups(nq * F_Q);
   if (wgs > 0x7fffffff) return hipErrorInvalidValue;
+  p.members = p.group * ((p.T + nq * F_Q - 1) / (nq * F_Q));
   // eight wavefronts per workgroup (two per SIMD of a CU) while a CU gets one workgroup; two
   // workgroups of four beyond, which leave a smaller last round
   const int nw = wgs <= cus ? 8 : 4;
-  const int64_t blocks = (int64_t)p.num_buckets * ((p.T + F_K - 1) / F_K);   // of a full ring
-  const bool split = (blocks + nw - 1) / nw >= split_rounds(DH);
-  const bool whole = p.T % F_K == 0;
-  auto pick = [&](auto waves) {
-    constexpr int NW = decltype(waves)::value;
-    return !split  ? reinterpret_cast<const void*>(&attn_ring_f32_kernel<DH, NW, false, false>)
-           : whole ? reinterpret_cast<const void*>(&attn_ring_f32_kernel<DH, NW, true, true>)
-                   : reinterpret_cast<const void*>(&attn_ring_f32_kernel<DH, NW, true, false>);
+  const bool split = (blocks + nw - 1) / nw >= split_rounds(DH), whole = p.T % F_K == 0;
+  const void* kernel = nullptr;
+  int lds = 0;
+  auto pick = [&](auto waves, auto groups, auto halves) {
+    constexpr int NW = decltype(waves)::value, NQ = decltype(groups)::value;
+    constexpr bool SPLIT = decltype(halves)::value;
+    kernel = SPLIT && whole ? reinterpret_cast<const void*>(&attn_ring_f32_kernel<DH, NW, NQ, SPLIT, SPLIT>)
+                            : reinterpret_cast<const void*>(&attn_ring_f32_kernel<DH, NW, NQ, SPLIT, false>);
+    lds = F32Lds<DH, NW, NQ, SPLIT>::kBytes;
   };
-  const void* kernel = nw == 8 ? pick(std::integral_constant<int, 8>()) : pick(std::integral_constant<int, 4>());
-  const int lds = nw == 8 ? (split ? F32Lds<DH, 8, true>::kBytes : F32Lds<DH, 8, false>::kBytes)
-                          : (split ? F32Lds<DH, 4, true>::kBytes : F32Lds<DH, 4, false>::kBytes);
+  const std::integral_constant<int, 8> w8; const std::integral_constant<int, 4> w4;
+  const std::integral_constant<int, 1> one; const std::integral_constant<int, 2> two;
+  if (nq == 2) nw == 8 ? pick(w8, two, std::true_type()) : pick(w4, two, std::true_type());
+  else if (split) nw == 8 ? pick(w8, one, std::true_type()) : pick(w4, one, std::true_type());
+  else nw == 8 ? pick(w8, one, std::false_type()) : pick(w4, one, std::false_type());
   void* args[] = {&p};
   return hipLaunchKernel(kernel, dim3((unsigned)wgs), dim3(64 * nw), args, lds, stream);
 }
 
-// The dynamic-LDS limit of the instances that need more than the default.
-template <bool WHOLE>
+// The dynamic-LDS limit of the instances that may need more than the default.
+template <int DH, int NQ, bool WHOLE>
 static hipError_t configure_f32() {
-  return hipFuncSetAttribute(reinterpret_cast<const void*>(&attn_ring_f32_kernel<128, 8, true, WHOLE>),
-                             hipFuncAttributeMaxDynamicSharedMemorySize, F32Lds<128, 8, true>::kBytes);
+  return hipFuncSetAttribute(reinterpret_cast<const void*>(&attn_ring_f32_kernel<DH, 8, NQ, true, WHOLE>),
+                             hipFuncAttributeMaxDynamicSharedMemorySize, F32Lds<DH, 8, NQ, true>::kBytes);
 }
 hipError_t configure_attn_ring_f32() {
-  const hipError_t e = configure_f32<true>();
-  return e == hipSuccess ? configure_f32<false>() : e;
+  hipError_t e = configure_f32<128, 1, true>();
+  if (e == hipSuccess) e = configure_f32<128, 1, false>();
+  if (e == hipSuccess) e = configure_f32<128, 2, true>();
+  if (e == hipSuccess) e = configure_f32<128, 2, false>();
+  if (e == hipSuccess) e = configure_f32<64, 2, true>();
+  return e == hipSuccess ? configure_f32<64, 2, false>() : e;
 }
 
 hipError_t launch_attn_ring_f32(const AttnParams& p, int Dh, int cus, hipStream_t stream) {
