@@ -144,6 +144,13 @@ size_t we_attn_workspace_bytes_for(int32_t B, int32_t H, int32_t Hkv, int32_t T,
                                    int32_t n_splits, int32_t q_tile, int32_t dtype);
 
 /*
+ * Bytes of workspace with which an fp32 call that leaves n_splits at 0 cuts its context into parts, 0 where it does
+ * not.  With fewer, or none, it takes the whole context in one pass; so does every call of
+ * we_attn_ring_fwd_static.
+ */
+size_t we_attn_f32_workspace_bytes(int32_t B, int32_t H, int32_t Hkv, int32_t T, int32_t Dh, int64_t L, int32_t dilation);
+
+/*
  * What the library would do with an attention call of these sizes (inspection helper without a
  * counterpart in the reference; launches nothing): plan[0] = queries per workgroup, [1] = context
  * parts of the units that are split, [2] = leading (batch, kv head) units left whole, [3] =

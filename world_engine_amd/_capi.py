@@ -122,6 +122,7 @@ SIGNATURES = {
 }
 
 SIGNATURES["we_attn_workspace_bytes_for"] = (c_size_t, [*SIGNATURES["we_attn_workspace_bytes"][1], c_int32])
+SIGNATURES["we_attn_f32_workspace_bytes"] = (c_size_t, [*SIGNATURES["we_attn_auto_splits"][1], c_int32])
 SIGNATURES["we_pos_check_guard_bytes"] = (c_size_t, [c_int32, c_int32, c_int32])
 SIGNATURES["we_linear_covers"] = (c_int32, [c_int32, c_int32, c_int32, c_int32])
 SIGNATURES["we_linear"] = (c_int32, [c_void_p, c_int64, c_void_p, c_int64, c_void_p, c_int64, c_int32, c_int32, c_int32,

@@ -3,6 +3,7 @@
 // measurement library's entry points (probe_capi.hip), so that both plan a call identically.
 #pragma once
 #include "../../include/we_attn.h"
+#include "f32_parts.h"
 #include "short_parts.h"
 #include "we_kernels.h"
 
@@ -244,9 +245,17 @@ inline int prepare_attn(const void* q, const int64_t* q_strides, const void* kv,
   if ((uint64_t)(L + T) * (uint64_t)Dh * 2u >= (1ull << 32)) return WE_ERR_UNSUPPORTED;  // 32-bit tile offsets
   if (!(scale > 0.f) || n_splits < 0 || n_splits > 64) return WE_ERR_BAD_SHAPE;
   if (variant_of(q_tile) < 0) return WE_ERR_UNSUPPORTED;
+  int f32_parts = 1;
   if (dtype == WE_DTYPE_F32) {
-    // fp32 caches take the one-pass kernel: no context splitting, no tile choice
+    // fp32 caches take a kernel of their own: no given number of parts, no tile choice
     if (n_splits > 1 || H > 65535 || B > 65535) return WE_ERR_UNSUPPORTED;
+    // (into parts where the caller leaves that to the library and has given memory for them; not in the library's own,
+    // which calls that overlap would share)
+    if (n_splits == 0 && workspace && aligned16(workspace) && workspace_limit == SIZE_MAX) {
+      F32Call call = {(int64_t)B * H, T, L / T / dilation, Dh, cus};
+      call.plan((int64_t)(workspace_bytes > (size_t)INT64_MAX ? (size_t)INT64_MAX : workspace_bytes));
+      f32_parts = call.parts;
+    }
     n_splits = 1;
   }
   if (!aligned16(q) || !aligned16(kv) || !aligned16(out) || !strides_ok(q_strides, dtype) ||
@@ -310,6 +319,11 @@ inline int prepare_attn(const void* q, const int64_t* q_strides, const void* kv,
   p.q_heads = shared ? 1 : p.group;
   p.unit_splits = pl.units_whole + (B * Hkv - pl.units_whole) * pl.n_splits;
   p.scale_log2 = scale * 1.4426950408889634f;
+  if (f32_parts > 1) {
+    p.n_splits = f32_parts;
+    p.ws_o = workspace;
+    p.ws_ml = reinterpret_cast<float*>(static_cast<char*>(workspace) + (size_t)f32_parts * (size_t)B * H * T * Dh * 4);
+  }
   p.gate = nullptr; p.gs_b = p.gs_h = p.gs_t = 0;
   p.gate_x = nullptr; p.gate_w = nullptr; p.gx_b = p.gx_t = 0;
   p.clock_out = nullptr;

@@ -38,6 +38,7 @@
 
 #include "attn_mma.h"
 #include "device_state.h"
+#include "f32_parts.h"
 #include "we_kernels.h"
 #include "../../include/we_attn.h"
 
@@ -47,9 +48,6 @@ namespace {
 constexpr int F_Q = 16;   // queries of a group
 constexpr int F_K = 16;   // keys per block
 constexpr float P_LOW = 10.f, P_HIGH = 15.f;   // exponents of split probabilities
-
-// Key blocks per wavefront from which on the split products are as exact as the fp32 ones (below).
-constexpr int split_rounds(int dh) { return dh == 64 ? 8 : 1; }
 
 // NQ: groups of queries per workgroup
 template <int DH, int NW, int NQ, bool SPLIT>
@@ -66,6 +64,11 @@ struct F32Lds {
   static constexpr int kBytes = kVis + (WE_MAX_SLOTS + 2) * 4;
 };
 }  // namespace
+
+struct F32Params {
+  AttnParams a;
+  int halves_from;   // blocks of visible keys from which on they go in halves
+};
 
 // maximum / sum over the four 16-lane groups of a wavefront, for each lane position in a group
 __device__ __forceinline__ float groups_max(float x) {
@@ -107,7 +110,8 @@ __device__ __forceinline__ float max_abs3(float m, float a, float b) {
 // block's vector instructions).
 template <int DH, int NW, int NQ, bool SPLIT, bool WHOLE>
 __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2)))
-attn_ring_f32_kernel(AttnParams p) {
+attn_ring_f32_kernel(F32Params fp) {
+  const AttnParams& p = fp.a;
   constexpr int NJ = DH / 16;    // 16-byte loads of K per lane and block
   constexpr int NH = DH / 64;    // 16-byte loads of V per lane and key
   constexpr int OROW = F32Lds<DH, NW, NQ, SPLIT>::OROW, NOUT = F32Lds<DH, NW, NQ, SPLIT>::NOUT;
@@ -124,22 +128,27 @@ attn_ring_f32_kernel(AttnParams p) {
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int c = lane & 15, g = lane >> 4;
 
-  // ---- which queries ----
-  // (spread over the XCDs by unit where every XCD gets the same number: a unit's workgroups share an L2)
-  const int units = p.B * p.Hkv, q_tiles = (p.T + BQ - 1) / BQ;
-  int unit, member;
-  if ((units & 7) == 0) {
+  // ---- which queries, which part of the keys ----
+  // (spread over the XCDs by unit part where every XCD gets the same number: its workgroups share an L2)
+  const int q_tiles = (p.T + BQ - 1) / BQ;
+  unsigned up, member;
+  if (((p.B * p.Hkv * p.n_splits) & 7) == 0) {
     const unsigned j = blockIdx.x >> 3;
     const unsigned u8 = j / (unsigned)p.members;
-    unit = (int)(u8 * 8 + (blockIdx.x & 7));
-    member = (int)(j - u8 * (unsigned)p.members);
+    up = u8 * 8 + (blockIdx.x & 7);
+    member = j - u8 * (unsigned)p.members;
   } else {
-    unit = (int)(blockIdx.x / (unsigned)p.members);
-    member = (int)(blockIdx.x - (unsigned)unit * (unsigned)p.members);
+    up = blockIdx.x / (unsigned)p.members;
+    member = blockIdx.x - up * (unsigned)p.members;
+  }
+  int unit = (int)up, part = 0;
+  if (p.n_splits > 1) {
+    unit = (int)(up / (unsigned)p.n_splits);
+    part = (int)(up - (unsigned)unit * (unsigned)p.n_splits);
   }
   const int b = unit / p.Hkv, hkv = unit - b * p.Hkv;
-  const int hq_in = member / q_tiles, h = hkv * p.group + hq_in;
-  const int q0 = (member - hq_in * q_tiles) * BQ;
+  const int hq_in = (int)member / q_tiles, h = hkv * p.group + hq_in;
+  const int q0 = ((int)member - hq_in * q_tiles) * BQ;
 
   // ---- list of visible slots; the tail is pseudo-slot n_slots ----
   if (wave == 0) {
@@ -244,13 +253,19 @@ attn_ring_f32_kernel(AttnParams p) {
   // different lines at any one time, and each line comes from memory at one member's request (184
   // against 192 us for the 1024-query shape above when it took 184; groups of 8 or 16: the same, then and now).
   const int bps = (p.T + F_K - 1) / F_K;  // blocks per slot; the last one may be short
-  const int nblk = nvis * bps, rounds = (nblk + NW - 1) / NW;
+  const int all_blk = nvis * bps;
+  int blk0 = 0, nblk = all_blk;
+  if (p.n_splits > 1) {
+    blk0 = (int)((unsigned)part * (unsigned)all_blk / (unsigned)p.n_splits);
+    nblk = (int)((unsigned)(part + 1) * (unsigned)all_blk / (unsigned)p.n_splits) - blk0;
+  }
+  const int rounds = (nblk + NW - 1) / NW;
   int rot_g = 1;
   while (rot_g * 2 <= p.members && rot_g < 4) rot_g *= 2;
   const int rot_end = (nblk / NW) & ~(rot_g - 1);
   auto block_of = [&](int k) __attribute__((always_inline)) {
-    const int kk = k < rot_end ? (k & ~(rot_g - 1)) | ((k + member) & (rot_g - 1)) : k;
-    return kk * NW + wave;
+    const int kk = k < rot_end ? (k & ~(rot_g - 1)) | ((k + (int)member) & (rot_g - 1)) : k;
+    return blk0 + kk * NW + wave;
   };
 
   // (uniform base and 32-bit lane offsets; rows past the frame repeat its last one)
@@ -337,7 +352,7 @@ attn_ring_f32_kernel(AttnParams p) {
 
   // ---- blocks whose values two f16 halves hold ----
   int k = 0;
-  if (SPLIT && split && rounds >= split_rounds(DH) && mine_n > 0) {
+  if (SPLIT && split && all_blk >= fp.halves_from && mine_n > 0) {
     // The keys come row by row, whole cache lines a request, and change places with the other lanes' through LDS, halved.
     constexpr int CPR = DH / 4, RPL = 64 / CPR;   // 16-byte chunks per row, rows per request
     unsigned char* const k_to = smem + wave * Lds::kWave + (lane / CPR) * Lds::KROW + (lane % CPR) * 8;
@@ -590,11 +605,12 @@ attn_ring_f32_kernel(AttnParams p) {
     }
   }
   __syncthreads();   // (and everybody is done with the keys)
-  float lt[NQ];
+  float lt[NQ], mt[NQ];
 #pragma unroll
   for (int qi = 0; qi < NQ; ++qi) {
     const int at = qi * F_Q + c;
-    float mm = -INFINITY;
+    float& mm = mt[qi];
+    mm = -INFINITY;
     lt[qi] = 0.f;
 #pragma unroll
     for (int w = 0; w < NW; ++w)
@@ -632,7 +648,10 @@ attn_ring_f32_kernel(AttnParams p) {
   }
   if (wave == 0 && g == 0) {  // (every wavefront has read the sums before the barrier above)
 #pragma unroll
-    for (int qi = 0; qi < NQ; ++qi) lsh[0][qi * F_Q + c] = lt[qi];
+    for (int qi = 0; qi < NQ; ++qi) {
+      lsh[0][qi * F_Q + c] = lt[qi];
+      msh[0][qi * F_Q + c] = mt[qi];
+    }
   }
   __syncthreads();
   for (int item = tid; item < BQ * DH / 4; item += 64 * NW) {
@@ -642,6 +661,12 @@ attn_ring_f32_kernel(AttnParams p) {
     f32x4_t y = *reinterpret_cast<const f32x4_t*>(&osh[0][qi][d]);
 #pragma unroll
     for (int w = 1; w < NOUT; ++w) y += *reinterpret_cast<const f32x4_t*>(&osh[w][qi][d]);
+    if (p.n_splits > 1) {  // (a part: merged by the second pass)
+      const int64_t row = ((int64_t)part * p.B * p.H + (int64_t)b * p.H + h) * p.T + qrow;
+      *reinterpret_cast<f32x4_t*>(static_cast<float*>(p.ws_o) + row * DH + d) = y;
+      if (d == 0) *reinterpret_cast<float2_t*>(p.ws_ml + row * 2) = float2_t{msh[0][qi], lsh[0][qi]};
+      continue;
+    }
     y *= 1.f / lsh[0][qi];
     // the gate multiplies the rounded attention output, as the module's own multiply does
     if (p.gate != nullptr) y *= reinterpret_cast<const float*>(p.gate)[b * p.gs_b + h * p.gs_h + (int64_t)qrow * p.gs_t];
@@ -649,19 +674,63 @@ attn_ring_f32_kernel(AttnParams p) {
   }
 }
 
+// Second pass of a context in parts: one thread per four columns of a query row.
+template <int DH>
+__global__ void __launch_bounds__(256) f32_combine_kernel(AttnParams p) {
+  const unsigned item = blockIdx.x * 256 + threadIdx.x, row = item / (DH / 4), d = item % (DH / 4) * 4;
+  const unsigned rows = (unsigned)(p.B * p.H * p.T);
+  if (row >= rows) return;
+  float m = -INFINITY, l = 0.f;
+  f32x4_t y = {0.f, 0.f, 0.f, 0.f};
+#pragma nounroll
+  for (int s0 = 0; s0 < p.n_splits; s0 += 4) {
+    float2_t ml[4];
+    f32x4_t o[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      if (s0 + j < p.n_splits) {
+        const int64_t at = (int64_t)(s0 + j) * rows + row;
+        ml[j] = *reinterpret_cast<const float2_t*>(p.ws_ml + at * 2);
+        o[j] = *reinterpret_cast<const f32x4_t*>(static_cast<const float*>(p.ws_o) + at * DH + d);
+      } else {
+        ml[j] = float2_t{-INFINITY, 0.f};
+        o[j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+      }
+    }
+    float mx = m;
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      if (ml[j][1] != 0.f) mx = fmaxf(mx, ml[j][0]);  // (a part without keys has no say)
+    const float carry = l != 0.f ? __builtin_amdgcn_exp2f(m - mx) : 0.f;
+    l *= carry;
+    y *= carry;
+    m = mx;
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      if (ml[j][1] != 0.f) {
+        const float w = __builtin_amdgcn_exp2f(ml[j][0] - mx);
+        l += w * ml[j][1];
+        y += w * o[j];
+      }
+  }
+  const int t = (int)(row % (unsigned)p.T), bh = (int)(row / (unsigned)p.T), b = bh / p.H, h = bh - b * p.H;
+  y *= 1.f / l;
+  if (p.gate != nullptr) y *= reinterpret_cast<const float*>(p.gate)[b * p.gs_b + h * p.gs_h + (int64_t)t * p.gs_t];
+  *reinterpret_cast<f32x4_t*>(reinterpret_cast<float*>(p.out) + b * p.os_b + h * p.os_h + (int64_t)t * p.os_t + d) = y;
+}
+
 template <int DH>
 static hipError_t launch_f32(AttnParams p, int cus, hipStream_t stream) {
-  const auto workgroups = [&](int queries) { return (int64_t)p.B * p.H * ((p.T + queries - 1) / queries); };
-  const int64_t blocks = (int64_t)p.num_buckets * ((p.T + F_K - 1) / F_K);   // of a full ring
-  // Two groups of queries share what is halved where one a workgroup would be more than one a CU.
-  const int nq = workgroups(F_Q) > cus && (blocks + 7) / 8 >= split_rounds(DH) ? 2 : 1;
-  const int64_t wgs = workgroups(nq * F_Q);
+  F32Call call = {(int64_t)p.B * p.H, p.T, p.num_buckets, DH, cus};
+  call.plan(p.n_splits > 1 ? INT64_MAX : 0);   // (parts as the host planned them, or none)
+  const int nq = call.groups;
+  const int64_t wgs = call.tiles(nq) * p.n_splits;
   if (wgs > 0x7fffffff) return hipErrorInvalidValue;
   p.members = p.group * ((p.T + nq * F_Q - 1) / (nq * F_Q));
   // eight wavefronts per workgroup (two per SIMD of a CU) while a CU gets one workgroup; two
   // workgroups of four beyond, which leave a smaller last round
   const int nw = wgs <= cus ? 8 : 4;
-  const bool split = (blocks + nw - 1) / nw >= split_rounds(DH), whole = p.T % F_K == 0;
+  const bool split = call.blocks() >= call.halves_from(), whole = p.T % F_K == 0;
   const void* kernel = nullptr;
   int lds = 0;
   auto pick = [&](auto waves, auto groups, auto halves) {
@@ -676,8 +745,13 @@ static hipError_t launch_f32(AttnParams p, int cus, hipStream_t stream) {
   if (nq == 2) nw == 8 ? pick(w8, two, std::true_type()) : pick(w4, two, std::true_type());
   else if (split) nw == 8 ? pick(w8, one, std::true_type()) : pick(w4, one, std::true_type());
   else nw == 8 ? pick(w8, one, std::false_type()) : pick(w4, one, std::false_type());
-  void* args[] = {&p};
-  return hipLaunchKernel(kernel, dim3((unsigned)wgs), dim3(64 * nw), args, lds, stream);
+  F32Params fp = {p, (int)call.halves_from()};
+  void* args[] = {&fp};
+  const hipError_t e = hipLaunchKernel(kernel, dim3((unsigned)wgs), dim3(64 * nw), args, lds, stream);
+  if (e != hipSuccess || p.n_splits == 1) return e;
+  const int64_t items = (int64_t)p.B * p.H * p.T * (DH / 4);
+  hipLaunchKernelGGL(f32_combine_kernel<DH>, dim3((unsigned)((items + 255) / 256)), dim3(256), 0, stream, p);
+  return hipGetLastError();
 }
 
 // The dynamic-LDS limit of the instances that may need more than the default.

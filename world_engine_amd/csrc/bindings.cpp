@@ -215,8 +215,18 @@ struct Workspace {
   Tensor t;
   void* ptr = nullptr;
   size_t bytes = 0;
-  Workspace(const Tensor* given, int64_t B, int64_t H, int64_t Hkv, int64_t T, int64_t Dh, int64_t L, int splits,
+  Workspace(const Tensor* given, int64_t B, int64_t H, int64_t Hkv, int64_t T, int64_t Dh, int64_t L, int64_t dilation, int splits,
             int q_tile, const Tensor& like) {
+    if (like.scalar_type() == at::kFloat) {  // (no caller has to know of it: a given one that does not do is passed over)
+      const size_t wanted = splits == 0 ? we_attn_f32_workspace_bytes((int)B, (int)H, (int)Hkv, (int)T, (int)Dh, L, (int)dilation) : 0;
+      if (wanted == 0) return;
+      const bool fits = given != nullptr && given->device() == like.device() && given->is_contiguous() &&
+                        (size_t)given->numel() * given->element_size() >= wanted && ((uintptr_t)given->data_ptr() & 15u) == 0;
+      t = fits ? *given : at::empty({(int64_t)wanted}, like.options().dtype(at::kByte));
+      ptr = t.data_ptr();
+      bytes = (size_t)t.numel() * t.element_size();
+      return;
+    }
     const size_t need = we_attn_workspace_bytes_for((int)B, (int)H, (int)Hkv, (int)T, (int)Dh, L, splits, q_tile, dtype_code(like));
     if (need == 0) return;
     if (given != nullptr && given->device() != like.device()) fail("workspace must be on the call's device, " + like.device().str());
@@ -520,7 +530,7 @@ PyObject* attn_ring(PyObject*, PyObject* const* argv, Py_ssize_t n) {
     const bool token_major = a.flag();
     const Strides qs(q, "q");
     const OnDevice on(dev);
-    const Workspace ws(ws_in, B, H, Hkv, T, Dh, L, splits, q_tile, q);
+    const Workspace ws(ws_in, B, H, Hkv, T, Dh, L, dilation, splits, q_tile, q);
     const Tensor out = output_or_new(out_in, token_major, q, dev, B, H, T, Dh);
     const Strides os(out, "out");
     run("we_attn_ring_fwd", nullptr, [&] { return we_attn_ring_fwd(q.data_ptr(), qs.s, kv.data_ptr(), static_cast<const uint8_t*>(written.data_ptr()),
@@ -588,7 +598,7 @@ PyObject* rope_kv_attn(PyObject*, PyObject* const* argv, Py_ssize_t n) {
     const Extras extras(eps, v1, v_lamb, gate, gate_x, gate_w, q.scalar_type(), B, H, Hkv, T, Dh);
     const OnDevice on(dev);
     const hipStream_t st = stream_of(dev);
-    const Workspace ws(ws_in, B, H, Hkv, T, Dh, L, splits, q_tile, q);
+    const Workspace ws(ws_in, B, H, Hkv, T, Dh, L, dilation, splits, q_tile, q);
     Tensor q_rot;
     if (q_rot_in == nullptr) {
       q_rot = new_heads(q, B, H, T, Dh);
@@ -668,7 +678,7 @@ PyObject* qkv_rope_kv_attn(PyObject*, PyObject* const* argv, Py_ssize_t n) {
                                           static_cast<uint8_t*>(written.data_ptr()), (int)B, (int)H, (int)Hkv, (int)T, (int)Dh,
                                           L, (int)dilation, frozen ? 1 : 0, code_t, extras.ptr(), st); });
     } else {
-      const Workspace ws(ws_in, B, H, Hkv, T, Dh, L, splits, q_tile, x);
+      const Workspace ws(ws_in, B, H, Hkv, T, Dh, L, dilation, splits, q_tile, x);
       out = output_or_new(out_in, true, x, dev, B, H, T, Dh);
       const Strides os(out, "out");
       const bool refused = run("we_qkv_rope_kv_attn_fwd", &check, [&] { return we_qkv_rope_kv_attn_fwd_checked(

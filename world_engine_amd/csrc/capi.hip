@@ -331,6 +331,13 @@ size_t we_attn_workspace_bytes_for(int32_t B, int32_t H, int32_t Hkv, int32_t T,
   return workspace_bytes_of(plan_cached(B, H, Hkv, T, Dh, L, n_splits, variant_of(q_tile), we::host::compute_units()), Dh, true);
 }
 
+size_t we_attn_f32_workspace_bytes(int32_t B, int32_t H, int32_t Hkv, int32_t T, int32_t Dh, int64_t L, int32_t dilation) {
+  if (B <= 0 || H <= 0 || Hkv <= 0 || (Dh != 64 && Dh != 128) || we::host::ring_shape_ok(B, H, Hkv, T, Dh, L, dilation) != WE_OK) return 0;
+  we::F32Call call = {(int64_t)B * H, T, L / T / dilation, Dh, we::host::compute_units()};
+  call.plan(INT64_MAX);
+  return (size_t)call.bytes(call.parts);
+}
+
 int we_attn_plan(int32_t B, int32_t H, int32_t Hkv, int32_t T, int32_t Dh, int64_t L, int32_t n_splits,
                  int32_t q_tile, int32_t compute_units, int32_t plan[WE_PLAN_FIELDS]) {
   if (!plan) return WE_ERR_NULL_POINTER;
