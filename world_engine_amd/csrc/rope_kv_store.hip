@@ -151,10 +151,13 @@ static void launch_store(const StoreParams& p, hipStream_t stream) {
   const auto grid = [&](int elements) {
     return dim3((unsigned)((p.T * (p.Dh / elements) + 255) / 256), (unsigned)heads, (unsigned)p.B);
   };
-  // (16 elements of half precision are what one request takes in whole, and the larger launches take them faster: 24 heads, 3600
-  // tokens 32.9 / 33.6 us with 8, 4 x 24 heads, 1024 tokens 31.9 either way)
+  // (16 elements of half precision are what one request takes in whole.  A frame's store, attention and second pass, 16 / 8
+  // elements, by the launch's workgroups of 16: up to 720 of them 0.2 to 0.3 us less with 8, none of 60 shapes slower by more than its
+  // runs differ; from 738 on as much lost as gained and up to 2.7 us more a pass: 810 34.0 / 35.1, 1008 24.9 / 25.6, 1276 45.3 /
+  // 46.3, 1386 229 / 241, 3536 72.5 / 74.7 - twice the workgroups, which no longer find room at once.  fp32 calls 3 to 8 % less at
+  // 405 to 1170.)
   const dim3 whole = grid(16);
-  const bool large = Tag::kBytes == 2 && (int64_t)whole.x * whole.y * whole.z > 4096;
+  const bool large = Tag::kBytes == 2 && (int64_t)whole.x * whole.y * whole.z > 720;
   if (p.norm_eps > 0.f || p.v1 != nullptr || large) {
     if (p.check != 0) hipLaunchKernelGGL((rope_kv_store_kernel<Tag, true>), grid(16), dim3(256), 0, stream, p);
     else hipLaunchKernelGGL((rope_kv_store_kernel<Tag, false>), grid(16), dim3(256), 0, stream, p);
