@@ -33,7 +33,7 @@ extern "C" {
 /* element types of q/k/v, the cache buffer and the attention output */
 #define WE_DTYPE_BF16 0
 #define WE_DTYPE_F16 1
-#define WE_DTYPE_F32 2 /* fp32 caches: the store rotates in fp32, the attention takes a one-pass fp32 kernel */
+#define WE_DTYPE_F32 2 /* fp32 caches: the store rotates in fp32, the attention takes a kernel of its own */
 
 #define WE_OK 0
 #define WE_ERR_NULL_POINTER (-1)
@@ -138,7 +138,7 @@ size_t we_attn_workspace_bytes(int32_t B, int32_t H, int32_t Hkv, int32_t T, int
 /*
  * The same for an element type: what lets an f16 call keep its partial results in fp32 (about twice
  * the bytes above; an f16 call with a shorter workspace splits less where it can, and holds them in
- * 16 bits otherwise), 0 for fp32 calls, which split nothing.
+ * 16 bits otherwise), 0 for fp32 calls (see we_attn_f32_workspace_bytes).
  */
 size_t we_attn_workspace_bytes_for(int32_t B, int32_t H, int32_t Hkv, int32_t T, int32_t Dh, int64_t L,
                                    int32_t n_splits, int32_t q_tile, int32_t dtype);
@@ -189,7 +189,7 @@ int we_attn_plan(int32_t B, int32_t H, int32_t Hkv, int32_t T, int32_t Dh, int64
  *   q_tile               queries per workgroup: 0 = choose automatically, or 128 / 256.
  *   scale                softmax scale (> 0); the reference uses 1/sqrt(Dh).
  *
- * Requirements: dtype bf16 or f16 or f32 (a one-pass kernel of its own, fp32 arithmetic
+ * Requirements: dtype bf16 or f16 or f32 (a kernel of its own, of fp32 precision
  * throughout, n_splits 0 or 1, q_tile ignored); Dh in {64, 128};
  * any T (frames that are not a multiple of the 64-key tile cost one masked tile per slot);
  * L/T <= WE_MAX_SLOTS; H % Hkv == 0; pointers and row starts 16-byte aligned.

@@ -1,6 +1,6 @@
 // fp32 attention over the KV ring buffer (gfx950): the same visibility rule and ring walk as the
-// half-precision kernel (attn_ring.hip), fp32 throughout (fp32 scores, softmax and P V,
-// src/model/attn.py:116 in eager mode) on the fp32 matrix instructions.
+// half-precision kernel (attn_ring.hip), of fp32 precision throughout (scores, softmax and P V,
+// src/model/attn.py:116 in eager mode).
 //
 // One workgroup = one or two groups of 16 queries of one (batch, head) and NW wavefronts that share out its keys: blocks
 // of 16 keys go round the wavefronts, each keeps its own running (reference, sum, O) and they merge
@@ -17,7 +17,7 @@
 // O's are added by the vector unit, so that no chain of products loses more than its own size.  Relative
 // error against 64 bits, fp32 products / halves: 16 heads of 128, 2048 keys 3.9e-7 / 3.0e-7, 8 heads, 4096
 // keys 6.3e-7 / 3.4e-7, 4 heads, 128 keys 2.3e-7 / 2.2e-7; heads of 64, 2880 keys 5.2e-7 / 3.2e-7, 1024 keys
-// 2.9e-7 / 2.8e-7, but 512 keys 2.4e-7 / 2.6e-7: their short contexts stay with fp32 products (split_rounds).
+// 2.9e-7 / 2.8e-7, but 512 keys 2.4e-7 / 2.6e-7: their short contexts stay with fp32 products (F32Call::halves_from).
 // Halves hold values of a certain size only; each wavefront looks at its own as they come and goes on with fp32
 // products where they do not (a block in front of which it notices costs it one round trip).
 //
@@ -251,7 +251,7 @@ attn_ring_f32_kernel(F32Params fp) {
   // Blocks go round the wavefronts in rounds of NW.  The workgroups that share a K/V stream take the
   // rounds in groups of rot_g, member m starting at round m of every group: they then ask for
   // different lines at any one time, and each line comes from memory at one member's request (184
-  // against 192 us for the 1024-query shape above when it took 184; groups of 8 or 16: the same, then and now).
+  // against 192 us for 8 heads, 1024 queries, 4096 keys when they took 184; groups of 8 or 16: the same, then and now).
   const int bps = (p.T + F_K - 1) / F_K;  // blocks per slot; the last one may be short
   const int all_blk = nvis * bps;
   int blk0 = 0, nblk = all_blk;
@@ -303,7 +303,7 @@ attn_ring_f32_kernel(F32Params fp) {
         s1 = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[j + 1][i], qf[j + 1][i], s1, 0, 0, 0);
       }
     // (the next block's loads go out between these products: together they keep a wavefront from issuing anything
-    // else while the CU's address path takes them, 47.0 against 45.5 us for the first shape above)
+    // else while the CU's address path takes them, 45.5 against 47.0 us for 16 heads of 128, 256 queries, 2048 keys)
 #pragma unroll
     for (int i = 0; i < NJ + 4 * NH; ++i) {
       __builtin_amdgcn_sched_group_barrier(0x20, 1, 0);
@@ -339,7 +339,7 @@ attn_ring_f32_kernel(F32Params fp) {
       for (int hh = 0; hh < NH; ++hh)
 #pragma unroll
         for (int e = 0; e < 4; ++e) o[qi][hh][e] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[i][hh][e], pr[i], o[qi][hh][e], 0, 0, 0);
-    // (two blocks in a row are not scheduled as one: 44.4 against 46.8 us for the first shape above)
+    // (two blocks in a row are not scheduled as one: 44.4 against 46.8 us for the same shape)
     __builtin_amdgcn_sched_barrier(0);
   };
   const int mine_n = rounds - (nblk - (rounds - 1) * NW > wave ? 0 : 1);  // rounds this wavefront takes part in

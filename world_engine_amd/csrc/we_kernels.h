@@ -123,7 +123,7 @@ hipError_t launch_attn_ring_short_f16(const AttnParams& p, int Dh, int ksplit, h
 // grouped heads that share query tiles (q_heads != group)
 hipError_t launch_attn_ring_shared_bf16(const AttnParams& p, int Dh, int ksplit, hipStream_t stream);
 hipError_t launch_attn_ring_shared_f16(const AttnParams& p, int Dh, int ksplit, hipStream_t stream);
-// fp32 caches: one pass on the fp32 matrix instructions, no context splitting
+// fp32 caches (f32_parts.h: whether in parts, merged by a second pass of their own)
 hipError_t launch_attn_ring_f32(const AttnParams& p, int Dh, int cus, hipStream_t stream);
 hipError_t launch_attn_combine(const AttnParams& p, int Dh, int dtype, hipStream_t stream);
 // Measurement library only (stream_probe.hip): the 256-token-frame tile stream without the arithmetic.
