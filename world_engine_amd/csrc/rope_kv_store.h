@@ -65,46 +65,47 @@ __device__ __forceinline__ void store8(void* p, const Chunk8<Tag>& c) {
   for (int i = 0; i < nvec; ++i) dst[i] = src[i];
 }
 
-// Weightless RMS norm of a row held 16 elements per lane by `cpr` consecutive lanes (a power of
+// Weightless RMS norm of a row held N = 16 or 8 elements per lane by `cpr` consecutive lanes (a power of
 // two, at most 64): x * rsqrt(mean(x^2) + eps) in fp32, rounded to the element type, as
 // F.rms_norm on a low-precision tensor does (src/model/nn.py:55-56).  The squares are added in the order
 // that torch 2.10's norm shows on this GPU - four neighbours one after the other, then halves onto halves:
 // half-precision squares are exact in fp32, so the order is all that decides a sum's bits, and of the orders
 // tried (groups of 1 to 16, neighbouring or strided, sequential or as trees) this one, with this reciprocal
 // root, gives every bit of 2*10^5 rows of 64 and of 128.
-template <typename Tag>
-__device__ __forceinline__ void rms_norm_chunk(Chunk16<Tag>& c, int cpr, int Dh, float eps) {
-  float x[16], part[4];
+template <typename Tag, int N, typename E>
+__device__ __forceinline__ void rms_norm_chunk(E& e, int cpr, int Dh, float eps) {
+  float x[N], part[N / 4];
 #pragma unroll
-  for (int j = 0; j < 4; ++j) {
+  for (int j = 0; j < N / 4; ++j) {
     part[j] = 0.f;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      x[4 * j + i] = Tag::to_f32(c.e[4 * j + i]);
+      x[4 * j + i] = Tag::to_f32(e[4 * j + i]);
       part[j] += x[4 * j + i] * x[4 * j + i];
     }
   }
   for (int m = cpr >> 1; m > 0; m >>= 1)
 #pragma unroll
-    for (int j = 0; j < 4; ++j) part[j] += __shfl_xor(part[j], m);
-  const float r = rsqrtf(((part[0] + part[2]) + (part[1] + part[3])) / (float)Dh + eps);
+    for (int j = 0; j < N / 4; ++j) part[j] += __shfl_xor(part[j], m);
+  const float sum = N == 16 ? (part[0] + part[N / 4 - 2]) + (part[1] + part[N / 4 - 1]) : part[0] + part[1];
+  const float r = rsqrtf(sum / (float)Dh + eps);
 #pragma unroll
-  for (int i = 0; i < 16; ++i) {
+  for (int i = 0; i < N; ++i) {
     float y = x[i] * r;
     asm("" : "+v"(y));  // (fused with the conversion to f16 the product of a negative value and 0 loses its sign)
-    c.e[i] = Tag::from_f32(y);
+    e[i] = Tag::from_f32(y);
   }
 }
 
-// torch.lerp(v, v1, w) on 16 elements: fp32 arithmetic, the formula switches at |w| = 0.5
+// torch.lerp(v, v1, w) on N elements: fp32 arithmetic, the formula switches at |w| = 0.5
 // (ATen/native/Lerp.h), result rounded to the element type.
-template <typename Tag>
-__device__ __forceinline__ void lerp_chunk(Chunk16<Tag>& v, const Chunk16<Tag>& v1, float w) {
+template <typename Tag, int N, typename E>
+__device__ __forceinline__ void lerp_chunk(E& v, const E& v1, float w) {
 #pragma unroll
-  for (int i = 0; i < 16; ++i) {
-    const float a = Tag::to_f32(v.e[i]), b = Tag::to_f32(v1.e[i]);
+  for (int i = 0; i < N; ++i) {
+    const float a = Tag::to_f32(v[i]), b = Tag::to_f32(v1[i]);
     const float d = b - a;
-    v.e[i] = Tag::from_f32(fabsf(w) < 0.5f ? a + w * d : b - d * (1.f - w));
+    v[i] = Tag::from_f32(fabsf(w) < 0.5f ? a + w * d : b - d * (1.f - w));
   }
 }
 
@@ -190,8 +191,8 @@ __device__ __forceinline__ void finish_kv_chunk(const StoreParams& p, int which,
                                                 const SlotInfo& si, Chunk16<Tag>& in, bool rotate,
                                                 const float (&c)[8], const float (&s)[8], const Chunk16<Tag>& res,
                                                 float lamb) {
-  if (which == 1 && p.norm_eps > 0.f) rms_norm_chunk<Tag>(in, p.Dh >> 4, p.Dh, p.norm_eps);
-  if (which == 2 && p.v1 != nullptr) lerp_chunk<Tag>(in, res, lamb);
+  if (which == 1 && p.norm_eps > 0.f) rms_norm_chunk<Tag, 16>(in.e, p.Dh >> 4, p.Dh, p.norm_eps);
+  if (which == 2 && p.v1 != nullptr) lerp_chunk<Tag, 16>(in.e, res.e, lamb);
   Chunk8<Tag> lo, hi;
   if (rotate) rotate_values<Tag>(in, c, s, lo, hi);
   store_kv_rows<Tag>(p, which, b, h, t, chunk, si, rotate, in, lo, hi);
@@ -204,7 +205,7 @@ __device__ __forceinline__ void finish_q_chunk(const StoreParams& p, int b, int 
                                                Chunk16<Tag>& in, bool rotate, const float (&c)[8],
                                                const float (&s)[8]) {
   typedef typename Tag::store_t st_t;
-  if (p.norm_eps > 0.f) rms_norm_chunk<Tag>(in, p.Dh >> 4, p.Dh, p.norm_eps);
+  if (p.norm_eps > 0.f) rms_norm_chunk<Tag, 16>(in.e, p.Dh >> 4, p.Dh, p.norm_eps);
   st_t* dst = (st_t*)p.q_out + (((int64_t)b * p.H + h) * p.T + t) * p.Dh;
   if (rotate) {
     Chunk8<Tag> lo, hi;

@@ -56,11 +56,11 @@ __global__ void __launch_bounds__(256) rope_kv_store_kernel(StoreParams p) {
   }
 }
 
-// The same without a norm or a blend, 8 elements a thread: bound by its trips to memory where the launch is small, and of fp32
+// The same with 8 elements a thread (EXTRAS: a norm or a blend too): bound by its trips to memory where the launch is small, and of fp32
 // rows by the requests, each of which takes a quarter of every 64 bytes with 16 elements a thread (us, 16 / 8
 // elements, persisting calls in a graph: fp32, 16 heads of 128, 256 tokens 5.94 / 4.42, 8 heads, 1024 tokens 9.50 / 7.28, 8 heads
 // of 64, 64 tokens 3.02 / 2.45; bf16, 16 heads of 128, 256 tokens 3.53 / 3.39, 16 of 64, 64 tokens 2.74 / 2.53).
-template <typename Tag, bool CHECK>
+template <typename Tag, bool CHECK, bool EXTRAS>
 __global__ void __launch_bounds__(256) rope_kv_store_8_kernel(StoreParams p) {
   touch_args<StoreParams>();
   typedef typename Tag::store_t st_t;
@@ -80,7 +80,9 @@ __global__ void __launch_bounds__(256) rope_kv_store_8_kernel(StoreParams p) {
   const bool bad = CHECK && own_ids_bad(p);
   const int64_t frame_t = p.t_pos[0];
   const bool rotate = which != 2 && p.cos_t != nullptr;
-  eight_t in;
+  const bool blend = EXTRAS && which == 2 && p.v1 != nullptr;
+  eight_t in, res;
+  float lamb = 0.f;
   f32x4_t c, s;
   if (live) {
     const st_t* src = which == 0   ? (const st_t*)p.q + b * p.qs_b + h * p.qs_h + t * p.qs_t
@@ -94,9 +96,17 @@ __global__ void __launch_bounds__(256) rope_kv_store_8_kernel(StoreParams p) {
       c = *reinterpret_cast<const f32x4_t*>(p.cos_t + at);
       s = *reinterpret_cast<const f32x4_t*>(p.sin_t + at);
     }
+    if (blend) {
+      const st_t* from = (const st_t*)p.v1 + b * p.v1s_b + h * p.v1s_h + t * p.v1s_t + chunk * 8;
+#pragma unroll
+      for (int i = 0; i < Tag::kBytes / 2; ++i) reinterpret_cast<uint4*>(&res)[i] = reinterpret_cast<const uint4*>(from)[i];
+      lamb = Tag::to_f32(*reinterpret_cast<const st_t*>(p.v_lamb));
+    }
   }
   if (CHECK && frame_refused(p, bad)) return;
   if (!live) return;
+  if (EXTRAS && which != 2 && p.norm_eps > 0.f) rms_norm_chunk<Tag, 8>(in, cpr, p.Dh, p.norm_eps);
+  if (blend) lerp_chunk<Tag, 8>(in, res, lamb);
   four_t lo = __builtin_shufflevector(in, in, 0, 1, 2, 3), hi = __builtin_shufflevector(in, in, 4, 5, 6, 7);
   if (rotate) {
 #pragma clang fp contract(off)
@@ -155,15 +165,20 @@ static void launch_store(const StoreParams& p, hipStream_t stream) {
   // elements, by the launch's workgroups of 16: up to 720 of them 0.2 to 0.3 us less with 8, none of 60 shapes slower by more than its
   // runs differ; from 738 on as much lost as gained and up to 2.7 us more a pass: 810 34.0 / 35.1, 1008 24.9 / 25.6, 1276 45.3 /
   // 46.3, 1386 229 / 241, 3536 72.5 / 74.7 - twice the workgroups, which no longer find room at once.  fp32 calls 3 to 8 % less at
-  // 405 to 1170.)
+  // 405 to 1170.  With a norm or a blend the same 0.3 us: 34 module passes of 24 to 1188 1.009 times as fast, 0.99 at worst with
+  // runs 1 % apart.)
   const dim3 whole = grid(16);
   const bool large = Tag::kBytes == 2 && (int64_t)whole.x * whole.y * whole.z > 720;
-  if (p.norm_eps > 0.f || p.v1 != nullptr || large) {
-    if (p.check != 0) hipLaunchKernelGGL((rope_kv_store_kernel<Tag, true>), grid(16), dim3(256), 0, stream, p);
-    else hipLaunchKernelGGL((rope_kv_store_kernel<Tag, false>), grid(16), dim3(256), 0, stream, p);
+  const bool extras = p.norm_eps > 0.f || p.v1 != nullptr;
+  const auto run = [&](auto kernel, int elements) {
+    hipLaunchKernelGGL(kernel, grid(elements), dim3(256), 0, stream, p);
+  };
+  if (large) {
+    p.check != 0 ? run(rope_kv_store_kernel<Tag, true>, 16) : run(rope_kv_store_kernel<Tag, false>, 16);
+  } else if (extras) {
+    p.check != 0 ? run(rope_kv_store_8_kernel<Tag, true, true>, 8) : run(rope_kv_store_8_kernel<Tag, false, true>, 8);
   } else {
-    if (p.check != 0) hipLaunchKernelGGL((rope_kv_store_8_kernel<Tag, true>), grid(8), dim3(256), 0, stream, p);
-    else hipLaunchKernelGGL((rope_kv_store_8_kernel<Tag, false>), grid(8), dim3(256), 0, stream, p);
+    p.check != 0 ? run(rope_kv_store_8_kernel<Tag, true, false>, 8) : run(rope_kv_store_8_kernel<Tag, false, false>, 8);
   }
 }
 
