@@ -166,9 +166,12 @@ static void launch_store(const StoreParams& p, hipStream_t stream) {
   // runs differ; from 738 on as much lost as gained and up to 2.7 us more a pass: 810 34.0 / 35.1, 1008 24.9 / 25.6, 1276 45.3 /
   // 46.3, 1386 229 / 241, 3536 72.5 / 74.7 - twice the workgroups, which no longer find room at once.  fp32 calls 3 to 8 % less at
   // 405 to 1170.  With a norm or a blend the same 0.3 us: 34 module passes of 24 to 1188 1.009 times as fast, 0.99 at worst with
-  // runs 1 % apart.)
+  // runs 1 % apart.  A rotation alone: 360 3.25 / 3.05, 456 3.35 / 3.48, 720 4.06 / 4.36; half the line also because a layer that
+  // rotates q and k and then stores both should find one kernel: 24 heads, 588 tokens, four layers of five passes 735 us with 16
+  // elements in all three launches, 742 with 8, 763 with 8 in one kind only.)
   const dim3 whole = grid(16);
-  const bool large = Tag::kBytes == 2 && (int64_t)whole.x * whole.y * whole.z > 720;
+  const int64_t most = p.k == nullptr ? 360 : 720;
+  const bool large = Tag::kBytes == 2 && (int64_t)whole.x * whole.y * whole.z > most;
   const bool extras = p.norm_eps > 0.f || p.v1 != nullptr;
   const auto run = [&](auto kernel, int elements) {
     hipLaunchKernelGGL(kernel, grid(elements), dim3(256), 0, stream, p);
