@@ -46,6 +46,22 @@ def test_both_items_store_the_same_bits(gpu_device, dtype, extras, B, T, Dh):
         assert_bits_equal(written_one, written_all, "written")
 
 
+# (a rotation alone: more than 360 workgroups against less)
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("B,T,Dh", [(8, 100, 128), (31, 33, 64)])
+def test_both_items_rotate_to_the_same_bits(gpu_device, dtype, B, T, Dh):
+    x = torch.randn(B, T, 16, Dh, device="cuda", generator=torch.Generator("cuda").manual_seed(T)).to(dtype).transpose(1, 2)
+    rope = RoPE(*ro.rope_table_1d(4 * T, Dh), 1, T).to(gpu_device)
+    pos = to_dev(ro.synth_pos_ids(1, B, T, T), gpu_device)
+
+    def rotated(at):
+        return ops.rope_apply(x[at], {n: t[at] for n, t in pos.items()}, rope.cos, rope.sin, rope.height, rope.width)
+
+    every = rotated(slice(None))
+    for b in (0, B // 2, B - 1):
+        assert_bits_equal(rotated(slice(b, b + 1)), every[b:b + 1], "RoPE(x)")
+
+
 # A norm's sum of at most 128 squares is off by at most 4 + 5 roundings, its root by half of that and 2 more, the product, the
 # blend and the rotation by 2 each: less than 12 units of 2^-24 on either side, of values up to sqrt(2) times the row's largest.
 @pytest.mark.parametrize("T,Dh", [(16, 64), (33, 128), (100, 64), (256, 128)])
