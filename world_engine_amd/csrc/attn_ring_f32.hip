@@ -132,7 +132,8 @@ attn_ring_f32_kernel(F32Params fp) {
   // (spread over the XCDs by unit part where every XCD gets the same number: its workgroups share an L2)
   const int q_tiles = (p.T + BQ - 1) / BQ;
   unsigned up, member;
-  if (((p.B * p.Hkv * p.n_splits) & 7) == 0) {
+  const int n_parts = SPLIT ? p.n_splits : 1;   // (F32Call::plan: parts in halves only)
+  if (((p.B * p.Hkv * n_parts) & 7) == 0) {
     const unsigned j = blockIdx.x >> 3;
     const unsigned u8 = j / (unsigned)p.members;
     up = u8 * 8 + (blockIdx.x & 7);
@@ -142,9 +143,9 @@ attn_ring_f32_kernel(F32Params fp) {
     member = blockIdx.x - up * (unsigned)p.members;
   }
   int unit = (int)up, part = 0;
-  if (p.n_splits > 1) {
-    unit = (int)(up / (unsigned)p.n_splits);
-    part = (int)(up - (unsigned)unit * (unsigned)p.n_splits);
+  if (n_parts > 1) {
+    unit = (int)(up / (unsigned)n_parts);
+    part = (int)(up - (unsigned)unit * (unsigned)n_parts);
   }
   const int b = unit / p.Hkv, hkv = unit - b * p.Hkv;
   const int hq_in = (int)member / q_tiles, h = hkv * p.group + hq_in;
@@ -255,9 +256,9 @@ attn_ring_f32_kernel(F32Params fp) {
   const int bps = (p.T + F_K - 1) / F_K;  // blocks per slot; the last one may be short
   const int all_blk = nvis * bps;
   int blk0 = 0, nblk = all_blk;
-  if (p.n_splits > 1) {
-    blk0 = (int)((unsigned)part * (unsigned)all_blk / (unsigned)p.n_splits);
-    nblk = (int)((unsigned)(part + 1) * (unsigned)all_blk / (unsigned)p.n_splits) - blk0;
+  if (n_parts > 1) {
+    blk0 = (int)((unsigned)part * (unsigned)all_blk / (unsigned)n_parts);
+    nblk = (int)((unsigned)(part + 1) * (unsigned)all_blk / (unsigned)n_parts) - blk0;
   }
   const int rounds = (nblk + NW - 1) / NW;
   int rot_g = 1;
@@ -661,7 +662,7 @@ attn_ring_f32_kernel(F32Params fp) {
     f32x4_t y = *reinterpret_cast<const f32x4_t*>(&osh[0][qi][d]);
 #pragma unroll
     for (int w = 1; w < NOUT; ++w) y += *reinterpret_cast<const f32x4_t*>(&osh[w][qi][d]);
-    if (p.n_splits > 1) {  // (a part: merged by the second pass)
+    if (n_parts > 1) {  // (a part: merged by the second pass)
       const int64_t row = ((int64_t)part * p.B * p.H + (int64_t)b * p.H + h) * p.T + qrow;
       *reinterpret_cast<f32x4_t*>(static_cast<float*>(p.ws_o) + row * DH + d) = y;
       if (d == 0) *reinterpret_cast<float2_t*>(p.ws_ml + row * 2) = float2_t{msh[0][qi], lsh[0][qi]};
