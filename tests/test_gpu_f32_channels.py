@@ -1,0 +1,49 @@
+"""fp32 attention where channels or keys differ in size by orders of magnitude: every output channel and every row is as exact
+as fp32 sums are, whatever the others hold."""
+import math
+
+import pytest
+import torch
+
+from world_engine_amd import ops
+
+pytestmark = pytest.mark.gpu
+
+# Relative errors (2-norms) against 64 bits.  fp32 products and sums over logits of a few units: 3 to 6e-7 of the whole output;
+# the worst of a few thousand channels or rows is up to three times that.
+REL, REL_ONE = 1e-6, 4e-6
+
+# (16 queries a workgroup, in one pass and in parts; 32 queries, frames on and off the blocks; heads of 64)
+SHAPES = [(1, 16, 16, 128, 128, 5), (1, 2, 2, 64, 128, 20), (2, 24, 24, 96, 128, 4), (3, 30, 10, 49, 128, 6), (2, 30, 6, 81, 64, 11)]
+
+
+def _errors(dev, shape, change):
+    """(whole, worst output channel, worst row) of the last frame over a full ring; ``change(q, k, v)`` alters inputs in place."""
+    B, H, Hkv, T, Dh, n = shape
+    g = torch.Generator(dev).manual_seed(T + Dh)
+    q = torch.randn(B, H, T, Dh, device=dev, generator=g)
+    kv = torch.randn(2, B, Hkv, (n + 1) * T, Dh, device=dev, generator=g)
+    written = torch.ones((n + 1) * T, dtype=torch.bool, device=dev)
+    k, v = kv[:, :, :, T:]          # (frame 0: the slot that it replaces, the first, is hidden)
+    change(q, k, v)
+    out = ops.attn_ring(q, kv, written, torch.zeros(B, T, dtype=torch.long, device=dev), n * T, 1).double()
+    ref = torch.empty_like(out)
+    for b in range(B):
+        for h in range(H):
+            kh = k[b, h // (H // Hkv)].double().t().contiguous()
+            ref[b, h] = torch.softmax(q[b, h].double() @ kh / math.sqrt(Dh), -1) @ v[b, h // (H // Hkv)].double()
+    d = out - ref
+    return [(d.norm() / ref.norm()).item()] + [(d.norm(dim=i) / ref.norm(dim=i)).max().item() for i in (2, 3)]
+
+
+@pytest.mark.parametrize("shape", SHAPES)
+@pytest.mark.parametrize("factor", [1e-4, 30.0, 1e3, 1e4, 1e6])
+def test_large_queries_meet_small_keys(gpu_device, shape, factor):
+    """Logits of the usual size, one channel of them from queries `factor` times as large and keys as much smaller."""
+    def change(q, k, v):
+        q[..., 5].mul_(factor)
+        k[..., 5].div_(factor)
+
+    whole, channel, row = _errors(gpu_device, shape, change)
+    print(f"f32 channels {shape} q x {factor:g}: {whole:.2e}, channel {channel:.2e}, row {row:.2e}", flush=True)
+    assert whole <= REL and channel <= REL_ONE and row <= REL_ONE

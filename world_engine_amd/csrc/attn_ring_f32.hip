@@ -18,8 +18,8 @@
 // error against 64 bits, fp32 products / halves: 16 heads of 128, 2048 keys 3.9e-7 / 3.0e-7, 8 heads, 4096
 // keys 6.3e-7 / 3.4e-7, 4 heads, 128 keys 2.3e-7 / 2.2e-7; heads of 64, 2880 keys 5.2e-7 / 3.2e-7, 1024 keys
 // 2.9e-7 / 2.8e-7, but 512 keys 2.4e-7 / 2.6e-7: their short contexts stay with fp32 products (F32Call::halves_from).
-// Halves hold values of a certain size only; each wavefront looks at its own as they come and goes on with fp32
-// products where they do not (a block in front of which it notices costs it one round trip).
+// Halves hold keys and values of a certain size only.  For the keys the queries' size tells (below); each wavefront looks at its
+// values as they come and goes on with fp32 products where they do not fit.
 //
 // Blocks through v_mfma_f32_16x16x4_f32: the contraction of S is taken in an order that lets a lane load four of its
 // head-dim values at once (lane group g of step (j, i) has value 16 j + 4 g + i of both operands), and output rows
@@ -48,6 +48,8 @@ namespace {
 constexpr int F_Q = 16;   // queries of a group
 constexpr int F_K = 16;   // keys per block
 constexpr float P_LOW = 10.f, P_HIGH = 15.f;   // exponents of split probabilities
+constexpr int K_UP = 5;          // exponent of the scale for the keys of large queries
+constexpr float Q_MOST = 4.f;    // 2-norm of a query, times scale * log2(e) (normalised queries: 1.44)
 
 // NQ: groups of queries per workgroup
 template <int DH, int NW, int NQ, bool SPLIT>
@@ -87,20 +89,42 @@ __device__ __forceinline__ float groups_sum(float x) {
 }
 
 typedef float float2_t __attribute__((ext_vector_type(2)));
-typedef _Float16 f16x4_t __attribute__((ext_vector_type(4)));
 
-// fp32 values as sums of two f16 ones: the value rounded, and what that leaves, rounded.
-struct Halves {
-  f16x8_t hi, lo;
-  // (minus_one: -1 that the compiler does not know, so that the rest stays one v_fma_mix)
-  __device__ __forceinline__ void set(int i, float a, float b, float minus_one) {
-    const f16x2_t h = __builtin_convertvector((float2_t{a, b}), f16x2_t);
-    hi[i] = h[0];
-    hi[i + 1] = h[1];
-    lo[i] = (_Float16)__builtin_fmaf((float)h[0], minus_one, a);
-    lo[i + 1] = (_Float16)__builtin_fmaf((float)h[1], minus_one, b);
+__device__ __forceinline__ uint32_t f16_pair(float a, float b) {
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector((float2_t{a, b}), f16x2_t));
+}
+// Four fp32 values as sums of two f16 ones: rounded (hi), and what that leaves, rounded; or both `up` times as large (a power of
+// two, f16_pow2).  All at the full rate, which conversions to one half of a register (v_fma_mixlo_f16) do not have: 36.9 -> 42
+// us for the first shape above.
+struct Halves4 {
+  u32x2_t hi, lo;
+  __device__ __forceinline__ Halves4(float a, float b, float c, float d) : Halves4(a, b, c, d, f16_pair(a, b), f16_pair(c, d), 1.f) {}
+  __device__ __forceinline__ Halves4(float a, float b, float c, float d, float up, uint32_t up16)
+      : Halves4(a, b, c, d, times(f16_pair(a, b), up16), times(f16_pair(c, d), up16), up) {}
+
+ private:
+  static __device__ __forceinline__ uint32_t times(uint32_t h, uint32_t by) {
+    uint32_t y;
+    asm("v_pk_mul_f16 %0, %1, %2" : "=v"(y) : "v"(h), "s"(by));
+    return y;
+  }
+  __device__ __forceinline__ Halves4(float a, float b, float c, float d, uint32_t h0, uint32_t h1, float up) : hi{h0, h1} {
+    float r[4];
+    asm("v_fma_mix_f32 %0, %1, %2, -%3 op_sel_hi:[0,0,1]" : "=v"(r[0]) : "v"(a), "s"(up), "v"(h0));
+    asm("v_fma_mix_f32 %0, %1, %2, -%3 op_sel:[0,0,1] op_sel_hi:[0,0,1]" : "=v"(r[1]) : "v"(b), "s"(up), "v"(h0));
+    asm("v_fma_mix_f32 %0, %1, %2, -%3 op_sel_hi:[0,0,1]" : "=v"(r[2]) : "v"(c), "s"(up), "v"(h1));
+    asm("v_fma_mix_f32 %0, %1, %2, -%3 op_sel:[0,0,1] op_sel_hi:[0,0,1]" : "=v"(r[3]) : "v"(d), "s"(up), "v"(h1));
+    lo = u32x2_t{f16_pair(r[0], r[1]), f16_pair(r[2], r[3])};
   }
 };
+// eight f16 values: the four of `a` and the four of `b`
+__device__ __forceinline__ f16x8_t f16x8_of(u32x2_t a, u32x2_t b) {
+  return __builtin_bit_cast(f16x8_t, (u32x4_t{a[0], a[1], b[0], b[1]}));
+}
+// 2^e, -126 <= e <= 127
+__device__ __forceinline__ float pow2(int e) { return __uint_as_float((uint32_t)(e + 127) << 23); }
+// twice in f16, -14 <= e <= 15
+__device__ __forceinline__ uint32_t f16_pow2(int e) { return (uint32_t)(e + 15) * 0x04000400u; }
 __device__ __forceinline__ float max_abs3(float m, float a, float b) {
   asm("v_max3_f32 %0, %0, |%1|, |%2|" : "+v"(m) : "v"(a), "v"(b));
   return m;
@@ -173,8 +197,6 @@ attn_ring_f32_kernel(F32Params fp) {
     const int qr = q0 + qi * F_Q + c < p.T ? q0 + qi * F_Q + c : p.T - 1;
     return reinterpret_cast<const float*>(p.q) + b * p.qs_b + h * p.qs_h + (int64_t)qr * p.qs_t;
   };
-  float minus_one = -1.f;
-  asm volatile("" : "+s"(minus_one));
   // ---- query c of a group, values 16 j + 4 g + i, pre-multiplied by scale * log2(e) ----
   f32x4_t qf[NJ];
   auto load_q = [&](int qi) __attribute__((always_inline)) {
@@ -183,28 +205,40 @@ attn_ring_f32_kernel(F32Params fp) {
     for (int j = 0; j < NJ; ++j) qf[j] = *reinterpret_cast<const f32x4_t*>(row + 16 * j + 4 * g) * p.scale_log2;
   };
   if (!SPLIT) load_q(0);
-  // ---- or in halves, values 32 j + 8 g + i, and by a power of two that brings the row's largest value to 2^10 .. 2^11; in
+  // ---- or in halves, values 32 j + 8 g + i, and by a power of two that brings the row's largest value to 2^14 .. 2^15; in
   // registers, or where there are several groups in LDS ----
-  Halves qs[NJ / 2];
-  float q_back[NQ];    // the power's inverse
-  float k_low = 0.f;   // smallest key value (below) that halves stand for
-  bool split = false;
+  // A key's halves are off by up to 2^-22 of it and by up to 2^-25 (half the smallest f16 number).  Under a query of norm Q_MOST
+  // the latter moves a logit by 2^-24 or so, as far as an exponential is off.  For larger queries keys are halved 2^K_UP times
+  // as large, and beyond that there are fp32 products: q x 1e3 and k / 1e3 in one channel gave errors of 2e-6, 1e6 of 2e-3,
+  // while the largest key of a few channels and keys stood for all (3 to 5e-7 now, as with fp32 products).
+  f16x8_t q_hi[NJ / 2], q_lo[NJ / 2];
+  float q_back[NQ];    // what undoes the queries' and the keys' scales
+  bool split = false, scale_keys = false;
   auto halve_q = [&](int qi, float& undo) __attribute__((always_inline)) {
     const float* row = query(qi);
-    float top = 0.f;
+    float top = 0.f, square = 0.f;
 #pragma unroll
     for (int j = 0; j < NJ; ++j) qf[j] = *reinterpret_cast<const f32x4_t*>(row + 32 * (j / 2) + 8 * g + 4 * (j & 1)) * p.scale_log2;
 #pragma unroll
-    for (int j = 0; j < NJ; ++j) top = max_abs3(max_abs3(top, qf[j][0], qf[j][1]), qf[j][2], qf[j][3]);
+    for (int j = 0; j < NJ; ++j) {
+      top = max_abs3(max_abs3(top, qf[j][0], qf[j][1]), qf[j][2], qf[j][3]);
+      square += (qf[j][0] * qf[j][0] + qf[j][1] * qf[j][1]) + (qf[j][2] * qf[j][2] + qf[j][3] * qf[j][3]);
+    }
     top = groups_max(top);
-    int e = 11 - __builtin_amdgcn_frexp_expf(top);
+    int e = 15 - __builtin_amdgcn_frexp_expf(top);
     e = e < 100 ? e : 100;
-    undo = top < 0x1p100f ? __builtin_amdgcn_ldexpf(1.f, -e) : INFINITY;
+    square = groups_sum(square);
+    undo = __builtin_amdgcn_ldexpf(1.f, -e);
+    if (!(square <= Q_MOST * Q_MOST)) undo = square <= Q_MOST * Q_MOST * pow2(2 * K_UP) ? -undo : INFINITY;   // (NaN: not halved)
 #pragma unroll
-    for (int j = 0; j < NJ; ++j)
+    for (int j = 0; j < NJ; ++j) qf[j] *= __builtin_amdgcn_ldexpf(1.f, e);
 #pragma unroll
-      for (int i = 0; i < 4; i += 2)
-        qs[j / 2].set(4 * (j & 1) + i, __builtin_amdgcn_ldexpf(qf[j][i], e), __builtin_amdgcn_ldexpf(qf[j][i + 1], e), minus_one);
+    for (int j = 0; j < NJ / 2; ++j) {
+      const Halves4 a(qf[2 * j][0], qf[2 * j][1], qf[2 * j][2], qf[2 * j][3]);
+      const Halves4 b(qf[2 * j + 1][0], qf[2 * j + 1][1], qf[2 * j + 1][2], qf[2 * j + 1][3]);
+      q_hi[j] = f16x8_of(a.hi, b.hi);
+      q_lo[j] = f16x8_of(a.lo, b.lo);
+    }
   };
   if (SPLIT && NQ == 1) halve_q(0, q_back[0]);
   if (SPLIT && NQ > 1 && wave >= 1 && wave <= NQ) {
@@ -213,21 +247,24 @@ attn_ring_f32_kernel(F32Params fp) {
     if (g == 0) back[(wave - 1) * F_Q + c] = undo;
 #pragma unroll
     for (int j = 0; j < NJ / 2; ++j) {
-      qsh[((wave - 1) * NJ + j) * 64 + lane] = qs[j].hi;
-      qsh[((wave - 1) * NJ + NJ / 2 + j) * 64 + lane] = qs[j].lo;
+      qsh[((wave - 1) * NJ + j) * 64 + lane] = q_hi[j];
+      qsh[((wave - 1) * NJ + NJ / 2 + j) * 64 + lane] = q_lo[j];
     }
   }
   __syncthreads();
   const int nvis = vis[WE_MAX_SLOTS + 1];
   if (SPLIT) {
-    float most = 0.f;
+    float most = -INFINITY, least = INFINITY;
 #pragma unroll
     for (int qi = 0; qi < NQ; ++qi) {
       if (NQ > 1) q_back[qi] = back[qi * F_Q + c];
       most = fmaxf(most, q_back[qi]);
+      least = fminf(least, q_back[qi]);
     }
     split = __ballot(!(most < INFINITY)) == 0ull;
-    k_low = __ballot(most > 0x1p-10f) == 0ull ? 0.f : 0.25f;   // (a row's largest value below 2, 1 on average)
+    scale_keys = __ballot(least < 0.f) != 0ull;
+#pragma unroll
+    for (int qi = 0; qi < NQ; ++qi) q_back[qi] = __builtin_fabsf(q_back[qi]) * (scale_keys ? pow2(-K_UP) : 1.f);
   }
 
   f32x4_t o[NQ][NH][4];  // o[qi][hh][e] register i: query c of group qi, value 64 hh + 16 g + 4 i + e
@@ -393,15 +430,8 @@ attn_ring_f32_kernel(F32Params fp) {
     load_rows(at);
     load_values(at);
     // The rest of a rounded value is off by up to 2^-22 of it and by up to 2^-25 (the smallest f16 numbers): next to values
-    // of 1/8 and more that is less than what an fp32 sum over them loses, for the keys so long as the queries are not large.
+    // of 1/8 and more that is less than what an fp32 sum over them loses.
     // (Values too large for f16 are infinite and their rest the other infinity: what they meet is no number, at the end.)
-    auto keys_fit = [&]() __attribute__((always_inline)) {
-      if (k_low == 0.f) return true;
-      float top = 0.f;
-#pragma unroll
-      for (int j = 0; j < NJ; ++j) top = max_abs3(max_abs3(top, kf[j][0], kf[j][1]), kf[j][2], kf[j][3]);
-      return __ballot(top < k_low) == 0ull;
-    };
     auto values_fit = [&]() __attribute__((always_inline)) {
       float top = 0.f;
 #pragma unroll
@@ -413,13 +443,19 @@ attn_ring_f32_kernel(F32Params fp) {
     f32x4_t s[NQ];
     int keys = 0;
     auto logits = [&](auto more) __attribute__((always_inline)) {
+      auto to_lds = [&](int j, auto scaled) __attribute__((always_inline)) {
+        const f32x4_t r = kf[j];
+        const Halves4 x = decltype(scaled)::value ? Halves4(r[0], r[1], r[2], r[3], pow2(K_UP), f16_pow2(K_UP))
+                                                  : Halves4(r[0], r[1], r[2], r[3]);
+        *reinterpret_cast<u32x2_t*>(k_to + RPL * j * Lds::KROW) = x.hi;
+        *reinterpret_cast<u32x2_t*>(k_to + (F_K + RPL * j) * Lds::KROW) = x.lo;
+      };
+      if (scale_keys) {
 #pragma unroll
-      for (int j = 0; j < NJ; ++j) {
-        Halves x;
-        x.set(0, kf[j][0], kf[j][1], minus_one);
-        x.set(2, kf[j][2], kf[j][3], minus_one);
-        *reinterpret_cast<f16x4_t*>(k_to + RPL * j * Lds::KROW) = f16x4_t{x.hi[0], x.hi[1], x.hi[2], x.hi[3]};
-        *reinterpret_cast<f16x4_t*>(k_to + (F_K + RPL * j) * Lds::KROW) = f16x4_t{x.lo[0], x.lo[1], x.lo[2], x.lo[3]};
+        for (int j = 0; j < NJ; ++j) to_lds(j, std::true_type());
+      } else {
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) to_lds(j, std::false_type());
       }
       asm volatile("" ::: "memory");
       keys = at.last + 1;   // (16 or more: a whole block)
@@ -432,17 +468,16 @@ attn_ring_f32_kernel(F32Params fp) {
       for (int qi = 0; qi < NQ; ++qi) sl[qi] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int j = 0; j < NJ / 2; ++j) {
-        Halves x;
-        x.hi = *reinterpret_cast<const f16x8_t*>(k_from + 64 * j);
-        x.lo = *reinterpret_cast<const f16x8_t*>(k_from + F_K * Lds::KROW + 64 * j);
+        const f16x8_t k_hi = *reinterpret_cast<const f16x8_t*>(k_from + 64 * j);
+        const f16x8_t k_lo = *reinterpret_cast<const f16x8_t*>(k_from + F_K * Lds::KROW + 64 * j);
 #pragma unroll
         for (int qi = 0; qi < NQ; ++qi) {
-          const f16x8_t q_hi = NQ > 1 ? qsh[(qi * NJ + j) * 64 + lane_q] : qs[j].hi;
-          const f16x8_t q_lo = NQ > 1 ? qsh[(qi * NJ + NJ / 2 + j) * 64 + lane_q] : qs[j].lo;
-          sh[qi][j] = F16Mma::mma16(x.hi, q_hi, f32x4_t{0.f, 0.f, 0.f, 0.f});
-          sl[qi] = F16Mma::mma16(x.lo, q_lo, sl[qi]);
-          sl[qi] = F16Mma::mma16(x.lo, q_hi, sl[qi]);
-          sl[qi] = F16Mma::mma16(x.hi, q_lo, sl[qi]);
+          const f16x8_t qh = NQ > 1 ? qsh[(qi * NJ + j) * 64 + lane_q] : q_hi[j];
+          const f16x8_t ql = NQ > 1 ? qsh[(qi * NJ + NJ / 2 + j) * 64 + lane_q] : q_lo[j];
+          sh[qi][j] = F16Mma::mma16(k_hi, qh, f32x4_t{0.f, 0.f, 0.f, 0.f});
+          sl[qi] = F16Mma::mma16(k_lo, ql, sl[qi]);
+          sl[qi] = F16Mma::mma16(k_lo, qh, sl[qi]);
+          sl[qi] = F16Mma::mma16(k_hi, ql, sl[qi]);
         }
         if (NQ > 1) __builtin_amdgcn_sched_barrier(0);
       }
@@ -475,7 +510,7 @@ attn_ring_f32_kernel(F32Params fp) {
             for (int hh = 0; hh < NH; ++hh) vf[i][hh] = f32x4_t{0.f, 0.f, 0.f, 0.f};
           }
       }
-      Halves ps[NQ];
+      f16x8_t p_hi[NQ], p_lo[NQ];
 #pragma unroll
       for (int qi = 0; qi < NQ; ++qi) {
         // (o and l_run are relative to m_run, P_LOW to P_HIGH below the largest logit: probabilities are up to 2^15)
@@ -493,31 +528,20 @@ attn_ring_f32_kernel(F32Params fp) {
 #pragma unroll
         for (int i = 0; i < 4; ++i) pr[i] = __builtin_amdgcn_exp2f(s[qi][i] - m_run[qi]);
         l_run[qi] += (pr[0] + pr[1]) + (pr[2] + pr[3]);
-        ps[qi].set(0, pr[0], pr[1], minus_one);
-        ps[qi].set(2, pr[2], pr[3], minus_one);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          ps[qi].hi[4 + i] = ps[qi].hi[i];
-          ps[qi].lo[4 + i] = ps[qi].lo[i];
-        }
+        const Halves4 x(pr[0], pr[1], pr[2], pr[3]);
+        p_hi[qi] = f16x8_of(x.hi, x.hi);
+        p_lo[qi] = f16x8_of(x.lo, x.lo);
       }
 #pragma unroll
       for (int hh = 0; hh < NH; ++hh) {
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          f16x8_t v;   // value 64 hh + 4 c + e of the lane's four keys: rounded, and the rest
-#pragma unroll
-          for (int i = 0; i < 4; i += 2) {
-            Halves x;
-            x.set(0, vf[i][hh][e], vf[i + 1][hh][e], minus_one);
-            v[i] = x.hi[0];
-            v[i + 1] = x.hi[1];
-            v[4 + i] = x.lo[0];
-            v[5 + i] = x.lo[1];
-          }
+          // value 64 hh + 4 c + e of the lane's four keys: rounded, and the rest
+          const Halves4 x(vf[0][hh][e], vf[1][hh][e], vf[2][hh][e], vf[3][hh][e]);
+          const f16x8_t v = f16x8_of(x.hi, x.lo);
 #pragma unroll
           for (int qi = 0; qi < NQ; ++qi) {
-            const f32x4_t d = F16Mma::mma16(v, ps[qi].hi, F16Mma::mma16(v, ps[qi].lo, f32x4_t{0.f, 0.f, 0.f, 0.f}));
+            const f32x4_t d = F16Mma::mma16(v, p_hi[qi], F16Mma::mma16(v, p_lo[qi], f32x4_t{0.f, 0.f, 0.f, 0.f}));
 #pragma unroll
             for (int i = 0; i < 4; ++i) o[qi][hh][e][i] += d[i];
           }
@@ -529,9 +553,8 @@ attn_ring_f32_kernel(F32Params fp) {
     };
     // (one way out, at the end: with two the compiler copies o from one set of registers to another in every block)
     auto block_of_halves = [&](auto more) __attribute__((always_inline)) {
-      const bool fit = keys_fit();
       logits(more);
-      const bool good = fit && values_fit();
+      const bool good = values_fit();
       if (good) outputs();
       if (decltype(more)::value) load_values(at);   // (either way: the keys' requests are counted from here)
       return good;
