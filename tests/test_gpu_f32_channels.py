@@ -47,3 +47,47 @@ def test_large_queries_meet_small_keys(gpu_device, shape, factor):
     whole, channel, row = _errors(gpu_device, shape, change)
     print(f"f32 channels {shape} q x {factor:g}: {whole:.2e}, channel {channel:.2e}, row {row:.2e}", flush=True)
     assert whole <= REL and channel <= REL_ONE and row <= REL_ONE
+
+
+@pytest.mark.parametrize("shape", SHAPES)
+@pytest.mark.parametrize("factor", [1e-2, 1e-4, 1e-6, 1e-12, 1e3])
+def test_one_channel_of_small_values(gpu_device, shape, factor):
+    whole, channel, row = _errors(gpu_device, shape, lambda q, k, v: v[..., 5].mul_(factor))
+    print(f"f32 channels {shape} v x {factor:g}: {whole:.2e}, channel {channel:.2e}, row {row:.2e}", flush=True)
+    assert whole <= REL and channel <= REL_ONE
+    assert row <= REL_ONE or factor > 1   # (a channel that is nearly all of a row, and whose sum may be next to nothing)
+
+
+# (Every query looks at one key, with a logit of `logit` units where the others have ones of 1 or so; its values are `factor` times the
+# others'.  A logit's own rounding, 2^-24 of it for every one of a few sums, goes into the probabilities of the keys that are left
+# over: eight times the bound above for 30.)
+@pytest.mark.parametrize("shape", SHAPES)
+@pytest.mark.parametrize("logit", [6.0, 12.0, 20.0])
+@pytest.mark.parametrize("factor", [1.0, 1e-2, 1e-4, 1e-6, 1e-8])
+def test_one_key_that_every_query_looks_at(gpu_device, shape, logit, factor):
+    T, Dh = shape[3:5]
+    unit = torch.randn(Dh, device=gpu_device, generator=torch.Generator(gpu_device).manual_seed(1))
+    unit /= unit.norm()
+
+    def change(q, k, v):
+        q.add_(8 * unit)
+        k[..., T + 7, :] = unit * (logit * math.sqrt(Dh) / 8)
+        v[..., T + 7, :] *= factor
+
+    whole, channel, row = _errors(gpu_device, shape, change)
+    print(f"f32 channels {shape} key of logit {logit:g}, v x {factor:g}: {whole:.2e}, channel {channel:.2e}, row {row:.2e}", flush=True)
+    assert whole <= 2 * REL and row <= 2 * REL_ONE
+
+
+@pytest.mark.parametrize("shape", SHAPES)
+@pytest.mark.parametrize("frame,factor", [(0, 0.0), (0, 1e-4), (0, 10.0), (1, 0.0), (1, 50.0), (None, 0.05), (None, 1e-3), (None, 1e3)])
+def test_frames_of_other_sizes(gpu_device, shape, frame, factor):
+    """The first visible frame, whose values the scale is chosen for, or the next one; or all."""
+    T = shape[3]
+
+    def change(q, k, v):
+        (v if frame is None else v[:, :, frame * T:(frame + 1) * T]).mul_(factor)
+
+    whole, channel, row = _errors(gpu_device, shape, change)
+    print(f"f32 channels {shape} v x {factor:g} in {frame}: {whole:.2e}, channel {channel:.2e}, row {row:.2e}", flush=True)
+    assert whole <= REL and channel <= REL_ONE and row <= REL_ONE

@@ -1,39 +1,38 @@
 // fp32 attention over the KV ring buffer (gfx950): the same visibility rule and ring walk as the
-// half-precision kernel (attn_ring.hip), of fp32 precision throughout (scores, softmax and P V,
-// src/model/attn.py:116 in eager mode).
+// half-precision kernel (attn_ring.hip), scores, softmax and P V as exact as fp32 products and sums make them
+// (src/model/attn.py:116 in eager mode).
 //
 // One workgroup = one or two groups of 16 queries of one (batch, head) and NW wavefronts that share out its keys: blocks
 // of 16 keys go round the wavefronts, each keeps its own running (reference, sum, O) and they merge
 // through LDS at the end.  A wavefront's keys are nobody else's, so K and V go from memory straight
 // into registers, one block ahead, without a barrier in the loop.
 //
-// Most blocks go through the f16 matrix instructions, sixteen times the fp32 ones' rate, as sums of two
+// Most products go through the f16 matrix instructions, sixteen times the fp32 ones' rate, as sums of two
 // halves (x = hi + lo, 22 bits; four products per pair).  S^T = K Q^T: K comes row by row - whole lines; read
 // in the operands' layout every request touches 64 of them - and changes places between the lanes through the
 // wavefront's own 8 KB of LDS, halved.  O^T += V^T P^T: the S^T accumulators are the B operand as they are (lane
 // group g, register i = key 4 g + i), and one instruction's 32 places take 16 keys' hi and lo of V.  What a
 // product of these instructions adds is cut off at the last bit of the largest one in its group of eight, and
 // so is the sum it is carried into where that is smaller: the large products of S start from zero each and
-// O's are added by the vector unit, so that no chain of products loses more than its own size.  Relative
-// error against 64 bits, fp32 products / halves: 16 heads of 128, 2048 keys 3.9e-7 / 3.0e-7, 8 heads, 4096
-// keys 6.3e-7 / 3.4e-7, 4 heads, 128 keys 2.3e-7 / 2.2e-7; heads of 64, 2880 keys 5.2e-7 / 3.2e-7, 1024 keys
-// 2.9e-7 / 2.8e-7, but 512 keys 2.4e-7 / 2.6e-7: their short contexts stay with fp32 products (F32Call::halves_from).
-// Halves hold keys and values of a certain size only.  For the keys the queries' size tells (below); each wavefront looks at its
-// values as they come and goes on with fp32 products where they do not fit.
+// O's are added by the vector unit, so that no chain of products loses more than its own size.  f16 numbers
+// have a smallest step: what is halved is scaled so that its halves are 22 bits (2^-21 at worst) of every single key,
+// value and probability that counts, or goes through fp32 products (queries, values and probabilities below).
+// Relative error against 64 bits, fp32 products / halves, normal inputs: 16 heads of 128, 2048 keys 3.9e-7 / 2.3e-7, 8 heads,
+// 4096 keys 6.3e-7 / 2.7e-7, 4 heads, 128 keys 2.5e-7 / 1.8e-7; heads of 64, 2880 keys 5.2e-7 / 2.6e-7, 1024 keys 2.9e-7 / 2.1e-7.
 //
 // Blocks through v_mfma_f32_16x16x4_f32: the contraction of S is taken in an order that lets a lane load four of its
 // head-dim values at once (lane group g of step (j, i) has value 16 j + 4 g + i of both operands), and output rows
 // are numbered so that a lane's four values of V are consecutive: one 16-byte load per key and 64 head-dim values.
 //
 // Bound by the vector unit and the trips through LDS: at 16 queries a workgroup every CU halves all of its unit's keys and
-// values itself, 128 of some 270 vector instructions per block and wavefront (57 % of the time they issue, 32 f16 MFMAs of 16
-// cycles beside them; a request for V a whole block ahead, into registers of its own, changes nothing).  Where that is more
-// than a workgroup a CU, two groups share what is halved (some 340 instructions for both; the queries' halves in LDS then).
-// us, fp32 products / halves / of two groups: 16 heads of 128, 256 queries, 2048 keys 49.5 / 40.4 (106 TFLOP/s), 8 heads, 1024
-// queries, 4096 keys 156 / 126 / 103 (167 TFLOP/s, where a large fp32 matrix product reaches 153), 24 heads of 64 on 8, 720
-// queries, 2880 keys 140 / 107 / 99.7, 16 heads, 272 queries, 2176 keys - / 63.5 / 52.8, 8 heads of 128, 64 queries, 512 keys 17.0 /
-// 12.5, 4 heads, 128 keys 9.0 / 7.9 (the loads' addresses in vector registers, o copied at a way out in mid-block and
-// a check of every key's size cost another 44.3, 133, 120, -, 13.2, 8.0).  Values that halves do not hold: 49 -> 52 for the first shape.
+// values itself, half of a block's vector instructions.  Where that is more than a workgroup a CU, two groups share what is
+// halved (some 370 instructions a block for both, which issue 60 % of the time of 8 heads, 1024 queries, 4096 keys, beside 64
+// f16 MFMAs of 16 cycles, 33 %).  us in one pass, fp32 products / halves: 16 heads of 128, 256 queries, 2048 keys 44.9 / 36.1 (119
+// TFLOP/s), 8 heads of 128, 64 queries, 512 keys 17.0 / 13.5, 4 heads, 128 keys 9.0 / 8.7; of two groups: 8 heads, 1024 queries, 4096
+// keys 151 / 94 (183 TFLOP/s, where a large fp32 matrix product reaches 153), 24 heads of 64 on 8, 720 queries, 2880 keys 136 / 99,
+// 16 heads, 272 queries, 2176 keys 83 / 50.7.  Other inputs, first and fourth shape: values of standard deviation 0.05 36.9 and
+// 96, queries of 30 37.1 and 96; queries of 1e4 in one channel, which take fp32 products, 46.9 and 156; values above 65504,
+// for which a wavefront does everything a second time, 71 and 225.
 #include <type_traits>
 
 #include "attn_mma.h"
@@ -47,9 +46,10 @@ namespace we {
 namespace {
 constexpr int F_Q = 16;   // queries of a group
 constexpr int F_K = 16;   // keys per block
-constexpr float P_LOW = 10.f, P_HIGH = 15.f;   // exponents of split probabilities
 constexpr int K_UP = 5;          // exponent of the scale for the keys of large queries
 constexpr float Q_MOST = 4.f;    // 2-norm of a query, times scale * log2(e) (normalised queries: 1.44)
+constexpr int P_UP = 15;         // exponent of the scale for a block's probabilities
+constexpr float M_SLACK = 8.f;   // how far above the running reference a logit may be
 
 // NQ: groups of queries per workgroup
 template <int DH, int NW, int NQ, bool SPLIT>
@@ -128,6 +128,19 @@ __device__ __forceinline__ uint32_t f16_pow2(int e) { return (uint32_t)(e + 15) 
 __device__ __forceinline__ float max_abs3(float m, float a, float b) {
   asm("v_max3_f32 %0, %0, |%1|, |%2|" : "+v"(m) : "v"(a), "v"(b));
   return m;
+}
+__device__ __forceinline__ float min_abs3(float m, float a, float b) {
+  asm("v_min3_f32 %0, %0, |%1|, |%2|" : "+v"(m) : "v"(a), "v"(b));
+  return m;
+}
+// the largest x >= 0 of a wavefront
+template <int ROR>
+__device__ __forceinline__ float max_ror(float x) {
+  return fmaxf(x, __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), 0x120 | ROR, 0xf, 0xf, false)));
+}
+__device__ __forceinline__ float wave_max(float x) {
+  x = max_ror<1>(max_ror<2>(max_ror<4>(max_ror<8>(groups_max(x)))));
+  return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(x)));
 }
 
 // WHOLE: T % 16 == 0, every block has 16 keys (a separate instance: what the others work out per request is a tenth of a
@@ -429,18 +442,37 @@ attn_ring_f32_kernel(F32Params fp) {
     Place at = place(0);
     load_rows(at);
     load_values(at);
-    // The rest of a rounded value is off by up to 2^-22 of it and by up to 2^-25 (the smallest f16 numbers): next to values
-    // of 1/8 and more that is less than what an fp32 sum over them loses.
-    // (Values too large for f16 are infinite and their rest the other infinity: what they meet is no number, at the end.)
-    auto values_fit = [&]() __attribute__((always_inline)) {
+    // Values are halved 2^e times as large, which brings the largest of a wavefront's first block to 2^12 .. 2^13 (e up to 13:
+    // should that block be empty, the next may have values of 8).  Halves are then off by up to 2^-22 of a value and by up to
+    // 2^-25, which is 2^-21 of 2^-4.  Tiles of 16 keys and 16 channels with a smaller value take fp32 products, one block in twenty of
+    // normal values has one.  By value: an output channel is a sum over keys only, and nearly all weight may be on one of them.
+    // While the largest of a lane's values stood for all, a channel times 1e-4 was off by 3e-4 of itself, a row that looks at
+    // one key with values times 1e-4 by 2e-4 (4e-7 to 1e-6 and 5e-7 to 2e-6 now, as with fp32 products).
+    // (Keys and values too large for f16 are infinite and their rest the other infinity: what they meet is no number, at the end.)
+    float v_up = 0.f, v_back = 0.f, v_low = 0.f;
+    uint32_t v_up16 = 0;
+    auto scale_values = [&]() __attribute__((always_inline)) {
       float top = 0.f;
 #pragma unroll
       for (int i = 0; i < 4; ++i)
 #pragma unroll
         for (int hh = 0; hh < NH; ++hh) top = max_abs3(max_abs3(top, vf[i][hh][0], vf[i][hh][1]), vf[i][hh][2], vf[i][hh][3]);
-      return __ballot(top < 0.125f) == 0ull;
+      int e = 139 - (int)(__float_as_uint(wave_max(top)) >> 23);
+      e = e < -14 ? -14 : (e > 13 ? 13 : e);
+      v_up = pow2(e);
+      v_up16 = f16_pow2(e);
+      v_back = pow2(-e - P_UP);
+      v_low = pow2(-e - 4);
     };
-    f32x4_t s[NQ];
+    auto values_fit = [&]() __attribute__((always_inline)) {
+      float least = INFINITY;
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int hh = 0; hh < NH; ++hh) least = min_abs3(min_abs3(least, vf[i][hh][0], vf[i][hh][1]), vf[i][hh][2], vf[i][hh][3]);
+      return __ballot(least < v_low) == 0ull;
+    };
+    f32x4_t s[NQ];   // logits / q_back
     int keys = 0;
     auto logits = [&](auto more) __attribute__((always_inline)) {
       auto to_lds = [&](int j, auto scaled) __attribute__((always_inline)) {
@@ -450,7 +482,7 @@ attn_ring_f32_kernel(F32Params fp) {
         *reinterpret_cast<u32x2_t*>(k_to + RPL * j * Lds::KROW) = x.hi;
         *reinterpret_cast<u32x2_t*>(k_to + (F_K + RPL * j) * Lds::KROW) = x.lo;
       };
-      if (scale_keys) {
+      if (__builtin_expect(scale_keys, 0)) {
 #pragma unroll
         for (int j = 0; j < NJ; ++j) to_lds(j, std::true_type());
       } else {
@@ -488,35 +520,32 @@ attn_ring_f32_kernel(F32Params fp) {
       }
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int qi = 0; qi < NQ; ++qi) {
-        float undo = q_back[qi];
-        asm volatile("" : "+v"(undo));
+      for (int qi = 0; qi < NQ; ++qi)
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           s[qi][i] = sh[qi][0][i] + sh[qi][1][i];
           if (NJ == 8) s[qi][i] += sh[qi][NJ / 2 - 2][i] + sh[qi][NJ / 2 - 1][i];
-          s[qi][i] = (s[qi][i] + sl[qi][i]) * undo;
+          s[qi][i] += sl[qi][i];
         }
-      }
     };
     auto outputs = [&]() __attribute__((always_inline)) {
-      if (!WHOLE && keys < F_K) {  // missing keys: no weight, and nothing for a zero weight to meet but zeros
+      if (!WHOLE && keys < F_K) {  // missing keys: no weight (their values are the last key's)
 #pragma unroll
         for (int i = 0; i < 4; ++i)
-          if (4 * g + i >= keys) {
 #pragma unroll
-            for (int qi = 0; qi < NQ; ++qi) s[qi][i] = -INFINITY;
-#pragma unroll
-            for (int hh = 0; hh < NH; ++hh) vf[i][hh] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-          }
+          for (int qi = 0; qi < NQ; ++qi) s[qi][i] = 4 * g + i < keys ? s[qi][i] : -INFINITY;
       }
-      f16x8_t p_hi[NQ], p_lo[NQ];
+      // Probabilities are relative to the block's largest (and near 1 lose nothing in the exponent's subtraction), of which their halves are off
+      // by up to 2^-40: the keys next to one that has nearly all weight, but no value to speak of, keep their bits.  `part`
+      // takes the block's sums to the running reference.
+      const bool fit = values_fit();
+      f32x4_t pr[NQ];
+      float part[NQ];
 #pragma unroll
       for (int qi = 0; qi < NQ; ++qi) {
-        // (o and l_run are relative to m_run, P_LOW to P_HIGH below the largest logit: probabilities are up to 2^15)
-        const float top = groups_max(fmaxf(fmaxf(s[qi][0], s[qi][1]), fmaxf(s[qi][2], s[qi][3])));
-        if (__ballot(top > m_run[qi] + P_HIGH) != 0ull) {
-          const float mx = fmaxf(m_run[qi], top - P_LOW), alpha = __builtin_amdgcn_exp2f(m_run[qi] - mx);  // 0 on the first block
+        const float top = groups_max(fmaxf(fmaxf(s[qi][0], s[qi][1]), fmaxf(s[qi][2], s[qi][3]))) * q_back[qi];
+        if (__ballot(top > m_run[qi] + M_SLACK) != 0ull) {
+          const float mx = fmaxf(m_run[qi], top), alpha = __builtin_amdgcn_exp2f(m_run[qi] - mx);  // 0 on the first block
           l_run[qi] *= alpha;
 #pragma unroll
           for (int hh = 0; hh < NH; ++hh)
@@ -524,26 +553,50 @@ attn_ring_f32_kernel(F32Params fp) {
             for (int e = 0; e < 4; ++e) o[qi][hh][e] *= alpha;
           m_run[qi] = mx;
         }
-        f32x4_t pr;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) pr[i] = __builtin_amdgcn_exp2f(s[qi][i] - m_run[qi]);
-        l_run[qi] += (pr[0] + pr[1]) + (pr[2] + pr[3]);
-        const Halves4 x(pr[0], pr[1], pr[2], pr[3]);
+        for (int i = 0; i < 4; ++i) pr[qi][i] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[qi][i], q_back[qi], -top));
+        part[qi] = __builtin_amdgcn_exp2f(top - m_run[qi]);
+        l_run[qi] += ((pr[qi][0] + pr[qi][1]) + (pr[qi][2] + pr[qi][3])) * part[qi];
+      }
+      if (__builtin_expect(!fit, 0)) {   // (then zeros to the products below: a branch around them would move o from registers to registers)
+        f32x4_t w[NQ];
+#pragma unroll
+        for (int qi = 0; qi < NQ; ++qi) w[qi] = pr[qi] * part[qi];
+#pragma unroll
+        for (int hh = 0; hh < NH; ++hh)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const float least = min_abs3(min_abs3(INFINITY, vf[0][hh][e], vf[1][hh][e]), vf[2][hh][e], vf[3][hh][e]);
+            if (__ballot(least < v_low) != 0ull) {
+#pragma unroll
+              for (int i = 0; i < 4; ++i) {
+#pragma unroll
+                for (int qi = 0; qi < NQ; ++qi) o[qi][hh][e] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[i][hh][e], w[qi][i], o[qi][hh][e], 0, 0, 0);
+                vf[i][hh][e] = 0.f;
+              }
+            }
+          }
+      }
+      f16x8_t p_hi[NQ], p_lo[NQ];
+#pragma unroll
+      for (int qi = 0; qi < NQ; ++qi) {
+        const Halves4 x(pr[qi][0], pr[qi][1], pr[qi][2], pr[qi][3], pow2(P_UP), f16_pow2(P_UP));
         p_hi[qi] = f16x8_of(x.hi, x.hi);
         p_lo[qi] = f16x8_of(x.lo, x.lo);
+        part[qi] *= v_back;
       }
 #pragma unroll
       for (int hh = 0; hh < NH; ++hh) {
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
           // value 64 hh + 4 c + e of the lane's four keys: rounded, and the rest
-          const Halves4 x(vf[0][hh][e], vf[1][hh][e], vf[2][hh][e], vf[3][hh][e]);
+          const Halves4 x(vf[0][hh][e], vf[1][hh][e], vf[2][hh][e], vf[3][hh][e], v_up, v_up16);
           const f16x8_t v = f16x8_of(x.hi, x.lo);
 #pragma unroll
           for (int qi = 0; qi < NQ; ++qi) {
             const f32x4_t d = F16Mma::mma16(v, p_hi[qi], F16Mma::mma16(v, p_lo[qi], f32x4_t{0.f, 0.f, 0.f, 0.f}));
 #pragma unroll
-            for (int i = 0; i < 4; ++i) o[qi][hh][e][i] += d[i];
+            for (int i = 0; i < 4; ++i) o[qi][hh][e][i] += d[i] * part[qi];
           }
         }
       }
@@ -551,17 +604,14 @@ attn_ring_f32_kernel(F32Params fp) {
       __builtin_amdgcn_sched_barrier(0);
       ++k;
     };
-    // (one way out, at the end: with two the compiler copies o from one set of registers to another in every block)
     auto block_of_halves = [&](auto more) __attribute__((always_inline)) {
       logits(more);
-      const bool good = values_fit();
-      if (good) outputs();
-      if (decltype(more)::value) load_values(at);   // (either way: the keys' requests are counted from here)
-      return good;
+      if (k == 0) scale_values();
+      outputs();
+      if (decltype(more)::value) load_values(at);
     };
-    bool good = true;
-    while (good && k + 1 < mine_n) good = block_of_halves(std::true_type());
-    if (good) block_of_halves(std::false_type());
+    while (k + 1 < mine_n) block_of_halves(std::true_type());
+    block_of_halves(std::false_type());
     float all = 0.f;
 #pragma unroll
     for (int qi = 0; qi < NQ; ++qi) {
@@ -574,22 +624,11 @@ attn_ring_f32_kernel(F32Params fp) {
     if (__ballot(!(__builtin_fabsf(all) < INFINITY)) != 0ull) {  // all of it once more
       k = 0;
       nothing_yet();
-    } else if (k < mine_n) {  // (the blocks below may have values that 2^15 times as much of would be too much)
-      const float less = __builtin_amdgcn_exp2f(-P_LOW);
-#pragma unroll
-      for (int qi = 0; qi < NQ; ++qi) {
-        m_run[qi] += P_LOW;
-        l_run[qi] *= less;
-#pragma unroll
-        for (int hh = 0; hh < NH; ++hh)
-#pragma unroll
-          for (int e = 0; e < 4; ++e) o[qi][hh][e] *= less;
-      }
     }
   }
 
-  // ---- the others ----
-  auto others = [&](auto group, int from) __attribute__((always_inline)) {
+  // ---- or all blocks through fp32 products ----
+  auto others = [&](auto group) __attribute__((always_inline)) {
     if (SPLIT) load_q(decltype(group)::value);
     f32x4_t ka[NJ], va[4][NH], kb[NJ], vb[4][NH];
     // The loop always requests the next block - behind a branch the compiler counts the loads in flight as if it had
@@ -597,9 +636,8 @@ attn_ring_f32_kernel(F32Params fp) {
     // requested a second time, for nothing, costs wavefronts with one or two of them most: attention alone, 4 heads of 128,
     // 64 queries, 128 keys 9.8 -> 8.75 us, 8 heads, 256 keys 12.25 -> 11.4, 8 heads of 64, 256 keys 7.64 -> 7.40, 128 keys
     // 6.43 -> 6.11.)
-    int k = from;
-    int keys_a = fetch(ka, va, k);
-    ++k;
+    int k = 1;
+    int keys_a = fetch(ka, va, 0);
     for (; k + 1 < mine_n; k += 2) {
       const int keys_b = fetch(kb, vb, k);
       block(group, ka, va, keys_a);
@@ -615,8 +653,8 @@ attn_ring_f32_kernel(F32Params fp) {
     }
   };
   if (k < mine_n) {
-    others(std::integral_constant<int, 0>(), k);
-    if constexpr (NQ > 1) others(std::integral_constant<int, 1>(), k);
+    others(std::integral_constant<int, 0>());
+    if constexpr (NQ > 1) others(std::integral_constant<int, 1>());
   }
 
   // ---- the wavefronts merge ----

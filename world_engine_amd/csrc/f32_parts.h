@@ -5,10 +5,9 @@
 // two groups share what the rounds halve (attn_ring_f32.hip).  Where they do not, a context in parts fills the CUs - or the
 // CUs take two groups of queries each and a part of the keys - at the price of a second pass over the parts' rows.
 // The cost is a fit to single calls; parts are taken where it says 7 % less.  us, one pass / parts: 2 heads of 128, 64 tokens, 64
-// slots 55.4 / 15.1 (16 parts), 2 heads, 256 tokens, 16 slots 56.2 / 20.4, 4 heads, 128 tokens, 16 slots 32.4 / 14.5, 8 heads,
-// 256 tokens, 8 slots 33.4 / 24.9, 16 heads 41.5 / 39.3, 8 heads, 64 tokens, 8 slots 12.6 / 11.1; heads of 64: 3 of 100 tokens, 40
-// slots 41.2 / 16.6, 8 of 64 tokens, 16 slots 12.5 / 10.1.  Over 39 of 70 drawn shapes that take parts 0.66 of the time on
-// average, 0.98 at worst.
+// slots 58.2 / 15.5 (16 parts), 2 heads, 256 tokens, 16 slots 58.8 / 20.3, 4 heads, 128 tokens, 16 slots 33.7 / 15.0, 8 heads,
+// 256 tokens, 8 slots 33.2 / 23.6, 16 heads 36.1 / 34.8, 8 heads, 64 tokens, 8 slots 13.5 / 11.5; heads of 64: 3 of 100 tokens, 40
+// slots 43.0 / 16.4, 8 of 64 tokens, 16 slots 13.3 / 10.5.  (The fit is from halves that took 3 to 6 % less.)
 #pragma once
 
 #include <stdint.h>
@@ -25,7 +24,9 @@ struct F32Call {
 
   int64_t tiles(int g) const { return heads * ((T + 16 * g - 1) / (16 * g)); }
   int64_t blocks() const { return slots * ((T + 15) / 16); }
-  // keys from which on a call's halves are as exact as fp32 products in one chain per wavefront
+  // Blocks of keys from which on a call's products go in halves.  (The lines for heads of 64 are from halves that were less exact
+  // than fp32 products in one short chain per wavefront, 512 keys 2.6e-7 against 2.45e-7.  The present ones are at 1.9e-7 there
+  // and faster from some 24 blocks on, 512 keys 10.3 -> 9.6 us, but 128 keys 6.4 -> 6.75.)
   int64_t halves_from() const { return dh == 64 ? (tiles(1) > cus ? 32 : 64) : 1; }
   int64_t row_bytes() const { return (int64_t)dh * 4 + 8; }
   int64_t bytes(int p) const { return p > 1 ? heads * T * p * row_bytes() : 0; }
