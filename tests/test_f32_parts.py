@@ -41,6 +41,63 @@ def test_parts_and_groups(tmp_path):
     assert cases > 1000 and wrong == 0
 
 
+LAUNCHED = r"""
+#include <cstdio>
+#include <cstring>
+#include <initializer_list>
+#include "attn_plan.h"
+
+static int parts, groups;
+namespace we {
+hipError_t launch_attn_ring_f32(const AttnParams& p, int, int q_groups, int, hipStream_t) {
+  parts = p.n_splits;
+  groups = q_groups;
+  return hipSuccess;
+}
+#define OTHER(name, ...) hipError_t name(const AttnParams&, __VA_ARGS__, hipStream_t) { return hipErrorUnknown; }
+OTHER(launch_attn_ring_bf16_128, int) OTHER(launch_attn_ring_bf16_64, int) OTHER(launch_attn_ring_f16_128, int) OTHER(launch_attn_ring_f16_64, int)
+OTHER(launch_attn_ring_short_bf16, int, int) OTHER(launch_attn_ring_short_f16, int, int) OTHER(launch_attn_ring_shared_bf16, int, int)
+OTHER(launch_attn_ring_shared_f16, int, int) OTHER(launch_attn_combine, int, int)
+}
+
+int main() {
+  long cases = 0, wrong = 0, less = 0;
+  const int64_t st[3] = {1 << 20, 1 << 10, 128};
+  uint8_t* at = reinterpret_cast<uint8_t*>(4096);   // (no memory is touched)
+  int64_t* t_pos = reinterpret_cast<int64_t*>(at);
+  for (int heads : {1, 2, 3, 8, 16, 40}) for (int T : {16, 33, 64, 256}) for (int slots : {2, 8, 16, 64}) for (int dh : {64, 128})
+    for (int d : {1, 2}) for (int share : {0, 16, 8, 4, 2, 1}) for (int splits : {0, 1}) {
+      we::F32Call want = {heads, T, slots / d, dh, 256};
+      want.plan(INT64_MAX);
+      const int64_t all = want.bytes(want.parts), given = share ? all / share : 0;
+      want.plan(splits ? 0 : given);
+      we::AttnParams p;
+      we::host::AttnPlan pl;
+      const int rc = we::host::prepare_attn(at, st, at, at, t_pos, at, st, given ? at : nullptr, (size_t)given, 1, heads, heads, T, dh,
+                                            (int64_t)slots * T, d, 0.1f, splits, 0, WE_DTYPE_F32, 256, p, pl);
+      parts = groups = 0;
+      wrong += rc != WE_OK || we::host::launch_attn(p, pl, dh, WE_DTYPE_F32, nullptr) != WE_OK;
+      wrong += parts != want.parts || groups != want.groups || (parts > 1 && want.bytes(parts) > given);
+      if (share > 1 && parts > 1) ++less;
+      ++cases;
+    }
+  printf("%ld %ld %ld\n", cases, wrong, less);
+  return 0;
+}
+"""
+
+
+def test_what_is_launched_is_what_was_planned(tmp_path):
+    """Parts and groups of queries together, also with a workspace that holds fewer parts than the best plan has."""
+    cxx, rocm = os.environ.get("CXX") or shutil.which("g++"), os.environ.get("ROCM_PATH", "/opt/rocm")
+    src, exe = tmp_path / "launched.cpp", tmp_path / "launched"
+    src.write_text(LAUNCHED)
+    subprocess.run([cxx, "-std=c++17", "-O1", "-D__HIP_PLATFORM_AMD__=1", f"-I{CSRC}", f"-isystem{rocm}/include", str(src), "-o", str(exe)],
+                   check=True)
+    cases, wrong, less = map(int, subprocess.run([str(exe)], capture_output=True, text=True, timeout=60, check=True).stdout.split())
+    assert cases > 1000 and less > 50 and wrong == 0
+
+
 def test_workspace_of_an_fp32_call():
     lib = _capi.lib()
     bytes_of = lib.we_attn_f32_workspace_bytes

@@ -33,6 +33,7 @@ struct AttnPlan {
   int units_whole;  // leading (batch, kv head) units that are not split
   int64_t ws_rows;  // query rows that go through the split-context workspace
   int cus;          // compute units planned for
+  int f32_groups = 1;   // fp32 calls: groups of 16 queries per workgroup, for the parts in AttnParams
 };
 
 inline int variant_of(int q_tile) {
@@ -245,17 +246,17 @@ inline int prepare_attn(const void* q, const int64_t* q_strides, const void* kv,
   if ((uint64_t)(L + T) * (uint64_t)Dh * 2u >= (1ull << 32)) return WE_ERR_UNSUPPORTED;  // 32-bit tile offsets
   if (!(scale > 0.f) || n_splits < 0 || n_splits > 64) return WE_ERR_BAD_SHAPE;
   if (variant_of(q_tile) < 0) return WE_ERR_UNSUPPORTED;
-  int f32_parts = 1;
+  int f32_parts = 1, f32_groups = 1;
   if (dtype == WE_DTYPE_F32) {
     // fp32 caches take a kernel of their own: no given number of parts, no tile choice
     if (n_splits > 1 || H > 65535 || B > 65535) return WE_ERR_UNSUPPORTED;
     // (into parts where the caller leaves that to the library and has given memory for them; not in the library's own,
     // which calls that overlap would share)
-    if (n_splits == 0 && workspace && aligned16(workspace) && workspace_limit == SIZE_MAX) {
-      F32Call call = {(int64_t)B * H, T, L / T / dilation, Dh, cus};
-      call.plan((int64_t)(workspace_bytes > (size_t)INT64_MAX ? (size_t)INT64_MAX : workspace_bytes));
-      f32_parts = call.parts;
-    }
+    const bool room = n_splits == 0 && workspace && aligned16(workspace) && workspace_limit == SIZE_MAX;
+    F32Call call = {(int64_t)B * H, T, L / T / dilation, Dh, cus};
+    call.plan(!room ? 0 : (int64_t)(workspace_bytes > (size_t)INT64_MAX ? (size_t)INT64_MAX : workspace_bytes));
+    f32_parts = call.parts;
+    f32_groups = call.groups;
     n_splits = 1;
   }
   if (!aligned16(q) || !aligned16(kv) || !aligned16(out) || !strides_ok(q_strides, dtype) ||
@@ -319,6 +320,7 @@ inline int prepare_attn(const void* q, const int64_t* q_strides, const void* kv,
   p.q_heads = shared ? 1 : p.group;
   p.unit_splits = pl.units_whole + (B * Hkv - pl.units_whole) * pl.n_splits;
   p.scale_log2 = scale * 1.4426950408889634f;
+  pl.f32_groups = f32_groups;
   if (f32_parts > 1) {
     p.n_splits = f32_parts;
     p.ws_o = workspace;
@@ -338,7 +340,7 @@ inline int prepare_attn(const void* q, const int64_t* q_strides, const void* kv,
 
 // The launches of one planned attention call.
 inline int launch_attn(const AttnParams& p, const AttnPlan& pl, int Dh, int dtype, hipStream_t st) {
-  if (dtype == WE_DTYPE_F32) return launch_attn_ring_f32(p, Dh, pl.cus, st) == hipSuccess ? WE_OK : WE_ERR_LAUNCH;
+  if (dtype == WE_DTYPE_F32) return launch_attn_ring_f32(p, Dh, pl.f32_groups, pl.cus, st) == hipSuccess ? WE_OK : WE_ERR_LAUNCH;
   const int ksplit = pl.variant == 1 ? 2 : 1;
   hipError_t e;
   if (p.T < 64) e = dtype == WE_DTYPE_BF16 ? launch_attn_ring_short_bf16(p, Dh, ksplit, st) : launch_attn_ring_short_f16(p, Dh, ksplit, st);

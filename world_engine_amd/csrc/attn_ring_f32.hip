@@ -782,10 +782,8 @@ __global__ void __launch_bounds__(256) f32_combine_kernel(AttnParams p) {
 }
 
 template <int DH>
-static hipError_t launch_f32(AttnParams p, int cus, hipStream_t stream) {
-  F32Call call = {(int64_t)p.B * p.H, p.T, p.num_buckets, DH, cus};
-  call.plan(p.n_splits > 1 ? INT64_MAX : 0);   // (parts as the host planned them, or none)
-  const int nq = call.groups;
+static hipError_t launch_f32(AttnParams p, int nq, int cus, hipStream_t stream) {
+  const F32Call call = {(int64_t)p.B * p.H, p.T, p.num_buckets, DH, cus};
   const int64_t wgs = call.tiles(nq) * p.n_splits;
   if (wgs > 0x7fffffff) return hipErrorInvalidValue;
   p.members = p.group * ((p.T + nq * F_Q - 1) / (nq * F_Q));
@@ -831,9 +829,9 @@ hipError_t configure_attn_ring_f32() {
   return e == hipSuccess ? configure_f32<64, 2, false>() : e;
 }
 
-hipError_t launch_attn_ring_f32(const AttnParams& p, int Dh, int cus, hipStream_t stream) {
-  if (Dh == 128) return launch_f32<128>(p, cus, stream);
-  if (Dh == 64) return launch_f32<64>(p, cus, stream);
+hipError_t launch_attn_ring_f32(const AttnParams& p, int Dh, int groups, int cus, hipStream_t stream) {
+  if (Dh == 128) return launch_f32<128>(p, groups, cus, stream);
+  if (Dh == 64) return launch_f32<64>(p, groups, cus, stream);
   return hipErrorInvalidValue;
 }
 

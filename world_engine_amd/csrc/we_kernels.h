@@ -123,8 +123,8 @@ hipError_t launch_attn_ring_short_f16(const AttnParams& p, int Dh, int ksplit, h
 // grouped heads that share query tiles (q_heads != group)
 hipError_t launch_attn_ring_shared_bf16(const AttnParams& p, int Dh, int ksplit, hipStream_t stream);
 hipError_t launch_attn_ring_shared_f16(const AttnParams& p, int Dh, int ksplit, hipStream_t stream);
-// fp32 caches (f32_parts.h: whether in parts, merged by a second pass of their own)
-hipError_t launch_attn_ring_f32(const AttnParams& p, int Dh, int cus, hipStream_t stream);
+// fp32 caches, in n_splits parts (merged by a second pass of their own) and groups of queries as F32Call::plan has them
+hipError_t launch_attn_ring_f32(const AttnParams& p, int Dh, int groups, int cus, hipStream_t stream);
 hipError_t launch_attn_combine(const AttnParams& p, int Dh, int dtype, hipStream_t stream);
 // Measurement library only (stream_probe.hip): the 256-token-frame tile stream without the arithmetic.
 hipError_t launch_stream_probe(const void* src, int workgroups, int tiles, int share, hipStream_t stream);
