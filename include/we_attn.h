@@ -144,9 +144,11 @@ size_t we_attn_workspace_bytes_for(int32_t B, int32_t H, int32_t Hkv, int32_t T,
                                    int32_t n_splits, int32_t q_tile, int32_t dtype);
 
 /*
- * Bytes of workspace with which an fp32 call that leaves n_splits at 0 cuts its context into parts, 0 where it does
- * not.  With fewer, or none, it takes the whole context in one pass; so does every call of
- * we_attn_ring_fwd_static.
+ * Bytes of workspace with which an fp32 call that leaves n_splits at 0 cuts its context into as many parts as
+ * are fastest, 0 where it takes one pass.  With fewer bytes it takes as many parts as they hold where that is
+ * still the faster way, else one pass, as with none (the results then differ in the last bits); so does every
+ * call with n_splits = 1 or of we_attn_ring_fwd_static.  An fp32 call writes to a workspace of any size that it
+ * is given.
  */
 size_t we_attn_f32_workspace_bytes(int32_t B, int32_t H, int32_t Hkv, int32_t T, int32_t Dh, int64_t L, int32_t dilation);
 
@@ -178,7 +180,8 @@ int we_attn_plan(int32_t B, int32_t H, int32_t Hkv, int32_t T, int32_t Dh, int64
  *   out  [B, H, T, Dh]   element strides out_strides = {batch, head, token}; Dh contiguous.
  *   workspace            device scratch of at least we_attn_workspace_bytes(...) bytes (f16: better
  *                        we_attn_workspace_bytes_for) for the
- *                        same sizes, n_splits and q_tile; may be NULL when that is 0.  Nothing in
+ *                        same sizes, n_splits and q_tile; may be NULL when that is 0.  fp32 calls need
+ *                        none and take what they get (we_attn_f32_workspace_bytes).  Nothing in
  *                        it has to start at any value; calls that overlap in time need a
  *                        workspace each.
  *   n_splits             0 = choose automatically (every (batch, kv head) unit in as many parts as
@@ -189,8 +192,9 @@ int we_attn_plan(int32_t B, int32_t H, int32_t Hkv, int32_t T, int32_t Dh, int64
  *   q_tile               queries per workgroup: 0 = choose automatically, or 128 / 256.
  *   scale                softmax scale (> 0); the reference uses 1/sqrt(Dh).
  *
- * Requirements: dtype bf16 or f16 or f32 (a kernel of its own, of fp32 precision
- * throughout, n_splits 0 or 1, q_tile ignored); Dh in {64, 128};
+ * Requirements: dtype bf16 or f16 or f32 (a kernel of its own, n_splits 0 or 1, q_tile ignored; fp32
+ * sums and softmax, products of fp32 values or of two f16 halves of each, 22 bits together and 21 at worst,
+ * as exact for every output channel and row as fp32 products in a chain are); Dh in {64, 128};
  * any T (frames that are not a multiple of the 64-key tile cost one masked tile per slot);
  * L/T <= WE_MAX_SLOTS; H % Hkv == 0; pointers and row starts 16-byte aligned.
  */
@@ -207,7 +211,7 @@ int we_attn_ring_fwd(const void* q, const int64_t q_strides[3],
  * under HIP graph capture, tight serving loops, harnesses that forbid hipMalloc.  It has no
  * counterpart in the reference (whose attention call allocates through torch as it pleases).
  * Arguments, requirements and results are those of we_attn_ring_fwd with a workspace of
- * WE_STATIC_SCRATCH_BYTES, bit for bit, without the workspace pair: the split-context partial
+ * WE_STATIC_SCRATCH_BYTES (fp32: with none, in one pass), bit for bit, without the workspace pair: the split-context partial
  * results go to a buffer of WE_STATIC_SCRATCH_BYTES that is part of the library's device image (every GPU the library runs on holds one copy until the
  * process ends; its address is looked up once per device by that device's set-up, see we_init:
  * under stream capture the device must have been set up beforehand).  Sizes whose

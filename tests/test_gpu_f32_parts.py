@@ -65,7 +65,8 @@ def _call(gpu_device, shape, seed=0):
 
 
 def test_f32_parts_need_their_workspace(gpu_device):
-    """A short workspace at the C entry point, none and the static entry point: one pass, bit for bit."""
+    """No workspace at the C entry point, one that holds no two parts, and the static entry point: one pass, bit for bit.
+    One that holds fewer parts than the best plan: as many as it holds."""
     shape = SHAPES[0]
     B, H, Hkv, T, Dh, n, d = shape
     q, kv, written, t_pos = _call(gpu_device, shape)
@@ -74,17 +75,17 @@ def test_f32_parts_need_their_workspace(gpu_device):
     assert not torch.equal(one, parts) and (one - parts).abs().max() < 1e-5
     need = _bytes(*shape)
     lib, st = _capi.lib(), torch.cuda.current_stream().cuda_stream
-    for bytes_, want in ((0, one), (16, one), (need // 16, one), (need, parts), (need + 4096, parts)):
+    for bytes_, want in ((0, one), (16, one), (need // 16, one), (need // 2, None), (need, parts), (need + 4096, parts)):
         ws = torch.empty(max(bytes_, 16), dtype=torch.uint8, device=gpu_device)
         out = torch.empty(B, T, H, Dh, device=gpu_device).transpose(1, 2)
         strides = lambda x: ops._bhtd_strides(x, "x")
         rc = lib.we_attn_ring_fwd(q.data_ptr(), strides(q), kv.data_ptr(), written.data_ptr(), t_pos.data_ptr(), out.data_ptr(), strides(out),
                                   ws.data_ptr() if bytes_ else None, bytes_, B, H, Hkv, T, Dh, n * T, d, 1 / math.sqrt(Dh), 0, 0, _capi.WE_DTYPE_F32, st)
         assert rc == 0
-        if bytes_ in (0, 16, need, need + 4096):
+        if want is not None:
             assert torch.equal(out, want), bytes_
         else:
-            assert (out - want).abs().max() < 1e-5
+            assert not torch.equal(out, one) and not torch.equal(out, parts) and (out - parts).abs().max() < 1e-5
     out = torch.empty(B, T, H, Dh, device=gpu_device).transpose(1, 2)
     ops.attn_ring_static(q, kv, written, t_pos, n * T, d, out)
     assert torch.equal(out, one)
@@ -121,3 +122,23 @@ def test_f32_parts_with_a_gate(gpu_device):
     plain = p.hip.rope_upsert_attend(q, k, v, pos, p.rope, 0)
     gated = p.hip.rope_upsert_attend(q, k, v, pos, p.rope, 0, gate=gate)
     assert torch.equal(gated, plain * gate[..., None])
+
+
+@pytest.mark.parametrize("d", [1, 2])
+def test_f32_calls_that_bring_or_keep_a_workspace_allocate_none(gpu_device, d):
+    """``ops.attn_f32_workspace_bytes`` is what such a call asks for; per-layer kept buffers hold it."""
+    B, H, Hkv, T, Dh, n = 1, 4, 4, 128, 128, 16
+    q, kv, written, t_pos = _call(gpu_device, (B, H, Hkv, T, Dh, n, d))
+    need = ops.attn_f32_workspace_bytes(B, H, Hkv, T, Dh, n * T, d)
+    assert need == _bytes(B, H, Hkv, T, Dh, n, d) > 0
+    out = torch.empty(B, T, H, Dh, device=gpu_device).transpose(1, 2)
+    ws = torch.empty(need, dtype=torch.uint8, device=gpu_device)
+    want = ops.attn_ring(q, kv, written, t_pos, n * T, d)
+    kept = {}
+    for _ in range(2):
+        assert ops.kept_buffers(kept, "attn", q, H, Hkv, T, Dh, n * T, dilation=d)[2].numel() == need
+    torch.cuda.synchronize()
+    before = torch.cuda.memory_stats(gpu_device)["allocation.all.allocated"]
+    ops.attn_ring(q, kv, written, t_pos, n * T, d, out=out, workspace=ws)
+    assert torch.cuda.memory_stats(gpu_device)["allocation.all.allocated"] == before
+    assert torch.equal(out, want)

@@ -158,7 +158,7 @@ class LayerKVCache(nn.Module):
                 rope.width, self.kv, self.written, self.L, self.pinned_dilation, bool(is_frozen), s,
                 float(qk_norm_eps), v1, v_lamb, gate, gate_x, gate_w)
         q_rot, out, workspace = ops.kept_buffers(self._reusable(reuse_buffers), "attn", q, q.shape[1], k.shape[1], q.shape[2],
-                                                 q.shape[3], self.L)
+                                                 q.shape[3], self.L, dilation=self.pinned_dilation)
         own = self._buffers
         res = native.rope_kv_attn(q, k, v, pos_ids["t_pos"], pos_ids["y_pos"], pos_ids["x_pos"], rope.cos, rope.sin, rope.height,
                                   rope.width, own["kv"], own["written"], self.L, self.pinned_dilation, is_frozen, scale, 0, 0,
@@ -187,7 +187,7 @@ class LayerKVCache(nn.Module):
             return y, (v if want_v else None)
         kv = self.kv
         q_rot, out, workspace = ops.kept_buffers(self._reusable(reuse_buffers), "qkv", x, n_heads, n_kv, x.shape[1], kv.shape[4],
-                                                 self.L)
+                                                 self.L, dilation=self.pinned_dilation)
         res = native.qkv_rope_kv_attn(x, w_qkv, n_heads, n_kv, pos_ids["t_pos"], pos_ids["y_pos"], pos_ids["x_pos"], rope.cos,
                                       rope.sin, rope.height, rope.width, kv, self.written, self.L, self.pinned_dilation,
                                       is_frozen, scale, 0, 0, True, want_v, qk_norm_eps, v1, v_lamb, None, gate_x, gate_w, out,

@@ -125,6 +125,12 @@ def attn_workspace_bytes(B: int, H: int, Hkv: int, T: int, Dh: int, L: int, n_sp
     return int(_capi.lib().we_attn_workspace_bytes_for(B, H, Hkv, T, Dh, L, n_splits, q_tile, _dtype_code(dtype)))
 
 
+def attn_f32_workspace_bytes(B: int, H: int, Hkv: int, T: int, Dh: int, L: int, dilation: int = 1) -> int:
+    """Bytes of workspace with which an fp32 call without a given ``n_splits`` cuts its context into parts, 0 where it
+    takes one pass.  Such a call allocates them itself when ``workspace`` is not given or is shorter."""
+    return int(_capi.lib().we_attn_f32_workspace_bytes(B, H, Hkv, T, Dh, L, dilation))
+
+
 def attn_plan(B: int, H: int, Hkv: int, T: int, Dh: int, L: int, n_splits: int = 0, q_tile: int = 0,
               compute_units: int = 0) -> dict:
     """What the library would do with an attention call of these sizes (``we_attn_plan``; launches
@@ -146,8 +152,8 @@ def attn_ring(q: Tensor, kv: Tensor, written: Tensor, t_pos: Tensor, L: int, dil
     ``[2,B,Hkv,L+T,Dh]``, ``written`` ``[L+T]`` bool, ``t_pos`` int64 with the frame index at
     element 0.  Returns ``[B,H,T,Dh]``; with ``token_major_out`` its memory is ``[B,T,H,Dh]`` so
     that ``y.transpose(1, 2).reshape(B, T, H*Dh)`` is a view (``src/patch_model.py:139``).
-    ``workspace`` (split-context scratch, uint8, ``attn_workspace_bytes`` long for q's element type) is allocated
-    when not given, or when it is shorter.
+    ``workspace`` (split-context scratch, uint8, ``attn_workspace_bytes`` long for q's element type, for fp32
+    ``attn_f32_workspace_bytes``) is allocated when not given, or when it is shorter; calls that overlap in time need one each.
     ``clocks`` (int64 device tensor): the call goes through the measurement library
     (``libwe_probe.so``, ``we_attn_ring_fwd_clocked``), which also leaves, per workgroup of the main
     kernel, its duration in shader-clock cycles and in ticks of the constant 100 MHz counter.
@@ -248,7 +254,8 @@ def qkv_rope_kv_attn(x: Tensor, w_qkv: Tensor, n_heads: int, n_kv_heads: int, po
     from a BLAS library's: they can differ from ``F.linear``'s in the last bit.
     ``buffers``: a dict the call keeps its ``q_rot`` / ``out`` / ``workspace`` tensors in and takes
     them from next time (shapes permitting), for callers that step the same layer again and again."""
-    q_rot, out, workspace = kept_buffers(buffers, "qkv", x, n_heads, n_kv_heads, x.shape[1], kv.shape[-1], L, n_splits, q_tile)
+    q_rot, out, workspace = kept_buffers(buffers, "qkv", x, n_heads, n_kv_heads, x.shape[1], kv.shape[-1], L, n_splits, q_tile,
+                                        dilation)
     return native.qkv_rope_kv_attn(x, w_qkv, n_heads, n_kv_heads, pos_ids["t_pos"], pos_ids["y_pos"], pos_ids["x_pos"],
                                    cos_table, sin_table, grid_h, grid_w, kv, written, L, dilation, is_frozen, scale, n_splits,
                                    q_tile, attend, want_v, qk_norm_eps, v1, v_lamb, gate, gate_x, gate_w, out, workspace,
@@ -256,17 +263,20 @@ def qkv_rope_kv_attn(x: Tensor, w_qkv: Tensor, n_heads: int, n_kv_heads: int, po
 
 
 def kept_buffers(buffers: Optional[dict], kind: str, like: Tensor, H: int, Hkv: int, T: int, Dh: int, L: int,
-                 n_splits: int = 0, q_tile: int = 0):
+                 n_splits: int = 0, q_tile: int = 0, dilation: int = 1):
     """``(q_rot, out, workspace)`` of a call kept in ``buffers`` from an earlier one (all None, i.e. made
     by the call itself, when there is no dict to keep them in)."""
     if buffers is None:
         return None, None, None
     B, dtype, dev = like.shape[0], like.dtype, like.device
-    key = (kind, B, H, Hkv, T, Dh, dtype, dev, n_splits, q_tile)
+    key = (kind, B, H, Hkv, T, Dh, dtype, dev, n_splits, q_tile, dilation)
     kept = buffers.get(key)
     if kept is None:
         with torch.cuda.device(dev):      # (the size depends on the device's compute-unit count)
-            ws_bytes = attn_workspace_bytes(B, H, Hkv, T, Dh, L, n_splits, q_tile, dtype)
+            if dtype == torch.float32:
+                ws_bytes = attn_f32_workspace_bytes(B, H, Hkv, T, Dh, L, dilation) if n_splits == 0 else 0
+            else:
+                ws_bytes = attn_workspace_bytes(B, H, Hkv, T, Dh, L, n_splits, q_tile, dtype)
         kept = buffers[key] = (torch.empty((B, H, T, Dh), dtype=dtype, device=dev),
                                torch.empty((B, T, H, Dh), dtype=dtype, device=dev).transpose(1, 2),
                                torch.empty(ws_bytes, dtype=torch.uint8, device=dev) if ws_bytes else None)
