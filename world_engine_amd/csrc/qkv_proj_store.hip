@@ -163,7 +163,7 @@ qkv_rope_store_kernel(ProjParams p) {
       for (int i = 0; i < 16; ++i) acc[nb][mb][i] = 0.f;
 
   // ---- what the item needs besides the projection (as it comes: a conversion here would wait for it) ----
-  ItemSide<Tag> side;
+  ItemSide<Tag, 16> side;
   u32x4_t res_raw[2];
   st_t lamb_raw;
   uint32_t guard;
@@ -173,7 +173,7 @@ qkv_rope_store_kernel(ProjParams p) {
     if (side.rotate) {
       const int64_t* ids = reinterpret_cast<const int64_t*>(smem + IDS_OFF + wave * 256) + (e_row & 7);
       const int64_t at = rope_table_row(s, ids[0], ids[8], ids[16]) * (s.Dh >> 1);
-      load_cos_sin(s.cos_t + at, s.sin_t + at, e_chunk, side.c, side.s);
+      load_cos_sin<16>(s.cos_t + at, s.sin_t + at, e_chunk, side.c, side.s);
     }
     if (blend) {
       const u32x4_t* src = reinterpret_cast<const u32x4_t*>((const st_t*)s.v1 + b * s.v1s_b + e_h * s.v1s_h + e_tc * s.v1s_t + e_chunk * 16);
@@ -235,7 +235,7 @@ qkv_rope_store_kernel(ProjParams p) {
         xch[(((nh * 4 + kg) * 4 + 2 * nb + mb) * 4 + g) * 64 + (lane ^ (2 * (nh * 4 + nb * 2 + (g >> 1))))] =
             f32x4_t{acc[nb][mb][4 * g], acc[nb][mb][4 * g + 1], acc[nb][mb][4 * g + 2], acc[nb][mb][4 * g + 3]};
   __syncthreads();
-  Chunk16<Tag> in;
+  Chunk<Tag, 16> in;
   {
     const int item = tid & 7, blk = (item & 2) + (e_row >> 5);
     const f32x4_t* src = xch + ((item >> 2) * 16 + blk) * 256 + (item & 1) * 128;
@@ -256,17 +256,17 @@ qkv_rope_store_kernel(ProjParams p) {
   asm volatile("" : "+v"(frame_t));
   if (!e_live || (s.guard != nullptr && guard != 0u)) return;  // (refused position ids: nothing is written)
   if (blend) {
-    *reinterpret_cast<u32x4_t*>(side.res.e) = res_raw[0];
-    *reinterpret_cast<u32x4_t*>(side.res.e + 8) = res_raw[1];
+    reinterpret_cast<u32x4_t*>(&side.res.e)[0] = res_raw[0];
+    reinterpret_cast<u32x4_t*>(&side.res.e)[1] = res_raw[1];
     side.lamb = Tag::to_f32(lamb_raw);
   }
   if (which == 0) {
-    finish_q_chunk<Tag>(s, b, e_h, e_t, e_chunk, in, side.rotate, side.c, side.s);
+    finish_q_chunk(s, b, e_h, e_t, e_chunk, in, side);
   } else {
     if (which == 2 && p.v_out != nullptr)
-      store16<Tag>((st_t*)p.v_out + b * p.vo_b + e_h * p.vo_h + e_t * p.vo_t + e_chunk * 16, in);
+      store_chunk((st_t*)p.v_out + b * p.vo_b + e_h * p.vo_h + e_t * p.vo_t + e_chunk * 16, in);
     const SlotInfo si = ring_slot((int64_t)uniform64((uint64_t)frame_t), s.dilation, s.num_buckets);
-    finish_kv_chunk<Tag>(s, which, b, e_h, e_t, e_chunk, si, in, side.rotate, side.c, side.s, side.res, side.lamb);
+    finish_kv_chunk(s, which, b, e_h, e_t, e_chunk, si, in, side);
   }
 }
 

@@ -1,6 +1,8 @@
 // Per-item work of the fused RoPE + ring-slot K/V store kernel (rope_kv_store.hip, gfx950): one
-// item = 16 consecutive input elements of one (tensor, batch, head, token) row.
+// item = N = 16 or 8 consecutive input elements of one (tensor, batch, head, token) row.
 #pragma once
+#include <type_traits>
+
 #include "we_common.h"
 #include "we_kernels.h"
 #include "../../include/we_attn.h"
@@ -30,39 +32,32 @@ struct F32Tag {
   __device__ static float from_f32(float f) { return f; }
 };
 
-// 16 elements of a row as raw storage.
-template <typename Tag>
-struct Chunk16 {
-  typename Tag::store_t e[16];
-};
-template <typename Tag>
-struct Chunk8 {
-  typename Tag::store_t e[8];
+// N elements of a row as raw storage.
+template <typename Tag, int N>
+struct Chunk {
+  typedef typename Tag::store_t values_t __attribute__((ext_vector_type(N)));
+  values_t e;
 };
 
-template <typename Tag>
-__device__ __forceinline__ void load16(Chunk16<Tag>& c, const void* p) {
-  constexpr int nvec = 16 * Tag::kBytes / 16;
-  const uint4* src = reinterpret_cast<const uint4*>(p);
-  uint4* dst = reinterpret_cast<uint4*>(c.e);
+template <typename Tag, int N>
+struct ChunkWords {   // what a chunk is loaded and stored as
+  static constexpr int kBytes = N * Tag::kBytes;
+  typedef typename std::conditional<kBytes % 16 == 0, uint4, uint2>::type word_t;
+  static constexpr int kWords = kBytes / (int)sizeof(word_t);
+};
+template <typename Tag, int N>
+__device__ __forceinline__ void load_chunk(Chunk<Tag, N>& c, const void* p) {
+  typedef ChunkWords<Tag, N> W;
 #pragma unroll
-  for (int i = 0; i < nvec; ++i) dst[i] = src[i];
+  for (int i = 0; i < W::kWords; ++i)
+    reinterpret_cast<typename W::word_t*>(&c.e)[i] = reinterpret_cast<const typename W::word_t*>(p)[i];
 }
-template <typename Tag>
-__device__ __forceinline__ void store16(void* p, const Chunk16<Tag>& c) {
-  constexpr int nvec = 16 * Tag::kBytes / 16;
-  uint4* dst = reinterpret_cast<uint4*>(p);
-  const uint4* src = reinterpret_cast<const uint4*>(c.e);
+template <typename Tag, int N>
+__device__ __forceinline__ void store_chunk(void* p, const Chunk<Tag, N>& c) {
+  typedef ChunkWords<Tag, N> W;
 #pragma unroll
-  for (int i = 0; i < nvec; ++i) dst[i] = src[i];
-}
-template <typename Tag>
-__device__ __forceinline__ void store8(void* p, const Chunk8<Tag>& c) {
-  constexpr int nvec = 8 * Tag::kBytes / 16;
-  uint4* dst = reinterpret_cast<uint4*>(p);
-  const uint4* src = reinterpret_cast<const uint4*>(c.e);
-#pragma unroll
-  for (int i = 0; i < nvec; ++i) dst[i] = src[i];
+  for (int i = 0; i < W::kWords; ++i)
+    reinterpret_cast<typename W::word_t*>(p)[i] = reinterpret_cast<const typename W::word_t*>(&c.e)[i];
 }
 
 // Weightless RMS norm of a row held N = 16 or 8 elements per lane by `cpr` consecutive lanes (a power of
@@ -72,15 +67,15 @@ __device__ __forceinline__ void store8(void* p, const Chunk8<Tag>& c) {
 // half-precision squares are exact in fp32, so the order is all that decides a sum's bits, and of the orders
 // tried (groups of 1 to 16, neighbouring or strided, sequential or as trees) this one, with this reciprocal
 // root, gives every bit of 2*10^5 rows of 64 and of 128.
-template <typename Tag, int N, typename E>
-__device__ __forceinline__ void rms_norm_chunk(E& e, int cpr, int Dh, float eps) {
+template <typename Tag, int N>
+__device__ __forceinline__ void rms_norm_chunk(Chunk<Tag, N>& c, int cpr, int Dh, float eps) {
   float x[N], part[N / 4];
 #pragma unroll
   for (int j = 0; j < N / 4; ++j) {
     part[j] = 0.f;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      x[4 * j + i] = Tag::to_f32(e[4 * j + i]);
+      x[4 * j + i] = Tag::to_f32(c.e[4 * j + i]);
       part[j] += x[4 * j + i] * x[4 * j + i];
     }
   }
@@ -93,19 +88,19 @@ __device__ __forceinline__ void rms_norm_chunk(E& e, int cpr, int Dh, float eps)
   for (int i = 0; i < N; ++i) {
     float y = x[i] * r;
     asm("" : "+v"(y));  // (fused with the conversion to f16 the product of a negative value and 0 loses its sign)
-    e[i] = Tag::from_f32(y);
+    c.e[i] = Tag::from_f32(y);
   }
 }
 
 // torch.lerp(v, v1, w) on N elements: fp32 arithmetic, the formula switches at |w| = 0.5
 // (ATen/native/Lerp.h), result rounded to the element type.
-template <typename Tag, int N, typename E>
-__device__ __forceinline__ void lerp_chunk(E& v, const E& v1, float w) {
+template <typename Tag, int N>
+__device__ __forceinline__ void lerp_chunk(Chunk<Tag, N>& v, const Chunk<Tag, N>& v1, float w) {
 #pragma unroll
   for (int i = 0; i < N; ++i) {
-    const float a = Tag::to_f32(v[i]), b = Tag::to_f32(v1[i]);
+    const float a = Tag::to_f32(v.e[i]), b = Tag::to_f32(v1.e[i]);
     const float d = b - a;
-    v[i] = Tag::from_f32(fabsf(w) < 0.5f ? a + w * d : b - d * (1.f - w));
+    v.e[i] = Tag::from_f32(fabsf(w) < 0.5f ? a + w * d : b - d * (1.f - w));
   }
 }
 
@@ -120,28 +115,28 @@ __device__ __forceinline__ int64_t rope_table_row(const StoreParams& p, int b, i
   return rope_table_row(p, p.t_pos[at], p.y_pos[at], p.x_pos[at]);
 }
 
-// cos / sin of the 8 pairs of chunk `chunk` of a table row.
-__device__ __forceinline__ void load_cos_sin(const float* cos_row, const float* sin_row, int chunk, float (&c)[8],
-                                             float (&s)[8]) {
-  const float4* cp = reinterpret_cast<const float4*>(cos_row + chunk * 8);
-  const float4* sp = reinterpret_cast<const float4*>(sin_row + chunk * 8);
-  *reinterpret_cast<float4*>(c) = cp[0];
-  *reinterpret_cast<float4*>(c + 4) = cp[1];
-  *reinterpret_cast<float4*>(s) = sp[0];
-  *reinterpret_cast<float4*>(s + 4) = sp[1];
+// cos / sin of the N / 2 pairs of chunk `chunk` of a table row.
+template <int N>
+__device__ __forceinline__ void load_cos_sin(const float* cos_row, const float* sin_row, int chunk, float (&c)[N / 2],
+                                             float (&s)[N / 2]) {
+#pragma unroll
+  for (int i = 0; i < N / 2; i += 4) {
+    *reinterpret_cast<float4*>(c + i) = *reinterpret_cast<const float4*>(cos_row + chunk * (N / 2) + i);
+    *reinterpret_cast<float4*>(s + i) = *reinterpret_cast<const float4*>(sin_row + chunk * (N / 2) + i);
+  }
 }
 
-// Rotation of the 8 (even, odd) pairs of one 16-element chunk: lo gets x0*cos - x1*sin (elements
-// [8*chunk, 8*chunk+8) of the output row), hi gets x1*cos + x0*sin (the same range of the second
+// Rotation of the N / 2 (even, odd) pairs of one N-element chunk: lo gets x0*cos - x1*sin (elements
+// [N / 2 * chunk, N / 2 * (chunk + 1)) of the output row), hi gets x1*cos + x0*sin (the same range of the second
 // half; the reference concatenates the rotated halves, attn.py:38-40).  Every product and sum is
 // rounded separately, as eager fp32 tensor ops do: contraction into fused multiply-adds is
 // switched off for this function (plain operators; the pragma does not govern inlined intrinsics).
-template <typename Tag>
-__device__ __forceinline__ void rotate_values(const Chunk16<Tag>& in, const float (&c)[8], const float (&s)[8],
-                                              Chunk8<Tag>& lo, Chunk8<Tag>& hi) {
+template <typename Tag, int N>
+__device__ __forceinline__ void rotate_values(const Chunk<Tag, N>& in, const float (&c)[N / 2], const float (&s)[N / 2],
+                                              Chunk<Tag, N / 2>& lo, Chunk<Tag, N / 2>& hi) {
 #pragma clang fp contract(off)
 #pragma unroll
-  for (int i = 0; i < 8; ++i) {
+  for (int i = 0; i < N / 2; ++i) {
     const float x0 = Tag::to_f32(in.e[2 * i]);
     const float x1 = Tag::to_f32(in.e[2 * i + 1]);
     const float p0 = x0 * c[i], p1 = x1 * s[i], p2 = x1 * c[i], p3 = x0 * s[i];
@@ -151,11 +146,23 @@ __device__ __forceinline__ void rotate_values(const Chunk16<Tag>& in, const floa
     hi.e[i] = Tag::from_f32(y1);
   }
 }
+// A rotated item's halves, or the item itself, into the row `to`.
+template <typename Tag, int N>
+__device__ __forceinline__ void store_item(typename Tag::store_t* to, int Dh, int chunk, bool rotated, const Chunk<Tag, N>& in,
+                                           const Chunk<Tag, N / 2>& lo, const Chunk<Tag, N / 2>& hi) {
+  if (rotated) {
+    store_chunk(to + chunk * (N / 2), lo);
+    store_chunk(to + (Dh >> 1) + chunk * (N / 2), hi);
+  } else {
+    store_chunk(to + chunk * N, in);
+  }
+}
+
 // Destination rows of a K/V item: tail always, ring slot on an unfrozen persisting frame.
-template <typename Tag>
+template <typename Tag, int N>
 __device__ __forceinline__ void store_kv_rows(const StoreParams& p, int which, int b, int h, int t, int chunk,
-                                              const SlotInfo& si, bool rotated, const Chunk16<Tag>& in,
-                                              const Chunk8<Tag>& lo, const Chunk8<Tag>& hi) {
+                                              const SlotInfo& si, bool rotated, const Chunk<Tag, N>& in,
+                                              const Chunk<Tag, N / 2>& lo, const Chunk<Tag, N / 2>& hi) {
   typedef typename Tag::store_t st_t;
   const int64_t cap = p.L + p.T;
   const int plane = which - 1;
@@ -163,85 +170,67 @@ __device__ __forceinline__ void store_kv_rows(const StoreParams& p, int which, i
   const bool to_ring = (!p.frozen) && si.write_step;
   const int64_t tail_row = p.L + t;
   const int64_t ring_row = (int64_t)si.slot * p.T + t;
-  st_t* d0 = plane_base + tail_row * p.Dh;
-  st_t* d1 = plane_base + ring_row * p.Dh;
-  if (rotated) {
-    store8<Tag>(d0 + chunk * 8, lo);
-    store8<Tag>(d0 + (p.Dh >> 1) + chunk * 8, hi);
-    if (to_ring) {
-      store8<Tag>(d1 + chunk * 8, lo);
-      store8<Tag>(d1 + (p.Dh >> 1) + chunk * 8, hi);
-    }
-  } else {
-    store16<Tag>(d0 + chunk * 16, in);
-    if (to_ring) store16<Tag>(d1 + chunk * 16, in);
-  }
+  store_item(plane_base + tail_row * p.Dh, p.Dh, chunk, rotated, in, lo, hi);
+  if (to_ring) store_item(plane_base + ring_row * p.Dh, p.Dh, chunk, rotated, in, lo, hi);
   // written[dst] = True for the rows the unfrozen write went to (kv_cache.py:149-151).
   if (!p.frozen && which == 1 && b == 0 && h == 0 && chunk == 0) p.written[to_ring ? ring_row : tail_row] = 1;
 }
 
-// Everything after the load of a K (which = 1) or V (which = 2) item: K is normalised (optional)
-// and rotated, V is blended with the value residual (optional); the tail row is written always
-// and the ring-slot row when this is an unfrozen persisting frame; `written` is marked
-// (src/model/attn.py:105-110, src/model/kv_cache.py:138,147-151).  cos / sin are the item's 8
-// table values (used when `rotate`), `res` the matching 16 elements of the value residual (used
-// when p.v1 is set).
-template <typename Tag>
-__device__ __forceinline__ void finish_kv_chunk(const StoreParams& p, int which, int b, int h, int t, int chunk,
-                                                const SlotInfo& si, Chunk16<Tag>& in, bool rotate,
-                                                const float (&c)[8], const float (&s)[8], const Chunk16<Tag>& res,
-                                                float lamb) {
-  if (which == 1 && p.norm_eps > 0.f) rms_norm_chunk<Tag, 16>(in.e, p.Dh >> 4, p.Dh, p.norm_eps);
-  if (which == 2 && p.v1 != nullptr) lerp_chunk<Tag, 16>(in.e, res.e, lamb);
-  Chunk8<Tag> lo, hi;
-  if (rotate) rotate_values<Tag>(in, c, s, lo, hi);
-  store_kv_rows<Tag>(p, which, b, h, t, chunk, si, rotate, in, lo, hi);
-}
-
-// Everything after the load of a Q item: optional norm, rotation (or plain copy when there is no
-// table), store into the contiguous [B, H, T, Dh] output.
-template <typename Tag>
-__device__ __forceinline__ void finish_q_chunk(const StoreParams& p, int b, int h, int t, int chunk,
-                                               Chunk16<Tag>& in, bool rotate, const float (&c)[8],
-                                               const float (&s)[8]) {
-  typedef typename Tag::store_t st_t;
-  if (p.norm_eps > 0.f) rms_norm_chunk<Tag, 16>(in.e, p.Dh >> 4, p.Dh, p.norm_eps);
-  st_t* dst = (st_t*)p.q_out + (((int64_t)b * p.H + h) * p.T + t) * p.Dh;
-  if (rotate) {
-    Chunk8<Tag> lo, hi;
-    rotate_values<Tag>(in, c, s, lo, hi);
-    store8<Tag>(dst + chunk * 8, lo);
-    store8<Tag>(dst + (p.Dh >> 1) + chunk * 8, hi);
-  } else {
-    store16<Tag>(dst + chunk * 16, in);
-  }
-}
-
-// What an item needs besides its own 16 elements: the 8 cos / sin values of its pairs (rotated
-// items) and the value residual's 16 elements with the blend weight (V items of a layer that has
+// What an item needs besides its own N elements: the N / 2 cos / sin values of its pairs (rotated
+// items) and the value residual's N elements with the blend weight (V items of a layer that has
 // one).  Separate from the arithmetic so that a caller can request them long before it has the
-// item's own values.
-template <typename Tag>
+// item's own values.  EXTRAS: whether a norm or a blend can be asked for at all.
+template <typename Tag, int N>
 struct ItemSide {
-  float c[8], s[8];
-  Chunk16<Tag> res;
+  float c[N / 2], s[N / 2];
+  Chunk<Tag, N> res;
   float lamb;
   bool rotate;
 };
-template <typename Tag>
+template <typename Tag, int N, bool EXTRAS = true>
 __device__ __forceinline__ void load_item_side(const StoreParams& p, int which, int b, int h, int t, int chunk,
-                                               ItemSide<Tag>& sd) {
+                                               ItemSide<Tag, N>& sd) {
   typedef typename Tag::store_t st_t;
   sd.rotate = which != 2 && p.cos_t != nullptr;
   sd.lamb = 0.f;
   if (sd.rotate) {
     const int64_t pos = rope_table_row(p, b, t);
     const int half = p.Dh >> 1;
-    load_cos_sin(p.cos_t + pos * half, p.sin_t + pos * half, chunk, sd.c, sd.s);
+    load_cos_sin<N>(p.cos_t + pos * half, p.sin_t + pos * half, chunk, sd.c, sd.s);
   }
-  if (which == 2 && p.v1 != nullptr) {
-    load16<Tag>(sd.res, (const st_t*)p.v1 + b * p.v1s_b + h * p.v1s_h + t * p.v1s_t + chunk * 16);
+  if (EXTRAS && which == 2 && p.v1 != nullptr) {
+    load_chunk(sd.res, (const st_t*)p.v1 + b * p.v1s_b + h * p.v1s_h + t * p.v1s_t + chunk * N);
     sd.lamb = Tag::to_f32(*reinterpret_cast<const st_t*>(p.v_lamb));
+  }
+}
+
+// Everything after the load of a K (which = 1) or V (which = 2) item: K is normalised (optional)
+// and rotated, V is blended with the value residual (optional); the tail row is written always
+// and the ring-slot row when this is an unfrozen persisting frame; `written` is marked
+// (src/model/attn.py:105-110, src/model/kv_cache.py:138,147-151).
+template <typename Tag, int N, bool EXTRAS = true>
+__device__ __forceinline__ void finish_kv_chunk(const StoreParams& p, int which, int b, int h, int t, int chunk,
+                                                const SlotInfo& si, Chunk<Tag, N>& in, const ItemSide<Tag, N>& sd) {
+  if (EXTRAS && which == 1 && p.norm_eps > 0.f) rms_norm_chunk(in, (int)((unsigned)p.Dh / (unsigned)N), p.Dh, p.norm_eps);
+  if (EXTRAS && which == 2 && p.v1 != nullptr) lerp_chunk(in, sd.res, sd.lamb);
+  Chunk<Tag, N / 2> lo, hi;
+  if (sd.rotate) rotate_values(in, sd.c, sd.s, lo, hi);
+  store_kv_rows(p, which, b, h, t, chunk, si, sd.rotate, in, lo, hi);
+}
+
+// Everything after the load of a Q item: optional norm, rotation (or plain copy when there is no
+// table), store into the contiguous [B, H, T, Dh] output.
+template <typename Tag, int N, bool EXTRAS = true>
+__device__ __forceinline__ void finish_q_chunk(const StoreParams& p, int b, int h, int t, int chunk,
+                                               Chunk<Tag, N>& in, const ItemSide<Tag, N>& sd) {
+  if (EXTRAS && p.norm_eps > 0.f) rms_norm_chunk(in, (int)((unsigned)p.Dh / (unsigned)N), p.Dh, p.norm_eps);
+  typename Tag::store_t* const to = (typename Tag::store_t*)p.q_out + (((int64_t)b * p.H + h) * p.T + t) * p.Dh;
+  Chunk<Tag, N / 2> lo, hi;
+  if (sd.rotate) {
+    rotate_values(in, sd.c, sd.s, lo, hi);
+    store_item(to, p.Dh, chunk, true, in, lo, hi);
+  } else {
+    store_item(to, p.Dh, chunk, false, in, lo, hi);
   }
 }
 
