@@ -243,3 +243,15 @@ def test_autocast_over_fp32_parameters(gpu_device):
                 pytest.skip("this torch normalises in fp32 under autocast, which a bf16 cache has never taken")
             raise
     assert torch.allclose(got.float(), want.float(), rtol=2e-2, atol=2e-2)
+
+
+def test_a_compiled_projection_takes_frames_of_several_lengths():
+    """From the second length on torch.compile traces with symbolic sizes."""
+    from world_engine_amd.attn import _plain_weight
+    lin = torch.nn.Linear(100, 60, bias=False).to(torch.bfloat16)
+    torch._dynamo.reset()
+    compiled = torch.compile(lambda x: _project(lin, x, _plain_weight(lin)), backend="eager", fullgraph=True)
+    with torch.no_grad():
+        for n in (5, 7, 9):
+            x = torch.randn(1, n, 100, dtype=torch.bfloat16)
+            assert torch.equal(compiled(x), lin(x))

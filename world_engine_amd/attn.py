@@ -15,6 +15,7 @@ on the same device.
 from __future__ import annotations
 
 import math
+from operator import index
 from typing import Mapping, Optional
 
 import torch
@@ -181,9 +182,11 @@ def _project(lin: nn.Module, x: Tensor, w: Optional[Tensor]) -> Tensor:
     of the host's time, most of it the BLAS routine's choice of a kernel).  fp32 sums rounded once, as there.  ``w`` is the
     layer's ``_plain_weight``."""
     if w is not None and type(x) is Tensor and not torch.is_autocast_enabled():
-        if torch.compiler.is_compiling():        # the opaque op where the kernel covers the shape, for the same bits as eager
+        # (the opaque op where the kernel covers the shape, for the same bits as eager; which sizes it covers is asked of
+        # numbers, so that a graph of symbolic sizes becomes one for these)
+        if torch.compiler.is_compiling():
             if (x.dtype in (torch.bfloat16, torch.float16) and w.dtype == x.dtype and not torch.is_grad_enabled()
-                    and _kernel_covers(x.numel() // x.shape[-1], w.shape[0], x.shape[-1], x.dtype is torch.float16)):
+                    and _kernel_covers(index(x.numel() // x.shape[-1]), index(w.shape[0]), index(x.shape[-1]), x.dtype is torch.float16)):
                 return torch.ops.world_engine_amd.linear(x, w)
         else:
             y = native.linear(x, w)
