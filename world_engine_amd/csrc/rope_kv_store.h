@@ -146,36 +146,6 @@ __device__ __forceinline__ void rotate_values(const Chunk<Tag, N>& in, const flo
     hi.e[i] = Tag::from_f32(y1);
   }
 }
-// A rotated item's halves, or the item itself, into the row `to`.
-template <typename Tag, int N>
-__device__ __forceinline__ void store_item(typename Tag::store_t* to, int Dh, int chunk, bool rotated, const Chunk<Tag, N>& in,
-                                           const Chunk<Tag, N / 2>& lo, const Chunk<Tag, N / 2>& hi) {
-  if (rotated) {
-    store_chunk(to + chunk * (N / 2), lo);
-    store_chunk(to + (Dh >> 1) + chunk * (N / 2), hi);
-  } else {
-    store_chunk(to + chunk * N, in);
-  }
-}
-
-// Destination rows of a K/V item: tail always, ring slot on an unfrozen persisting frame.
-template <typename Tag, int N>
-__device__ __forceinline__ void store_kv_rows(const StoreParams& p, int which, int b, int h, int t, int chunk,
-                                              const SlotInfo& si, bool rotated, const Chunk<Tag, N>& in,
-                                              const Chunk<Tag, N / 2>& lo, const Chunk<Tag, N / 2>& hi) {
-  typedef typename Tag::store_t st_t;
-  const int64_t cap = p.L + p.T;
-  const int plane = which - 1;
-  st_t* plane_base = (st_t*)p.kv + (((int64_t)plane * p.B + b) * p.Hkv + h) * cap * p.Dh;
-  const bool to_ring = (!p.frozen) && si.write_step;
-  const int64_t tail_row = p.L + t;
-  const int64_t ring_row = (int64_t)si.slot * p.T + t;
-  store_item(plane_base + tail_row * p.Dh, p.Dh, chunk, rotated, in, lo, hi);
-  if (to_ring) store_item(plane_base + ring_row * p.Dh, p.Dh, chunk, rotated, in, lo, hi);
-  // written[dst] = True for the rows the unfrozen write went to (kv_cache.py:149-151).
-  if (!p.frozen && which == 1 && b == 0 && h == 0 && chunk == 0) p.written[to_ring ? ring_row : tail_row] = 1;
-}
-
 // What an item needs besides its own N elements: the N / 2 cos / sin values of its pairs (rotated
 // items) and the value residual's N elements with the blend weight (V items of a layer that has
 // one).  Separate from the arithmetic so that a caller can request them long before it has the
@@ -204,6 +174,42 @@ __device__ __forceinline__ void load_item_side(const StoreParams& p, int which, 
   }
 }
 
+// An item's two halves for the output row: rotated, or as they are.
+template <typename Tag, int N>
+__device__ __forceinline__ void item_halves(const Chunk<Tag, N>& in, const ItemSide<Tag, N>& sd, Chunk<Tag, N / 2>& lo, Chunk<Tag, N / 2>& hi) {
+#pragma unroll
+  for (int i = 0; i < N / 2; ++i) {
+    lo.e[i] = in.e[i];
+    hi.e[i] = in.e[N / 2 + i];
+  }
+  if (sd.rotate) rotate_values(in, sd.c, sd.s, lo, hi);
+}
+// Into the row `to`: into its two halves, or next to each other (no branch: small launches wait for their code).
+template <typename Tag, int N>
+__device__ __forceinline__ void store_halves(typename Tag::store_t* to, int Dh, int chunk, bool rotated, const Chunk<Tag, N>& lo,
+                                             const Chunk<Tag, N>& hi) {
+  store_chunk(to + (rotated ? chunk * N : chunk * 2 * N), lo);
+  store_chunk(to + (rotated ? (Dh >> 1) + chunk * N : chunk * 2 * N + N), hi);
+}
+
+// Destination rows of a K/V item: tail always, ring slot on an unfrozen persisting frame.
+template <typename Tag, int N>
+__device__ __forceinline__ void store_kv_rows(const StoreParams& p, int which, int b, int h, int t, int chunk,
+                                              const SlotInfo& si, bool rotated, const Chunk<Tag, N>& lo,
+                                              const Chunk<Tag, N>& hi) {
+  typedef typename Tag::store_t st_t;
+  const int64_t cap = p.L + p.T;
+  const int plane = which - 1;
+  st_t* plane_base = (st_t*)p.kv + (((int64_t)plane * p.B + b) * p.Hkv + h) * cap * p.Dh;
+  const bool to_ring = (!p.frozen) && si.write_step;
+  const int64_t tail_row = p.L + t;
+  const int64_t ring_row = (int64_t)si.slot * p.T + t;
+  store_halves(plane_base + tail_row * p.Dh, p.Dh, chunk, rotated, lo, hi);
+  if (to_ring) store_halves(plane_base + ring_row * p.Dh, p.Dh, chunk, rotated, lo, hi);
+  // written[dst] = True for the rows the unfrozen write went to (kv_cache.py:149-151).
+  if (!p.frozen && which == 1 && b == 0 && h == 0 && chunk == 0) p.written[to_ring ? ring_row : tail_row] = 1;
+}
+
 // Everything after the load of a K (which = 1) or V (which = 2) item: K is normalised (optional)
 // and rotated, V is blended with the value residual (optional); the tail row is written always
 // and the ring-slot row when this is an unfrozen persisting frame; `written` is marked
@@ -214,8 +220,8 @@ __device__ __forceinline__ void finish_kv_chunk(const StoreParams& p, int which,
   if (EXTRAS && which == 1 && p.norm_eps > 0.f) rms_norm_chunk(in, (int)((unsigned)p.Dh / (unsigned)N), p.Dh, p.norm_eps);
   if (EXTRAS && which == 2 && p.v1 != nullptr) lerp_chunk(in, sd.res, sd.lamb);
   Chunk<Tag, N / 2> lo, hi;
-  if (sd.rotate) rotate_values(in, sd.c, sd.s, lo, hi);
-  store_kv_rows(p, which, b, h, t, chunk, si, sd.rotate, in, lo, hi);
+  item_halves(in, sd, lo, hi);
+  store_kv_rows(p, which, b, h, t, chunk, si, sd.rotate, lo, hi);
 }
 
 // Everything after the load of a Q item: optional norm, rotation (or plain copy when there is no
@@ -224,14 +230,9 @@ template <typename Tag, int N, bool EXTRAS = true>
 __device__ __forceinline__ void finish_q_chunk(const StoreParams& p, int b, int h, int t, int chunk,
                                                Chunk<Tag, N>& in, const ItemSide<Tag, N>& sd) {
   if (EXTRAS && p.norm_eps > 0.f) rms_norm_chunk(in, (int)((unsigned)p.Dh / (unsigned)N), p.Dh, p.norm_eps);
-  typename Tag::store_t* const to = (typename Tag::store_t*)p.q_out + (((int64_t)b * p.H + h) * p.T + t) * p.Dh;
   Chunk<Tag, N / 2> lo, hi;
-  if (sd.rotate) {
-    rotate_values(in, sd.c, sd.s, lo, hi);
-    store_item(to, p.Dh, chunk, true, in, lo, hi);
-  } else {
-    store_item(to, p.Dh, chunk, false, in, lo, hi);
-  }
+  item_halves(in, sd, lo, hi);
+  store_halves((typename Tag::store_t*)p.q_out + (((int64_t)b * p.H + h) * p.T + t) * p.Dh, p.Dh, chunk, sd.rotate, lo, hi);
 }
 
 // Whether the position ids of token i (0 .. B * T) break one of the rules asked for: the frame index
