@@ -13,7 +13,7 @@
 // HBM-bound: bytes = elements read once + written once (twice for K/V on a persisting call); small launches by their
 // trips to memory, and fp32 rows by the requests, each of which takes a quarter of every 64 bytes with 16 elements a thread (us, 16 / 8
 // elements, persisting calls in a graph: fp32, 16 heads of 128, 256 tokens 5.94 / 4.42, 8 heads, 1024 tokens 9.50 / 7.28, 8 heads
-// of 64, 64 tokens 3.02 / 2.45; bf16, 16 heads of 128, 256 tokens 3.53 / 3.39, 16 of 64, 64 tokens 2.74 / 2.53).
+// of 64, 64 tokens 3.02 / 2.45; bf16, 16 of 64, 64 tokens 2.74 / 2.53).
 #include "rope_kv_store.h"
 
 namespace we {
@@ -82,12 +82,13 @@ static void launch_store(const StoreParams& p, hipStream_t stream) {
   const auto grid = [&](int elements) {
     return dim3((unsigned)((p.T * (p.Dh / elements) + 255) / 256), (unsigned)heads, (unsigned)p.B);
   };
-  // (16 elements of half precision are what one request takes in whole.  A frame's store, attention and second pass, 16 / 8
-  // elements, by the launch's workgroups of 16: up to 720 of them 0.2 to 0.3 us less with 8, none of 60 shapes slower by more than its
-  // runs differ; from 738 on as much lost as gained and up to 2.7 us more a pass: 810 34.0 / 35.1, 1008 24.9 / 25.6, 1276 45.3 /
-  // 46.3, 1386 229 / 241, 3536 72.5 / 74.7 - twice the workgroups, which no longer find room at once.  fp32 calls 3 to 8 % less at
-  // 405 to 1170.  With a norm or a blend the same 0.3 us: 34 module passes of 24 to 1188 1.009 times as fast, 0.99 at worst with
-  // runs 1 % apart.  A rotation alone: 360 3.25 / 3.05, 456 3.35 / 3.48, 720 4.06 / 4.36; half the line also because a layer that
+  // (16 elements of half precision are what one request takes in whole; 8 are twice the workgroups, which beyond some number no
+  // longer find room at once.  A frame's store, attention and second pass, us with 16 / 8 elements, by the launch's workgroups
+  // of 16: 384 24.57 / 24.37, 480 42.07 / 41.97, 700 35.64 / 35.75, 720 25.48 / 25.71, 810 30.13 / 29.98, 1008 32.5 / 33.2 and 35.8 /
+  // 36.35, 1276 30.5 / 30.8, 1536 34.9 / 34.7, 2592 75.4 / 74.5; the store alone from 360 on as fast or faster with 16, 1008 5.68 /
+  // 6.09.  The line is from 100 drawn passes with kernels of 16 that held more registers: 0.2 to 0.3 us less with 8 up to 720
+  // workgroups, with a norm or a blend too, as much lost as gained beyond.  fp32 calls 3 to 8 % less at 405 to 1170.  A rotation
+  // alone: 128 2.86 / 2.72, 360 3.37 / 3.33, 456 3.52 / 3.68, 512 3.56 / 3.78, 720 4.18 / 4.45; half the line also because a layer that
   // rotates q and k and then stores both should find one kernel: 24 heads, 588 tokens, four layers of five passes 735 us with 16
   // elements in all three launches, 742 with 8, 763 with 8 in one kind only.)
   const dim3 whole = grid(16);
