@@ -1,6 +1,6 @@
 """fp32 attention on values split into f16 halves: against 64-bit attention at the edges of the rule that takes a
-wavefront there (key blocks per wavefront, frames off the 16-key block) and out of there again (values that halves do
-not hold, in the first, a middle or the last block of a ring, in keys, values or queries)."""
+wavefront there (key blocks per wavefront, frames off the 16-key block), and with what halves do not hold (in the first, a
+middle or the last block of a ring, in keys, values or queries): fp32 products in their place, or the wavefront's keys once more."""
 import pytest
 import torch
 
@@ -69,7 +69,7 @@ def test_f32_halves_of_two_groups_of_queries(gpu_device, B, H, Hkv, T, Dh, n):
 @pytest.mark.parametrize("Dh,n", [(128, 4), (64, 22)])
 @pytest.mark.parametrize("what,frame,factor", [("v", 2, 1e-4), ("v", None, 1e-20), ("v", 3, 1e30), ("k", 2, 1e6), ("q", None, 1e-30)])
 def test_f32_two_groups_without_halves(gpu_device, Dh, n, what, frame, factor):
-    """Both groups go on with fp32 products from the same block on, or start over."""
+    """Both groups take fp32 products of the same tiles, or start over."""
     def change(t, q, k, v):
         if frame is None or t == frame:
             {"q": q, "k": k, "v": v}[what].mul_(factor)

@@ -43,7 +43,7 @@ def test_f32_parts_of_a_ring_that_fills(gpu_device, B, H, Hkv, T, Dh, n, d):
 
 @pytest.mark.parametrize("what,frame,factor", [("v", 7, 1e-4), ("v", 20, 1e30), ("v", None, 1e-20), ("q", None, 1e-30)])
 def test_f32_parts_without_halves(gpu_device, what, frame, factor):
-    """One part goes on with fp32 products, the others with halves."""
+    """One part takes fp32 products or starts over, the others have halves."""
     B, H, Hkv, T, Dh, n, d = SHAPES[1]
     p = Pair(gpu_device, torch.float32, B=B, H=H, Hkv=Hkv, T=T, Dh=Dh, n_slots=n, d=d, cfg_id=95)
     for t in range(n + 1):
