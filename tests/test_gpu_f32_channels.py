@@ -91,3 +91,35 @@ def test_frames_of_other_sizes(gpu_device, shape, frame, factor):
     whole, channel, row = _errors(gpu_device, shape, change)
     print(f"f32 channels {shape} v x {factor:g} in {frame}: {whole:.2e}, channel {channel:.2e}, row {row:.2e}", flush=True)
     assert whole <= REL and channel <= REL_ONE and row <= REL_ONE
+
+
+@pytest.mark.parametrize("seed", range(40))
+def test_every_element_against_its_own_sum(gpu_device, seed):
+    """Channels, keys, single values and channels of queries against keys, each over orders of magnitude (or not): an element is
+    off by no more than 2^-22 of what its own sums add up, weights times |values| and, for the weights, times the logits' |q k|
+    (1.1e-7 at most over these)."""
+    import random
+    rng = random.Random(seed)
+    B, H, Hkv, T, Dh, n = SHAPES[seed % len(SHAPES)]
+    g = torch.Generator(gpu_device).manual_seed(seed)
+    spread = lambda shape, octaves: torch.exp2((torch.rand(shape, device=gpu_device, generator=g) - 0.5) * octaves)
+    q = torch.randn(B, H, T, Dh, device=gpu_device, generator=g)
+    kv = torch.randn(2, B, Hkv, (n + 1) * T, Dh, device=gpu_device, generator=g)
+    kv[1] *= spread((Dh,), rng.choice([0, 4, 30, 60])) * spread(((n + 1) * T, 1), rng.choice([0, 4, 30, 60]))
+    kv[1] *= spread(kv[1].shape, rng.choice([0, 0, 20]))
+    channels = spread((Dh,), rng.choice([0, 4, 20]))
+    q *= channels * rng.choice([1, 4, 8])
+    kv[0] /= channels
+    written = torch.ones((n + 1) * T, dtype=torch.bool, device=gpu_device)
+    out = ops.attn_ring(q, kv, written, torch.zeros(B, T, dtype=torch.long, device=gpu_device), n * T, 1).double()
+    worst = 0.0
+    for b in range(B):
+        for h in range(H):
+            k, v = (x[b, h // (H // Hkv), T:].double() for x in kv)
+            qk, size = q[b, h].double() @ k.t().contiguous(), q[b, h].double().abs() @ k.t().abs().contiguous() / math.sqrt(Dh)
+            p = torch.softmax(qk / math.sqrt(Dh), -1)
+            terms = p @ v.abs()
+            terms = terms * (1 + (p * size).sum(-1, keepdim=True)) + (p * size) @ v.abs()
+            worst = max(worst, ((out[b, h] - p @ v).abs() / terms).max().item())
+    print(f"f32 channels, elements, seed {seed}: {worst:.2e}", flush=True)
+    assert worst <= 2.0 ** -22
